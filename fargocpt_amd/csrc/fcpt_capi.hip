@@ -48,8 +48,12 @@ struct fcpt_ctx {
     // a device ring array for re-expressing a field about a new background
     std::vector<double> hbg[FCPT_NUM_FIELDS];
     double *bg_tmp = nullptr;
-    // fused FP64 adiabatic steps leave c_s, nu and T to be formed (lazy_derived)
+    // the fused step leaves derived fields to be formed (lazy_derived)
     bool derived_stale = false;
+    // the derived fields are those of the current E and Sigma (stored or
+    // stale); false once a caller has set a field or stage of its own, which
+    // the next step then reads as stored (one iteration of separate kernels)
+    bool derived_own = true;
     // split storage: steps between background moves (FCPT_PARAM_REBASE_INTERVAL;
     // 0 = only on request) and steps since the last one
     int rebase_interval = 0;
@@ -91,26 +95,27 @@ int fail(fcpt_ctx *c, int code, const char *fmt, ...)
             return fail((ctx), FCPT_ERR_DEVICE, "hipSetDevice: %s", hipGetErrorString(e_)); \
     } while (0)
 
-// When the fused Euler step of an adiabatic disk runs the kick and viscous
-// walks, the step forms c_s, nu and T where it needs them
-// (KParams::lazy_derived); in split storage the kick walk also forms the
-// pressure from E and passes E to the viscous walk through its partner buffer
-// (KParams::e_partner), so the end of the step does not store the pressure
-// (which saves a decode and an encode per cell where the split kernels are
-// bound by their arithmetic; in FP64 storage, bound by the bytes, measured
-// 0.5 % slower, so not used there).  Afterwards those fields are stale until
+// When the fused step runs the kick walk, the derived fields are formed where
+// the step needs them and left stale (KParams::lazy_derived) until
 // sync_derived stores them (the same expressions on the stored E and Sigma).
-static bool lazy_applies(const fcpt_ctx *ctx)
+static bool lazy_applies(const fcpt_ctx *ctx) { return ctx->fused && kv_walk_applies(ctx->P); }
+// whether the next iteration runs fused, and the parameters it runs with
+// (the fused step of an isothermal disk forms its pressure from Sigma anyway)
+static bool next_fused(const fcpt_ctx *ctx)
 {
-    const KParams &P = ctx->P;
-    return ctx->fused && P.adiabatic && P.integrator == FCPT_INTEGRATOR_EULER && kick_walk_applies(P);
+    return ctx->fused && (ctx->derived_own || !ctx->P.adiabatic || !lazy_applies(ctx));
 }
-static KParams step_view(const fcpt_ctx *ctx)
+static KParams step_view(const fcpt_ctx *ctx, bool fused)
 {
     KParams P = ctx->P;
-    P.e_partner = lazy_applies(ctx) && P.split ? 1 : 0;
-    P.lazy_derived = lazy_applies(ctx) ? 1 : 0;
+    set_step_modes(P, fused);
     return P;
+}
+// after a whole iteration that ran with `fused`
+static void stepped(fcpt_ctx *ctx, bool fused)
+{
+    ctx->derived_stale = fused && lazy_applies(ctx);
+    ctx->derived_own = true;
 }
 static int sync_derived(fcpt_ctx *ctx)
 {
@@ -118,6 +123,12 @@ static int sync_derived(fcpt_ctx *ctx)
     launch_derived(ctx->P, ctx->stream);
     ctx->derived_stale = false;
     return FCPT_OK;
+}
+// the fields sync_derived stores (an isothermal disk: the pressure alone)
+static bool derived_field(int f)
+{
+    return f == FCPT_PRESSURE || f == FCPT_SOUNDSPEED || f == FCPT_SCALE_HEIGHT || f == FCPT_VISCOSITY ||
+           f == FCPT_TEMPERATURE;
 }
 // entry points that read or expose the fields: the context, with the derived
 // fields stored
@@ -307,8 +318,9 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
     P.radial_waves = 3;
     P.visc_tile = 0;
     P.kick_tile = 0;
+    P.kv_tile = 0;
     P.lazy_derived = 0;
-    P.e_partner = 0;
+    P.split_emul = 0;
     P.ealt = nullptr;
     init_launch_fields(P);
     // Interpret.cpp:230-231
@@ -354,6 +366,11 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
     P.damping_time_factor = desc->damping_time_factor;
     P.damping_time_radius_outer = desc->damping_time_radius_outer;
     P.omega_frame = desc->omega_frame;
+    P.energy_per_t = P.Rgas / P.mu / (P.gamma - 1.0);
+    P.const_ok = 1;
+    for (double c : {P.Rgas, P.mu, P.gamma, P.gamma - 1.0, P.alpha, P.sigma_sb, P.c_light, P.G * P.mstar, P.radial_viscosity_factor, P.heating_viscous_factor})
+        if (!(c >= 0x1p-40 && c <= 0x1p40)) P.const_ok = 0;
+    if (!(desc->radii[0] >= 0x1p-20 && desc->radii[nr + 1] <= 0x1p20)) P.const_ok = 0;
     P.monitor_timestep = desc->monitor_timestep;
     int ids[4] = {desc->damp_inner_scalar, desc->damp_inner_vector, desc->damp_outer_scalar,
                   desc->damp_outer_vector};
@@ -425,7 +442,7 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
         rc = dev_alloc_bytes(c, &P.f[k], field_rows(k, nr) * ns * field_element_size(P, k));
     if (!rc) rc = dev_alloc_bytes(c, &P.valt[0], field_rows(FCPT_VRAD, nr) * ns * esz);
     if (!rc) rc = dev_alloc_bytes(c, &P.valt[1], field_rows(FCPT_VAZI, nr) * ns * esz);
-    if (!rc && P.adiabatic && P.split) rc = dev_alloc_bytes(c, &P.ealt, field_rows(FCPT_ENERGY, nr) * ns * esz);
+    if (!rc && P.adiabatic) rc = dev_alloc_bytes(c, &P.ealt, field_rows(FCPT_ENERGY, nr) * ns * esz);
     for (int k = 0; k < 4 && !rc; ++k) rc = dev_alloc_bytes(c, &P.mom[k], ncell * sizeof(double));  // FP64 in both modes
     for (int k = 0; k < 4 && !rc; ++k) rc = dev_alloc_bytes(c, &P.mom_b[k], ncell * esz);
     // the density and energy between the transport sweeps stay FP64 in both
@@ -587,6 +604,7 @@ int fcpt_upload_field(fcpt_ctx *ctx, int32_t field, const double *host)
 {
     CTX_SYNCED(ctx);
     if (field < 0 || field >= FCPT_NUM_FIELDS || !host) return fail(ctx, FCPT_ERR_ARG, "bad field");
+    if (field == FCPT_SIGMA || field == FCPT_ENERGY || derived_field(field)) ctx->derived_own = false;
     if (ctx->P.split && field != FCPT_POTENTIAL) return upload_split(ctx, field, host);
     const size_t n = field_rows(field, ctx->P.nr) * ctx->P.ns;
     HIP_TRY(ctx, hipMemcpyAsync(ctx->P.f[field], host, n * sizeof(double), hipMemcpyHostToDevice,
@@ -597,8 +615,9 @@ int fcpt_upload_field(fcpt_ctx *ctx, int32_t field, const double *host)
 
 int fcpt_download_field(fcpt_ctx *ctx, int32_t field, double *host)
 {
-    CTX_SYNCED(ctx);
+    CTX_CHECK(ctx);
     if (field < 0 || field >= FCPT_NUM_FIELDS || !host) return fail(ctx, FCPT_ERR_ARG, "bad field");
+    if (derived_field(field)) sync_derived(ctx);
     if (ctx->P.split && field != FCPT_POTENTIAL) return download_split(ctx, field, host);
     const size_t n = field_rows(field, ctx->P.nr) * ctx->P.ns;
     HIP_TRY(ctx, hipMemcpyAsync(host, ctx->P.f[field], n * sizeof(double), hipMemcpyDeviceToHost,
@@ -828,6 +847,7 @@ int fcpt_init_profiles(fcpt_ctx *ctx, const fcpt_ic_desc *ic)
     if (rc) return rc;
     if (le != hipSuccess) return fail(ctx, FCPT_ERR_DEVICE, "launch: %s", hipGetErrorString(le));
     if (se != hipSuccess) return fail(ctx, FCPT_ERR_DEVICE, "sync: %s", hipGetErrorString(se));
+    ctx->derived_own = true;
     return FCPT_OK;
 }
 
@@ -865,6 +885,7 @@ int fcpt_upload_state(fcpt_ctx *ctx, const double *sigma, const double *vrad, co
         launch_heatcool_cfl(P, ctx->stream);
     }
     LAUNCH_CHECK(ctx);
+    ctx->derived_own = true;
     if ((rc = clear_error_flags(ctx))) return rc;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     return FCPT_OK;
@@ -966,10 +987,10 @@ int fcpt_nbody_potential(fcpt_ctx *ctx)
         return FCPT_OK;                              \
     }
 
-DT_ENTRY(fcpt_update_with_sourceterms, launch_sources(ctx->P, ctx->stream))
-DT_ENTRY(fcpt_artificial_viscosity, launch_artificial_viscosity(ctx->P, ctx->stream, 0))
+DT_ENTRY(fcpt_update_with_sourceterms, launch_sources(ctx->P, ctx->stream); ctx->derived_own = false)
+DT_ENTRY(fcpt_artificial_viscosity, launch_artificial_viscosity(ctx->P, ctx->stream, 0); ctx->derived_own = false)
 DT_ENTRY(fcpt_update_velocities_with_viscosity, launch_visc_update(ctx->P, ctx->stream))
-DT_ENTRY(fcpt_transport, launch_transport(ctx->P, ctx->stream))
+DT_ENTRY(fcpt_transport, launch_transport(ctx->P, ctx->stream); ctx->derived_own = false)
 
 int fcpt_recalculate_viscosity(fcpt_ctx *ctx)
 {
@@ -994,6 +1015,7 @@ int fcpt_substep3(fcpt_ctx *ctx, double time, double dt)
     launch_set_clock(ctx->P, ctx->stream, time);
     launch_set_dt(ctx->P, ctx->stream, dt);
     launch_substep3(ctx->P, ctx->stream);
+    ctx->derived_own = false;
     LAUNCH_CHECK(ctx);
     return FCPT_OK;
 }
@@ -1003,6 +1025,9 @@ int fcpt_apply_boundary_condition(fcpt_ctx *ctx, double dt, int32_t final_call)
     CTX_SYNCED(ctx);
     launch_set_dt(ctx->P, ctx->stream, dt);
     launch_boundaries(ctx->P, ctx->stream, final_call, 0);
+    // the damping changes E and Sigma of rings whose derived fields the step
+    // reads; those of the ghost rings it does not
+    if (final_call && ctx->P.damping) ctx->derived_own = false;
     LAUNCH_CHECK(ctx);
     return FCPT_OK;
 }
@@ -1011,6 +1036,7 @@ int fcpt_recalculate_derived(fcpt_ctx *ctx)
 {
     CTX_SYNCED(ctx);
     launch_derived(ctx->P, ctx->stream);
+    ctx->derived_own = true;
     LAUNCH_CHECK(ctx);
     return FCPT_OK;
 }
@@ -1037,14 +1063,10 @@ int fcpt_get_nshift(fcpt_ctx *ctx, int32_t *nshift)
 static const KParams *enqueue_kick(const KParams &P, const KParams &Q, hipStream_t st, bool fused,
                                    bool pressure_first, int fold_mode = -1)
 {
-    if (fused && kick_walk_applies(P)) {
-        // the potential pass and two walks: sources and artificial
-        // viscosity; then the viscous stress and update (and SubStep3)
-        if (pressure_first && P.adiabatic) launch_pressure(P, st);
+    if (P.lazy_derived) {
+        // the potential pass and one walk, which forms the pressure itself
         launch_kick(P, st, fold_mode);
-        if (P.adiabatic) launch_visc_energy(Q, st);
-        else launch_visc_fused(Q, st);
-        return &P;
+        return &Q;
     }
     if (fused) launch_potential_fold(P, st, fold_mode);
     else launch_potential(P, st);
@@ -1131,16 +1153,15 @@ static void enqueue_step(const KParams &P, hipStream_t st, int count_monitor, bo
 // one sim::run iteration: CalculateTimeStep with the monitor clip (mode 2),
 // then the step; the fused Euler step folds the CFL minima inside its
 // potential launch (one launch less)
-static void enqueue_iteration(const fcpt_ctx *ctx)
+static void enqueue_iteration(const fcpt_ctx *ctx, bool fused)
 {
-    const KParams &P = ctx->P;
-    if (ctx->fused && P.integrator != FCPT_INTEGRATOR_LEAPFROG) {
-        const KParams V = step_view(ctx);
+    const KParams V = step_view(ctx, fused);
+    if (fused && V.integrator != FCPT_INTEGRATOR_LEAPFROG) {
         launch_cfl_cells(V, ctx->stream);
         enqueue_euler(V, ctx->stream, 1, true, 2);
     } else {
-        launch_cfl(P, ctx->stream, 2);
-        enqueue_step(P, ctx->stream, 1, ctx->fused);
+        launch_cfl(V, ctx->stream, 2);
+        enqueue_step(V, ctx->stream, 1, fused);
     }
 }
 
@@ -1148,9 +1169,10 @@ int fcpt_step_euler(fcpt_ctx *ctx, double dt)
 {
     CTX_SYNCED(ctx);
     launch_set_dt(ctx->P, ctx->stream, dt);
-    enqueue_euler(step_view(ctx), ctx->stream, 0, ctx->fused, -1);
+    const bool fused = next_fused(ctx);
+    enqueue_euler(step_view(ctx, fused), ctx->stream, 0, fused, -1);
     LAUNCH_CHECK(ctx);
-    ctx->derived_stale = lazy_applies(ctx);
+    stepped(ctx, fused);
     return FCPT_OK;
 }
 
@@ -1158,8 +1180,13 @@ int fcpt_step_leapfrog(fcpt_ctx *ctx, double dt)
 {
     CTX_SYNCED(ctx);
     launch_set_dt(ctx->P, ctx->stream, dt);
-    enqueue_leapfrog(ctx->P, ctx->stream, 0, ctx->fused);
+    const bool fused = next_fused(ctx);
+    KParams V = ctx->P;
+    V.integrator = FCPT_INTEGRATOR_LEAPFROG;  // the scheme, whatever the descriptor's own
+    set_step_modes(V, fused);
+    enqueue_leapfrog(V, ctx->stream, 0, fused);
     LAUNCH_CHECK(ctx);
+    stepped(ctx, fused);
     return FCPT_OK;
 }
 
@@ -1184,9 +1211,11 @@ int fcpt_set_midstep_params(fcpt_ctx *ctx, const fcpt_step_params *params)
 int fcpt_run_step(fcpt_ctx *ctx, double *dt_out)
 {
     CTX_CHECK(ctx);
-    enqueue_iteration(ctx);
+    const bool fused = next_fused(ctx);
+    if (!fused) sync_derived(ctx);
+    enqueue_iteration(ctx, fused);
     LAUNCH_CHECK(ctx);
-    if (lazy_applies(ctx)) ctx->derived_stale = true;
+    stepped(ctx, fused);
     int rc = read_scalars(ctx);
     if (rc) return rc;
     if (take_nonfinite(ctx))
@@ -1201,7 +1230,7 @@ static int ensure_step_graph(fcpt_ctx *ctx)
     if (ctx->step_graph) return FCPT_OK;
     hipGraph_t g = nullptr;
     HIP_TRY(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_iteration(ctx);
+    enqueue_iteration(ctx, ctx->fused);
     hipError_t e = hipStreamEndCapture(ctx->stream, &g);
     if (e != hipSuccess) return fail(ctx, FCPT_ERR_DEVICE, "graph capture: %s", hipGetErrorString(e));
     e = hipGraphInstantiate(&ctx->step_graph, g, nullptr, nullptr, 0);
@@ -1227,14 +1256,19 @@ int fcpt_run_steps(fcpt_ctx *ctx, int32_t n_steps, int32_t use_graph)
     for (int left = n_steps; left > 0;) {
         int m = left;
         if (periodic_rebase(ctx)) m = std::min(m, ctx->rebase_interval - ctx->steps_since_rebase);
-        if (use_graph) {
+        const bool fused = next_fused(ctx);
+        if (fused != ctx->fused) {  // fields of the caller's own: one step of separate kernels
+            m = 1;
+            sync_derived(ctx);
+        }
+        if (use_graph && fused == ctx->fused) {
             for (int k = 0; k < m; ++k) HIP_TRY(ctx, hipGraphLaunch(ctx->step_graph, ctx->stream));
         } else {
-            for (int k = 0; k < m; ++k) enqueue_iteration(ctx);
+            for (int k = 0; k < m; ++k) enqueue_iteration(ctx, fused);
             LAUNCH_CHECK(ctx);
         }
         left -= m;
-        if (lazy_applies(ctx)) ctx->derived_stale = true;
+        stepped(ctx, fused);
         if (periodic_rebase(ctx) && (ctx->steps_since_rebase += m) >= ctx->rebase_interval) {
             const int rc = rebase_backgrounds(ctx);
             if (rc) return rc;
@@ -1371,11 +1405,11 @@ int fcpt_set_launch_param(fcpt_ctx *ctx, int32_t param, int32_t value)
     return FCPT_OK;
 }
 
-// The walks' tiles by whole-step time: each candidate runs `reps` graph-replayed
+// The kick walk's tile (the viscous walk's in a disk without artificial
+// viscosity) by whole-step time: each candidate runs `reps` graph-replayed
 // sim::run iterations from the same state, which is saved first (every field
 // and the device scalars) and put back after each trial and at the end, so
-// the context's state and clock come out as they went in.  Tiles 2 .. 16
-// for each walk that applies, the kick walk's first, then the viscous walk's.
+// the context's state and clock come out as they went in.  Tiles 2 .. 32.
 int fcpt_autotune_walks(fcpt_ctx *ctx, int32_t reps, int32_t *kick_tile, int32_t *visc_tile)
 {
     CTX_SYNCED(ctx);
@@ -1385,7 +1419,9 @@ int fcpt_autotune_walks(fcpt_ctx *ctx, int32_t reps, int32_t *kick_tile, int32_t
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     KParams &P = ctx->P;
     const int kick0 = resolve_kick_tile(P), visc0 = resolve_visc_tile(P);
-    if (!ctx->fused || P.integrator != FCPT_INTEGRATOR_EULER || visc0 <= 1) {
+    const bool kv = walks_tunable(P);
+    if (!ctx->fused || P.integrator != FCPT_INTEGRATOR_EULER ||
+        !(kv || (P.artvisc == FCPT_ARTVISC_NONE && visc0 > 1))) {
         if (kick_tile) *kick_tile = kick0;
         if (visc_tile) *visc_tile = visc0;
         return FCPT_OK;  // the walks do not run in this context's step
@@ -1441,47 +1477,31 @@ int fcpt_autotune_walks(fcpt_ctx *ctx, int32_t reps, int32_t *kick_tile, int32_t
         if (!r && er != hipSuccess) r = fail(ctx, FCPT_ERR_DEVICE, "state restore: %s", hipGetErrorString(er));
         return r;
     };
-    const int cand[] = {2, 4, 8, 16};
-    int best_k = kick0, best_v = visc0;
+    const int cand[] = {2, 4, 8, 16, 32};
+    int best_t = visc0;
     rc = e == hipSuccess ? FCPT_OK : fail(ctx, FCPT_ERR_DEVICE, "state save: %s", hipGetErrorString(e));
-    if (!rc && kick_walk_applies(P)) {
-        double best = 1e300;
-        for (int t : cand) {
-            if (t > P.nr) continue;
-            P.kick_tile = t;
-            if (!kick_walk_applies(P)) continue;
-            double ms = 0.0;
-            if ((rc = trial(ms))) break;
-            if (ms < best) {
-                best = ms;
-                best_k = t;
-            }
+    double best = 1e300;
+    for (int t : cand) {
+        if (rc || t > P.nr) continue;
+        if (kv) P.kick_tile = t;
+        P.visc_tile = t;
+        double ms = 0.0;
+        if ((rc = trial(ms))) break;
+        if (ms < best) {
+            best = ms;
+            best_t = t;
         }
-        P.kick_tile = best_k;
     }
-    if (!rc) {
-        double best = 1e300;
-        for (int t : cand) {
-            if (t > P.nr) continue;
-            P.visc_tile = t;
-            if (P.kick_tile > 1 && !kick_walk_applies(P)) continue;
-            double ms = 0.0;
-            if ((rc = trial(ms))) break;
-            if (ms < best) {
-                best = ms;
-                best_v = t;
-            }
-        }
-        P.visc_tile = best_v;
-    }
+    if (kv) P.kick_tile = best_t;
+    P.visc_tile = best_t;
     hipFree(save);
     if (ctx->step_graph) {
         hipGraphExecDestroy(ctx->step_graph);
         ctx->step_graph = nullptr;
     }
     if (rc) return rc;
-    if (kick_tile) *kick_tile = best_k;
-    if (visc_tile) *visc_tile = best_v;
+    if (kick_tile) *kick_tile = resolve_kick_tile(P);
+    if (visc_tile) *visc_tile = resolve_visc_tile(P);
     return FCPT_OK;
 }
 
@@ -1548,7 +1568,7 @@ int fcpt_autotune(fcpt_ctx *ctx, int32_t reps, int32_t *radial_tile, int32_t *ra
 int fcpt_disk_on_planet_accel(fcpt_ctx *ctx, const fcpt_force_body *bodies, int32_t n_bodies,
                               int32_t flags, double *accel_xy)
 {
-    CTX_SYNCED(ctx);
+    CTX_CHECK(ctx);  // reads Sigma and H, which every step stores
     if (n_bodies < 0 || n_bodies > kForceMaxBodies || (n_bodies > 0 && (!bodies || !accel_xy)))
         return fail(ctx, FCPT_ERR_ARG, "1 .. %d bodies", kForceMaxBodies);
     if (flags & ~(FCPT_FORCE_NO_STAR_SMOOTHING | FCPT_FORCE_SMOOTHING_PLANETLOC |
@@ -1964,40 +1984,18 @@ int fcpt_batch_create(fcpt_ctx *const *disks, int32_t n_disks, fcpt_batch **out)
             }
         }
         KParams P = c->P;
-        // the radial tile is chosen below, over the whole batch; in split
-        // storage the walks' tiles as the disk's own launches choose them
-        // (whether the walks run decides where split storage rounds)
-        if (P.split) {
-            P.kick_tile = resolve_kick_tile(P);
-            P.visc_tile = resolve_visc_tile(P);
-        }
+        // the batch runs the fused step (its rounding points in split storage
+        // are the disk's own, whatever tile the batch chooses below)
+        set_step_modes(P, true);
+        b->lazy.push_back(P.lazy_derived != 0);
         host.push_back(P);
     }
-    // FP64 storage: the walks' tiles of the members that leave them to the
-    // size rule, chosen over the batch's wavefronts as the radial tile below
-    // (a member too small to fill the device alone still runs the walks;
-    // FP64 results do not depend on the tiles or on whether the walks run)
-    if (!b->split) {
-        auto waves = [&](int t) {
-            long w = 0;
-            for (const KParams &P : host) w += walk_waves(P, P.visc_tile > 0 ? P.visc_tile : t);
-            return w;
-        };
-        int t = 8;
-        while (t > 2 && waves(t) < 3072) t /= 2;
-        for (KParams &P : host) {
-            if (P.kick_tile <= 0) P.kick_tile = t;
-            if (P.visc_tile <= 0) P.visc_tile = t;
-        }
-    }
-    for (KParams &P : host) {
-        // the batch runs the fused step: c_s, nu and T formed where needed
-        // as in the disk's own fused step
-        const bool walks = P.adiabatic && kick_walk_applies(P);
-        P.e_partner = walks && P.split ? 1 : 0;
-        P.lazy_derived = walks ? 1 : 0;
-        b->lazy.push_back(walks);
-    }
+    // The walks' tiles of the members that leave them to the size rule,
+    // chosen over the batch's wavefronts as the radial tile below (results
+    // do not depend on the tiles).
+    resolve_kv_tiles(host);
+    for (KParams &P : host)
+        if (!kv_walk_applies(P)) P.visc_tile = resolve_visc_tile(P);
     // The radial sweep's tile of the members that leave it to the size rule.
     // A single disk's rule shrinks the tile until that disk alone fills the
     // device with wavefronts; in a batch all members' blocks share one
@@ -2089,6 +2087,14 @@ int fcpt_batch_run_steps(fcpt_batch *b, int32_t n_steps, int32_t use_graph)
             b->graph = nullptr;
             return bfail(b, FCPT_ERR_DEVICE, hipGetErrorString(e));
         }
+    }
+    if (n_steps > 0 && std::any_of(b->disks.begin(), b->disks.end(), [](fcpt_ctx *c) { return !c->derived_own; })) {
+        // a member with fields of its caller's own: one iteration disk by disk
+        for (fcpt_ctx *c : b->disks) {
+            if (fcpt_run_steps(c, 1, 0)) return bfail(b, FCPT_ERR_DEVICE, c->err.c_str());
+            BHIP(b, hipStreamSynchronize(c->stream));
+        }
+        --n_steps;
     }
     for (int left = n_steps; left > 0;) {
         // up to the next background move of a member in split storage

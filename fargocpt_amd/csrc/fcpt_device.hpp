@@ -16,8 +16,19 @@ namespace fcpt {
 
 constexpr int kMaxPlanets = FCPT_MAX_PLANETS;
 constexpr unsigned kCflMaxBlocks = 4096;  // slots of the block-minimum array
-// rows of KParams::ring_tab
-enum { TAB_SRC_INVDXTHETA = 0, TAB_INV_DXTHETA, TAB_INV_OMEGA_K, TAB_OMEGA_K, TAB_VISC_AREA, kRingTabs };
+// a ring's values in KParams::ring_tab: the metric the walks read, and the
+// ring-uniform products and quotients of their formulas
+enum {
+    TAB_RINF = 0, TAB_INV_RINF, TAB_RMED, TAB_INV_RMED, TAB_INV_DIFF_RMED, TAB_INV_DIFF_RSUP, TAB_INV_DIFF_RSUP_RB,
+    TAB_SRC_INVDXTHETA, TAB_INV_DXTHETA, TAB_INV_OMEGA_K, TAB_OMEGA_K, TAB_VISC_AREA, TAB_RINF_SQ, TAB_RINF_OMEGA,
+    TAB_TW_LSQ, TAB_RMED_SUM, TAB_RMED_SUM_RCP, TAB_RSUP_RINF, TAB_RMED_SQ_DIFF, TAB_RMED_SQ_DIFF_RCP,
+    TAB_RMED_DIFF, TAB_E_LO, TAB_E_HI, TAB_SQRT_GAMMA, TAB_SQRT_GAMMA_RCP, TAB_C_LIGHT, TAB_C_LIGHT_RCP,
+    TAB_G_GM1, TAB_MU_GM1, TAB_SIGMA_FLOOR10, TAB_BETA_INV, TAB_ARTVISC_SQ, kRingTabs
+};
+
+// KParams::split_emul: c_s, H, nu and the pressure; the source-term velocities
+// and the viscous heating's stress tensor
+enum { SPLIT_EMUL_DERIVED = 1, SPLIT_EMUL_STAGES = 2 };
 
 struct DevPlanet {
     double x, y, mass, r_cubic;
@@ -87,16 +98,16 @@ struct KParams {
     int radial_waves;    // register budget of the radial sweep: wavefronts per SIMD (2 or 3)
     int visc_tile;       // rings per thread of the fused viscous pass (0: size-based choice)
     int kick_tile;       // rings per thread of the kick walk (0: size-based choice, 1: off)
-    // the fused Euler step of an adiabatic disk (either storage): the sound
-    // speed, viscosity and temperature are formed from E and Sigma where the
-    // step needs them instead of stored (the kick walk stores nu only); the
-    // host stores them all (k_derived) before anything else reads the fields
+    int kv_tile;         // batches: the kick walk's rings per thread, chosen over the batch
+    // the fused step with the kick walk: the derived fields (the sound speed,
+    // viscosity, temperature and pressure; the pressure of an isothermal
+    // disk) are formed from E and Sigma where the step needs them instead of
+    // stored, and the walk writes the updated E to its partner ealt; the host
+    // stores the fields (k_derived) before anything else reads them
     int lazy_derived;
-    // the fused step's walks of an adiabatic disk (split storage): the kick walk
-    // forms the pressure from E and writes the updated E to the partner buffer
-    // ealt, which the viscous walk reads (its SubStep3 writes E back); the end
-    // of the step does not store the pressure
-    int e_partner;
+    // split storage: values the kick walk and the CFL round as if stored
+    // (SPLIT_EMUL_*), in disks whose step keeps fewer values in FP64
+    int split_emul;
     int cfl_gx, cfl_gy;  // grid of the CFL cell kernel (its block-minimum slots)
     // fields in HBM (indexed by fcpt_field): double, or float when split
     void *f[FCPT_NUM_FIELDS];
@@ -112,13 +123,14 @@ struct KParams {
     void *sig_b, *en_b;  // radial-sweep outputs
     void *sig_c, *en_c;  // azimuthal-sweep outputs
     void *valt[2];       // partners of v_r and v_phi for the fused step kernels
-    void *ealt;          // partner of E (adiabatic disks in split storage; e_partner)
+    void *ealt;          // partner of E (adiabatic disks)
     double *bgm[4];      // backgrounds of the four momenta (split storage)
     double *iso_cs, *iso_h, *iso_nu;  // locally isothermal ring profiles of c_s, H, nu
-    // ring-uniform quotients of the source terms, the artificial viscosity,
-    // the viscous update and the derived fields (k_ring_tables), kRingTabs
-    // rows of nr + 2 values
+    // kRingTabs values per ring, nr + 2 rings (k_ring_tables): one base pointer
+    // and one run of memory per ring for the walks' scalar loads
     double *ring_tab;
+    double energy_per_t;  // R / mu / (gamma - 1): energy_at's factor, to rounding
+    int const_ok;         // the physical constants lie in the range quot_in assumes
     double *vmean;       // per-ring mean azimuthal velocity
     double *vuni;        // per-ring uniform residual velocity (FARGO)
     int *nshift;         // per-ring integer shift

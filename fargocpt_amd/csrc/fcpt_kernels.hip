@@ -11,6 +11,8 @@
 // per-ring background (value = bg[ring] + (double)deviation), which halves the
 // HBM traffic; the arithmetic is FP64 in both instantiations and the FP64
 // instantiation performs exactly the operations of the reference.
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <vector>
 
@@ -84,6 +86,36 @@ __device__ __forceinline__ double shared_div(double n, const SharedDen &D)
     return q;
 }
 
+// A denominator with its refined reciprocal, shared by several quotients: in
+// FP64 storage shared_den's, so that in range (ok) the quotient is the IEEE one
+// at three instructions; in split storage recip<true>'s, a product.  ok says
+// that the denominator lies in [2^-100, 2^100) and the numerators the caller
+// forms are within [2^-400, 2^250) or zero (quot_range); others divide.
+__device__ __forceinline__ bool quot_range(double x)
+{
+    const unsigned e = (unsigned)((unsigned long long)__double_as_longlong(x) >> 52) & 0x7ffu;
+    return e - 923u < 200u;
+}
+struct Den {
+    double d, r;
+    bool ok;
+};
+template <bool SPLIT>
+__device__ __forceinline__ double quot_by(double n, const Den &D)
+{
+    if constexpr (SPLIT) {
+        return n * D.r;
+    } else {
+        const double q0 = n * D.r;
+        double q = fma(fma(-D.d, q0, n), D.r, q0);
+        if (!D.ok) {
+            __builtin_amdgcn_s_sleep(0);  // a branch: the division is not formed and selected
+            q = n / D.d;
+        }
+        return q;
+    }
+}
+
 // IEEE FP64 square root.  The compiler's sqrt on gfx950 scales x by 2^256
 // below 2^-767, refines v_rsq by one Goldschmidt step and two Newton
 // corrections, scales back, and passes zeros and +inf through a class test.
@@ -151,6 +183,11 @@ __device__ __forceinline__ double omega_kepler(const KParams &P, double r)
 }
 
 
+// dt and time of the running kick (no kernel that reads them writes them, so they
+// are scalar loads that stores do not repeat)
+__device__ __forceinline__ double kick_dt(const KParams &P) { return *(const __attribute__((address_space(4))) double *)&P.s->dt; }
+__device__ __forceinline__ double kick_time(const KParams &P) { return *(const __attribute__((address_space(4))) double *)&P.s->time; }
+
 // Per-ring arrays (metric, backgrounds, ring means, shifts) are never written
 // by the kernel that reads them.  Reading them through the constant address
 // space says so: with a wave-uniform index they become scalar loads, which
@@ -191,7 +228,7 @@ __device__ __forceinline__ unsigned sr_bits(unsigned x)
     x ^= x >> 15;
     return x;
 }
-__device__ __forceinline__ float round_dev(double d, unsigned key, size_t c)
+__device__ __forceinline__ float round_dev(double d, unsigned key, unsigned c)
 {
     if (!key) return (float)d;
     // add a 29-bit variate below the FP32 unit of the FP64 deviation and drop
@@ -200,7 +237,7 @@ __device__ __forceinline__ float round_dev(double d, unsigned key, size_t c)
     // reached); smaller deviations are rounded once more by the conversion,
     // infinities stay infinite.
     const unsigned long long b0 = (unsigned long long)__double_as_longlong(d);
-    const unsigned u = sr_bits((unsigned)c ^ key ^ (unsigned)(b0 >> 32)) >> 3;
+    const unsigned u = sr_bits(c ^ key ^ (unsigned)(b0 >> 32)) >> 3;
     const unsigned long long b = b0 + (unsigned long long)u;
     return (float)__longlong_as_double((long long)(b & ~0x1fffffffull));
 }
@@ -209,7 +246,10 @@ __device__ __forceinline__ unsigned sr_key(int id, unsigned step)
     return sr_hash(step * 0x85ebca77u + (unsigned)id * 0xc2b2ae3du) | 1u;
 }
 
-// field accessor: an FP64 array, or FP32 deviations from an FP64 ring background
+// field accessor: an FP64 array, or FP32 deviations from an FP64 ring background.
+// An element's address is its row's (scalar where the ring is) plus a 32-bit
+// byte offset along the ring, which the load and store instructions add
+// themselves: no 64-bit address per lane (a row is at most 2 MiB).
 template <bool SPLIT>
 struct Fld {
     using T = typename std::conditional<SPLIT, float, double>::type;
@@ -217,41 +257,44 @@ struct Fld {
     const double *bg;
     int ns;
     unsigned key;  // split storage: 0 rounds to nearest, else the stochastic rounding's key
+    __device__ __forceinline__ T &at(int i, int j) const
+    {
+        char *row = reinterpret_cast<char *>(p) + (size_t)i * (size_t)ns * sizeof(T);
+        return *reinterpret_cast<T *>(row + (unsigned)j * (unsigned)sizeof(T));
+    }
+    // the rounding's cell number (its low 32 bits)
+    __device__ __forceinline__ unsigned cell(int i, int j) const { return (unsigned)i * (unsigned)ns + (unsigned)j; }
     __device__ __forceinline__ double operator()(int i, int j) const
     {
-        const size_t c = (size_t)i * (size_t)ns + (size_t)j;
-        if constexpr (SPLIT) return cst(bg)[i] + (double)p[c];
-        else return p[c];
+        if constexpr (SPLIT) return cst(bg)[i] + (double)at(i, j);
+        else return at(i, j);
     }
     __device__ __forceinline__ void set(int i, int j, double v) const
     {
-        const size_t c = (size_t)i * (size_t)ns + (size_t)j;
-        if constexpr (SPLIT) p[c] = round_dev(v - cst(bg)[i], key, c);
-        else p[c] = v;
+        if constexpr (SPLIT) at(i, j) = round_dev(v - cst(bg)[i], key, cell(i, j));
+        else at(i, j) = v;
     }
     // the stored value alone, and its decoding: lets a kernel issue a load
     // early and pay for it where the value is used
-    __device__ __forceinline__ T raw(int i, int j) const { return p[(size_t)i * (size_t)ns + (size_t)j]; }
-    __device__ __forceinline__ void set_raw(int i, int j, T x) const { p[(size_t)i * (size_t)ns + (size_t)j] = x; }
+    __device__ __forceinline__ T raw(int i, int j) const { return at(i, j); }
+    __device__ __forceinline__ void set_raw(int i, int j, T x) const { at(i, j) = x; }
     // store v at (i, j) and return it as a later load of it returns it
     __device__ __forceinline__ double set_get(int i, int j, double v) const
     {
-        const size_t c = (size_t)i * (size_t)ns + (size_t)j;
         if constexpr (SPLIT) {
             const double b = cst(bg)[i];
-            const float x = round_dev(v - b, key, c);
-            p[c] = x;
+            const float x = round_dev(v - b, key, cell(i, j));
+            at(i, j) = x;
             return b + (double)x;
         } else {
-            p[c] = v;
+            at(i, j) = v;
             return v;
         }
     }
     // v as a later load of the value stored at (i, j) returns it
     __device__ __forceinline__ double stored(int i, int j, double v) const
     {
-        const size_t c = (size_t)i * (size_t)ns + (size_t)j;
-        if constexpr (SPLIT) return cst(bg)[i] + (double)round_dev(v - cst(bg)[i], key, c);
+        if constexpr (SPLIT) return cst(bg)[i] + (double)round_dev(v - cst(bg)[i], key, cell(i, j));
         else return v;
     }
     __device__ __forceinline__ double dec(int i, T x) const
@@ -261,11 +304,22 @@ struct Fld {
     }
 };
 
-// a ring-uniform quotient of ring i (row t of KParams::ring_tab, formed once
-// by k_ring_tables with the expression its users had inline: the same bits)
+// value t of ring i in KParams::ring_tab (formed once by k_ring_tables with
+// the expressions of its users: the same bits)
 __device__ __forceinline__ double ring_tab(const KParams &P, int t, int i)
 {
-    return cst(P.ring_tab)[(size_t)t * (size_t)(P.nr + 2) + (size_t)i];
+    return cst(P.ring_tab)[i * kRingTabs + t];
+}
+// the same for a ring walk, whose wavefront holds the rows of its rings in LDS
+// from row0 on: a scalar load per value and ring misses the scalar cache once
+// per ring and stalls the walk at every use
+struct KWalk : KParams {
+    const double *rows;
+    int row0;
+};
+__device__ __forceinline__ double ring_tab(const KWalk &P, int t, int i)
+{
+    return P.rows[(i - P.row0) * kRingTabs + t];
 }
 
 // the rounding key of split-storage stores of field (or buffer) `id` in the
@@ -603,6 +657,16 @@ __device__ __forceinline__ void b_cfl_finalize(const KParams &P, int mode) { b_c
 
 // adiabatic sound speed, scale height and viscosity of one cell
 // (compute_sound_speed, compute_scale_height, compute_viscosity)
+template <bool SPLIT>
+__device__ __forceinline__ Den make_den(double d, bool in_range)
+{
+    if constexpr (SPLIT) {
+        return Den{d, recip<true>(d), true};
+    } else {
+        const SharedDen s = shared_den(d);
+        return Den{d, s.r, in_range && quot_range(d)};
+    }
+}
 struct AdiDerived {
     double cs, h, nu;
 };
@@ -624,11 +688,34 @@ __device__ __forceinline__ AdiDerived adi_derived(const KParams &P, int i, doubl
     return d;
 }
 
-// true where the fused step forms c_s, nu and T instead of storing them
-template <bool SPLIT>
-__device__ __forceinline__ bool lazy_derived(const KParams &P)
+// the same (FP64 storage) with the quotients by Sigma and sqrt(gamma) through
+// their reciprocals where `fine` says that E, Sigma and the constants are in range
+template <bool SPLIT, class PP>
+__device__ __forceinline__ AdiDerived adi_derived_in(const PP &P, int i, double e, double sig, bool fine)
 {
-    return P.lazy_derived != 0 && P.adiabatic;
+    if constexpr (SPLIT) {
+        return adi_derived<true>(P, i, e, sig);
+    } else {
+        AdiDerived d;
+        d.cs = sqrt_ieee(quot_by<false>(ring_tab(P, TAB_G_GM1, i) * e, Den{sig, shared_den(sig).r, fine}));
+        const Den sg{ring_tab(P, TAB_SQRT_GAMMA, i), ring_tab(P, TAB_SQRT_GAMMA_RCP, i), fine};
+        d.h = quot_by<false>(d.cs, sg) * ring_tab(P, TAB_INV_OMEGA_K, i);
+        const double alpha = P.alpha;
+        d.nu = alpha * d.h * d.cs;
+        return d;
+    }
+}
+
+// split storage: c_s and nu as a step that stores them reads them back
+template <bool SPLIT>
+__device__ __forceinline__ AdiDerived adi_derived_stored(const KParams &P, int i, int j, double e, double sig)
+{
+    AdiDerived a = adi_derived<SPLIT>(P, i, e, sig);
+    if (SPLIT && (P.split_emul & SPLIT_EMUL_DERIVED)) {
+        a.cs = fld<SPLIT>(P, FCPT_SOUNDSPEED).stored(i, j, a.cs);
+        a.nu = fld<SPLIT>(P, FCPT_VISCOSITY).stored(i, j, a.nu);
+    }
+    return a;
 }
 
 // the CFL limit of cell (i, j) (cfl.cpp:235-376), vm_i the ring's mean v_phi
@@ -657,9 +744,10 @@ __device__ __forceinline__ double cfl_cell(const KParams &P, int i, int j, doubl
     if (iso) {
         csv = cst(P.iso_cs)[i];
         nuv = cst(P.iso_nu)[i];
-    } else if (lazy_derived<SPLIT>(P)) {
-        // as the end of the last step formed them from the same E and Sigma
-        const AdiDerived a = adi_derived<SPLIT>(P, i, fld<SPLIT>(P, FCPT_ENERGY)(i, j), fld<SPLIT>(P, FCPT_SIGMA)(i, j));
+    } else if (P.lazy_derived) {
+        // as recalculate_derived forms them from the same E and Sigma
+        const AdiDerived a = adi_derived_stored<SPLIT>(P, i, j, fld<SPLIT>(P, FCPT_ENERGY)(i, j),
+                                                       fld<SPLIT>(P, FCPT_SIGMA)(i, j));
         csv = a.cs;
         nuv = a.nu;
     } else {
@@ -1006,32 +1094,47 @@ __global__ void __launch_bounds__(256) k_potential_fold(KParams P, int fold_mode
 // momentum_update_radial, SourceEuler.cpp:325-372, for one cell: pressure and
 // potential gradients between rings i - 1 and i, and the centrifugal term of
 // the four v_phi around the interface (summed in that order)
+// inv = 2 / (Sigma(i) + Sigma(i - 1))
+template <class PP>
+__device__ __forceinline__ double src_vr_by(const PP &P, int i, double dt, double v, double inv, double p0,
+                                            double pm, double phi0, double phim, double va00, double va01,
+                                            double va10, double va11)
+{
+    double gradp = inv;
+    gradp *= (p0 - pm);
+    gradp *= ring_tab(P, TAB_INV_DIFF_RMED, i);
+    const double gradphi = (phi0 - phim) * ring_tab(P, TAB_INV_DIFF_RMED, i);
+    const double vsum = va00 + va01 + va10 + va11;
+    const double vt = 0.25 * vsum + ring_tab(P, TAB_RINF_OMEGA, i);
+    const double vt2 = vt * vt;
+    const double centrifugal_accel = vt2 * ring_tab(P, TAB_INV_RINF, i);
+    return v + dt * (-gradp - gradphi + centrifugal_accel);
+}
 template <bool SPLIT = false>
 __device__ __forceinline__ double src_vr_new(const KParams &P, int i, double dt, double v, double s0,
                                              double sm, double p0, double pm, double phi0, double phim,
                                              double va00, double va01, double va10, double va11)
 {
-    double gradp = quot<SPLIT>(2.0, s0 + sm);
-    gradp *= (p0 - pm);
-    gradp *= cst(P.InvDiffRmed)[i];
-    const double gradphi = (phi0 - phim) * cst(P.InvDiffRmed)[i];
-    const double vsum = va00 + va01 + va10 + va11;
-    const double vt = 0.25 * vsum + cst(P.Rinf)[i] * P.omega_frame;
-    const double vt2 = vt * vt;
-    const double centrifugal_accel = vt2 * cst(P.InvRinf)[i];
-    return v + dt * (-gradp - gradphi + centrifugal_accel);
+    return src_vr_by(P, i, dt, v, quot<SPLIT>(2.0, s0 + sm), p0, pm, phi0, phim, va00, va01, va10, va11);
 }
 
 // momentum_update_azimuthal, SourceEuler.cpp:375-428, for one cell
+// inv = 2 / (Sigma(j) + Sigma(j - 1))
+template <class PP>
+__device__ __forceinline__ double src_vphi_by(const PP &P, int i, double dt, double va, double inv, double p0,
+                                              double pjp, double phi0, double phijp)
+{
+    const double invdxtheta = ring_tab(P, TAB_SRC_INVDXTHETA, i);  // 2 / (dphi (Rsup + Rinf))
+    const double gradp = inv * (p0 - pjp) * invdxtheta;
+    const double gradphi = (phi0 - phijp) * invdxtheta;
+    return va + dt * (-gradp - gradphi);
+}
 template <bool SPLIT = false>
 __device__ __forceinline__ double src_vphi_new(const KParams &P, int i, double dt, double va, double s0,
                                                double sjp, double p0, double pjp, double phi0,
                                                double phijp)
 {
-    const double invdxtheta = ring_tab(P, TAB_SRC_INVDXTHETA, i);  // 2 / (dphi (Rsup + Rinf))
-    const double gradp = quot<SPLIT>(2.0, s0 + sjp) * (p0 - pjp) * invdxtheta;
-    const double gradphi = (phi0 - phijp) * invdxtheta;
-    return va + dt * (-gradp - gradphi);
+    return src_vphi_by(P, i, dt, va, quot<SPLIT>(2.0, s0 + sjp), p0, pjp, phi0, phijp);
 }
 
 // momentum_update_radial, SourceEuler.cpp:325-372
@@ -1069,11 +1172,12 @@ FCPT_PAIR0(src_vphi, 256)
 
 // compression_heating, SourceEuler.cpp:459-493, for one cell (rings 0 .. nr-2)
 // from v_r(i), v_r(i + 1), v_phi(j), v_phi(j + 1)
-__device__ __forceinline__ double src_energy_new(const KParams &P, int i, double dt, double e, double vr0,
+template <class PP>
+__device__ __forceinline__ double src_energy_new(const PP &P, int i, double dt, double e, double vr0,
                                                  double vr1, double va0, double va1)
 {
-    const double DIV_V = (vr1 * cst(P.Rinf)[i + 1] - vr0 * cst(P.Rinf)[i]) * cst(P.InvDiffRsupRb)[i] +
-                         (va1 - va0) * P.invdphi * cst(P.InvRmed)[i];
+    const double DIV_V = (vr1 * ring_tab(P, TAB_RINF, i + 1) - vr0 * ring_tab(P, TAB_RINF, i)) * ring_tab(P, TAB_INV_DIFF_RSUP_RB, i) +
+                         (va1 - va0) * P.invdphi * ring_tab(P, TAB_INV_RMED, i);
     return e * exp(-(P.gamma - 1.0) * dt * DIV_V);
 }
 
@@ -1104,14 +1208,34 @@ __device__ __forceinline__ double energy_floor(const KParams &P, double sigma)
     return energy_at<SPLIT>(P, P.t_min, sigma);
 }
 // assure_temperature_range for one cell, SourceEuler.cpp:136-202
+// (FP64 storage: an e clear of both limits by more than the rounding of the
+// limits' products is unchanged, so the limits' four divisions are formed
+// only for the others)
 template <bool SPLIT = false>
 __device__ __forceinline__ double temperature_floor(const KParams &P, double e, double sigma)
 {
+    if constexpr (!SPLIT) {
+        const double es = sigma * P.energy_per_t;
+        const double lo = P.t_min * es, hi = P.t_max * es;
+        if (lo >= 0x1p-900 && e > lo * (1.0 + 0x1p-40) && e < hi * (1.0 - 0x1p-40)) return e;
+        __builtin_amdgcn_s_sleep(0);  // a branch: the divisions are not formed and selected
+    }
     const double minimum_energy = energy_floor<SPLIT>(P, sigma);
     const double maximum_energy = energy_at<SPLIT>(P, P.t_max, sigma);
     if (!(e > minimum_energy)) e = minimum_energy;
     if (!(e < maximum_energy)) e = maximum_energy;
     return e;
+}
+
+// temperature_floor at a cell of ring i whose Sigma is in range (fine)
+template <bool SPLIT, class PP>
+__device__ __forceinline__ double temperature_floor_in(const PP &P, int i, double e, double sig, bool fine)
+{
+    if constexpr (!SPLIT) {
+        if (fine && e > sig * ring_tab(P, TAB_E_LO, i) && e < sig * ring_tab(P, TAB_E_HI, i)) return e;
+        __builtin_amdgcn_s_sleep(0);
+    }
+    return temperature_floor<SPLIT>(P, e, sig);
 }
 
 template <bool SPLIT>
@@ -1162,13 +1286,9 @@ __device__ __forceinline__ void derived_store(const KParams &P, int i, int j, co
                                              bool force_nu = false)
 {
     double c_s, h;
-    // the fused step's kick walk forms the pressure from E itself
-    if (P.e_partner) with_pressure = false;
-    if (lazy_derived<SPLIT>(P)) {
-        // the field the step reads stored: H (the potential's smoothing)
-        const AdiDerived a = adi_derived<SPLIT>(P, i, d.e, d.sig);
-        fld<SPLIT>(P, FCPT_SCALE_HEIGHT).set(i, j, a.h);
-        if (with_pressure) fld<SPLIT>(P, FCPT_PRESSURE).set(i, j, (P.gamma - 1.0) * d.e);
+    if (P.lazy_derived) {
+        // the only derived field the step reads stored: H (the potential's smoothing)
+        if (P.adiabatic) fld<SPLIT>(P, FCPT_SCALE_HEIGHT).set(i, j, adi_derived<SPLIT>(P, i, d.e, d.sig).h);
         return;
     }
     if (P.adiabatic) {
@@ -1203,19 +1323,15 @@ struct TwQ {
     double qr, qp, eps_rr, eps_pp, div_V, l_sq;
 };
 
-__device__ __forceinline__ TwQ tw_q_cell(const KParams &P, int i, double vr0, double vr1, double va0,
+template <class PP>
+__device__ __forceinline__ TwQ tw_q_cell(const PP &P, int i, double vr0, double vr1, double va0,
                                          double va1, double sig)
 {
-    const int ns = P.ns;
     TwQ q;
-    q.eps_rr = (vr1 - vr0) * cst(P.InvDiffRsup)[i];
-    q.eps_pp = cst(P.InvRmed)[i] * ((va1 - va0) * P.invdphi + 0.5 * (vr1 + vr0));
+    q.eps_rr = (vr1 - vr0) * ring_tab(P, TAB_INV_DIFF_RSUP, i);
+    q.eps_pp = ring_tab(P, TAB_INV_RMED, i) * ((va1 - va0) * P.invdphi + 0.5 * (vr1 + vr0));
     q.div_V = std_min(q.eps_rr + q.eps_pp, 0.0);
-    const double Dr = cst(P.Rinf)[i + 1] - cst(P.Rinf)[i];
-    const double rDphi = cst(P.Rmed)[i] * P.dphi;
-    const double dxm = (ns <= 16) ? std_min(Dr, rDphi) : std_max(Dr, rDphi);
-    const double dx_sq = dxm * dxm;
-    q.l_sq = (P.artvisc_factor * P.artvisc_factor) * dx_sq;
+    q.l_sq = ring_tab(P, TAB_TW_LSQ, i);
     q.qr = q.l_sq * sig * -q.div_V * (q.eps_rr - 1.0 / 3.0 * q.div_V);
     q.qp = q.l_sq * sig * -q.div_V * (q.eps_pp - 1.0 / 3.0 * q.div_V);
     return q;
@@ -1223,8 +1339,8 @@ __device__ __forceinline__ TwQ tw_q_cell(const KParams &P, int i, double vr0, do
 
 // energy after the TW dissipation and the temperature floor
 // (artificial_viscosity.cpp:72-86, then SetTemperatureFloorCeilValues, :19-21)
-__device__ __forceinline__ double tw_dissipation(const KParams &P, int i, const TwQ &q, double sig,
-                                                 double dt, double e)
+template <class PP>
+__device__ __forceinline__ double tw_heat(const PP &P, int i, const TwQ &q, double sig, double dt, double e)
 {
     if (i > 1 && i < P.nr - 1) {
         const double d = q.eps_rr - q.eps_pp;
@@ -1232,7 +1348,13 @@ __device__ __forceinline__ double tw_dissipation(const KParams &P, int i, const 
             -q.l_sq * q.div_V * sig * 1.0 / 3.0 * (q.eps_rr * q.eps_rr + q.eps_pp * q.eps_pp + d * d);
         e += Qplus * dt;
     }
-    return temperature_floor(P, e, sig);
+    return e;
+}
+template <class PP>
+__device__ __forceinline__ double tw_dissipation(const PP &P, int i, const TwQ &q, double sig,
+                                                 double dt, double e)
+{
+    return temperature_floor(P, tw_heat(P, i, q, sig, dt, e), sig);
 }
 
 // update_with_artificial_viscosity_TW, artificial_viscosity.cpp:35-88
@@ -1259,25 +1381,38 @@ FCPT_PAIR0(tw_q, 256)
 
 // the TW velocity updates of one cell from the tensors around it
 // (artificial_viscosity.cpp:90-139)
+// (inv = 2 dt / ((Rsup + Rinf) Sigma_avg))
+template <class PP>
+__device__ __forceinline__ double tw_vphi_by(const PP &P, double va, double inv, double qp0, double qpj)
+{
+    const double dVp = inv * (qp0 - qpj) * P.invdphi;
+    return va + dVp;
+}
 template <bool SPLIT = false>
 __device__ __forceinline__ double tw_vphi_new(const KParams &P, int i, double dt, double va, double s0,
                                               double sjp, double qp0, double qpj)
 {
     const double sigma_phi_avg = 0.5 * (s0 + sjp);
-    const double dVp =
-        quot<SPLIT>(2.0 * dt, (cst(P.Rsup)[i] + cst(P.Rinf)[i]) * sigma_phi_avg) * (qp0 - qpj) * P.invdphi;
-    return va + dVp;
+    return tw_vphi_by(P, va, quot<SPLIT>(2.0 * dt, ring_tab(P, TAB_RSUP_RINF, i) * sigma_phi_avg), qp0, qpj);
 }
 
+// (c = f dt / Sigma_avg 2 / (Rmed(i)^2 - Rmed(i - 1)^2))
+template <class PP>
+__device__ __forceinline__ double tw_vr_by(const PP &P, int i, double v, double c, double qr0, double qrm,
+                                           double qp0, double qpm)
+{
+    const double r0 = ring_tab(P, TAB_RMED, i), r1 = ring_tab(P, TAB_RMED, i - 1);
+    const double dVr = c * ((qr0 * r0 - qrm * r1) - 0.5 * (qp0 + qpm) * ring_tab(P, TAB_RMED_DIFF, i));
+    return v + dVr;
+}
 template <bool SPLIT = false>
 __device__ __forceinline__ double tw_vr_new(const KParams &P, int i, double dt, double v, double s0,
                                             double sm, double qr0, double qrm, double qp0, double qpm)
 {
     const double sigma_r_avg = 0.5 * (s0 + sm);
-    const double r0 = cst(P.Rmed)[i], r1 = cst(P.Rmed)[i - 1];
-    const double dVr = quot<SPLIT>(quot<SPLIT>(P.radial_viscosity_factor * dt, sigma_r_avg) * 2.0, r0 * r0 - r1 * r1) *
-                       ((qr0 * r0 - qrm * r1) - 0.5 * (qp0 + qpm) * (r0 - r1));
-    return v + dVr;
+    const double c = quot<SPLIT>(quot<SPLIT>(P.radial_viscosity_factor * dt, sigma_r_avg) * 2.0,
+                                 ring_tab(P, TAB_RMED_SQ_DIFF, i));
+    return tw_vr_by(P, i, v, c, qr0, qrm, qp0, qpm);
 }
 
 template <bool SPLIT>
@@ -1327,11 +1462,12 @@ struct SnQ {
     double qr, qp, dv_r, dv_phi;
 };
 
-__device__ __forceinline__ SnQ sn_q_cell(const KParams &P, double vr0, double vr1, double va0,
+template <class PP>
+__device__ __forceinline__ SnQ sn_q_cell(const PP &P, int i, double vr0, double vr1, double va0,
                                          double va1, double sig)
 {
     SnQ q;
-    const double fac2 = P.artvisc_factor * P.artvisc_factor;
+    const double fac2 = ring_tab(P, TAB_ARTVISC_SQ, i);
     q.dv_r = vr1 - vr0;
     q.qr = q.dv_r < 0.0 ? fac2 * sig * (q.dv_r * q.dv_r) : 0.0;
     q.dv_phi = va1 - va0;
@@ -1341,14 +1477,20 @@ __device__ __forceinline__ SnQ sn_q_cell(const KParams &P, double vr0, double vr
 
 // energy after the SN dissipation and the temperature floor
 // (artificial_viscosity.cpp:187-205, then SetTemperatureFloorCeilValues)
-__device__ __forceinline__ double sn_dissipation(const KParams &P, int i, const SnQ &q, double sig,
-                                                 double dt, double e)
+template <class PP>
+__device__ __forceinline__ double sn_heat(const PP &P, int i, const SnQ &q, double dt, double e)
 {
     if (i >= 1 && i < P.nr - 1) {
         const double invdxtheta = ring_tab(P, TAB_INV_DXTHETA, i);  // 1 / (dphi Rmed)
-        e = e - dt * q.qr * q.dv_r * cst(P.InvDiffRsup)[i] - dt * q.qp * q.dv_phi * invdxtheta;
+        e = e - dt * q.qr * q.dv_r * ring_tab(P, TAB_INV_DIFF_RSUP, i) - dt * q.qp * q.dv_phi * invdxtheta;
     }
-    return temperature_floor(P, e, sig);
+    return e;
+}
+template <class PP>
+__device__ __forceinline__ double sn_dissipation(const PP &P, int i, const SnQ &q, double sig,
+                                                 double dt, double e)
+{
+    return temperature_floor(P, sn_heat(P, i, q, dt, e), sig);
 }
 
 // update_with_artificial_viscosity_SN, artificial_viscosity.cpp:148-211
@@ -1366,7 +1508,7 @@ __device__ __forceinline__ void b_sn_q(const KParams &P, int bx, int by)
     const double vr0 = vr(i, j), vr1 = vr(i + 1, j), va0 = vaz(i, j), va1 = vaz(i, jn);
     const double sig = S(i, j);
     const double e_in = diss ? E(i, j) : 0.0;
-    const SnQ q = sn_q_cell(P, vr0, vr1, va0, va1, sig);
+    const SnQ q = sn_q_cell(P, i, vr0, vr1, va0, va1, sig);
     fld<SPLIT>(P, FCPT_Q_R).set(i, j, q.qr);
     fld<SPLIT>(P, FCPT_Q_PHI).set(i, j, q.qp);
     if (diss) E.set(i, j, sn_dissipation(P, i, q, sig, dt, e_in));
@@ -1374,19 +1516,29 @@ __device__ __forceinline__ void b_sn_q(const KParams &P, int bx, int by)
 FCPT_PAIR0(sn_q, 256)
 
 // the SN velocity updates of one cell (artificial_viscosity.cpp:214-248)
+// (inv = 2 dt / (Sigma + its neighbour's))
+template <class PP>
+__device__ __forceinline__ double sn_vr_by(const PP &P, int i, double v, double inv, double qr0, double qrm)
+{
+    return v - inv * (qr0 - qrm) * ring_tab(P, TAB_INV_DIFF_RMED, i);
+}
+template <class PP>
+__device__ __forceinline__ double sn_vphi_by(const PP &P, int i, double va, double inv, double qp0, double qpj)
+{
+    return va - inv * (qp0 - qpj) * ring_tab(P, TAB_INV_DXTHETA, i);  // 1 / (dphi Rmed)
+}
 template <bool SPLIT = false>
 __device__ __forceinline__ double sn_vr_new(const KParams &P, int i, double dt, double v, double s0,
                                             double sm, double qr0, double qrm)
 {
-    return v - quot<SPLIT>(dt * 2.0, s0 + sm) * (qr0 - qrm) * cst(P.InvDiffRmed)[i];
+    return sn_vr_by(P, i, v, quot<SPLIT>(dt * 2.0, s0 + sm), qr0, qrm);
 }
 
 template <bool SPLIT = false>
 __device__ __forceinline__ double sn_vphi_new(const KParams &P, int i, double dt, double va, double s0,
                                               double sjp, double qp0, double qpj)
 {
-    const double invdxtheta = ring_tab(P, TAB_INV_DXTHETA, i);  // 1 / (dphi Rmed)
-    return va - quot<SPLIT>(dt * 2.0, s0 + sjp) * (qp0 - qpj) * invdxtheta;
+    return sn_vphi_by(P, i, va, quot<SPLIT>(dt * 2.0, s0 + sjp), qp0, qpj);
 }
 
 template <bool SPLIT>
@@ -1467,7 +1619,7 @@ template <bool SPLIT>
 __device__ __forceinline__ void b_iso_profile(const KParams &P, int bx, int by)
 {
     CELL_LOOP_HEAD(0, P.nr)
-    const double r = cst(P.Rmed)[i];
+    const double r = ring_tab(P, TAB_RMED, i);
     const double vK = sqrt(P.G * P.mstar / r);
     const double h = P.aspect_ratio * pow(r, P.flaring);
     const double c_s = h * vK;
@@ -1481,28 +1633,61 @@ __device__ __forceinline__ void b_iso_profile(const KParams &P, int bx, int by)
 }
 FCPT_PAIR0(iso_profile, 256)
 
-// the ring-uniform quotients of KParams::ring_tab, each with the expression
-// its users had inline (the same bits): 2 / (dphi (Rsup + Rinf)) of the
-// azimuthal source term, 1 / (dphi Rmed) of the SN viscosity, 1 / Omega_K
-// and Omega_K at Rmed, and 2 / (Rinf(i+1)^2 - Rinf(i)^2) of the viscous v_phi
-// update
-__global__ void __launch_bounds__(256) k_ring_tables(KParams P, double *tab)
+// KParams::ring_tab: the metric, and each ring-uniform product or quotient
+// with the expression of the cell formula that reads it (the same bits)
+__global__ void __launch_bounds__(256) k_ring_tables(KParams P, double *out)
 {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= P.nr) return;
-    const size_t w = (size_t)P.nr + 2;
-    tab[TAB_SRC_INVDXTHETA * w + i] = 2.0 / (P.dphi * (P.Rsup[i] + P.Rinf[i]));
+    if (i > P.nr) return;
+    double *tab = out + (size_t)i * kRingTabs;
+    tab[TAB_RINF] = P.Rinf[i];
+    tab[TAB_INV_RINF] = P.InvRinf[i];
+    tab[TAB_RMED] = P.Rmed[i];
+    tab[TAB_INV_RMED] = P.InvRmed[i];
+    tab[TAB_INV_DIFF_RMED] = P.InvDiffRmed[i];
+    tab[TAB_INV_DIFF_RSUP] = P.InvDiffRsup[i];
+    tab[TAB_INV_DIFF_RSUP_RB] = P.InvDiffRsupRb[i];
+    tab[TAB_SRC_INVDXTHETA] = 2.0 / (P.dphi * (P.Rsup[i] + P.Rinf[i]));
     const double dxtheta = P.dphi * P.Rmed[i];
-    tab[TAB_INV_DXTHETA * w + i] = 1.0 / dxtheta;
-    tab[TAB_INV_OMEGA_K * w + i] = 1.0 / omega_kepler(P, P.Rmed[i]);
-    tab[TAB_OMEGA_K * w + i] = omega_kepler(P, P.Rmed[i]);
-    const double a1 = P.Rinf[i + 1] * P.Rinf[i + 1], a0 = P.Rinf[i] * P.Rinf[i];
-    tab[TAB_VISC_AREA * w + i] = 2.0 / (a1 - a0);
+    tab[TAB_INV_DXTHETA] = 1.0 / dxtheta;
+    tab[TAB_INV_OMEGA_K] = 1.0 / omega_kepler(P, P.Rmed[i]);
+    tab[TAB_OMEGA_K] = omega_kepler(P, P.Rmed[i]);
+    const double a0 = P.Rinf[i] * P.Rinf[i], a1 = P.Rsup[i] * P.Rsup[i];  // Rsup[i] is Rinf[i + 1]
+    tab[TAB_VISC_AREA] = 2.0 / (a1 - a0);
+    tab[TAB_RINF_SQ] = a0;
+    tab[TAB_RINF_OMEGA] = P.Rinf[i] * P.omega_frame;
+    // the length scale of the TW tensor (artificial_viscosity.cpp:52-62)
+    const double Dr = P.Rsup[i] - P.Rinf[i], rDphi = P.Rmed[i] * P.dphi;
+    const double dxm = (P.ns <= 16) ? std_min(Dr, rDphi) : std_max(Dr, rDphi);
+    tab[TAB_TW_LSQ] = (P.artvisc_factor * P.artvisc_factor) * (dxm * dxm);
+    tab[TAB_RSUP_RINF] = P.Rsup[i] + P.Rinf[i];
+    const double r0 = P.Rmed[i], r1 = i > 0 ? P.Rmed[i - 1] : 0.0;
+    const SharedDen sum = shared_den(r0 + r1);
+    tab[TAB_RMED_SUM] = sum.d;
+    tab[TAB_RMED_SUM_RCP] = P.split ? recip<true>(sum.d) : sum.r;
+    const SharedDen sq = shared_den(r0 * r0 - r1 * r1);
+    tab[TAB_RMED_SQ_DIFF] = sq.d;
+    tab[TAB_RMED_SQ_DIFF_RCP] = P.split ? recip<true>(sq.d) : sq.r;
+    tab[TAB_RMED_DIFF] = r0 - r1;
+    // disk-wide constants, repeated per ring: the walks load them with the
+    // ring's values instead of holding them in registers throughout
+    tab[TAB_E_LO] = P.t_min * P.energy_per_t * (1.0 + 0x1p-40);
+    tab[TAB_E_HI] = P.t_max * P.energy_per_t * (1.0 - 0x1p-40);
+    const SharedDen sg = shared_den(sqrt(P.gamma)), cl = shared_den(P.c_light);
+    tab[TAB_SQRT_GAMMA] = sg.d;
+    tab[TAB_SQRT_GAMMA_RCP] = sg.r;
+    tab[TAB_C_LIGHT] = cl.d;
+    tab[TAB_C_LIGHT_RCP] = cl.r;
+    tab[TAB_G_GM1] = P.gamma * (P.gamma - 1.0);
+    tab[TAB_MU_GM1] = P.mu * (P.gamma - 1.0);
+    tab[TAB_SIGMA_FLOOR10] = 10.0 * P.sigma0 * P.sigma_floor;
+    tab[TAB_BETA_INV] = 1 / P.cooling_beta;
+    tab[TAB_ARTVISC_SQ] = P.artvisc_factor * P.artvisc_factor;
 }
 
 void launch_ring_tables(const KParams &P, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_ring_tables, dim3((unsigned)((P.nr + 255) / 256)), dim3(256), 0, st, P, P.ring_tab);
+    hipLaunchKernelGGL(k_ring_tables, dim3((unsigned)((P.nr + 256) / 256)), dim3(256), 0, st, P, P.ring_tab);
 }
 
 // the locally isothermal ring profiles c_s, H and nu = alpha H c_s, with the
@@ -1511,7 +1696,7 @@ __global__ void __launch_bounds__(256) k_iso_rings(KParams P)
 {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= P.nr) return;
-    const double r = cst(P.Rmed)[i];
+    const double r = ring_tab(P, TAB_RMED, i);
     const double vK = sqrt(P.G * P.mstar / r);
     const double h = P.aspect_ratio * pow(r, P.flaring);
     const double c_s = h * vK;
@@ -1531,28 +1716,30 @@ struct StressDiag {
     double divv, trr, tpp;
 };
 
-__device__ __forceinline__ StressDiag stress_diag(const KParams &P, int i, double vr0, double vr1,
+template <class PP>
+__device__ __forceinline__ StressDiag stress_diag(const PP &P, int i, double vr0, double vr1,
                                                   double va0, double va1, double n, double s)
 {
     StressDiag d;
-    d.divv = (vr1 * cst(P.Rinf)[i + 1] - vr0 * cst(P.Rinf)[i]) * cst(P.InvDiffRsupRb)[i] +
-             (va1 - va0) * P.invdphi * cst(P.InvRmed)[i];
-    const double drr = (vr1 - vr0) * cst(P.InvDiffRsup)[i];
+    d.divv = (vr1 * ring_tab(P, TAB_RINF, i + 1) - vr0 * ring_tab(P, TAB_RINF, i)) * ring_tab(P, TAB_INV_DIFF_RSUP_RB, i) +
+             (va1 - va0) * P.invdphi * ring_tab(P, TAB_INV_RMED, i);
+    const double drr = (vr1 - vr0) * ring_tab(P, TAB_INV_DIFF_RSUP, i);
     d.trr = 2.0 * n * s * (drr - 1.0 / 3.0 * d.divv);
-    const double dpp = (va1 - va0) * P.invdphi * cst(P.InvRmed)[i] + 0.5 * (vr1 + vr0) * cst(P.InvRmed)[i];
+    const double dpp = (va1 - va0) * P.invdphi * ring_tab(P, TAB_INV_RMED, i) + 0.5 * (vr1 + vr0) * ring_tab(P, TAB_INV_RMED, i);
     d.tpp = 2.0 * n * s * (dpp - 1.0 / 3.0 * d.divv);
     return d;
 }
 
 // the corner component tau_r_phi at (i >= 1, j) from v_phi(i), v_phi(i - 1),
 // v_r(j), v_r(j - 1) and nu, Sigma of the four cells around the corner
-__device__ __forceinline__ double stress_rp(const KParams &P, int i, double va0, double vam, double vr0,
+template <class PP>
+__device__ __forceinline__ double stress_rp(const PP &P, int i, double va0, double vam, double vr0,
                                             double vrp, double n, double nm, double njp, double nmp,
                                             double s, double sm, double sjp, double smp)
 {
-    const double dvazirdr = (va0 * cst(P.InvRmed)[i] - vam * cst(P.InvRmed)[i - 1]) * cst(P.InvDiffRmed)[i];
+    const double dvazirdr = (va0 * ring_tab(P, TAB_INV_RMED, i) - vam * ring_tab(P, TAB_INV_RMED, i - 1)) * ring_tab(P, TAB_INV_DIFF_RMED, i);
     const double dvrdphi = (vr0 - vrp) * P.invdphi;
-    const double drp = cst(P.Rinf)[i] * dvazirdr + dvrdphi * cst(P.InvRinf)[i];
+    const double drp = ring_tab(P, TAB_RINF, i) * dvazirdr + dvrdphi * ring_tab(P, TAB_INV_RINF, i);
     const double n4 = 0.25 * (n + nm + njp + nmp);
     const double s4 = 0.25 * (s + sm + sjp + smp);
     return n4 * s4 * drp;
@@ -1586,29 +1773,43 @@ __device__ __forceinline__ void b_stress(const KParams &P, int bx, int by)
 FCPT_PAIR0(stress, 256)
 
 // update_velocities_with_viscosity, viscosity.cpp:355-426, for one cell
+// (inv = dt / Rmed / Sigma_avg)
+template <class PP>
+__device__ __forceinline__ double visc_vphi_by(const PP &P, int i, double va, double inv, double trp0,
+                                               double trp1, double tpp0, double tppj)
+{
+    const double a1 = ring_tab(P, TAB_RINF_SQ, i + 1), a0 = ring_tab(P, TAB_RINF_SQ, i);
+    const double dVp = inv * (ring_tab(P, TAB_VISC_AREA, i) * (a1 * trp1 - a0 * trp0) + (tpp0 - tppj) * P.invdphi);
+    return va + dVp;
+}
 template <bool SPLIT = false>
 __device__ __forceinline__ double visc_vphi_new(const KParams &P, int i, double dt, double va, double s0,
                                                 double sjp, double trp0, double trp1, double tpp0,
                                                 double tppj)
 {
     const double sigma_avg = 0.5 * (s0 + sjp);
-    const double a1 = cst(P.Rinf)[i + 1] * cst(P.Rinf)[i + 1], a0 = cst(P.Rinf)[i] * cst(P.Rinf)[i];
-    const double dVp = quot<SPLIT>(dt * cst(P.InvRmed)[i], sigma_avg) *
-                       (ring_tab(P, TAB_VISC_AREA, i) * (a1 * trp1 - a0 * trp0) + (tpp0 - tppj) * P.invdphi);
-    return va + dVp;
+    return visc_vphi_by(P, i, va, quot<SPLIT>(dt * ring_tab(P, TAB_INV_RMED, i), sigma_avg), trp0, trp1, tpp0, tppj);
 }
 
+// (c = dt / Sigma_avg f 2 / (Rmed(i) + Rmed(i - 1)))
+template <class PP>
+__device__ __forceinline__ double visc_vr_by(const PP &P, int i, double v, double c, double trr0, double trrm,
+                                             double trp0, double trpn, double tpp0, double tppm)
+{
+    const double dVr = c * ((ring_tab(P, TAB_RMED, i) * trr0 - ring_tab(P, TAB_RMED, i - 1) * trrm) *
+                                ring_tab(P, TAB_INV_DIFF_RMED, i) +
+                            (trpn - trp0) * P.invdphi - 0.5 * (tpp0 + tppm));
+    return v + dVr;
+}
 template <bool SPLIT = false>
 __device__ __forceinline__ double visc_vr_new(const KParams &P, int i, double dt, double v, double s0,
                                               double sm, double trr0, double trrm, double trp0,
                                               double trpn, double tpp0, double tppm)
 {
     const double sigma_avg = 0.5 * (s0 + sm);
-    const double dVr = quot<SPLIT>(quot<SPLIT>(dt, sigma_avg) * P.radial_viscosity_factor * 2.0,
-                                   cst(P.Rmed)[i] + cst(P.Rmed)[i - 1]) *
-                       ((cst(P.Rmed)[i] * trr0 - cst(P.Rmed)[i - 1] * trrm) * cst(P.InvDiffRmed)[i] +
-                        (trpn - trp0) * P.invdphi - 0.5 * (tpp0 + tppm));
-    return v + dVr;
+    const double c = quot<SPLIT>(quot<SPLIT>(dt, sigma_avg) * P.radial_viscosity_factor * 2.0,
+                                 ring_tab(P, TAB_RMED_SUM, i));
+    return visc_vr_by(P, i, v, c, trr0, trrm, trp0, trpn, tpp0, tppm);
 }
 
 template <bool SPLIT>
@@ -1752,12 +1953,12 @@ __device__ __forceinline__ void b_av_fused(const KParams &P, int bx, int by, int
     }
     double qr0, qp0, qpj = 0.0, qrm = 0.0, qpm = 0.0, e = e_in;
     if (sn) {
-        const SnQ q = sn_q_cell(P, vr0, vr1, va0, va1, sig);
+        const SnQ q = sn_q_cell(P, i, vr0, vr1, va0, va1, sig);
         qr0 = q.qr;
         qp0 = q.qp;
         if (diss) e = sn_dissipation(P, i, q, sig, dt, e_in);
-        if (inner) qpj = sn_q_cell(P, vrj0, vrj1, vaj0, va0, sjp).qp;
-        if (radial) qrm = sn_q_cell(P, vrm0, vr0, vam0, vam1, sm).qr;
+        if (inner) qpj = sn_q_cell(P, i, vrj0, vrj1, vaj0, va0, sjp).qp;
+        if (radial) qrm = sn_q_cell(P, im, vrm0, vr0, vam0, vam1, sm).qr;
     } else {
         const TwQ q = tw_q_cell(P, i, vr0, vr1, va0, va1, sig);
         qr0 = q.qr;
@@ -1784,183 +1985,6 @@ __device__ __forceinline__ void b_av_fused(const KParams &P, int bx, int by, int
         vr_o.set_raw(i, j, vr_raw);
 }
 FCPT_PAIR1(av_fused, 256, int, with_viscosity)
-
-// The kick's source terms and artificial viscosity as one radial walk:
-// update_with_sourceterms, compression_heating (adiabatic) and the TW or SN
-// artificial viscosity with its dissipation and recalculate_viscosity, the
-// per-cell steps of b_src_fused, b_src_energy and b_av_fused in that order,
-// after the potential pass.  A wavefront owns kKickSegW consecutive sectors
-// and `tile` consecutive rings: lane k holds sector j0 - 2 + k (lanes 0, 1,
-// 62 and 63 are the halo) and walks the rings outwards.  Each ring is loaded
-// once (v_r, v_phi, Sigma, the potential, and the pressure of an adiabatic
-// disk); the source-term velocities of a ring are formed one ring ahead of the
-// artificial viscosity that reads them, the neighbouring sectors' values come
-// from the adjacent lanes by DPP moves (each stage spoils one more lane at
-// either edge), and the tensor of ring i - 1 carries over.  E is read and
-// written only at the lane's own cells, so no wavefront reads what another
-// writes, and the derived fields it stores (c_s, H, nu) are not read here.
-// Every value goes through the helpers
-// of the separate kernels with the same arguments, so FP64 storage gives the
-// same fields bit for bit; in split storage the source-term velocities stay
-// in FP64 between the stages.
-constexpr int kKickSegW = 60;
-
-struct KickRing {
-    double vr, va, s, p, phi, e;  // the lane's sector (p: pressure, phi: potential, e: E)
-    double sL, vaR;               // Sigma of sector j - 1, v_phi of sector j + 1
-};
-
-template <bool SPLIT, bool ADI, bool SN>
-__device__ __forceinline__ void b_kick_walk(const KParams &P, int bx, int by, int tile)
-{
-    const int ns = P.ns, nr = P.nr;
-    const int k = (int)threadIdx.x;  // lane
-    const int i0 = __builtin_amdgcn_readfirstlane((by * (int)blockDim.y + (int)threadIdx.y) * tile);
-    if (i0 >= nr) return;
-    const int i1 = i0 + tile < nr ? i0 + tile : nr;  // rings [i0, i1)
-    const int j0 = bx * kKickSegW;
-    const int Ls = ns - j0 < kKickSegW ? ns - j0 : kKickSegW;
-    const int j = (j0 - 2 + k + 2 * ns) % ns;
-    const bool own = k >= 2 && k < 2 + Ls;  // lanes that write
-    FLD(vr, FCPT_VRAD);
-    FLD(vaz, FCPT_VAZI);
-    FLD(S, FCPT_SIGMA);
-    FLD(E, FCPT_ENERGY);
-    const Fld<SPLIT> vr_o = alt_vr<SPLIT>(P);
-    const Fld<SPLIT> vaz_o = alt_vaz<SPLIT>(P);
-    const double dt = P.s->dt;
-    constexpr bool sn = SN;
-    const bool diss = ADI && P.artvisc_dissipation;
-    auto load = [&](int r) {
-        KickRing w;
-        w.vr = vr(r, j);
-        if (r < nr) {
-            w.va = vaz(r, j);
-            w.s = S(r, j);
-            // P = (gamma - 1) E as the last step stored it (compute_pressure):
-            // with the partner buffer no wavefront writes E during the walk
-            w.e = ADI ? E(r, j) : 0.0;
-            w.p = ADI ? (P.e_partner ? (P.gamma - 1.0) * w.e : fld<SPLIT>(P, FCPT_PRESSURE)(r, j))
-                      : iso_pressure(P, r, w.s);
-            w.phi = phi_fld(P)(r, j);
-        } else {
-            w.va = w.s = w.p = w.phi = w.e = 0.0;
-        }
-        w.sL = from_left(w.s);
-        w.vaR = from_right(w.va);
-        return w;
-    };
-    // the source-term velocities of ring r (b) from ring r - 1 (a); rows
-    // that are not updated keep their values
-    auto src = [&](int r, const KickRing &a, const KickRing &b, double &v1r, double &v1a) {
-        const double pjp = from_left(b.p), phijp = from_left(b.phi);
-        const bool upd_p = r >= 1 && r < nr - 1;
-        const bool upd_r = r >= 2 && upd_p;
-        v1a = upd_p ? src_vphi_new<SPLIT>(P, r, dt, b.va, b.s, b.sL, b.p, pjp, b.phi, phijp) : b.va;
-        v1r = upd_r ? src_vr_new<SPLIT>(P, r, dt, b.vr, b.s, a.s, b.p, a.p, b.phi, a.phi, b.va, b.vaR, a.va, a.vaR)
-                    : b.vr;
-    };
-    // the tensor of cell (r, j) from the source-term velocities
-    struct Q {
-        TwQ tw;
-        SnQ sn;
-        double qr, qp;
-    };
-    auto qcell = [&](int r, double vr0, double vr1, double va0, double va1, double sig) {
-        Q q;
-        if constexpr (SN) {
-            q.sn = sn_q_cell(P, vr0, vr1, va0, va1, sig);
-            q.qr = q.sn.qr;
-            q.qp = q.sn.qp;
-        } else {
-            q.tw = tw_q_cell(P, r, vr0, vr1, va0, va1, sig);
-            q.qr = q.tw.qr;
-            q.qp = q.tw.qp;
-        }
-        return q;
-    };
-    KickRing R0, R1;  // rings i, i + 1
-    double v1r0 = 0.0, v1a0 = 0.0;  // source-term velocities of ring i
-    double qr_m = 0.0, qp_m = 0.0, s_m = 0.0;  // tensor and Sigma of cell (i - 1, j)
-    if (i0 >= 1) {
-        const KickRing Rm2 = load(i0 >= 2 ? i0 - 2 : 0);  // unused by ring 0
-        const KickRing Rm = load(i0 - 1);
-        R0 = load(i0);
-        double v1rm, v1am;
-        src(i0 - 1, Rm2, Rm, v1rm, v1am);
-        src(i0, Rm, R0, v1r0, v1a0);
-        const Q qm = qcell(i0 - 1, v1rm, v1r0, v1am, from_right(v1am), Rm.s);
-        qr_m = qm.qr;
-        qp_m = qm.qp;
-        s_m = Rm.s;
-    } else {
-        R0 = load(i0);
-        src(i0, R0, R0, v1r0, v1a0);  // ring 0 is passed through
-    }
-    for (int i = i0; i < i1; ++i) {
-        R1 = load(i + 1);  // ring nr holds only v_r
-        double v1r1, v1a1;
-        src(i + 1, R0, R1, v1r1, v1a1);
-        const double v1aR = from_right(v1a0);  // v_phi of sector j + 1
-        const Q q = qcell(i, v1r0, v1r1, v1a0, v1aR, R0.s);
-        const double qpj = from_left(q.qp);  // tensor of cell (i, j - 1)
-        const bool inner = i >= 1 && i < nr - 1;
-        const bool radial = i >= 2 && inner;
-        if (own) {
-            if constexpr (ADI) {
-                // compression_heating (rings 0 .. nr-2), then the dissipation;
-                // the result to E or (e_partner) to its partner buffer, every cell
-                const Fld<SPLIT> Eo = P.e_partner ? buf<SPLIT>(P, P.ealt, P.bg[FCPT_ENERGY], FCPT_ENERGY) : E;
-                double e = R0.e;
-                if (i < nr - 1) e = E.stored(i, j, src_energy_new(P, i, dt, e, v1r0, v1r1, v1a0, v1aR));
-                if (diss) e = sn ? sn_dissipation(P, i, q.sn, R0.s, dt, e) : tw_dissipation(P, i, q.tw, R0.s, dt, e);
-                if (i < nr - 1 || diss) {
-                    e = Eo.set_get(i, j, e);  // the partner has E's background and key
-                } else if (P.e_partner) {
-                    Eo.set_raw(i, j, E.raw(i, j));
-                }
-                // recalculate_viscosity
-                const AdiDerived d = adi_derived<SPLIT>(P, i, e, R0.s);
-                if (!lazy_derived<SPLIT>(P)) {
-                    fld<SPLIT>(P, FCPT_SOUNDSPEED).set(i, j, d.cs);
-                    fld<SPLIT>(P, FCPT_SCALE_HEIGHT).set(i, j, d.h);
-                }
-                fld<SPLIT>(P, FCPT_VISCOSITY).set(i, j, d.nu);
-            }
-            if (inner)
-                vaz_o.set(i, j, sn ? sn_vphi_new<SPLIT>(P, i, dt, v1a0, R0.s, R0.sL, q.qp, qpj)
-                                   : tw_vphi_new<SPLIT>(P, i, dt, v1a0, R0.s, R0.sL, q.qp, qpj));
-            else
-                vaz_o.set_raw(i, j, vaz.raw(i, j));
-            if (radial)
-                vr_o.set(i, j, sn ? sn_vr_new<SPLIT>(P, i, dt, v1r0, R0.s, s_m, q.qr, qr_m)
-                                  : tw_vr_new<SPLIT>(P, i, dt, v1r0, R0.s, s_m, q.qr, qr_m, q.qp, qp_m));
-            else
-                vr_o.set_raw(i, j, vr.raw(i, j));
-        }
-        qr_m = q.qr;
-        qp_m = q.qp;
-        s_m = R0.s;
-        R0 = R1;
-        v1r0 = v1r1;
-        v1a0 = v1a1;
-    }
-    if (i1 == nr && own) vr_o.set_raw(nr, j, vr.raw(nr, j));  // the outer v_r row, untouched
-}
-template <bool SPLIT, bool ADI, bool SN>
-__global__ void __launch_bounds__(256) k_kick_walk(KParams P, int tile)
-{
-    const BlockXY bb = xcd_block();
-    b_kick_walk<SPLIT, ADI, SN>(P, bb.x, bb.y, tile);
-}
-// batched form: each disk's tile is its resolved kick_tile
-template <bool SPLIT, bool ADI, bool SN>
-__global__ void __launch_bounds__(256) kb_kick_walk(const KParams *Ps, const BatchEntry *map)
-{
-    const BatchEntry e = batch_entry(map);
-    const KParams &P = batch_disk(Ps, e.disk);
-    b_kick_walk<SPLIT, ADI, SN>(P, (int)(e.yx & 0xffffu), (int)(e.yx >> 16), P.kick_tile);
-}
 
 // compute_viscous_stress_tensor and update_velocities_with_viscosity
 // (viscosity.cpp:139-426) in one pass: the stress components a cell's update
@@ -2058,19 +2082,23 @@ __device__ __forceinline__ void b_copy_velocities(const KParams &P, int bx, int 
     FLD(vaz, FCPT_VAZI);
     alt_vr<SPLIT>(P).set_raw(i, j, vr.raw(i, j));
     if (i < P.nr) alt_vaz<SPLIT>(P).set_raw(i, j, vaz.raw(i, j));
+    if (i < P.nr && P.adiabatic && P.lazy_derived) {  // E is in its partner buffer too
+        FLD(E, FCPT_ENERGY);
+        buf<SPLIT>(P, P.ealt, P.bg[FCPT_ENERGY]).set_raw(i, j, E.raw(i, j));
+    }
 }
 FCPT_PAIR0(copy_velocities, 256)
 
 // ---------------------------------------------------------------------------
 // Q- of the beta cooling (thermal_relaxation, SourceEuler.cpp:632-690) for
 // one active cell
-template <bool SPLIT>
-__device__ __forceinline__ double cooling_beta_cell(const KParams &P, int i, int j, double time, double e,
+template <bool SPLIT, class PP>
+__device__ __forceinline__ double cooling_beta_cell(const PP &P, int i, int j, double time, double e,
                                                     double sig)
 {
     if (!P.cooling_beta_enabled) return 0.0;
     const double omega_k = ring_tab(P, TAB_OMEGA_K, i);  // Omega_K(Rmed)
-    double beta_inv = 1 / P.cooling_beta;
+    double beta_inv = ring_tab(P, TAB_BETA_INV, i);
     if (P.cooling_beta_ramp_up > 0.0) {
         const double x = 2 * time / P.cooling_beta_ramp_up;
         const double ramp_factor = 1 - exp(-(x * x));
@@ -2088,9 +2116,9 @@ __device__ __forceinline__ double cooling_beta_cell(const KParams &P, int i, int
 // the cell's stress tensor; tau_r_phi is the mean of the cell's four corners
 template <bool SPLIT = false>
 __device__ __forceinline__ double viscous_heating_q(const KParams &P, double nu, double sig, double trr,
-                                                    double tpp, double dv, double tau_r_phi)
+                                                    double tpp, double dv, double tau_r_phi, bool fine = false)
 {
-    double q = quot<SPLIT>(1.0, 2.0 * nu * sig) * (trr * trr + 2 * (tau_r_phi * tau_r_phi) + tpp * tpp);
+    double q = quot_by<SPLIT>(1.0, make_den<SPLIT>(2.0 * nu * sig, fine)) * (trr * trr + 2 * (tau_r_phi * tau_r_phi) + tpp * tpp);
     q += (2.0 / 9.0) * nu * sig * (dv * dv);
     q *= P.heating_viscous_factor;
     return 0.0 + q;
@@ -2127,19 +2155,34 @@ __device__ __forceinline__ double rad_alpha(const KParams &P, double h, double s
     const double inv_pow4 = pow4_comp(quot<SPLIT>(P.mu * (P.gamma - 1.0), P.Rgas * sig));
     return 1.0 + 2.0 * h * 4.0 * P.sigma_sb / P.c_light * inv_pow4 * pow3_comp(e);
 }
+// the same at a cell of ring i whose Sigma, E and H are in range (fine)
+template <bool SPLIT, class PP>
+__device__ __forceinline__ double rad_alpha_in(const PP &P, int i, double h, double sig, double e, bool fine)
+{
+    if constexpr (SPLIT) {
+        return rad_alpha<true>(P, h, sig, e);
+    } else {
+        const double d = P.Rgas * sig;
+        const double inv_pow4 = pow4_comp(quot_by<false>(ring_tab(P, TAB_MU_GM1, i), Den{d, shared_den(d).r, fine}));
+        const Den c{ring_tab(P, TAB_C_LIGHT, i), ring_tab(P, TAB_C_LIGHT_RCP, i), fine};
+        return 1.0 + quot_by<false>(2.0 * h * 4.0 * P.sigma_sb, c) * inv_pow4 * pow3_comp(e);
+    }
+}
 
 // SubStep3 (SourceEuler.cpp:859-954) at one cell from its Q+ and Q- before
-// the radiative correction; writes T, Q+, Q- and E
-template <bool SPLIT>
-__device__ __forceinline__ void substep3_cell(const KParams &P, int i, int j, double e, double sig, double h,
-                                              double qplus, double qminus)
+// the radiative correction; writes T, Q+, Q- and (to Eo) E
+template <bool SPLIT, class PP>
+__device__ __forceinline__ void substep3_cell(const PP &P, const Fld<SPLIT> &Eo, int i, int j, double e,
+                                              double sig, double h, double qplus, double qminus, bool fine = false)
 {
-    const double dt = P.s->dt;
-    // compute_temperature (SourceEuler.cpp:1378-1408) before the update
-    const double c_v_inv = P.mu / P.Rgas * (P.gamma - 1.0);
-    const double temperature = c_v_inv * e / sig;
+    const double dt = kick_dt(P);
+    if (!P.lazy_derived) {
+        // compute_temperature (SourceEuler.cpp:1378-1408) before the update
+        const double c_v_inv = P.mu / P.Rgas * (P.gamma - 1.0);
+        fld<SPLIT>(P, FCPT_TEMPERATURE).set(i, j, c_v_inv * e / sig);
+    }
     if (i >= 1 && i < P.nr - 1) {
-        const double alpha = rad_alpha<SPLIT>(P, h, sig, e);
+        const double alpha = rad_alpha_in<SPLIT>(P, i, h, sig, e, fine);
         if constexpr (SPLIT) {
             const double ra = recip<true>(alpha);
             qplus *= ra;
@@ -2150,8 +2193,7 @@ __device__ __forceinline__ void substep3_cell(const KParams &P, int i, int j, do
             qminus = shared_div(qminus, A);
         }
         double energy_new = e + dt * (qplus - qminus);
-        const double SigmaFloor = 10.0 * P.sigma0 * P.sigma_floor;
-        if ((sig < SigmaFloor)) {
+        if (sig < ring_tab(P, TAB_SIGMA_FLOOR10, i)) {
             // TAU_EFF is never computed without surface cooling: it holds 0
             const double tau_eff = 0.0;
             const double e4 = qplus * tau_eff / (2.0 * P.sigma_sb);
@@ -2163,10 +2205,9 @@ __device__ __forceinline__ void substep3_cell(const KParams &P, int i, int j, do
     } else {
         qplus = qminus = 0.0;
     }
-    if (!lazy_derived<SPLIT>(P)) fld<SPLIT>(P, FCPT_TEMPERATURE).set(i, j, temperature);
     fld<SPLIT>(P, FCPT_QPLUS).set(i, j, qplus);
     fld<SPLIT>(P, FCPT_QMINUS).set(i, j, qminus);
-    fld<SPLIT>(P, FCPT_ENERGY).set(i, j, temperature_floor<SPLIT>(P, e, sig));
+    Eo.set(i, j, temperature_floor_in<SPLIT>(P, i, e, sig, fine));
 }
 
 template <bool SPLIT>
@@ -2178,7 +2219,7 @@ __device__ __forceinline__ void b_substep3(const KParams &P, int bx, int by)
     const double h = fld<SPLIT>(P, FCPT_SCALE_HEIGHT)(i, j);
     double qplus = 0.0, qminus = 0.0;
     if (i >= 1 && i < P.nr - 1) heating_cooling_cell<SPLIT>(P, i, j, P.s->time, e, sig, qplus, qminus);
-    substep3_cell<SPLIT>(P, i, j, e, sig, h, qplus, qminus);
+    substep3_cell<SPLIT>(P, fld<SPLIT>(P, FCPT_ENERGY), i, j, e, sig, h, qplus, qminus);
 }
 FCPT_PAIR0(substep3, 256)
 
@@ -2318,11 +2359,9 @@ __device__ __forceinline__ void b_visc_walk(const KParams &P, int bx, int by, in
             else
                 vr_o.set_raw(i, j, vr.raw(i, j));
             if constexpr (ENERGY) {
-                const double e = P.e_partner ? buf<SPLIT>(P, P.ealt, P.bg[FCPT_ENERGY])(i, j)
-                                             : fld<SPLIT>(P, FCPT_ENERGY)(i, j);
-                // H as the kick walk formed it from the same E and Sigma
-                const double h = lazy_derived<SPLIT>(P) ? adi_derived<SPLIT>(P, i, e, A.s).h
-                                                         : fld<SPLIT>(P, FCPT_SCALE_HEIGHT)(i, j);
+                FLD(E, FCPT_ENERGY);
+                const double e = E(i, j);
+                const double h = fld<SPLIT>(P, FCPT_SCALE_HEIGHT)(i, j);
                 double qplus = 0.0, qminus = 0.0;
                 if (upd_p) {
                     qminus = cooling_beta_cell<SPLIT>(P, i, j, P.s->time, e, A.s);
@@ -2330,7 +2369,7 @@ __device__ __forceinline__ void b_visc_walk(const KParams &P, int bx, int by, in
                         qplus = viscous_heating_q<SPLIT>(P, A.n, A.s, d.trr, d.tpp, d.divv,
                                                   0.25 * (trp_c + trp1 + trp_n + trp1_n));
                 }
-                substep3_cell<SPLIT>(P, i, j, e, A.s, h, qplus, qminus);
+                substep3_cell<SPLIT>(P, E, i, j, e, A.s, h, qplus, qminus);
             }
         }
         dprev = d;
@@ -2354,6 +2393,355 @@ __global__ void __launch_bounds__(256) kb_visc_walk(const KParams *Ps, const Bat
     const BatchEntry e = batch_entry(map);
     const KParams &P = batch_disk(Ps, e.disk);
     b_visc_walk<SPLIT, ENERGY>(P, (int)(e.yx & 0xffffu), (int)(e.yx >> 16), P.visc_tile);
+}
+
+// The whole kick of the fused step as one radial walk, after the potential
+// pass: update_with_sourceterms, compression_heating (adiabatic), the TW or SN
+// artificial viscosity with its dissipation and recalculate_viscosity, then
+// the viscous stress, the velocity update and (adiabatic) SubStep3: the
+// per-cell steps of b_src_fused, b_src_energy, b_av_fused, b_visc_fused and
+// b_substep3 in that order.
+//
+// A wavefront owns kKvSegW consecutive sectors and `tile` consecutive rings:
+// lane k holds sector j0 - 3 + k and walks the rings outwards.  Each ring is
+// loaded once (v_r, v_phi, Sigma, the potential, and E of an adiabatic disk,
+// whose pressure is (gamma - 1) E); neighbouring sectors' values come from the
+// adjacent lanes by DPP moves, and every stage runs one ring behind the one it
+// reads: the source-term velocities at ring m + 1, the artificial viscosity at
+// m, the viscous update and SubStep3 at m - 1.  The stages spoil three lanes
+// at the lower and two at the upper edge: the source terms read sectors j - 1
+// and j + 1, the artificial viscosity the tensor of j - 1 and v_phi of j + 1,
+// the viscous update tau_phi_phi of j - 1 and tau_r_phi of j + 1.  Results go
+// to partner buffers (the velocities' valt, E's ealt), so no wavefront reads
+// what another writes; rows that are not updated are copied as stored.
+//
+// Every value goes through the helpers of the separate kernels with the same
+// arguments, so FP64 storage gives the same fields bit for bit.  Split storage
+// rounds what the stages hand over (v_r, v_phi, E and nu between the
+// artificial viscosity and the viscous update) as if it had been stored;
+// KParams::split_emul adds the roundings of the forms that store more.
+//
+// What bounds it: the latency of its chain of stages, at the 3 wavefronts per
+// SIMD (4 isothermal) that its registers allow; VALU issue is about half of
+// its time.  Hence one pass for the whole kick (a walk for the sources and
+// artificial viscosity and one for the rest moved 188 B/cell at 4096 x 12288
+// adiabatic, 2161 us; this one 88 B/cell, 1390 us; 2048 x 6144 isothermal 256
+// -> 185 us), the loads of ring m + 2 in flight during ring m, no load behind
+// a store in the loop (rows that are only copied are copied after it: 240 us
+// at 4096 x 12288), the ring's metric in LDS (KWalk), and quotients that share
+// a denominator through one reciprocal.
+// doubles of LDS per wavefront: the ring-table rows of its rings
+__host__ __device__ inline int kv_lds_doubles(int tile) { return (tile + 5) * kRingTabs; }
+extern __shared__ __align__(16) double kv_lds[];
+
+constexpr int kKvSegW = 59;   // sectors written per wavefront
+constexpr int kKvHalo = 3;    // sectors before them
+template <bool SPLIT, bool ADI, bool SN, bool EMUL>
+__device__ __forceinline__ void b_kv_walk(const KParams &K, int bx, int by, int tile, double *lds)
+{
+    const int ns = K.ns, nr = K.nr;
+    const int k = (int)threadIdx.x;  // lane
+    const int i0 = __builtin_amdgcn_readfirstlane((by * (int)blockDim.y + (int)threadIdx.y) * tile);
+    if (i0 >= nr) return;
+    const int i1 = i0 + tile < nr ? i0 + tile : nr;  // rings [i0, i1)
+    const int j0 = bx * kKvSegW;
+    const int Ls = ns - j0 < kKvSegW ? ns - j0 : kKvSegW;
+    const int j = (j0 - kKvHalo + k + ns) % ns;
+    const bool own = k >= kKvHalo && k < kKvHalo + Ls;  // lanes that write
+    // this wavefront's rows of the ring table: rings i0 - 3 .. i1 + 1
+    const KWalk P{K, lds + (int)threadIdx.y * kv_lds_doubles(tile), i0 >= 3 ? i0 - 3 : 0};
+    {
+        const int last = i1 + 1 <= nr ? i1 + 1 : nr, n = (last - P.row0 + 1) * kRingTabs;
+        const double *src = K.ring_tab + (size_t)P.row0 * kRingTabs;
+        for (int t = k; t < n; t += 64) const_cast<double *>(P.rows)[t] = src[t];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    FLD(vr, FCPT_VRAD);
+    FLD(vaz, FCPT_VAZI);
+    FLD(S, FCPT_SIGMA);
+    FLD(E, FCPT_ENERGY);
+    const Fld<SPLIT> vr_o = alt_vr<SPLIT>(P);
+    const Fld<SPLIT> vaz_o = alt_vaz<SPLIT>(P);
+    const double dt = kick_dt(P);
+    const bool diss = ADI && P.artvisc_dissipation;
+    const bool emul_derived = EMUL && (P.split_emul & SPLIT_EMUL_DERIVED);
+    const bool emul_stages = EMUL && (P.split_emul & SPLIT_EMUL_STAGES);
+    const bool launch_ok = P.const_ok && quot_range(dt);  // the quotients' numerators are in range
+    // one ring of the lane's sector as loaded
+    struct Raw {
+        typename Fld<SPLIT>::T vr, va, s, e;
+        double phi;
+    };
+    auto load = [&](int r) {
+        Raw w;
+        const int c = r < nr ? r : nr - 1;  // ring nr holds only v_r
+        w.vr = vr.raw(r, j);
+        w.va = vaz.raw(c, j);
+        w.s = S.raw(c, j);
+        if constexpr (ADI) w.e = E.raw(c, j);
+        w.phi = phi_fld(P)(c, j);
+        return w;
+    };
+    struct Ring {
+        double vr, va, s, p, phi, e;  // p: pressure, phi: potential
+        double sL, vaR;               // Sigma of sector j - 1, v_phi of sector j + 1
+    };
+    auto ring = [&](int r, const Raw &w) {
+        Ring g;
+        const int c = r < nr ? r : nr - 1;
+        g.vr = vr.dec(r, w.vr);
+        g.va = vaz.dec(c, w.va);
+        g.s = S.dec(c, w.s);
+        if constexpr (ADI) {
+            g.e = E.dec(c, w.e);
+            g.p = (P.gamma - 1.0) * g.e;
+            if (emul_derived) g.p = fld<SPLIT>(P, FCPT_PRESSURE).stored(c, j, g.p);
+        } else {
+            g.e = 0.0;
+            g.p = iso_pressure(P, c, g.s);
+        }
+        g.phi = w.phi;
+        g.sL = from_left(g.s);
+        g.vaR = from_right(g.va);
+        return g;
+    };
+    // the reciprocals of a ring's Sigma sums with ring r - 1 and sector j - 1:
+    // the denominators of the source terms, the artificial viscosity and the
+    // viscous update (whose Sigma_avg is half the sum)
+    struct Rcp {
+        double r, p;
+        bool ok;
+    };
+    // the source-term velocities of ring r (b) from ring r - 1 (a); rows
+    // that are not updated keep their values
+    auto src = [&](int r, const Ring &a, const Ring &b, double &v1r, double &v1a) {
+        const double pjp = from_left(b.p), phijp = from_left(b.phi);
+        const bool upd_p = r >= 1 && r < nr - 1;
+        const bool upd_r = r >= 2 && upd_p;
+        const Den dr = make_den<SPLIT>(b.s + a.s, launch_ok), dp = make_den<SPLIT>(b.s + b.sL, launch_ok);
+        v1a = b.va;
+        v1r = b.vr;
+        if (upd_p) {
+            v1a = src_vphi_by(P, r, dt, b.va, quot_by<SPLIT>(2.0, dp), b.p, pjp, b.phi, phijp);
+            if (emul_stages) v1a = vaz_o.stored(r, j, v1a);
+        }
+        if (upd_r) {
+            v1r = src_vr_by(P, r, dt, b.vr, quot_by<SPLIT>(2.0, dr), b.p, a.p, b.phi, a.phi, b.va, b.vaR, a.va,
+                            a.vaR);
+            if (emul_stages) v1r = vr_o.stored(r, j, v1r);
+        }
+        return Rcp{dr.r, dp.r, dr.ok && dp.ok};
+    };
+    // the tensor of cell (r, j) from the source-term velocities
+    struct Q {
+        TwQ tw;
+        SnQ sn;
+        double qr, qp;
+    };
+    auto qcell = [&](int r, double vr0, double vr1, double va0, double va1, double sig) {
+        Q q;
+        if constexpr (SN) {
+            q.sn = sn_q_cell(P, r, vr0, vr1, va0, va1, sig);
+            q.qr = q.sn.qr;
+            q.qp = q.sn.qp;
+        } else {
+            q.tw = tw_q_cell(P, r, vr0, vr1, va0, va1, sig);
+            q.qr = q.tw.qr;
+            q.qp = q.tw.qp;
+        }
+        return q;
+    };
+    // a ring after the artificial viscosity, as the viscous stage reads it
+    struct Visc {
+        double vr, va, s, n, e, h;
+        Rcp rcp;
+        bool fine;  // its E and Sigma are in range
+    };
+    const int m0 = i0 >= 1 ? i0 - 1 : 0;  // the first ring of the artificial viscosity
+    Ring R0;                              // ring m
+    double v1r0, v1a0;                    // its source-term velocities
+    Rcp rcp0;
+    double qr_m = 0.0, qp_m = 0.0, s_m = 0.0;  // tensor and Sigma of cell (m - 1, j)
+    Raw X;                                // ring m + 1, in flight
+    {
+        const Raw x2 = load(m0 >= 2 ? m0 - 2 : 0), x1 = load(m0 >= 1 ? m0 - 1 : 0), x0 = load(m0);
+        X = load(m0 + 1);
+        const Ring Rm2 = ring(m0 >= 2 ? m0 - 2 : 0, x2);  // read by rings m0 - 1 >= 2 only
+        const Ring Rm = ring(m0 >= 1 ? m0 - 1 : 0, x1);
+        R0 = ring(m0, x0);
+        rcp0 = src(m0, Rm, R0, v1r0, v1a0);  // ring 0 is passed through
+        if (m0 >= 1) {
+            double v1rm, v1am;
+            src(m0 - 1, Rm2, Rm, v1rm, v1am);
+            const Q qm = qcell(m0 - 1, v1rm, v1r0, v1am, from_right(v1am), Rm.s);
+            qr_m = qm.qr;
+            qp_m = qm.qp;
+            s_m = Rm.s;
+        }
+    }
+    Visc A{};                              // ring m - 1
+    StressDiag dprev{0.0, 0.0, 0.0};       // its predecessor's diagonal
+    double trp_c = 0.0, s_prev = 0.0;      // tau_rp(m - 1, j), Sigma(m - 2, j)
+    for (int m = m0; m <= i1; ++m) {
+        // the artificial viscosity at ring m (ring nr holds only v_r)
+        Visc B;
+        if (m < nr) {
+            const Ring R1 = ring(m + 1, X);
+            if (m < i1) X = load(m + 2 <= nr ? m + 2 : nr);  // before this ring's stores
+            double v1r1, v1a1;
+            const Rcp rcp1 = src(m + 1, R0, R1, v1r1, v1a1);
+            const double v1aR = from_right(v1a0);  // v_phi of sector j + 1
+            const Q q = qcell(m, v1r0, v1r1, v1a0, v1aR, R0.s);
+            const double qpj = from_left(q.qp);  // tensor of cell (m, j - 1)
+            const bool inner = m >= 1 && m < nr - 1;
+            const bool radial = m >= 2 && inner;
+            B.s = R0.s;
+            if constexpr (ADI) {
+                // compression_heating (rings 0 .. nr-2), then the dissipation
+                double e = R0.e;
+                if (m < nr - 1) e = E.stored(m, j, src_energy_new(P, m, dt, e, v1r0, v1r1, v1a0, v1aR));
+                const bool s_ok = launch_ok && quot_range(R0.s);
+                if (diss) {
+                    if constexpr (SN) e = sn_heat(P, m, q.sn, dt, e);
+                    else e = tw_heat(P, m, q.tw, R0.s, dt, e);
+                    // the limits are FP64 quotients in both storage modes
+                    e = E.stored(m, j, temperature_floor_in<false>(P, m, e, R0.s, s_ok));
+                } else if (!emul_stages && m < nr - 1) {
+                    e = E.stored(m, j, e);
+                }
+                // recalculate_viscosity
+                B.fine = s_ok && quot_range(e);
+                const AdiDerived d = adi_derived_in<SPLIT>(P, m, e, R0.s, B.fine);
+                B.e = e;
+                B.h = emul_derived ? fld<SPLIT>(P, FCPT_SCALE_HEIGHT).stored(m, j, d.h) : d.h;
+                B.n = fld<SPLIT>(P, FCPT_VISCOSITY).stored(m, j, d.nu);
+                // the second kick of a LeapFrog step smooths its potential with this H
+                if (P.integrator == FCPT_INTEGRATOR_LEAPFROG && own && m >= i0 && m < i1)
+                    fld<SPLIT>(P, FCPT_SCALE_HEIGHT).set(m, j, d.h);
+            } else {
+                B.e = B.h = 0.0;
+                B.n = cst(P.iso_nu)[m];
+                B.fine = false;
+            }
+            B.rcp = rcp0;
+            B.va = v1a0;
+            if (inner) {
+                if constexpr (SN) {
+                    B.va = sn_vphi_by(P, m, v1a0, quot_by<SPLIT>(dt * 2.0, Den{R0.s + R0.sL, rcp0.p, rcp0.ok}), q.qp, qpj);
+                } else {
+                    const Den D = make_den<SPLIT>(ring_tab(P, TAB_RSUP_RINF, m) * (0.5 * (R0.s + R0.sL)), rcp0.ok);
+                    B.va = tw_vphi_by(P, v1a0, quot_by<SPLIT>(2.0 * dt, D), q.qp, qpj);
+                }
+                B.va = vaz_o.stored(m, j, B.va);
+            }
+            B.vr = v1r0;
+            if (radial) {
+                const Den D{R0.s + s_m, rcp0.r, rcp0.ok};
+                if constexpr (SN) {
+                    B.vr = sn_vr_by(P, m, v1r0, quot_by<SPLIT>(dt * 2.0, D), q.qr, qr_m);
+                } else {
+                    const Den R2{ring_tab(P, TAB_RMED_SQ_DIFF, m), ring_tab(P, TAB_RMED_SQ_DIFF_RCP, m), rcp0.ok};
+                    const double c = quot_by<SPLIT>(2.0 * (P.radial_viscosity_factor * dt), D) * 2.0;
+                    B.vr = tw_vr_by(P, m, v1r0, quot_by<SPLIT>(c, R2), q.qr, qr_m, q.qp, qp_m);
+                }
+                B.vr = vr_o.stored(m, j, B.vr);
+            }
+            qr_m = q.qr;
+            qp_m = q.qp;
+            s_m = R0.s;
+            R0 = R1;
+            v1r0 = v1r1;
+            v1a0 = v1a1;
+            rcp0 = rcp1;
+        } else {
+            B = Visc{R0.vr, 0.0, 0.0, 0.0, 0.0, 0.0, {0.0, 0.0, false}, false};
+        }
+        // the viscous stage at ring i = m - 1 (A), from rings i and i + 1 (B)
+        const int i = m - 1;
+        if (i >= m0) {
+            const StressDiag d = stress_diag(P, i, A.vr, B.vr, A.va, from_right(A.va), A.n, A.s);
+            double trp1 = 0.0;  // tau_rp at corner (i + 1, j)
+            if (m <= nr - 1) {
+                const double nB = ADI ? from_left(B.n) : B.n, nA = ADI ? from_left(A.n) : A.n;
+                trp1 = stress_rp(P, m, B.va, A.va, B.vr, from_left(B.vr), B.n, A.n, nB, nA, B.s, A.s,
+                                 from_left(B.s), from_left(A.s));
+            }
+            const bool upd_p = i >= 1 && i < nr - 1;
+            const bool upd_r = i >= 2 && upd_p;
+            const double tppj = from_left(d.tpp);    // diagonal of (i, j - 1)
+            const double trp_n = from_right(trp_c);  // corner (i, j + 1)
+            double qplus = 0.0, qminus = 0.0;
+            if constexpr (ADI) {
+                if (upd_p) {
+                    qminus = cooling_beta_cell<SPLIT>(P, i, j, kick_time(P), A.e, A.s);
+                    if (P.heating_viscous) {
+                        double trr = d.trr, tpp = d.tpp, dv = d.divv, c0 = trp_c, c1 = trp1;
+                        if (emul_stages) {
+                            trr = fld<SPLIT>(P, FCPT_TAU_R_R).stored(i, j, trr);
+                            tpp = fld<SPLIT>(P, FCPT_TAU_PHI_PHI).stored(i, j, tpp);
+                            dv = fld<SPLIT>(P, FCPT_DIV_V).stored(i, j, dv);
+                            c0 = fld<SPLIT>(P, FCPT_TAU_R_PHI).stored(i, j, c0);
+                            c1 = fld<SPLIT>(P, FCPT_TAU_R_PHI).stored(m, j, c1);
+                        }
+                        const double c0n = emul_stages ? from_right(c0) : trp_n;
+                        const double c1n = from_right(c1);  // corner (i + 1, j + 1)
+                        if (A.n != 0.0)
+                            qplus = viscous_heating_q<SPLIT>(P, A.n, A.s, trr, tpp, dv, 0.25 * (c0 + c1 + c0n + c1n),
+                                                             A.fine);
+                    }
+                }
+            }
+            const double sAL = from_left(A.s);
+            if (own && i >= i0) {
+                if (upd_p) {
+                    const Den D{A.s + sAL, A.rcp.p, A.rcp.ok};
+                    const double inv = quot_by<SPLIT>(2.0 * (dt * ring_tab(P, TAB_INV_RMED, i)), D);
+                    vaz_o.set(i, j, visc_vphi_by(P, i, A.va, inv, trp_c, trp1, d.tpp, tppj));
+                }
+                if (upd_r) {
+                    const Den D{A.s + s_prev, A.rcp.r, A.rcp.ok};
+                    const Den R{ring_tab(P, TAB_RMED_SUM, i), ring_tab(P, TAB_RMED_SUM_RCP, i), A.rcp.ok};
+                    const double c = quot_by<SPLIT>(quot_by<SPLIT>(2.0 * dt, D) * P.radial_viscosity_factor * 2.0, R);
+                    vr_o.set(i, j, visc_vr_by(P, i, A.vr, c, d.trr, dprev.trr, trp_c, trp_n, d.tpp, dprev.tpp));
+                }
+                if constexpr (ADI) {
+                    const Fld<SPLIT> Eo = buf<SPLIT>(P, P.ealt, P.bg[FCPT_ENERGY], FCPT_ENERGY);
+                    substep3_cell<SPLIT>(P, Eo, i, j, A.e, A.s, A.h, qplus, qminus, A.fine);
+                }
+            }
+            dprev = d;
+            trp_c = trp1;
+            s_prev = A.s;
+        }
+        A = B;
+    }
+    // the rows that are not updated, copied as stored (here and not in the
+    // loop: a load there would make every ring wait for its prefetch)
+    if (!own) return;
+    if (i0 == 0) {
+        vr_o.set_raw(0, j, vr.raw(0, j));
+        vaz_o.set_raw(0, j, vaz.raw(0, j));
+    }
+    if (i0 <= 1 && i1 > 1) vr_o.set_raw(1, j, vr.raw(1, j));
+    if (i1 == nr) {
+        vr_o.set_raw(nr - 1, j, vr.raw(nr - 1, j));
+        vaz_o.set_raw(nr - 1, j, vaz.raw(nr - 1, j));
+        vr_o.set_raw(nr, j, vr.raw(nr, j));
+    }
+}
+template <bool SPLIT, bool ADI, bool SN, bool EMUL>
+__global__ void __launch_bounds__(64, ADI ? 3 : 4) k_kv_walk(KParams P, int tile)
+{
+    const BlockXY bb = xcd_block();
+    b_kv_walk<SPLIT, ADI, SN, EMUL>(P, bb.x, bb.y, tile, kv_lds);
+}
+// batched form: each disk's tile is its kv_tile
+template <bool SPLIT, bool ADI, bool SN>
+__global__ void __launch_bounds__(256) kb_kv_walk(const KParams *Ps, const BatchEntry *map)
+{
+    const BatchEntry e = batch_entry(map);
+    const KParams &P = batch_disk(Ps, e.disk);
+    b_kv_walk<SPLIT, ADI, SN, SPLIT>(P, (int)(e.yx & 0xffffu), (int)(e.yx >> 16), P.kv_tile, kv_lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -3530,6 +3918,10 @@ KParams swapped_view(const KParams &P)
     Q.valt[0] = P.f[FCPT_VRAD];
     Q.f[FCPT_VAZI] = P.valt[1];
     Q.valt[1] = P.f[FCPT_VAZI];
+    if (P.lazy_derived && P.adiabatic) {  // the kick walk writes E to its partner too
+        Q.f[FCPT_ENERGY] = P.ealt;
+        Q.ealt = P.f[FCPT_ENERGY];
+    }
     return Q;
 }
 
@@ -3588,48 +3980,112 @@ void launch_visc_energy(const KParams &P, hipStream_t st)
     }
 }
 
-// rings per thread of the kick walk: 8, or 4, while that gives 3072
-// wavefronts, else 1 (the separate passes)
-static int kick_tile(const KParams &P)
+// Split storage's rounding points.  A disk large enough for 3072 wavefronts
+// of ring walks hands the source-term velocities on in FP64; a smaller one
+// rounds them, the viscous heating's tensor and the derived fields to their
+// stored form, as the separate passes store them.
+static bool walk_rounding(const KParams &P)
 {
-    if (P.kick_tile > 0) return P.kick_tile;
-    const long segs = (P.ns + kKickSegW - 1) / kKickSegW;
-    int tile = 8;
-    while (tile > 1 && segs * ((P.nr + tile - 1) / tile) < 3072) tile = tile > 4 ? tile / 2 : 1;
-    return tile;
+    auto tile = [&](int set, int seg) {
+        if (set > 0) return set;
+        const long segs = (P.ns + seg - 1) / seg;
+        int t = 8;
+        while (t > 1 && segs * ((P.nr + t - 1) / t) < 3072) t = t > 4 ? t / 2 : 1;
+        return t;
+    };
+    return tile(P.kick_tile, 60) > 1 && tile(P.visc_tile, 62) > 1;
 }
 
-int resolve_kick_tile(const KParams &P) { return kick_tile(P); }
-int resolve_visc_tile(const KParams &P) { return visc_tile(P); }
-long walk_waves(const KParams &P, int tile)
+bool kv_walk_applies(const KParams &P)
 {
-    const long rings = (P.nr + tile - 1) / tile;
-    return rings * ((P.ns + kKickSegW - 1) / kKickSegW + (P.ns + kViscSegW - 1) / kViscSegW) / 2;
+    return (P.artvisc == FCPT_ARTVISC_TW || P.artvisc == FCPT_ARTVISC_SN) && P.kick_tile != 1 && P.visc_tile != 1;
 }
 
-bool kick_walk_applies(const KParams &P)
+void set_step_modes(KParams &P, bool fused)
 {
-    return (P.artvisc == FCPT_ARTVISC_TW || P.artvisc == FCPT_ARTVISC_SN) && kick_tile(P) > 1 &&
-           visc_tile(P) > 1;
+    P.lazy_derived = fused && kv_walk_applies(P) ? 1 : 0;
+    P.split_emul = 0;
+    if (P.split && P.lazy_derived) {
+        const bool walk = walk_rounding(P);
+        if (!walk || P.integrator == FCPT_INTEGRATOR_LEAPFROG) P.split_emul |= SPLIT_EMUL_DERIVED;
+        if (!walk) P.split_emul |= SPLIT_EMUL_STAGES;
+    }
 }
+
+// Rings per thread of the kick walk: a walk of t rings costs about t + 3.5
+// (its window start), and the device holds `slots` of them at once, so the
+// tile with the fewest rounds of walks times their length.
+template <class Waves>
+static int kv_best_tile(Waves &&waves, long slots)
+{
+    int best = 1;
+    double best_cost = 1e300;
+    for (int t = 1; t <= 24; ++t) {
+        const double rounds = (double)waves(t) / (double)slots;
+        const double cost = (t + 3.5) * (rounds <= 3.0 ? std::ceil(rounds) : rounds + 0.5);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = t;
+        }
+    }
+    return best;
+}
+// walks resident at once: 3 wavefronts per SIMD of an adiabatic walk's
+// registers, 4 of an isothermal one's
+static long kv_slots(const KParams &P) { return P.adiabatic ? 3072 : 4096; }
+static int kv_tile(const KParams &P)
+{
+    if (P.kick_tile > 1) return P.kick_tile;
+    if (P.visc_tile > 1) return P.visc_tile;
+    return kv_best_tile([&](int t) { return kv_waves(P, t); }, kv_slots(P));
+}
+void resolve_kv_tiles(std::vector<KParams> &D)
+{
+    const KParams *any = nullptr;
+    for (const KParams &P : D)
+        if (kv_walk_applies(P)) any = &P;
+    if (!any) return;
+    const int t = kv_best_tile(
+        [&](int tile) {
+            long w = 0;
+            for (const KParams &P : D)
+                if (kv_walk_applies(P)) w += kv_waves(P, tile);
+            return w;
+        },
+        kv_slots(*any));
+    for (KParams &P : D)
+        if (kv_walk_applies(P)) P.kv_tile = P.kick_tile > 1 ? P.kick_tile : P.visc_tile > 1 ? P.visc_tile : t;
+}
+long kv_waves(const KParams &P, int tile)
+{
+    return (long)((P.ns + kKvSegW - 1) / kKvSegW) * ((P.nr + tile - 1) / tile);
+}
+
+int resolve_kick_tile(const KParams &P) { return kv_walk_applies(P) ? kv_tile(P) : 1; }
+int resolve_visc_tile(const KParams &P) { return kv_walk_applies(P) ? kv_tile(P) : visc_tile(P); }
+bool walks_tunable(const KParams &P) { return kv_walk_applies(P) && (!P.split || walk_rounding(P)); }
 
 void launch_kick(const KParams &P, hipStream_t st, int fold_mode)
 {
-    const int tile = kick_tile(P);
-    const int tiles = (P.nr + tile - 1) / tile;
-    const dim3 g((unsigned)((P.ns + kKickSegW - 1) / kKickSegW), (unsigned)((tiles + 3) / 4));
+    const int tile = kv_tile(P);
+    // one wavefront per block: with four, a block's registers and LDS stay
+    // taken until its last wavefront ends (1024 x 3072 adiabatic step 406 us
+    // with four, 370 with one)
+    const dim3 g((unsigned)((P.ns + kKvSegW - 1) / kKvSegW), (unsigned)((P.nr + tile - 1) / tile)), b(64);
+    const size_t lds = kv_lds_doubles(tile) * sizeof(double);
     launch_potential_fold(P, st, fold_mode);
-    const int v = (P.split ? 4 : 0) + (P.adiabatic ? 2 : 0) + (P.artvisc == FCPT_ARTVISC_SN ? 1 : 0);
-    switch (v) {
-    case 0: hipLaunchKernelGGL((k_kick_walk<false, false, false>), g, kBlock, 0, st, P, tile); break;
-    case 1: hipLaunchKernelGGL((k_kick_walk<false, false, true>), g, kBlock, 0, st, P, tile); break;
-    case 2: hipLaunchKernelGGL((k_kick_walk<false, true, false>), g, kBlock, 0, st, P, tile); break;
-    case 3: hipLaunchKernelGGL((k_kick_walk<false, true, true>), g, kBlock, 0, st, P, tile); break;
-    case 4: hipLaunchKernelGGL((k_kick_walk<true, false, false>), g, kBlock, 0, st, P, tile); break;
-    case 5: hipLaunchKernelGGL((k_kick_walk<true, false, true>), g, kBlock, 0, st, P, tile); break;
-    case 6: hipLaunchKernelGGL((k_kick_walk<true, true, false>), g, kBlock, 0, st, P, tile); break;
-    default: hipLaunchKernelGGL((k_kick_walk<true, true, true>), g, kBlock, 0, st, P, tile); break;
-    }
+#define KV(SP, EM)                                                                                        \
+    do {                                                                                                  \
+        const bool sn = P.artvisc == FCPT_ARTVISC_SN;                                                     \
+        if (P.adiabatic && sn) hipLaunchKernelGGL((k_kv_walk<SP, true, true, EM>), g, b, lds, st, P, tile);   \
+        else if (P.adiabatic) hipLaunchKernelGGL((k_kv_walk<SP, true, false, EM>), g, b, lds, st, P, tile);   \
+        else if (sn) hipLaunchKernelGGL((k_kv_walk<SP, false, true, EM>), g, b, lds, st, P, tile);            \
+        else hipLaunchKernelGGL((k_kv_walk<SP, false, false, EM>), g, b, lds, st, P, tile);                   \
+    } while (0)
+    if (!P.split) KV(false, false);
+    else if (P.split_emul) KV(true, true);
+    else KV(true, false);
+#undef KV
 }
 
 void launch_derived(const KParams &P, hipStream_t st) { LAUNCH(k_derived, cell_grid(P, P.nr), kBlock, st, P); }
@@ -3908,22 +4364,25 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
     stage(B_POTENTIAL, 0, all, [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         add_grid(v, d, (unsigned)((P.ns + 64 * kPotCells - 1) / (64 * kPotCells)), rows_grid(P, P.nr));
     });
-    // the kick: the two walks where the disk's own launch uses them
-    // (kick_walk_applies with the tiles resolved at batch creation), else the
-    // cell-parallel fused passes; each pass flips the disk's view
+    // the kick: the walk where the disk's own launch uses it (its tile in
+    // kv_tile), else the cell-parallel fused passes; each pass flips the
+    // disk's view
     auto flip = [&](int kind, int arg, auto pred, auto grid) { stage_v(kind, arg, pred, grid, true, false); };
-    auto walk = [](const KParams &P) { return kick_walk_applies(P); };
+    auto walk = [](const KParams &P) { return kv_walk_applies(P); };
     auto kick_grid = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
-        const int tiles = (P.nr + P.kick_tile - 1) / P.kick_tile;
-        add_grid(v, d, (unsigned)((P.ns + kKickSegW - 1) / kKickSegW), (unsigned)((tiles + 3) / 4));
+        const int tiles = (P.nr + P.kv_tile - 1) / P.kv_tile;
+        add_grid(v, d, (unsigned)((P.ns + kKvSegW - 1) / kKvSegW), (unsigned)((tiles + 3) / 4));
     };
     auto visc_grid = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         const int tiles = (P.nr + P.visc_tile - 1) / P.visc_tile;
         add_grid(v, d, (unsigned)((P.ns + kViscSegW - 1) / kViscSegW), (unsigned)((tiles + 3) / 4));
     };
+    int kv_most = 1;  // the longest walk, which sizes the launch's LDS
+    for (const KParams &P : D)
+        if (walk(P)) kv_most = std::max(kv_most, P.kv_tile);
     for (int a = 0; a < 2; ++a)
         for (int sn = 0; sn < 2; ++sn)
-            flip(B_KICK_WALK, 2 * a + sn,
+            flip(B_KV_WALK, 2 * a + sn + 4 * kv_most,
                  [&](const KParams &P) {
                      return walk(P) && P.adiabatic == a && (P.artvisc == FCPT_ARTVISC_SN) == (sn != 0);
                  },
@@ -3944,11 +4403,11 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
     stage(B_RECALC_VISC, 0, none, rows(0));
     // the viscous pass: the walk (with SubStep3 when adiabatic) where the
     // disk's tile is above 1, as launch_visc_fused / launch_visc_energy
-    auto vwalk = [](const KParams &P) { return P.visc_tile > 1; };
+    auto vwalk = [&](const KParams &P) { return cell(P) && P.visc_tile > 1; };
     for (int a = 0; a < 2; ++a)
         flip(B_VISC_WALK, a, [&](const KParams &P) { return vwalk(P) && P.adiabatic == a; }, visc_grid);
-    flip(B_VISC_FUSED, 0, [&](const KParams &P) { return !vwalk(P); }, rows(-1));
-    stage(B_SUBSTEP3, 0, [&](const KParams &P) { return !vwalk(P) && P.adiabatic; }, rows(0));
+    flip(B_VISC_FUSED, 0, [&](const KParams &P) { return cell(P) && !vwalk(P); }, rows(-1));
+    stage(B_SUBSTEP3, 0, [&](const KParams &P) { return cell(P) && !vwalk(P) && P.adiabatic; }, rows(0));
     // the boundary call before the transport with the FARGO ring means
     stage(B_GHOST_MEAN, 0, all, [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         add_grid(v, d, (unsigned)((P.ns + 255) / 256 + P.nr), 1);
@@ -4010,10 +4469,11 @@ void launch_batch_stage(const KParams *Ps, const BatchStageDev &S, int split, in
         break;
     case B_GHOST_MEAN: LAUNCHB(kb_ghost_ring_mean, b256); break;
     case B_VEL_FINAL: LAUNCHB(kb_velocities_final, kBlock, S.arg); break;
-    case B_KICK_WALK: {
+    case B_KV_WALK: {
         const dim3 g(S.n);
-#define KWB(SP, AD, SN)                                                                            hipLaunchKernelGGL((kb_kick_walk<SP, AD, SN>), g, kBlock, 0, st, Ps, S.map)
-        const int v = (split ? 4 : 0) + S.arg;
+#define KWB(SP, AD, SN)                                                                            hipLaunchKernelGGL((kb_kv_walk<SP, AD, SN>), g, kBlock, lds, st, Ps, S.map)
+        const int v = (split ? 4 : 0) + (S.arg & 3);
+        const size_t lds = 4 * kv_lds_doubles(S.arg >> 2) * sizeof(double);
         if (v == 0) KWB(false, false, false);
         else if (v == 1) KWB(false, false, true);
         else if (v == 2) KWB(false, true, false);

@@ -51,17 +51,21 @@ void launch_visc_fused(const KParams &P, hipStream_t st);
 // the fused viscous pass followed by SubStep3 (adiabatic disks); one walk
 // that does not store the stress tensor where the grid is large enough
 void launch_visc_energy(const KParams &P, hipStream_t st);
-// the kick's potential pass, then its source terms and artificial viscosity as
-// one walk (TW or SN artificial viscosity on a grid large enough for it),
-// velocities to the view's partner buffers; then launch_visc_energy
-// (adiabatic) or launch_visc_fused on the swapped view
-bool kick_walk_applies(const KParams &P);
+// the kick's potential pass, then the whole kick as one walk (TW or SN
+// artificial viscosity), results in the swapped view
+bool kv_walk_applies(const KParams &P);
+// how the step runs: lazy_derived and split_emul
+void set_step_modes(KParams &P, bool fused);
 // the rings per thread the walks use for this disk (1: the cell-parallel form)
 int resolve_kick_tile(const KParams &P);
 int resolve_visc_tile(const KParams &P);
-// wavefronts of one kick-walk or viscous-walk launch of a disk at `tile`
-// rings per thread (the mean of the two walks' segment counts)
-long walk_waves(const KParams &P, int tile);
+// whether the walk's tile may be set without changing results
+bool walks_tunable(const KParams &P);
+// wavefronts of one kick-walk launch of a disk at `tile` rings per thread
+long kv_waves(const KParams &P, int tile);
+// a batch: kv_tile of every member that runs the kick walk (its own, or the
+// one chosen over the batch's wavefronts)
+void resolve_kv_tiles(std::vector<KParams> &disks);
 void launch_kick(const KParams &P, hipStream_t st, int fold_mode);
 // the potential; fold_mode >= 0: in the same launch, the CFL fold of
 // k_cfl_rings' slots (launch_cfl_cells) with that mode
@@ -115,7 +119,7 @@ enum BatchKind {
     B_SRC_ENERGY, B_TW_Q, B_TW_VEL, B_SN_Q, B_SN_VEL, B_TEMP_FLOOR, B_RECALC_VISC, B_STRESS,
     B_VISC_UPDATE, B_SUBSTEP3, B_GHOST, B_RADIAL_ISO, B_RADIAL_ADI, B_AZIM_ISO, B_AZIM_ADI,
     B_VELOCITIES, B_DAMPING, B_DERIVED, B_SRC_FUSED, B_AV_FUSED, B_VISC_FUSED, B_FINAL_DERIVED,
-    B_CFL_RINGS, B_CFL_FINAL_RINGS, B_KICK_WALK, B_VISC_WALK, B_GHOST_MEAN, B_VEL_FINAL
+    B_CFL_RINGS, B_CFL_FINAL_RINGS, B_KV_WALK, B_VISC_WALK, B_GHOST_MEAN, B_VEL_FINAL
 };
 struct BatchStageHost {
     int kind, arg;

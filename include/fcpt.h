@@ -289,15 +289,18 @@ int fcpt_time_copy(fcpt_ctx *ctx, int32_t reps, double *ms_per_launch, double *b
                             (1 .. 64; 0 restores the size-based default);
    FCPT_PARAM_RADIAL_WAVES  the sweep's register budget in wavefronts per
                             SIMD (2 or 3; default 3);
-   FCPT_PARAM_VISC_TILE     rings walked by one thread of the fused viscous
-                            pass (1 .. 64, where 1 is the cell-parallel form;
-                            0 restores the size-based default);
    FCPT_PARAM_KICK_TILE     rings walked by one thread of the kick walk, which
-                            runs the source terms and the artificial
-                            viscosity of the fused step as one pass (1 .. 64,
-                            where 1 runs them as separate passes; 0 restores
-                            the size-based default; the walk needs the TW or
-                            SN artificial viscosity and a viscous tile above 1).
+                            runs the source terms, the artificial viscosity,
+                            the viscous update and SubStep3 of the fused step
+                            as one pass (1 .. 64, where 1 runs them as separate
+                            passes; 0 restores the size-based default; the
+                            walk needs the TW or SN artificial viscosity and
+                            a viscous tile other than 1);
+   FCPT_PARAM_VISC_TILE     the kick walk's tile where FCPT_PARAM_KICK_TILE is 0;
+                            where the kick walk does not run, rings walked by
+                            one thread of the fused viscous pass (1 .. 64, where
+                            1 is the cell-parallel form; 0 restores the
+                            size-based default).
    FCPT_PARAM_FUSED_STEP (default 1) makes fcpt_step_euler, fcpt_step_leapfrog,
    fcpt_run_step and fcpt_run_steps run the fused passes (the walks above,
    the ghost rings with the FARGO ring means, and for Euler the final
@@ -307,7 +310,11 @@ int fcpt_time_copy(fcpt_ctx *ctx, int32_t reps, double *ms_per_launch, double *b
    leave Q_R, Q_PHI, TAU_* and DIV_V unspecified (as they were, or, for an
    adiabatic disk with viscous heating on a grid below the walks' size, the
    step's tensor); 0 runs the separate kernels of the per-function entry
-   points above, which always store them.  Every parameter change drops a
+   points above, which always store them.  The derived fields a fused step
+   needs are formed from E and Sigma; a step that follows a field or stage of
+   the caller's own (fcpt_upload_field of Sigma, E or a derived field, or a
+   stage entry point that changes them) reads the fields as stored, through
+   the separate kernels.  Every parameter change drops a
    captured step graph so that the next fcpt_run_steps captures the new
    shape. */
 /* FCPT_PARAM_SPLIT_ROUNDING (split storage only; default 1) chooses how a
@@ -349,8 +356,9 @@ int fcpt_rebase_backgrounds(fcpt_ctx *ctx);
    the timed kernels write transport scratch only), keeps the fastest and
    returns it.  Drops a captured step graph. */
 int fcpt_autotune(fcpt_ctx *ctx, int32_t reps, int32_t *radial_tile, int32_t *radial_waves);
-/* Autotuner of the fused step's walks (no counterpart in the reference): the
-   kick walk's and the viscous walk's tiles (2 .. 16 rings) by the time of
+/* Autotuner of the fused step's walk (no counterpart in the reference): the
+   kick walk's tile, or the viscous walk's in a disk without artificial
+   viscosity (2 .. 32 rings), by the time of
    `reps` whole graph-replayed iterations each, every trial from the same
    state, which the call saves first and puts back (fields and clock as they
    were); keeps the fastest and returns the tiles.  A context whose step does
