@@ -5,12 +5,15 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -59,6 +62,9 @@ struct fcpt_ctx {
     int rebase_interval = 0;
     int steps_since_rebase = 0;
 };
+
+static void host_slots_join();
+static void host_slots_leave();
 
 namespace {
 
@@ -300,10 +306,12 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
     for (int i = 0; i + 1 < desc->nr + 2; ++i)
         if (!(desc->radii[i + 1] > desc->radii[i]) || !(desc->radii[i] > 0.0)) return FCPT_ERR_ARG;
     fcpt_ctx *c = new fcpt_ctx();
+    host_slots_join();
     c->desc = *desc;
     c->desc.radii = nullptr;
     hipError_t e = hipGetDevice(&c->device);
     if (e != hipSuccess) {
+        host_slots_leave();
         delete c;
         return FCPT_ERR_DEVICE;
     }
@@ -382,6 +390,7 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
         ids[3] = clampi(rinf_id_log(*desc, desc->rmax * desc->damping_outer_limit) + 1, nr);
     memcpy(P.damp_ids, ids, sizeof(ids));
     if (desc->damping && (ids[0] >= ids[2] || ids[1] >= ids[3])) {
+        host_slots_leave();
         delete c;
         return FCPT_ERR_ARG;  // inner and outer damping zones overlap
     }
@@ -525,6 +534,7 @@ int fcpt_destroy(fcpt_ctx *ctx)
     if (ctx->s_host) hipHostFree(ctx->s_host);
     if (ctx->totals_host) hipHostFree(ctx->totals_host);
     if (ctx->force_host) hipHostFree(ctx->force_host);
+    host_slots_leave();
     delete ctx;
     return FCPT_OK;
 }
@@ -584,20 +594,256 @@ static int upload_split(fcpt_ctx *ctx, int field, const double *host)
     return FCPT_OK;
 }
 
-static int download_split(fcpt_ctx *ctx, int field, double *host)
+// ---- fields to the host ----------------------------------------------------
+// A copy into the caller's pageable arrays is bound by the host: its pages are
+// touched for the first time (the kernel clears them) and written by one
+// thread, 1.6 GB in 158 ms where the link takes 30.  So the bytes go through
+// pinned slots, in pieces: the link fills a slot while kCopyThreads threads
+// move earlier ones to the caller (and decode split storage's FP32 deviations
+// there, so half the bytes cross the link): 37 ms, and 21 for split storage
+// instead of 292.  What fits the slots as a whole is decoded and written to
+// them by one kernel, all fields at once: each transfer and its event cost
+// tens of microseconds, more than the link's time below some MB (128 x 384:
+// 530 -> 70 us, 32 x 64: 80 -> 21 us; slots filled in smaller pieces were
+// slower than in one).
+//
+// The slots belong to the process (a disk's own would cost each disk their
+// pinning, ~10 ms): allocated by the first copy that needs them, leased to one
+// copy at a time, freed with the last context.
+constexpr size_t kSlotBytes = size_t(4) << 20;
+constexpr int kSlots = 12, kCopyThreads = 8;
+constexpr size_t kSmallBytes = size_t(1) << 20;  // copies up to this size have a buffer of their own
+
+struct HostSlots {
+    std::mutex life, lease;  // life: users and the allocations' existence
+    int users = 0;
+    char *small = nullptr, *slots = nullptr;
+};
+static HostSlots &host_slots()
 {
-    const int ns = ctx->P.ns;
-    const size_t rows = field_rows(field, ctx->P.nr);
-    std::vector<double> bg(rows);
-    std::vector<float> d(rows * ns);
-    HIP_TRY(ctx, hipMemcpyAsync(bg.data(), ctx->P.bg[field], rows * sizeof(double),
-                                hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(ctx, hipMemcpyAsync(d.data(), ctx->P.f[field], d.size() * sizeof(float),
-                                hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    for (size_t i = 0; i < rows; ++i)
-        for (int j = 0; j < ns; ++j) host[i * ns + j] = bg[i] + (double)d[i * ns + j];
+    static HostSlots *h = new HostSlots;  // outlives contexts that a program destroys at its end
+    return *h;
+}
+static void host_slots_join()
+{
+    std::lock_guard<std::mutex> g(host_slots().life);
+    ++host_slots().users;
+}
+static void host_slots_leave()
+{
+    HostSlots &h = host_slots();
+    std::lock_guard<std::mutex> g(h.life);
+    if (--h.users > 0) return;
+    if (h.small) hipHostFree(h.small);
+    if (h.slots) hipHostFree(h.slots);
+    h.small = h.slots = nullptr;
+}
+// (the caller holds the lease)
+static hipError_t host_slots_get(bool large, char **out)
+{
+    HostSlots &h = host_slots();
+    std::lock_guard<std::mutex> g(h.life);
+    char *&p = large ? h.slots : h.small;
+    if (!p) {
+        const hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&p), large ? kSlotBytes * kSlots : kSmallBytes,
+                                           hipHostMallocPortable);
+        if (e != hipSuccess) {
+            p = nullptr;
+            return e;
+        }
+    }
+    *out = p;
+    return hipSuccess;
+}
+
+struct HostCopy {
+    int field;
+    double *dst;
+};
+
+// one piece of a copy: n elements of fields[which] from element `first` on
+struct CopyPiece {
+    int which;
+    size_t first, n;
+};
+
+static int copy_large(fcpt_ctx *ctx, const std::vector<HostCopy> &fields)
+{
+    const KParams &P = ctx->P;
+    const size_t ns = (size_t)P.ns;
+    char *slots = nullptr;
+    HIP_TRY(ctx, host_slots_get(true, &slots));
+    std::vector<CopyPiece> pieces;
+    std::vector<std::vector<double>> bg(fields.size());
+    for (size_t k = 0; k < fields.size(); ++k) {
+        const int f = fields[k].field;
+        const size_t total = field_rows(f, P.nr) * ns, most = kSlotBytes / field_element_size(P, f);
+        for (size_t a = 0; a < total; a += most) pieces.push_back({(int)k, a, std::min(most, total - a)});
+        if (P.split && f != FCPT_POTENTIAL) {
+            bg[k].resize(field_rows(f, P.nr));
+            HIP_TRY(ctx, hipMemcpyAsync(bg[k].data(), P.bg[f], bg[k].size() * sizeof(double), hipMemcpyDeviceToHost,
+                                        ctx->stream));
+        }
+    }
+    hipEvent_t ev[kSlots] = {};
+    hipError_t err = hipSuccess;
+    for (int k = 0; k < kSlots && err == hipSuccess; ++k) err = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+    if (err == hipSuccess) err = hipStreamSynchronize(ctx->stream);  // the backgrounds
+    std::mutex m;
+    std::condition_variable cv;
+    size_t issued = 0, next = 0;
+    std::vector<char> done(pieces.size(), 0);
+    bool stop = err != hipSuccess;
+    // moves piece c, whose transfer has been issued, out of its slot
+    auto move_out = [&](size_t c) -> hipError_t {
+        const hipError_t e = hipEventSynchronize(ev[c % kSlots]);
+        if (e != hipSuccess) return e;
+        const CopyPiece &p = pieces[c];
+        const char *src = slots + (c % kSlots) * kSlotBytes;
+        double *dst = fields[(size_t)p.which].dst + p.first;
+        if (bg[(size_t)p.which].empty()) {
+            std::memcpy(dst, src, p.n * sizeof(double));
+            return hipSuccess;
+        }
+        const float *d = reinterpret_cast<const float *>(src);
+        const double *b = bg[(size_t)p.which].data();
+        for (size_t a = 0; a < p.n;) {
+            const size_t row = (p.first + a) / ns, end = std::min(p.n, (row + 1) * ns - p.first);
+            const double base = b[row];
+            for (; a < end; ++a) dst[a] = base + (double)d[a];
+        }
+        return hipSuccess;
+    };
+    auto work = [&]() {
+        hipError_t e = hipSetDevice(ctx->device);
+        for (;;) {
+            size_t c;
+            {
+                std::unique_lock<std::mutex> l(m);
+                if (e != hipSuccess) {
+                    err = e;
+                    stop = true;
+                    cv.notify_all();
+                }
+                cv.wait(l, [&] { return stop || next < issued || next >= pieces.size(); });
+                if (stop || next >= pieces.size()) return;
+                c = next++;
+            }
+            e = move_out(c);
+            std::lock_guard<std::mutex> l(m);
+            done[c] = 1;
+            cv.notify_all();
+        }
+    };
+    std::vector<std::thread> threads;
+    if (!stop) {
+        const size_t want = std::min<size_t>(kCopyThreads, pieces.size());
+        try {
+            threads.reserve(want);
+            for (size_t t = 0; t < want; ++t) threads.emplace_back(work);
+        } catch (...) {  // fewer threads than wanted; with none, this one moves the pieces
+        }
+    }
+    for (size_t c = 0; c < pieces.size(); ++c) {
+        {
+            std::unique_lock<std::mutex> l(m);
+            cv.wait(l, [&] { return stop || threads.empty() || c < kSlots || done[c - kSlots]; });
+            if (stop) break;
+        }
+        const CopyPiece &p = pieces[c];
+        const int f = fields[(size_t)p.which].field;
+        const size_t esz = field_element_size(P, f);
+        hipError_t e = hipMemcpyAsync(slots + (c % kSlots) * kSlotBytes, static_cast<const char *>(P.f[f]) + p.first * esz,
+                                      p.n * esz, hipMemcpyDeviceToHost, ctx->stream);
+        if (e == hipSuccess) e = hipEventRecord(ev[c % kSlots], ctx->stream);
+        if (e == hipSuccess && threads.empty()) e = move_out(c);
+        std::lock_guard<std::mutex> l(m);
+        if (e != hipSuccess) {
+            err = e;
+            stop = true;
+        } else {
+            issued = c + 1;
+        }
+        cv.notify_all();
+    }
+    for (std::thread &t : threads) t.join();
+    const hipError_t se = hipStreamSynchronize(ctx->stream);  // no transfer into a slot outlives the lease
+    for (hipEvent_t e : ev)
+        if (e) hipEventDestroy(e);
+    HIP_TRY(ctx, err);
+    HIP_TRY(ctx, se);
     return FCPT_OK;
+}
+
+// all fields by one kernel into the slots, then to the caller: by this thread
+// below 1 MB, by several above
+static int copy_export(fcpt_ctx *ctx, const std::vector<HostCopy> &fields, size_t total)
+{
+    const KParams &P = ctx->P;
+    char *out = nullptr;
+    HIP_TRY(ctx, host_slots_get(total > kSmallBytes, &out));
+    ExportFields x{};
+    size_t at = 0;
+    for (const HostCopy &f : fields) {
+        x.field[x.n] = f.field;
+        x.rows[x.n] = (int)field_rows(f.field, P.nr);
+        x.out[x.n] = reinterpret_cast<double *>(out) + at;
+        at += (size_t)x.rows[x.n++] * (size_t)P.ns;
+    }
+    launch_export(P, ctx->stream, x);
+    LAUNCH_CHECK(ctx);
+    // strip t of T of every field
+    auto strip = [&](size_t t, size_t T) {
+        for (int k = 0; k < x.n; ++k) {
+            const size_t n = (size_t)x.rows[k] * (size_t)P.ns, a = n * t / T, b = n * (t + 1) / T;
+            std::memcpy(fields[(size_t)k].dst + a, x.out[k] + a, (b - a) * sizeof(double));
+        }
+    };
+    const size_t T = std::max<size_t>(1, std::min<size_t>(kCopyThreads, total / kSmallBytes));
+    std::mutex m;
+    std::condition_variable cv;
+    int go = 0;  // 1: the slots are filled, -1: they will not be
+    std::vector<std::thread> threads;
+    try {
+        threads.reserve(T - 1);
+        for (size_t t = 1; t < T; ++t)
+            threads.emplace_back([&, t] {
+                {
+                    std::unique_lock<std::mutex> l(m);
+                    cv.wait(l, [&] { return go != 0; });
+                }
+                if (go > 0) strip(t, T);
+            });
+    } catch (...) {  // this thread takes the strips that have no other
+    }
+    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    {
+        std::lock_guard<std::mutex> l(m);
+        go = e == hipSuccess ? 1 : -1;
+    }
+    cv.notify_all();
+    if (e == hipSuccess) {
+        strip(0, T);
+        for (size_t t = threads.size() + 1; t < T; ++t) strip(t, T);
+    }
+    for (std::thread &t : threads) t.join();
+    HIP_TRY(ctx, e);
+    return FCPT_OK;
+}
+
+// the fields to the caller's arrays in FP64 (split storage: background +
+// deviation)
+static int copy_to_host(fcpt_ctx *ctx, const std::vector<HostCopy> &fields)
+{
+    const KParams &P = ctx->P;
+    size_t total = 0;
+    for (const HostCopy &f : fields) total += field_rows(f.field, P.nr) * (size_t)P.ns * sizeof(double);
+    std::lock_guard<std::mutex> lease(host_slots().lease);
+    try {
+        return total > kSlotBytes * kSlots ? copy_large(ctx, fields) : copy_export(ctx, fields, total);
+    } catch (const std::exception &e) {
+        return fail(ctx, FCPT_ERR_DEVICE, "copy to the host: %s", e.what());
+    }
 }
 
 int fcpt_upload_field(fcpt_ctx *ctx, int32_t field, const double *host)
@@ -618,12 +864,7 @@ int fcpt_download_field(fcpt_ctx *ctx, int32_t field, double *host)
     CTX_CHECK(ctx);
     if (field < 0 || field >= FCPT_NUM_FIELDS || !host) return fail(ctx, FCPT_ERR_ARG, "bad field");
     if (derived_field(field)) sync_derived(ctx);
-    if (ctx->P.split && field != FCPT_POTENTIAL) return download_split(ctx, field, host);
-    const size_t n = field_rows(field, ctx->P.nr) * ctx->P.ns;
-    HIP_TRY(ctx, hipMemcpyAsync(host, ctx->P.f[field], n * sizeof(double), hipMemcpyDeviceToHost,
-                                ctx->stream));
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    return FCPT_OK;
+    return copy_to_host(ctx, {{field, host}});
 }
 
 // split storage: re-express a field about a new host-given background
@@ -893,12 +1134,13 @@ int fcpt_upload_state(fcpt_ctx *ctx, const double *sigma, const double *vrad, co
 
 int fcpt_download_state(fcpt_ctx *ctx, double *sigma, double *vrad, double *vazi, double *energy)
 {
-    int rc;
-    if (sigma && (rc = fcpt_download_field(ctx, FCPT_SIGMA, sigma))) return rc;
-    if (vrad && (rc = fcpt_download_field(ctx, FCPT_VRAD, vrad))) return rc;
-    if (vazi && (rc = fcpt_download_field(ctx, FCPT_VAZI, vazi))) return rc;
-    if (energy && (rc = fcpt_download_field(ctx, FCPT_ENERGY, energy))) return rc;
-    return FCPT_OK;
+    CTX_CHECK(ctx);
+    std::vector<HostCopy> fields;
+    double *const dst[4] = {sigma, vrad, vazi, energy};
+    const int f[4] = {FCPT_SIGMA, FCPT_VRAD, FCPT_VAZI, FCPT_ENERGY};
+    for (int k = 0; k < 4; ++k)
+        if (dst[k]) fields.push_back({f[k], dst[k]});
+    return fields.empty() ? FCPT_OK : copy_to_host(ctx, fields);
 }
 
 int fcpt_set_time(fcpt_ctx *ctx, double time, double last_dt, int32_t n_monitor)

@@ -3766,6 +3766,21 @@ void launch_fill_rows(const KParams &P, hipStream_t st, void *dst, const double 
     if (P.split) hipLaunchKernelGGL(k_fill_rows<true>, g, kBlock, 0, st, dst, ring, bg, P.ns, rows);
     else hipLaunchKernelGGL(k_fill_rows<false>, g, kBlock, 0, st, dst, ring, bg, P.ns, rows);
 }
+// one block row of 64 x 4 threads per four rings, blockIdx.z the field
+template <bool SPLIT>
+__global__ void __launch_bounds__(256) k_export(KParams P, ExportFields x)
+{
+    const int j = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int i = wave_ring(0, (int)blockIdx.y), k = (int)blockIdx.z, f = x.field[k];
+    if (j >= P.ns || i >= x.rows[k]) return;
+    const double v = f == FCPT_POTENTIAL ? phi_fld(P)(i, j) : fld<SPLIT>(P, f)(i, j);
+    x.out[k][(size_t)i * (size_t)P.ns + (size_t)j] = v;
+}
+void launch_export(const KParams &P, hipStream_t st, const ExportFields &x)
+{
+    const dim3 c = cell_grid(P, P.nr + 1);
+    LAUNCH(k_export, dim3(c.x, c.y, (unsigned)x.n), kBlock, st, P, x);
+}
 void launch_copy_velocities(const KParams &P, hipStream_t st)
 {
     LAUNCH(k_copy_velocities, cell_grid(P, P.nr + 1), kBlock, st, P);

@@ -89,6 +89,13 @@ void launch_rebase(const KParams &P, hipStream_t st, void *field, const double *
 // split storage: out[i] = ring mean of the field's row i (rows rows)
 void launch_split_ring_mean(const KParams &P, hipStream_t st, const void *field, const double *bg,
                             int rows, double *out);
+// fields in FP64 (split storage: background + deviation) into host memory the
+// device can write, all in one launch
+struct ExportFields {
+    int n, field[4], rows[4];
+    double *out[4];
+};
+void launch_export(const KParams &P, hipStream_t st, const ExportFields &x);
 // bytes of one stored value of a 2-D field (8 in FP64 storage, 4 in split storage)
 size_t element_size(const KParams &P);
 // bytes per value of one field: the potential is FP64 in both storage modes
