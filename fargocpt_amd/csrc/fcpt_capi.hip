@@ -22,6 +22,12 @@
 
 using namespace fcpt;
 
+// Iterations in one captured graph.  A graph's start and end cost the device
+// 3 to 5 us beyond the kernels between them (32 x 64: 37.1 us per step with one
+// iteration per graph, 33.1 with 4, 32.2 with 16; 251 x 757: 60.3, 57.6, 56.3),
+// and every captured iteration costs its first use about 15 us.
+constexpr int kGraphSteps = 8;
+
 // split storage: steps of fcpt_run_steps between two moves of the ring
 // backgrounds unless the caller sets another interval
 constexpr int kDefaultRebaseInterval = 1000;
@@ -42,7 +48,7 @@ struct fcpt_ctx {
     double *force_part = nullptr;   // per-block partial sums
     double *force_out = nullptr;
     double *force_host = nullptr;
-    hipGraphExec_t step_graph = nullptr;
+    hipGraphExec_t step_graph[2] = {nullptr, nullptr};  // of one iteration and of kGraphSteps
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::string err;
     // host copies of the per-ring metric (split storage derives its backgrounds from them)
@@ -65,6 +71,19 @@ struct fcpt_ctx {
 
 static void host_slots_join();
 static void host_slots_leave();
+
+// both graphs of a context or a batch, to be captured again
+static hipError_t drop_graphs(hipGraphExec_t (&g)[2])
+{
+    hipError_t e = hipSuccess;
+    for (hipGraphExec_t &x : g) {
+        if (!x) continue;
+        const hipError_t d = hipGraphExecDestroy(x);
+        if (e == hipSuccess) e = d;
+        x = nullptr;
+    }
+    return e;
+}
 
 namespace {
 
@@ -527,7 +546,7 @@ int fcpt_destroy(fcpt_ctx *ctx)
         hipStreamSynchronize(ctx->stream);
         hipStreamDestroy(ctx->stream);
     }
-    if (ctx->step_graph) hipGraphExecDestroy(ctx->step_graph);
+    drop_graphs(ctx->step_graph);
     if (ctx->ev0) hipEventDestroy(ctx->ev0);
     if (ctx->ev1) hipEventDestroy(ctx->ev1);
     for (void *p : ctx->allocs) hipFree(p);
@@ -603,9 +622,9 @@ static int upload_split(fcpt_ctx *ctx, int field, const double *host)
 // there, so half the bytes cross the link): 37 ms, and 21 for split storage
 // instead of 292.  What fits the slots as a whole is decoded and written to
 // them by one kernel, all fields at once: each transfer and its event cost
-// tens of microseconds, more than the link's time below some MB (128 x 384:
-// 530 -> 70 us, 32 x 64: 80 -> 21 us; slots filled in smaller pieces were
-// slower than in one).
+// tens of microseconds, more than the link's time below some MB (512 x
+// 1536: 1.5 - 3.5 -> 0.9 - 1.5 ms, 32 x 64: 80 -> 21 us; slots filled in smaller
+// pieces were slower than in one).
 //
 // The slots belong to the process (a disk's own would cost each disk their
 // pinning, ~10 ms): allocated by the first copy that needs them, leased to one
@@ -1466,19 +1485,21 @@ int fcpt_run_step(fcpt_ctx *ctx, double *dt_out)
     return FCPT_OK;
 }
 
-// capture one sim::run iteration into a graph (once per context)
-static int ensure_step_graph(fcpt_ctx *ctx)
+// capture one iteration, or kGraphSteps of them (`many`), into a graph (each
+// once per context)
+static int ensure_step_graph(fcpt_ctx *ctx, bool many)
 {
-    if (ctx->step_graph) return FCPT_OK;
+    hipGraphExec_t &exec = ctx->step_graph[many ? 1 : 0];
+    if (exec) return FCPT_OK;
     hipGraph_t g = nullptr;
     HIP_TRY(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_iteration(ctx, ctx->fused);
+    for (int k = 0; k < (many ? kGraphSteps : 1); ++k) enqueue_iteration(ctx, ctx->fused);
     hipError_t e = hipStreamEndCapture(ctx->stream, &g);
     if (e != hipSuccess) return fail(ctx, FCPT_ERR_DEVICE, "graph capture: %s", hipGetErrorString(e));
-    e = hipGraphInstantiate(&ctx->step_graph, g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
     hipGraphDestroy(g);
     if (e != hipSuccess) {
-        ctx->step_graph = nullptr;
+        exec = nullptr;
         return fail(ctx, FCPT_ERR_DEVICE, "graph instantiate: %s", hipGetErrorString(e));
     }
     return FCPT_OK;
@@ -1491,8 +1512,11 @@ int fcpt_run_steps(fcpt_ctx *ctx, int32_t n_steps, int32_t use_graph)
 {
     CTX_CHECK(ctx);
     if (n_steps < 0) return fail(ctx, FCPT_ERR_ARG, "negative step count");
+    // calls of kGraphSteps or more replay that many per graph and launch the
+    // rest one by one; shorter ones replay single iterations
+    const bool many = n_steps >= kGraphSteps;
     if (use_graph) {
-        int rc = ensure_step_graph(ctx);
+        int rc = ensure_step_graph(ctx, many);
         if (rc) return rc;
     }
     for (int left = n_steps; left > 0;) {
@@ -1503,12 +1527,13 @@ int fcpt_run_steps(fcpt_ctx *ctx, int32_t n_steps, int32_t use_graph)
             m = 1;
             sync_derived(ctx);
         }
+        int k = 0;
         if (use_graph && fused == ctx->fused) {
-            for (int k = 0; k < m; ++k) HIP_TRY(ctx, hipGraphLaunch(ctx->step_graph, ctx->stream));
-        } else {
-            for (int k = 0; k < m; ++k) enqueue_iteration(ctx, fused);
-            LAUNCH_CHECK(ctx);
+            const int per = many ? kGraphSteps : 1;
+            for (; k + per <= m; k += per) HIP_TRY(ctx, hipGraphLaunch(ctx->step_graph[many ? 1 : 0], ctx->stream));
         }
+        for (; k < m; ++k) enqueue_iteration(ctx, fused);
+        LAUNCH_CHECK(ctx);
         left -= m;
         stepped(ctx, fused);
         if (periodic_rebase(ctx) && (ctx->steps_since_rebase += m) >= ctx->rebase_interval) {
@@ -1530,7 +1555,7 @@ int fcpt_time_steps(fcpt_ctx *ctx, int32_t n_steps, int32_t use_graph, double *m
 {
     CTX_CHECK(ctx);
     int rc = ensure_events(ctx);
-    if (!rc && use_graph) rc = ensure_step_graph(ctx);
+    if (!rc && use_graph) rc = ensure_step_graph(ctx, n_steps >= kGraphSteps);
     if (rc) return rc;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     HIP_TRY(ctx, hipEventRecord(ctx->ev0, ctx->stream));
@@ -1640,10 +1665,7 @@ int fcpt_set_launch_param(fcpt_ctx *ctx, int32_t param, int32_t value)
     else if (param == FCPT_PARAM_KICK_TILE) ctx->P.kick_tile = value;
     else if (param == FCPT_PARAM_SPLIT_ROUNDING) ctx->P.split_rounding = ctx->P.split ? value : 0;
     else ctx->fused = value != 0;
-    if (ctx->step_graph) {
-        HIP_TRY(ctx, hipGraphExecDestroy(ctx->step_graph));
-        ctx->step_graph = nullptr;
-    }
+    HIP_TRY(ctx, drop_graphs(ctx->step_graph));
     return FCPT_OK;
 }
 
@@ -1709,10 +1731,7 @@ int fcpt_autotune_walks(fcpt_ctx *ctx, int32_t reps, int32_t *kick_tile, int32_t
     hipError_t e = copy_fields(true);
     if (e == hipSuccess) e = hipMemcpy(&s0, ctx->s_dev, sizeof(DevScalars), hipMemcpyDeviceToHost);
     auto trial = [&](double &ms_out) -> int {
-        if (ctx->step_graph) {
-            hipGraphExecDestroy(ctx->step_graph);
-            ctx->step_graph = nullptr;
-        }
+        drop_graphs(ctx->step_graph);
         int r = fcpt_run_steps(ctx, 1, 1);  // capture + warm-up
         if (!r) r = fcpt_time_steps(ctx, reps, 1, &ms_out);
         const hipError_t er = restore();
@@ -1737,10 +1756,7 @@ int fcpt_autotune_walks(fcpt_ctx *ctx, int32_t reps, int32_t *kick_tile, int32_t
     if (kv) P.kick_tile = best_t;
     P.visc_tile = best_t;
     hipFree(save);
-    if (ctx->step_graph) {
-        hipGraphExecDestroy(ctx->step_graph);
-        ctx->step_graph = nullptr;
-    }
+    drop_graphs(ctx->step_graph);
     if (rc) return rc;
     if (kick_tile) *kick_tile = resolve_kick_tile(P);
     if (visc_tile) *visc_tile = resolve_visc_tile(P);
@@ -1798,10 +1814,7 @@ int fcpt_autotune(fcpt_ctx *ctx, int32_t reps, int32_t *radial_tile, int32_t *ra
     }
     P.radial_tile = best_t;
     P.radial_waves = best_w;
-    if (ctx->step_graph) {
-        HIP_TRY(ctx, hipGraphExecDestroy(ctx->step_graph));
-        ctx->step_graph = nullptr;
-    }
+    HIP_TRY(ctx, drop_graphs(ctx->step_graph));
     if (radial_tile) *radial_tile = best_t;
     if (radial_waves) *radial_waves = best_w;
     return FCPT_OK;
@@ -2130,7 +2143,7 @@ struct fcpt_batch {
     KParams *Ps = nullptr;  // device array: every disk's parameters, then their swapped views
     std::vector<BatchStageDev> stages;
     hipStream_t stream = nullptr;
-    hipGraphExec_t graph = nullptr;
+    hipGraphExec_t graph[2] = {nullptr, nullptr};  // as a context's step_graph
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t done = nullptr;  // end of the last batched run; every disk's stream waits for it
     std::string err;
@@ -2194,10 +2207,7 @@ static int upload_batch_plan(fcpt_batch *b)
         b->stages.push_back(
             BatchStageDev{h.kind, h.arg, static_cast<const BatchEntry *>(m), (unsigned)h.entries.size()});
     }
-    if (b->graph) {
-        hipGraphExecDestroy(b->graph);
-        b->graph = nullptr;
-    }
+    drop_graphs(b->graph);
     return FCPT_OK;
 }
 
@@ -2279,7 +2289,7 @@ int fcpt_batch_destroy(fcpt_batch *b)
         hipStreamSynchronize(b->stream);
         hipStreamDestroy(b->stream);
     }
-    if (b->graph) hipGraphExecDestroy(b->graph);
+    drop_graphs(b->graph);
     if (b->ev0) hipEventDestroy(b->ev0);
     if (b->ev1) hipEventDestroy(b->ev1);
     if (b->done) hipEventDestroy(b->done);
@@ -2295,10 +2305,7 @@ int fcpt_batch_set_radial_waves(fcpt_batch *b, int32_t waves)
     BHIP(b, hipSetDevice(b->device));
     BHIP(b, hipStreamSynchronize(b->stream));
     b->radial_waves = waves;
-    if (b->graph) {
-        BHIP(b, hipGraphExecDestroy(b->graph));
-        b->graph = nullptr;
-    }
+    BHIP(b, drop_graphs(b->graph));
     return FCPT_OK;
 }
 
@@ -2310,6 +2317,24 @@ int fcpt_batch_synchronize(fcpt_batch *b)
     return FCPT_OK;
 }
 
+static int ensure_batch_graph(fcpt_batch *b, bool many)
+{
+    hipGraphExec_t &exec = b->graph[many ? 1 : 0];
+    if (exec) return FCPT_OK;
+    hipGraph_t g = nullptr;
+    BHIP(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+    for (int k = 0; k < (many ? kGraphSteps : 1); ++k) enqueue_batch_step(b, b->stream);
+    hipError_t e = hipStreamEndCapture(b->stream, &g);
+    if (e != hipSuccess) return bfail(b, FCPT_ERR_DEVICE, hipGetErrorString(e));
+    e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+    hipGraphDestroy(g);
+    if (e != hipSuccess) {
+        exec = nullptr;
+        return bfail(b, FCPT_ERR_DEVICE, hipGetErrorString(e));
+    }
+    return FCPT_OK;
+}
+
 int fcpt_batch_run_steps(fcpt_batch *b, int32_t n_steps, int32_t use_graph)
 {
     if (!b) return FCPT_ERR_ARG;
@@ -2317,18 +2342,10 @@ int fcpt_batch_run_steps(fcpt_batch *b, int32_t n_steps, int32_t use_graph)
     BHIP(b, hipSetDevice(b->device));
     // the disks' own queued work (uploads, start-up calls) comes first
     for (fcpt_ctx *c : b->disks) BHIP(b, hipStreamSynchronize(c->stream));
-    if (use_graph && !b->graph) {
-        hipGraph_t g = nullptr;
-        BHIP(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-        enqueue_batch_step(b, b->stream);
-        hipError_t e = hipStreamEndCapture(b->stream, &g);
-        if (e != hipSuccess) return bfail(b, FCPT_ERR_DEVICE, hipGetErrorString(e));
-        e = hipGraphInstantiate(&b->graph, g, nullptr, nullptr, 0);
-        hipGraphDestroy(g);
-        if (e != hipSuccess) {
-            b->graph = nullptr;
-            return bfail(b, FCPT_ERR_DEVICE, hipGetErrorString(e));
-        }
+    const bool many = n_steps >= kGraphSteps;
+    if (use_graph) {
+        const int rc = ensure_batch_graph(b, many);
+        if (rc) return rc;
     }
     if (n_steps > 0 && std::any_of(b->disks.begin(), b->disks.end(), [](fcpt_ctx *c) { return !c->derived_own; })) {
         // a member with fields of its caller's own: one iteration disk by disk
@@ -2343,12 +2360,13 @@ int fcpt_batch_run_steps(fcpt_batch *b, int32_t n_steps, int32_t use_graph)
         int m = left;
         for (fcpt_ctx *c : b->disks)
             if (periodic_rebase(c)) m = std::min(m, c->rebase_interval - c->steps_since_rebase);
+        int k = 0;
         if (use_graph) {
-            for (int k = 0; k < m; ++k) BHIP(b, hipGraphLaunch(b->graph, b->stream));
-        } else {
-            for (int k = 0; k < m; ++k) enqueue_batch_step(b, b->stream);
-            BHIP(b, hipGetLastError());
+            const int per = many ? kGraphSteps : 1;
+            for (; k + per <= m; k += per) BHIP(b, hipGraphLaunch(b->graph[many ? 1 : 0], b->stream));
         }
+        for (; k < m; ++k) enqueue_batch_step(b, b->stream);
+        BHIP(b, hipGetLastError());
         left -= m;
         // a disk call made after this one (a download, the totals) is ordered
         // after the batched steps on the disk's own stream
@@ -2452,7 +2470,8 @@ int fcpt_batch_time_steps(fcpt_batch *b, int32_t n_steps, int32_t use_graph, dou
     BHIP(b, hipSetDevice(b->device));
     if (!b->ev0) BHIP(b, hipEventCreate(&b->ev0));
     if (!b->ev1) BHIP(b, hipEventCreate(&b->ev1));
-    int rc = fcpt_batch_run_steps(b, 0, use_graph);  // capture outside the timed region
+    int rc = use_graph ? ensure_batch_graph(b, n_steps >= kGraphSteps) : FCPT_OK;  // outside the timed region
+    if (!rc) rc = fcpt_batch_run_steps(b, 0, 0);  // waits for the disks' own queued work
     if (rc) return rc;
     BHIP(b, hipStreamSynchronize(b->stream));
     BHIP(b, hipEventRecord(b->ev0, b->stream));

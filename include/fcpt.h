@@ -251,8 +251,9 @@ int fcpt_run_step(fcpt_ctx *ctx, double *dt_out);
 
 /* n_steps iterations of sim::run entirely on the device: the CFL time step,
    the monitor clip and the time stay in device memory and the planets keep the
-   last step parameters.  use_graph != 0 replays one captured HIP graph per
-   iteration.  No host synchronisation; errors surface at the next sync. */
+   last step parameters.  use_graph != 0 replays captured HIP graphs (of one
+   iteration, or of several in longer calls).  No host synchronisation; errors
+   surface at the next sync. */
 int fcpt_run_steps(fcpt_ctx *ctx, int32_t n_steps, int32_t use_graph);
 
 /* Measurement hooks (no counterpart in the reference): elapsed device time of
@@ -391,8 +392,8 @@ int fcpt_batch_set_radial_waves(fcpt_batch *batch, int32_t waves);
    the transport's scratch arrays only).  Keeps and returns the fastest;
    drops a captured batch graph.  Results do not depend on the choice. */
 int fcpt_batch_autotune(fcpt_batch *batch, int32_t reps, int32_t *radial_tile, int32_t *radial_waves);
-/* n_steps sim::run iterations of every disk; use_graph != 0 replays one
-   captured HIP graph per iteration.  No host synchronisation. */
+/* n_steps sim::run iterations of every disk; use_graph != 0 replays captured
+   HIP graphs as fcpt_run_steps does.  No host synchronisation. */
 int fcpt_batch_run_steps(fcpt_batch *batch, int32_t n_steps, int32_t use_graph);
 /* as fcpt_batch_run_steps, timed with HIP events on the batch's stream */
 int fcpt_batch_time_steps(fcpt_batch *batch, int32_t n_steps, int32_t use_graph, double *ms_total);
