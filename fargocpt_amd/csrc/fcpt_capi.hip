@@ -348,6 +348,7 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
     P.kv_tile = 0;
     P.lazy_derived = 0;
     P.split_emul = 0;
+    P.kick = P.pad_ = 0;
     P.ealt = nullptr;
     init_launch_fields(P);
     // Interpret.cpp:230-231
@@ -1383,9 +1384,21 @@ static void enqueue_euler(const KParams &P, hipStream_t st, int count_monitor, b
 // bodies (compute_pressure first), final boundaries over dt, derived fields.
 // The isothermal unfused path needs the pressure of the transported Sigma,
 // as does the adiabatic one of the transported E.
-static void enqueue_leapfrog(const KParams &P, hipStream_t st, int count_monitor, bool fused)
+static void enqueue_leapfrog(const KParams &P, hipStream_t st, int count_monitor, bool fused, int fold_mode)
 {
     const KParams Q = swapped_view(P);
+    if (P.lazy_derived) {
+        // the walks take their half steps from KParams::kick, so the clock
+        // needs no launches of its own
+        KParams K = P;
+        K.kick = 1;
+        launch_kick(K, st, fold_mode);
+        launch_transport_ghost(Q, P, st, 0);
+        K.kick = 2;
+        launch_kick(K, st, -1);
+        launch_final_leapfrog(P, st, count_monitor ? 2 : 1);
+        return;
+    }
     launch_leapfrog_phase(P, st, 0);
     const KParams *cur = enqueue_kick(P, Q, st, fused, false);
     launch_leapfrog_phase(P, st, 1);
@@ -1407,7 +1420,7 @@ static void enqueue_leapfrog(const KParams &P, hipStream_t st, int count_monitor
 
 static void enqueue_step(const KParams &P, hipStream_t st, int count_monitor, bool fused)
 {
-    if (P.integrator == FCPT_INTEGRATOR_LEAPFROG) enqueue_leapfrog(P, st, count_monitor, fused);
+    if (P.integrator == FCPT_INTEGRATOR_LEAPFROG) enqueue_leapfrog(P, st, count_monitor, fused, -1);
     else enqueue_euler(P, st, count_monitor, fused, -1);
 }
 
@@ -1420,6 +1433,9 @@ static void enqueue_iteration(const fcpt_ctx *ctx, bool fused)
     if (fused && V.integrator != FCPT_INTEGRATOR_LEAPFROG) {
         launch_cfl_cells(V, ctx->stream);
         enqueue_euler(V, ctx->stream, 1, true, 2);
+    } else if (V.lazy_derived) {
+        launch_cfl_cells(V, ctx->stream);
+        enqueue_leapfrog(V, ctx->stream, 1, true, 2);
     } else {
         launch_cfl(V, ctx->stream, 2);
         enqueue_step(V, ctx->stream, 1, fused);
@@ -1445,7 +1461,7 @@ int fcpt_step_leapfrog(fcpt_ctx *ctx, double dt)
     KParams V = ctx->P;
     V.integrator = FCPT_INTEGRATOR_LEAPFROG;  // the scheme, whatever the descriptor's own
     set_step_modes(V, fused);
-    enqueue_leapfrog(V, ctx->stream, 0, fused);
+    enqueue_leapfrog(V, ctx->stream, 0, fused, -1);
     LAUNCH_CHECK(ctx);
     stepped(ctx, fused);
     return FCPT_OK;

@@ -108,6 +108,9 @@ struct KParams {
     // split storage: values the kick walk and the CFL round as if stored
     // (SPLIT_EMUL_*), in disks whose step keeps fewer values in FP64
     int split_emul;
+    // the fused LeapFrog step's kick: 1 and 2 run over dt / 2, 2 from the midstep
+    // time and with the midstep bodies; 0 elsewhere (the whole dt)
+    int kick, pad_;
     int cfl_gx, cfl_gy;  // grid of the CFL cell kernel (its block-minimum slots)
     // fields in HBM (indexed by fcpt_field): double, or float when split
     void *f[FCPT_NUM_FIELDS];

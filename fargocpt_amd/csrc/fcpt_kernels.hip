@@ -185,8 +185,16 @@ __device__ __forceinline__ double omega_kepler(const KParams &P, double r)
 
 // dt and time of the running kick (no kernel that reads them writes them, so they
 // are scalar loads that stores do not repeat)
-__device__ __forceinline__ double kick_dt(const KParams &P) { return *(const __attribute__((address_space(4))) double *)&P.s->dt; }
-__device__ __forceinline__ double kick_time(const KParams &P) { return *(const __attribute__((address_space(4))) double *)&P.s->time; }
+__device__ __forceinline__ double kick_dt(const KParams &P)
+{
+    const double dt = *(const __attribute__((address_space(4))) double *)&P.s->dt;
+    return P.kick ? dt / 2 : dt;
+}
+__device__ __forceinline__ double kick_time(const KParams &P)
+{
+    const double t = *(const __attribute__((address_space(4))) double *)&P.s->time;
+    return P.kick == 2 ? t + kick_dt(P) : t;
+}
 
 // Per-ring arrays (metric, backgrounds, ring means, shifts) are never written
 // by the kernel that reads them.  Reading them through the constant address
@@ -295,6 +303,12 @@ struct Fld {
     __device__ __forceinline__ double stored(int i, int j, double v) const
     {
         if constexpr (SPLIT) return cst(bg)[i] + (double)round_dev(v - cst(bg)[i], key, cell(i, j));
+        else return v;
+    }
+    // the stored form of v at (i, j)
+    __device__ __forceinline__ T enc(int i, int j, double v) const
+    {
+        if constexpr (SPLIT) return round_dev(v - cst(bg)[i], key, cell(i, j));
         else return v;
     }
     __device__ __forceinline__ double dec(int i, T x) const
@@ -1043,8 +1057,9 @@ __device__ __forceinline__ void potential_ring_cells(const KParams &P, int i, in
         acc[c] = 0.0;
     }
     // the bodies through scalar loads (this launch writes none of them)
-    const auto bodies = cst(s->planet);
-    const int np = *cst(&s->n_planets);
+    const bool mid = P.kick == 2 && *cst(&s->has_mid);
+    const auto bodies = mid ? cst(s->planet_mid) : cst(s->planet);
+    const int np = mid ? *cst(&s->n_planets_mid) : *cst(&s->n_planets);
     for (int k = 0; k < np; ++k) {
         const double px = bodies[k].x, py = bodies[k].y;
         const double mass = bodies[k].mass, r_sm = bodies[k].r_cubic;
@@ -1053,7 +1068,8 @@ __device__ __forceinline__ void potential_ring_cells(const KParams &P, int i, in
         for (int c = 0; c < kPotCells; ++c)
             acc[c] += potential_body<SPLIT>(P, x[c], y[c], smk >= 0.0 ? smk : sm[c], px, py, mass, r_sm);
     }
-    const double ix = *cst(&s->indirect_x), iy = *cst(&s->indirect_y);
+    const double ix = mid ? *cst(&s->indirect_mid_x) : *cst(&s->indirect_x);
+    const double iy = mid ? *cst(&s->indirect_mid_y) : *cst(&s->indirect_y);
 #pragma unroll
     for (int c = 0; c < kPotCells; ++c) {
         const int j = j0 + 64 * c;
@@ -2082,10 +2098,6 @@ __device__ __forceinline__ void b_copy_velocities(const KParams &P, int bx, int 
     FLD(vaz, FCPT_VAZI);
     alt_vr<SPLIT>(P).set_raw(i, j, vr.raw(i, j));
     if (i < P.nr) alt_vaz<SPLIT>(P).set_raw(i, j, vaz.raw(i, j));
-    if (i < P.nr && P.adiabatic && P.lazy_derived) {  // E is in its partner buffer too
-        FLD(E, FCPT_ENERGY);
-        buf<SPLIT>(P, P.ealt, P.bg[FCPT_ENERGY]).set_raw(i, j, E.raw(i, j));
-    }
 }
 FCPT_PAIR0(copy_velocities, 256)
 
@@ -2980,6 +2992,66 @@ __device__ __forceinline__ void b_final_derived(const KParams &P, int bx, int by
     derived_store<SPLIT>(P, i, j, derived_load<SPLIT>(P, i, j, true), true, true);
 }
 FCPT_PAIR1(final_derived, 256, int, advance_time)
+
+// The end of the fused LeapFrog step in one launch: the second kick's
+// velocities and E, in the partner buffers of view P, damped into the fields
+// with Sigma, then the ghost rings, the clock and the derived fields: what
+// copying them back, b_damping and b_final_derived do (three launches, 18 us
+// of a 307 x 1021 step; this one 10).  One thread per cell of the active rings;
+// a ghost ring's cells are written by the thread of the ring they copy, so
+// that no thread reads what another writes.
+template <bool SPLIT>
+__device__ __forceinline__ void b_final_leapfrog(const KParams &P, int bx, int by, int advance_time)
+{
+    CELL_LOOP_HEAD(1, P.nr - 1)
+    using T = typename Fld<SPLIT>::T;
+    const int nr = P.nr;
+    const double dt = P.s->dt;
+    FLD(S, FCPT_SIGMA);
+    FLD(E, FCPT_ENERGY);
+    FLD(vr, FCPT_VRAD);
+    FLD(vaz, FCPT_VAZI);
+    const Fld<SPLIT> vr_s = alt_vr<SPLIT>(P), vaz_s = alt_vaz<SPLIT>(P);
+    const Fld<SPLIT> E_s = P.adiabatic ? buf<SPLIT>(P, P.ealt, P.bg[FCPT_ENERGY]) : E;
+    // the stored form of (r, j) of a field after the damping
+    auto damped = [&](const Fld<SPLIT> &to, const Fld<SPLIT> &from, int f0, bool vector, int r) {
+        const T raw = from.raw(r, j);
+        if (!P.damping) return raw;
+        const bool in = damp_in_inner(P, vector, r);
+        if (!in && !damp_in_outer(P, vector, r)) return raw;
+        return to.enc(r, j, damp_apply(P, vector, in, r, dt, to.dec(r, raw), fld<SPLIT>(P, f0)(r, j)));
+    };
+    const T s = damped(S, S, FCPT_SIGMA0, false, i);
+    const T e = damped(E, E_s, FCPT_ENERGY0, false, i);
+    const T va = damped(vaz, vaz_s, FCPT_VAZI0, false, i);
+    const T v = damped(vr, vr_s, FCPT_VRAD0, true, i == 1 ? 2 : i);  // v_r(1) is a ghost value, from v_r(2)
+    S.set_raw(i, j, s);
+    E.set_raw(i, j, e);
+    vaz.set_raw(i, j, va);
+    const double sv = S.dec(i, s), ev = E.dec(i, e);
+    derived_store<SPLIT>(P, i, j, DerivedIn{ev, sv, 0.0, 0.0}, false, false);
+    double v0, v1;
+    if (i == 1) {
+        ghost_vr_inner(P, vr.dec(2, v), v0, v1);
+        vr.set(0, j, v0);
+        vr.set(1, j, v1);
+    } else {
+        vr.set_raw(i, j, v);
+    }
+    if (i == nr - 2) {
+        ghost_vr_outer(P, vr.dec(i, v), v0, v1);
+        vr.set(nr, j, v0);
+        vr.set(nr - 1, j, v1);
+    }
+    if (i == 1 || i == nr - 2) {
+        const int g = i == 1 ? 0 : nr - 1;  // the ghost ring
+        const double sg = S.set_get(g, j, sv), eg = E.set_get(g, j, ev);
+        vaz.set(g, j, ghost_vaz(P, g));
+        derived_store<SPLIT>(P, g, j, DerivedIn{eg, sg, 0.0, 0.0}, false, false);
+    }
+    if (advance_time && i == 1 && j == 0) advance_clock(P, advance_time);
+}
+FCPT_PAIR1(final_leapfrog, 256, int, advance_time)
 
 // ---------------------------------------------------------------------------
 // Transport
@@ -4116,6 +4188,10 @@ void launch_final_boundaries_derived(const KParams &P, hipStream_t st, int advan
         LAUNCH(k_damping, cell_grid(P, n_inner + n_outer), kBlock, st, P);
     }
     LAUNCH(k_final_derived, cell_grid(P, P.nr), kBlock, st, P, advance_time);
+}
+void launch_final_leapfrog(const KParams &P, hipStream_t st, int advance_time)
+{
+    LAUNCH(k_final_leapfrog, cell_grid(P, P.nr - 2), kBlock, st, P, advance_time);
 }
 void launch_iso_rings(const KParams &P, hipStream_t st)
 {

@@ -32,6 +32,7 @@ void launch_set_mid_params(const KParams &P, hipStream_t st, const fcpt_step_par
 void launch_leapfrog_phase(const KParams &P, hipStream_t st, int phase);
 void launch_pressure(const KParams &P, hipStream_t st);
 void launch_final_boundaries_derived(const KParams &P, hipStream_t st, int advance_time);
+void launch_final_leapfrog(const KParams &P, hipStream_t st, int advance_time);
 void launch_copy_velocities(const KParams &P, hipStream_t st);
 void launch_fill_rows(const KParams &P, hipStream_t st, void *dst, const double *ring,
                       const double *bg, int rows);
