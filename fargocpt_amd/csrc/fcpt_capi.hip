@@ -415,6 +415,20 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
         return FCPT_ERR_ARG;  // inner and outer damping zones overlap
     }
 
+    // the zones as damping_single_inner / _outer test them (damping.cpp:311-427)
+    for (int v = 0; v < 2; ++v) {
+        // radius[0] and radius[size_radial - 1] of the scalar (Rmed) and vector (Rinf) grids
+        auto rmed = [&](int i) {
+            const double a = desc->radii[i], b = desc->radii[i + 1];
+            double r = 2.0 / 3.0 * (std::pow(b, 3) - std::pow(a, 3));
+            return r / (std::pow(b, 2) - std::pow(a, 2));
+        };
+        const double first = v ? desc->radii[0] : rmed(0), last = v ? desc->radii[nr] : rmed(nr - 1);
+        const double lin = P.damping_inner_limit, lout = P.damping_outer_limit;
+        P.zone_in[v] = P.damping && lin > 1.0 && first < P.rmin * lin ? ids[v] : -1;
+        P.zone_out[v] = P.damping && lout < 1.0 && last > P.rmax * lout ? ids[2 + v] : INT32_MAX;
+    }
+
     // per-ring metric arrays, init_radialarrays (init.cpp:188-225), in FP64 on the host
     const int n1 = nr + 2;
     std::vector<double> Rinf(n1, 0), Rsup(n1, 0), Rmed(n1, 0), Surf(n1, 0), InvSurf(n1, 0),
@@ -490,6 +504,7 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
     if (!rc) rc = dev_alloc(c, &P.iso_h, (size_t)nr + 2);
     if (!rc) rc = dev_alloc(c, &P.iso_nu, (size_t)nr + 2);
     if (!rc) rc = dev_alloc(c, &P.ring_tab, (size_t)kRingTabs * ((size_t)nr + 2));
+    if (!rc) rc = dev_alloc(c, &P.damp_tab, 8 * ((size_t)nr + 2));
     if (!rc) rc = dev_alloc(c, &P.vmean, (size_t)nr + 1);
     if (!rc) rc = dev_alloc(c, &P.vuni, (size_t)nr + 1);
     if (!rc) rc = dev_alloc(c, &P.nshift, (size_t)nr + 1);

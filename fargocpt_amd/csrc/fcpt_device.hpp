@@ -77,6 +77,8 @@ struct KParams {
     int bc_inner, bc_outer;
     int damping;
     int damp_ids[4];
+    int zone_in[2], zone_out[2];  // last ring of the inner and first of the outer damping
+                                  // zone of the scalar [0] and vector [1] fields (none: -1, INT_MAX)
     double G, Rgas, sigma_sb, c_light, mstar, mu, gamma;
     double aspect_ratio, flaring, alpha, thickness_smoothing;
     double cfl, cfl_max_var, heating_cooling_cfl_limit;
@@ -132,6 +134,7 @@ struct KParams {
     // kRingTabs values per ring, nr + 2 rings (k_ring_tables): one base pointer
     // and one run of memory per ring for the walks' scalar loads
     double *ring_tab;
+    double *damp_tab;     // per ring: the damping's squared ramp and time scale: scalar inner, outer, vector inner, outer
     double energy_per_t;  // R / mu / (gamma - 1): energy_at's factor, to rounding
     int const_ok;         // the physical constants lie in the range quot_in assumes
     double *vmean;       // per-ring mean azimuthal velocity

@@ -1699,6 +1699,21 @@ __global__ void __launch_bounds__(256) k_ring_tables(KParams P, double *out)
     tab[TAB_SIGMA_FLOOR10] = 10.0 * P.sigma0 * P.sigma_floor;
     tab[TAB_BETA_INV] = 1 / P.cooling_beta;
     tab[TAB_ARTVISC_SQ] = P.artvisc_factor * P.artvisc_factor;
+    for (int v = 0; v < 2; ++v) {
+        double *t = P.damp_tab + 8 * i + 4 * v;
+        const double r = v ? P.Rinf[i] : P.Rmed[i < P.nr ? i : P.nr - 1];
+        const double lin = P.damping_inner_limit, lout = P.damping_outer_limit;
+        if (i <= P.zone_in[v]) {
+            const double a = (r - P.rmin * lin) / (P.rmin - P.rmin * lin);
+            t[0] = a * a;
+            t[1] = P.damping_time_factor * 2.0 * M_PI / omega_kepler(P, P.rmin);
+        }
+        if (i >= P.zone_out[v]) {
+            const double a = (r - P.rmax * lout) / (P.rmax - P.rmax * lout);
+            t[2] = a * a;
+            t[3] = P.damping_time_factor * 2.0 * M_PI / omega_kepler(P, P.damping_time_radius_outer);
+        }
+    }
 }
 
 void launch_ring_tables(const KParams &P, hipStream_t st)
@@ -2757,42 +2772,33 @@ __global__ void __launch_bounds__(256) kb_kv_walk(const KParams *Ps, const Batch
 }
 
 // ---------------------------------------------------------------------------
-// damping (boundary_conditions/damping.cpp:311-427, 754-776) of one value:
-// whether ring i of a vector (v_r) or scalar field lies in the inner or the
-// outer damping zone, and the value relaxed towards its reference x0
-__device__ __forceinline__ bool damp_in_inner(const KParams &P, bool vector, int i)
+// damping (boundary_conditions/damping.cpp:311-427, 754-776): whether ring i of
+// a vector (v_r) or scalar field lies in a damping zone, the relaxation of its
+// values over dt (the inner zone's, then the outer one's), and a value relaxed
+// towards its reference x0.  Ramp and time scale are per-ring constants
+// (k_ring_tables): a damped ring costs one division and one exponential,
+// shared by its scalar fields.
+__device__ __forceinline__ bool damped_ring(const KParams &P, bool vector, int i)
 {
-    const double *radius = vector ? P.Rinf : P.Rmed;
-    const int size_radial = vector ? P.nr + 1 : P.nr;
-    const double lin = P.damping_inner_limit;
-    if (i >= size_radial || !((lin > 1.0) && (radius[0] < P.rmin * lin))) return false;
-    return i <= (vector ? P.damp_ids[1] : P.damp_ids[0]);
+    return i <= P.zone_in[vector] || i >= P.zone_out[vector];
 }
-__device__ __forceinline__ bool damp_in_outer(const KParams &P, bool vector, int i)
+struct Damp {
+    bool in, out;
+    double f_in, f_out;
+};
+__device__ __forceinline__ Damp damp_ring(const KParams &P, bool vector, int i, double dt)
 {
-    const double *radius = vector ? P.Rinf : P.Rmed;
-    const int size_radial = vector ? P.nr + 1 : P.nr;
-    const double lout = P.damping_outer_limit;
-    if (i >= size_radial || !((lout < 1.0) && (radius[size_radial - 1] > P.rmax * lout))) return false;
-    return i >= (vector ? P.damp_ids[3] : P.damp_ids[2]);
+    const auto t = cst(P.damp_tab) + 8 * i + (vector ? 4 : 0);
+    Damp d{i <= P.zone_in[vector], i >= P.zone_out[vector], 1.0, 1.0};
+    if (d.in) d.f_in = exp(-dt * t[0] / t[1]);
+    if (d.out) d.f_out = exp(-dt * t[2] / t[3]);
+    return d;
 }
-__device__ __forceinline__ double damp_apply(const KParams &P, bool vector, bool inner, int i, double dt,
-                                             double x, double x0)
+__device__ __forceinline__ double damp_value(double x, double x0, const Damp &d)
 {
-    const double *radius = vector ? P.Rinf : P.Rmed;
-    const double RMIN = P.rmin, RMAX = P.rmax;
-    double tau, a;
-    if (inner) {
-        const double lin = P.damping_inner_limit;
-        tau = P.damping_time_factor * 2.0 * M_PI / omega_kepler(P, RMIN);
-        a = (radius[i] - RMIN * lin) / (RMIN - RMIN * lin);
-    } else {
-        const double lout = P.damping_outer_limit;
-        tau = P.damping_time_factor * 2.0 * M_PI / omega_kepler(P, P.damping_time_radius_outer);
-        a = (radius[i] - RMAX * lout) / (RMAX - RMAX * lout);
-    }
-    const double exp_factor = exp(-dt * (a * a) / tau);
-    return (x - x0) * exp_factor + x0;
+    if (d.in) x = (x - x0) * d.f_in + x0;
+    if (d.out) x = (x - x0) * d.f_out + x0;
+    return x;
 }
 
 // damping: block row y maps to an inner-zone ring (y < n_inner) or an
@@ -2807,25 +2813,22 @@ __device__ __forceinline__ void b_damping(const KParams &P, int bx, int by)
     if (j >= ns) return;
     const double dt = P.s->dt;
     int i;
-    bool inner;
     if (y < n_inner) {
         i = y;
-        inner = true;
     } else {
         // outer zone starts at the smaller of the scalar / vector limits
         const int o0 = P.damp_ids[2] < P.damp_ids[3] ? P.damp_ids[2] : P.damp_ids[3];
         i = o0 + (y - n_inner);
-        if (i > P.nr) return;
-        inner = false;
+        if (i < n_inner || i > P.nr) return;  // a ring of both zones is the inner row's
     }
     const int F0[4] = {FCPT_VRAD0, FCPT_VAZI0, FCPT_SIGMA0, FCPT_ENERGY0};
     const int F[4] = {FCPT_VRAD, FCPT_VAZI, FCPT_SIGMA, FCPT_ENERGY};
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const bool vector = q == 0;
-        if (!(inner ? damp_in_inner(P, vector, i) : damp_in_outer(P, vector, i))) continue;
+        if (i >= (vector ? P.nr + 1 : P.nr) || !damped_ring(P, vector, i)) continue;
         const Fld<SPLIT> X = fld<SPLIT>(P, F[q]), X0 = fld<SPLIT>(P, F0[q]);
-        X.set(i, j, damp_apply(P, vector, inner, i, dt, X(i, j), X0(i, j)));
+        X.set(i, j, damp_value(X(i, j), X0(i, j), damp_ring(P, vector, i, dt)));
     }
 }
 FCPT_PAIR0(damping, 256)
@@ -3014,17 +3017,18 @@ __device__ __forceinline__ void b_final_leapfrog(const KParams &P, int bx, int b
     const Fld<SPLIT> vr_s = alt_vr<SPLIT>(P), vaz_s = alt_vaz<SPLIT>(P);
     const Fld<SPLIT> E_s = P.adiabatic ? buf<SPLIT>(P, P.ealt, P.bg[FCPT_ENERGY]) : E;
     // the stored form of (r, j) of a field after the damping
-    auto damped = [&](const Fld<SPLIT> &to, const Fld<SPLIT> &from, int f0, bool vector, int r) {
-        const T raw = from.raw(r, j);
-        if (!P.damping) return raw;
-        const bool in = damp_in_inner(P, vector, r);
-        if (!in && !damp_in_outer(P, vector, r)) return raw;
-        return to.enc(r, j, damp_apply(P, vector, in, r, dt, to.dec(r, raw), fld<SPLIT>(P, f0)(r, j)));
-    };
-    const T s = damped(S, S, FCPT_SIGMA0, false, i);
-    const T e = damped(E, E_s, FCPT_ENERGY0, false, i);
-    const T va = damped(vaz, vaz_s, FCPT_VAZI0, false, i);
-    const T v = damped(vr, vr_s, FCPT_VRAD0, true, i == 1 ? 2 : i);  // v_r(1) is a ghost value, from v_r(2)
+    const int rv = i == 1 ? 2 : i;  // v_r(1) is a ghost value, from v_r(2)
+    const bool zs = damped_ring(P, false, i), zv = damped_ring(P, true, rv);
+    T s = S.raw(i, j), e = E_s.raw(i, j), va = vaz_s.raw(i, j), v = vr_s.raw(rv, j);
+    if (zs) {
+        const double s0 = fld<SPLIT>(P, FCPT_SIGMA0)(i, j), e0 = fld<SPLIT>(P, FCPT_ENERGY0)(i, j);
+        const double va0 = fld<SPLIT>(P, FCPT_VAZI0)(i, j);
+        const Damp f = damp_ring(P, false, i, dt);
+        s = S.enc(i, j, damp_value(S.dec(i, s), s0, f));
+        e = E.enc(i, j, damp_value(E.dec(i, e), e0, f));
+        va = vaz.enc(i, j, damp_value(vaz.dec(i, va), va0, f));
+    }
+    if (zv) v = vr.enc(rv, j, damp_value(vr.dec(rv, v), fld<SPLIT>(P, FCPT_VRAD0)(rv, j), damp_ring(P, true, rv, dt)));
     S.set_raw(i, j, s);
     E.set_raw(i, j, e);
     vaz.set_raw(i, j, va);
@@ -3509,123 +3513,105 @@ __device__ __forceinline__ void b_velocities(const KParams &P, int bx, int by)
 }
 FCPT_PAIR0(velocities, 256)
 
-// the damping of the final boundary call applied to a value the velocity
-// kernel stores: the value is damped as a later load of it returns it, so
-// the field is that of the velocity kernel followed by the damping kernel
-template <bool SPLIT>
-__device__ __forceinline__ double damp_stored(const KParams &P, const Fld<SPLIT> &X, int f0, bool vector,
-                                              int i, int j, double dt, double x)
-{
-    if (!P.damping) return x;
-    const bool in = damp_in_inner(P, vector, i), out = damp_in_outer(P, vector, i);
-    if (!in && !out) return x;
-    x = X.stored(i, j, x);
-    const double x0 = fld<SPLIT>(P, f0)(i, j);
-    if (in) x = damp_apply(P, vector, true, i, dt, x, x0);
-    if (out) x = damp_apply(P, vector, false, i, dt, x, x0);
-    return x;
-}
-
 // The end of the fused Euler step in one launch: the velocity kernel, the
 // final boundary call (damping, ghost rings, the clock) and
-// recalculate_derived_disk_quantities.  A cell forms its velocities, Sigma
-// and E as the velocity kernel and the damping store them, and its derived
-// fields from the stored values, as k_final_derived reads them.  The ghost
-// rings copy their neighbour ring, which another thread stores, so a
-// ghost-ring thread forms the neighbour's values itself (the same
-// expressions on the same inputs):
-// ring 0 takes Sigma and E of ring 1 and v_r from v_r(2), ring nr-1 those of
-// ring nr-2; v_r(1) is a ghost value too, so the ring-1 thread stores that
-// one instead of its own, and no cell is stored by two threads.
-template <bool SPLIT>
-__device__ __forceinline__ double vel_final_vr(const KParams &P, int r, int j, double dt)
-{
-    // v_r(r >= 1) as the velocity kernel and the damping pass it to set()
-    const Fld<false> Sb = buf<false>(P, P.sig_c, nullptr);
-    const Fld<false> m0 = mom_out(P, 0);
-    const Fld<false> m1 = mom_out(P, 1);
-    FLD(vr, FCPT_VRAD);
-    const double den = Sb(r - 1, j) + Sb(r, j);
-    const double v = SPLIT ? (m0(r - 1, j) + m1(r, j)) * recip<true>(den) : (m0(r - 1, j) + m1(r, j)) / den;
-    return damp_stored<SPLIT>(P, vr, FCPT_VRAD0, true, r, j, dt, v);
-}
-template <bool SPLIT>
-__device__ __forceinline__ void vel_final_sig_e(const KParams &P, int r, int j, double dt, double &sig,
-                                                double &e, bool need_e)
-{
-    // Sigma and (adiabatic) E of ring r as the velocity kernel and the
-    // damping pass them to set(); isothermal E is not touched there and is
-    // the stored value
-    FLD(S, FCPT_SIGMA);
-    FLD(E, FCPT_ENERGY);
-    const double floor_value = P.sigma_floor * P.sigma0;
-    double s0 = buf<false>(P, P.sig_c, nullptr)(r, j);
-    if (s0 < floor_value) s0 = floor_value;
-    sig = damp_stored<SPLIT>(P, S, FCPT_SIGMA0, false, r, j, dt, s0);
-    if (P.adiabatic) {
-        const double eb = buf<false>(P, P.en_c, nullptr)(r, j);
-        e = damp_stored<SPLIT>(P, E, FCPT_ENERGY0, false, r, j, dt, temperature_floor<SPLIT>(P, eb, s0));
-    } else {
-        e = need_e ? E(r, j) : 0.0;
-    }
-}
-
+// recalculate_derived_disk_quantities.  A thread owns one cell of an active
+// ring: it forms the velocities, Sigma and E as the velocity kernel and the
+// damping store them, and the derived fields from the stored values, as
+// k_final_derived reads them.  Every load is issued before the first use (the
+// damping references behind wave-uniform tests), so a wavefront waits once
+// and not at each damping branch.  The cells of a ghost ring are written by
+// the thread of the ring they copy, and v_r(1), a ghost value from v_r(2), by
+// that of ring 1: no thread reads what another writes.
+// Large grids are bound by bytes (88 per cell, adiabatic FP64), small ones by
+// the load latency.  Several rings per thread share the density and the
+// outward momentum of the ring inside, but lose more to fewer wavefronts:
+// 128x384 isothermal 36.7 us/step with one, 37.7 with two, 39.9 with four;
+// 2048x6144 split 1068, 1084, 1089; 4096x12288 FP64 5121, 5129, 5127.  With
+// the loads behind the branches and per-cell damping ramps the steps took
+// 37.7, 1141 and 5221 us.
 template <bool SPLIT>
 __device__ __forceinline__ void b_velocities_final(const KParams &P, int bx, int by, int advance_time)
 {
-    CELL_LOOP_HEAD(0, P.nr)
+    CELL_LOOP_HEAD(1, P.nr - 1)
     const int nr = P.nr;
-    const double dt = P.s->dt;
+    const int jm = j == 0 ? ns - 1 : j - 1;
+    const double dt = *cst(&P.s->dt);
+    const Fld<false> Sb = buf<false>(P, P.sig_c, nullptr), Eb = buf<false>(P, P.en_c, nullptr);
+    const Fld<false> m0 = mom_out(P, 0), m1 = mom_out(P, 1), m2 = mom_out(P, 2), m3 = mom_out(P, 3);
     FLD(vr, FCPT_VRAD);
     FLD(vaz, FCPT_VAZI);
     FLD(S, FCPT_SIGMA);
     FLD(E, FCPT_ENERGY);
-    const bool ghost = i == 0 || i == nr - 1;
-    // every value first, every store after (a load after a store waits for it)
-    double sr, er, va = 0.0, vb = 0.0, vphi = 0.0;
+    // v_r between rings r - 1 and r, as the velocity kernel and the damping
+    // pass it to set()
+    auto v_r = [&](int r, double p0, double p1, double sm, double s0, double x0) {
+        const double v = SPLIT ? (p0 + p1) * recip<true>(sm + s0) : (p0 + p1) / (sm + s0);
+        return damped_ring(P, true, r) ? damp_value(vr.stored(r, j, v), x0, damp_ring(P, true, r, dt)) : v;
+    };
+    auto v_r0 = [&](int r) { return damped_ring(P, true, r) ? fld<SPLIT>(P, FCPT_VRAD0)(r, j) : 0.0; };
+    const bool z = damped_ring(P, false, i);
+    const double sm = Sb(i - 1, j), s0 = Sb(i, j), sj = Sb(i, jm);
+    const double p0 = m0(i - 1, j), p1 = m1(i, j), p2 = m2(i, jm), p3 = m3(i, j);
+    const double e0 = P.adiabatic ? Eb(i, j) : 0.0;
+    double x_s = 0.0, x_e = 0.0, x_va = 0.0;
+    if (z) {
+        x_s = fld<SPLIT>(P, FCPT_SIGMA0)(i, j);
+        x_va = fld<SPLIT>(P, FCPT_VAZI0)(i, j);
+        if (P.adiabatic) x_e = fld<SPLIT>(P, FCPT_ENERGY0)(i, j);
+    }
+    const double x_vr = v_r0(i);
+    const bool ghost = i == 1 || i == nr - 2;
+    // an isothermal disk's E is only copied to the ghost rings
+    const double e_ghost = ghost && !P.adiabatic ? E(i, j) : 0.0;
+    double v2 = 0.0;
+    if (i == 1) v2 = vr.stored(2, j, v_r(2, m0(1, j), m1(2, j), s0, Sb(2, j), v_r0(2)));
+
+    const double floor_value = P.sigma_floor * P.sigma0;
+    double sig = s0;
+    if (sig < floor_value) sig = floor_value;
+    double en = P.adiabatic ? temperature_floor<SPLIT>(P, e0, sig) : 0.0;
+    double va = (SPLIT ? (p2 + p3) * recip<true>(sj + s0) : (p2 + p3) / (sj + s0)) * cst(P.InvRmed)[i] -
+                cst(P.Rmed)[i] * P.omega_frame;
+    const double v = v_r(i, p0, p1, sm, s0, x_vr);
+    if (z) {
+        const Damp f = damp_ring(P, false, i, dt);
+        sig = damp_value(S.stored(i, j, sig), x_s, f);
+        if (P.adiabatic) en = damp_value(E.stored(i, j, en), x_e, f);
+        va = damp_value(vaz.stored(i, j, va), x_va, f);
+    }
+    const double s_stored = S.set_get(i, j, sig);
+    const double e_stored = P.adiabatic ? E.set_get(i, j, en) : e_ghost;
+    vaz.set(i, j, va);
+    double g0, g1;  // ghost values of v_r
+    if (i == 1) {
+        ghost_vr_inner(P, v2, g0, g1);
+        vr.set(0, j, g0);
+        vr.set(1, j, g1);
+    } else {
+        vr.set(i, j, v);
+    }
+    if (i == nr - 2) {
+        ghost_vr_outer(P, vr.stored(i, j, v), g0, g1);
+        vr.set(nr, j, g0);
+        vr.set(nr - 1, j, g1);
+    }
+    auto derived = [&](int r, double e, double sv) {
+        DerivedIn d{e, sv, 0.0, 0.0};
+        if (!P.adiabatic) {
+            d.cs = cst(P.iso_cs)[r];
+            d.h = cst(P.iso_h)[r];
+        }
+        derived_store<SPLIT>(P, r, j, d, true, true);
+    };
+    derived(i, e_stored, s_stored);
     if (ghost) {
-        const int r = i == 0 ? 1 : nr - 2;  // the ring the ghost ring copies
-        vel_final_sig_e<SPLIT>(P, r, j, dt, sr, er, true);
-        // the ghost ring takes the neighbour's values as a load returns them
-        sr = S.stored(r, j, sr);
-        if (P.adiabatic) er = E.stored(r, j, er);
-        if (i == 0) ghost_vr_inner(P, vr.stored(2, j, vel_final_vr<SPLIT>(P, 2, j, dt)), va, vb);
-        else ghost_vr_outer(P, vr.stored(nr - 2, j, vel_final_vr<SPLIT>(P, nr - 2, j, dt)), va, vb);
-        vphi = ghost_vaz(P, i);
-    } else {
-        const Fld<false> Sb = buf<false>(P, P.sig_c, nullptr);
-        const Fld<false> m2 = mom_out(P, 2);
-        const Fld<false> m3 = mom_out(P, 3);
-        const int jm = j == 0 ? ns - 1 : j - 1;
-        const double s0 = Sb(i, j), sjm = Sb(i, jm);
-        const double msum = m2(i, jm) + m3(i, j);
-        const double v_phi = (SPLIT ? msum * recip<true>(sjm + s0) : msum / (sjm + s0)) * cst(P.InvRmed)[i] -
-                             cst(P.Rmed)[i] * P.omega_frame;
-        vphi = damp_stored<SPLIT>(P, vaz, FCPT_VAZI0, false, i, j, dt, v_phi);
-        if (i == 1) ghost_vr_inner(P, vr.stored(2, j, vel_final_vr<SPLIT>(P, 2, j, dt)), va, vb);
-        else vb = vel_final_vr<SPLIT>(P, i, j, dt);
-        vel_final_sig_e<SPLIT>(P, i, j, dt, sr, er, false);
+        const int g = i == 1 ? 0 : nr - 1;  // the ghost ring
+        const double sg = S.set_get(g, j, s_stored), eg = E.set_get(g, j, e_stored);
+        vaz.set(g, j, ghost_vaz(P, g));
+        derived(g, eg, sg);
     }
-    // stores: the ghost rings, v_r(1) of the ring-1 thread, or the cell's own
-    const double s_stored = S.set_get(i, j, sr);
-    double e_stored = 0.0;
-    if (ghost || P.adiabatic) e_stored = E.set_get(i, j, er);
-    vaz.set(i, j, vphi);
-    if (i == 0) {
-        vr.set(0, j, va);
-    } else if (i == nr - 1) {
-        vr.set(nr, j, va);
-        vr.set(nr - 1, j, vb);
-    } else {
-        vr.set(i, j, vb);  // v_r(1): the ghost value
-    }
-    if (advance_time && i == 0 && j == 0) advance_clock(P, advance_time);
-    DerivedIn d{P.adiabatic ? e_stored : 0.0, s_stored, 0.0, 0.0};
-    if (!P.adiabatic) {
-        d.cs = cst(P.iso_cs)[i];
-        d.h = cst(P.iso_h)[i];
-    }
-    derived_store<SPLIT>(P, i, j, d, true, true);
+    if (advance_time && i == 1 && j == 0) advance_clock(P, advance_time);
 }
 FCPT_PAIR1(velocities_final, 256, int, advance_time)
 
@@ -3994,7 +3980,7 @@ void launch_transport_ghost(const KParams &P, const KParams &out, hipStream_t st
     LAUNCH(k_ghost_ring_mean, dim3((unsigned)(gb + P.nr)), dim3(256), st, P);
     launch_radial_sweep(P, st);
     launch_azimuthal_sweep(P, st);
-    if (final_advance) LAUNCH(k_velocities_final, cell_grid(out, out.nr), kBlock, st, out, final_advance);
+    if (final_advance) LAUNCH(k_velocities_final, cell_grid(out, out.nr - 2), kBlock, st, out, final_advance);
     else LAUNCH(k_velocities, cell_grid(out, out.nr), kBlock, st, out);
 }
 
@@ -4509,7 +4495,7 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
     stage(B_AZIM_ADI, 0, adi, azim);
     // the velocity kernel with the final boundary call and the derived
     // fields writes the fields of every disk
-    stage_v(B_VEL_FINAL, 2, all, rows(0), false, true);
+    stage_v(B_VEL_FINAL, 2, all, rows(2), false, true);
     std::fill(view.begin(), view.end(), 0u);
     (void)ghosts;
     (void)cfl;
