@@ -481,7 +481,7 @@ class Disk:
         self._check(self.lib.fcpt_set_launch_param(self.h, PARAM_FUSED_STEP, 1 if fused else 0))
 
     def set_radial_tile(self, rings):
-        """Rings walked by one radial-sweep thread (0: size-based default)."""
+        """Rings per walk of the transport's sweeps (0: size-based default)."""
         self._check(self.lib.fcpt_set_launch_param(self.h, PARAM_RADIAL_TILE, rings))
 
     def set_visc_tile(self, rings):
@@ -533,7 +533,7 @@ class Disk:
         return {"kick_tile": k.value, "visc_tile": v.value}
 
     def set_radial_waves(self, waves):
-        """Register budget of the radial sweep in wavefronts per SIMD (2 or 3)."""
+        """Kept as set (2 or 3), without effect: the sweeps have one register budget."""
         self._check(self.lib.fcpt_set_launch_param(self.h, PARAM_RADIAL_WAVES, waves))
 
 
@@ -569,9 +569,8 @@ class Batch:
             pass
 
     def autotune(self, reps=10):
-        """Time the batched radial sweep's tiles and register budgets on the
-        current state and keep the fastest; returns {"radial_tile": t,
-        "radial_waves": w}."""
+        """Time the batched sweeps' tiles on the current state and keep the
+        fastest; returns {"radial_tile": t, "radial_waves": w} (w as set)."""
         t, w = C.c_int32(), C.c_int32()
         self._check(self.lib.fcpt_batch_autotune(self.h, reps, C.byref(t), C.byref(w)))
         return {"radial_tile": t.value, "radial_waves": w.value}

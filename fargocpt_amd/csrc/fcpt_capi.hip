@@ -487,11 +487,6 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
     if (!rc) rc = dev_alloc_bytes(c, &P.valt[1], field_rows(FCPT_VAZI, nr) * ns * esz);
     if (!rc && P.adiabatic) rc = dev_alloc_bytes(c, &P.ealt, field_rows(FCPT_ENERGY, nr) * ns * esz);
     for (int k = 0; k < 4 && !rc; ++k) rc = dev_alloc_bytes(c, &P.mom[k], ncell * sizeof(double));  // FP64 in both modes
-    for (int k = 0; k < 4 && !rc; ++k) rc = dev_alloc_bytes(c, &P.mom_b[k], ncell * esz);
-    // the density and energy between the transport sweeps stay FP64 in both
-    // storage modes: they are rounded once per step, on the final store
-    if (!rc) rc = dev_alloc_bytes(c, &P.sig_b, ncell * sizeof(double));
-    if (!rc) rc = dev_alloc_bytes(c, &P.en_b, ncell * sizeof(double));
     if (!rc) rc = dev_alloc_bytes(c, &P.sig_c, ncell * sizeof(double));
     if (!rc) rc = dev_alloc_bytes(c, &P.en_c, ncell * sizeof(double));
     if (P.split) {
@@ -504,6 +499,7 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
     if (!rc) rc = dev_alloc(c, &P.iso_h, (size_t)nr + 2);
     if (!rc) rc = dev_alloc(c, &P.iso_nu, (size_t)nr + 2);
     if (!rc) rc = dev_alloc(c, &P.ring_tab, (size_t)kRingTabs * ((size_t)nr + 2));
+    if (!rc) rc = dev_alloc(c, &P.sweep_tab, kSweepTabs * ((size_t)nr + 2));
     if (!rc) rc = dev_alloc(c, &P.damp_tab, 8 * ((size_t)nr + 2));
     if (!rc) rc = dev_alloc(c, &P.vmean, (size_t)nr + 1);
     if (!rc) rc = dev_alloc(c, &P.vuni, (size_t)nr + 1);
@@ -1622,8 +1618,8 @@ int fcpt_time_kernel(fcpt_ctx *ctx, int32_t kernel, int32_t reps, double *ms_per
             launch_disk_force(ctx->P, ctx->stream, fb, ctx->force_sig1d, ctx->force_part,
                               ctx->force_out);
             break;
-        case FCPT_KERNEL_RADIAL_SWEEP: launch_radial_sweep(ctx->P, ctx->stream); break;
-        case FCPT_KERNEL_AZIMUTHAL: launch_azimuthal_sweep(ctx->P, ctx->stream); break;
+        case FCPT_KERNEL_RADIAL_SWEEP:  // one kernel runs both sweeps
+        case FCPT_KERNEL_AZIMUTHAL: launch_sweeps(ctx->P, ctx->stream); break;
         case FCPT_KERNEL_CFL: launch_cfl_cells(ctx->P, ctx->stream); break;
         case FCPT_KERNEL_STRESS: launch_stress(ctx->P, ctx->stream); break;
         case FCPT_KERNEL_POTENTIAL: launch_potential(ctx->P, ctx->stream); break;
@@ -1799,7 +1795,7 @@ int fcpt_get_launch_param(fcpt_ctx *ctx, int32_t param, int32_t *value)
     if (!ctx || !value) return FCPT_ERR_ARG;
     const KParams &P = ctx->P;
     switch (param) {
-    case FCPT_PARAM_RADIAL_TILE: *value = radial_tile_for(P.nr, P.ns, P.radial_tile); break;
+    case FCPT_PARAM_RADIAL_TILE: *value = resolve_sweep_tile(P); break;
     case FCPT_PARAM_RADIAL_WAVES: *value = P.radial_waves; break;
     case FCPT_PARAM_FUSED_STEP: *value = ctx->fused ? 1 : 0; break;
     case FCPT_PARAM_VISC_TILE: *value = resolve_visc_tile(P); break;
@@ -1820,34 +1816,28 @@ int fcpt_autotune(fcpt_ctx *ctx, int32_t reps, int32_t *radial_tile, int32_t *ra
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     KParams &P = ctx->P;
     const int tiles[] = {1, 2, 4, 8, 16, 32};
-    const int waves[] = {3, 2};
     double best = 1e300;
-    int best_t = radial_tile_for(P.nr, P.ns, 0), best_w = 3;
-    for (int w : waves) {
-        for (int t : tiles) {
-            if (t > P.nr) continue;
-            P.radial_tile = t;
-            P.radial_waves = w;
-            launch_radial_sweep(P, ctx->stream);  // warm-up
-            HIP_TRY(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-            for (int k = 0; k < reps; ++k) launch_radial_sweep(P, ctx->stream);
-            HIP_TRY(ctx, hipEventRecord(ctx->ev1, ctx->stream));
-            LAUNCH_CHECK(ctx);
-            HIP_TRY(ctx, hipEventSynchronize(ctx->ev1));
-            float ms = 0.f;
-            HIP_TRY(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-            if (ms < best) {
-                best = ms;
-                best_t = t;
-                best_w = w;
-            }
+    int best_t = resolve_sweep_tile(P);
+    for (int t : tiles) {
+        if (t > P.nr) continue;
+        P.radial_tile = t;
+        launch_sweeps(P, ctx->stream);  // warm-up
+        HIP_TRY(ctx, hipEventRecord(ctx->ev0, ctx->stream));
+        for (int k = 0; k < reps; ++k) launch_sweeps(P, ctx->stream);
+        HIP_TRY(ctx, hipEventRecord(ctx->ev1, ctx->stream));
+        LAUNCH_CHECK(ctx);
+        HIP_TRY(ctx, hipEventSynchronize(ctx->ev1));
+        float ms = 0.f;
+        HIP_TRY(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+        if (ms < best) {
+            best = ms;
+            best_t = t;
         }
     }
     P.radial_tile = best_t;
-    P.radial_waves = best_w;
     HIP_TRY(ctx, drop_graphs(ctx->step_graph));
     if (radial_tile) *radial_tile = best_t;
-    if (radial_waves) *radial_waves = best_w;
+    if (radial_waves) *radial_waves = P.radial_waves;
     return FCPT_OK;
 }
 
@@ -2202,7 +2192,7 @@ int bfail(fcpt_batch *b, int code, const char *msg)
 
 void enqueue_batch_step(const fcpt_batch *b, hipStream_t st)
 {
-    for (const BatchStageDev &s : b->stages) launch_batch_stage(b->Ps, s, b->split, b->radial_waves, st);
+    for (const BatchStageDev &s : b->stages) launch_batch_stage(b->Ps, s, b->split, st);
 }
 }  // namespace
 
@@ -2274,31 +2264,18 @@ int fcpt_batch_create(fcpt_ctx *const *disks, int32_t n_disks, fcpt_batch **out)
         host.push_back(P);
     }
     // The walks' tiles of the members that leave them to the size rule,
-    // chosen over the batch's wavefronts as the radial tile below (results
+    // chosen over the batch's wavefronts as the sweeps' tile below (results
     // do not depend on the tiles).
     resolve_kv_tiles(host);
     for (KParams &P : host)
         if (!kv_walk_applies(P)) P.visc_tile = resolve_visc_tile(P);
-    // The radial sweep's tile of the members that leave it to the size rule.
-    // A single disk's rule shrinks the tile until that disk alone fills the
-    // device with wavefronts; in a batch all members' blocks share one
-    // launch, so the tile is the largest that fills the device with the
-    // batch's wavefronts (fewer tiles, hence fewer window reloads at tile
-    // starts; the sweep's results do not depend on the tile).
+    // The sweeps' tile of the members that leave it to the size rule: all
+    // members' blocks share one launch, so one tile by the batch's wavefronts
+    // (the results do not depend on it).
     for (const KParams &P : host) b->auto_radial.push_back(P.radial_tile <= 0);
-    {
-        auto waves = [&](int t) {
-            long w = 0;
-            for (const KParams &P : host)
-                w += (long)((P.ns + 63) / 64) * ((P.nr + (P.radial_tile > 0 ? P.radial_tile : t) - 1) /
-                                                  (P.radial_tile > 0 ? P.radial_tile : t));
-            return w;
-        };
-        int t = 32;
-        while (t > 2 && waves(t) < 3072) t /= 2;
-        for (KParams &P : host)
-            if (P.radial_tile <= 0) P.radial_tile = t;
-    }
+    const int sweep_tile = resolve_sweep_tile(host);
+    for (KParams &P : host)
+        if (P.radial_tile <= 0) P.radial_tile = sweep_tile;
     b->host = host;
     int rc = hipSetDevice(b->device) == hipSuccess ? FCPT_OK : FCPT_ERR_DEVICE;
     if (!rc) rc = upload_batch_plan(b);
@@ -2419,8 +2396,8 @@ int fcpt_batch_time_kernel(fcpt_batch *b, int32_t kernel, int32_t reps, double *
     if (reps <= 0) return bfail(b, FCPT_ERR_ARG, "reps must be positive");
     int kinds[2] = {-1, -1};
     switch (kernel) {
-    case FCPT_KERNEL_RADIAL_SWEEP: kinds[0] = B_RADIAL_ISO; kinds[1] = B_RADIAL_ADI; break;
-    case FCPT_KERNEL_AZIMUTHAL: kinds[0] = B_AZIM_ISO; kinds[1] = B_AZIM_ADI; break;
+    case FCPT_KERNEL_RADIAL_SWEEP:  // one kernel runs both sweeps
+    case FCPT_KERNEL_AZIMUTHAL: kinds[0] = B_SWEEPS_ISO; kinds[1] = B_SWEEPS_ADI; break;
     case FCPT_KERNEL_CFL: kinds[0] = B_CFL_RINGS; break;
     case FCPT_KERNEL_POTENTIAL: kinds[0] = B_POTENTIAL; break;
     case FCPT_KERNEL_STRESS:
@@ -2436,7 +2413,7 @@ int fcpt_batch_time_kernel(fcpt_batch *b, int32_t kernel, int32_t reps, double *
     auto one = [&]() {
         for (const BatchStageDev &s : b->stages) {
             if (s.kind != kinds[0] && s.kind != kinds[1]) continue;
-            launch_batch_stage(b->Ps, s, b->split, b->radial_waves, b->stream);
+            launch_batch_stage(b->Ps, s, b->split, b->stream);
         }
     };
     BHIP(b, hipStreamSynchronize(b->stream));
@@ -2452,10 +2429,10 @@ int fcpt_batch_time_kernel(fcpt_batch *b, int32_t kernel, int32_t reps, double *
     return FCPT_OK;
 }
 
-// The batch's radial tile (for the members that leave it to the size rule)
-// and register budget by the radial stage's time: each candidate's plan is
-// uploaded and its radial stage timed over `reps` launches, which write the
-// transport's scratch arrays only, so the disks' state is untouched.
+// The batch's sweep tile (for the members that leave it to the size rule) by
+// the sweeps' time: each candidate's plan is uploaded and the sweeps timed over
+// `reps` launches, which write the transport's scratch arrays only, so the
+// disks' state is untouched.
 int fcpt_batch_autotune(fcpt_batch *b, int32_t reps, int32_t *radial_tile, int32_t *radial_waves)
 {
     if (!b) return FCPT_ERR_ARG;
@@ -2465,33 +2442,28 @@ int fcpt_batch_autotune(fcpt_batch *b, int32_t reps, int32_t *radial_tile, int32
     int cur_t = 0;
     for (size_t k = 0; k < b->host.size(); ++k)
         if (b->auto_radial[k]) cur_t = b->host[k].radial_tile;
-    int best_t = cur_t, best_w = b->radial_waves;
+    int best_t = cur_t;
     double best = 1e300;
     const int tiles[] = {4, 8, 16, 32};
-    for (int w : {3, 2}) {
-        for (int t : tiles) {
-            if (cur_t == 0 && t != tiles[0]) break;  // no member's tile is the batch's to choose
-            for (size_t k = 0; k < b->host.size(); ++k)
-                if (b->auto_radial[k]) b->host[k].radial_tile = t;
-            int rc = upload_batch_plan(b);
-            b->radial_waves = w;
-            double ms = 0.0;
-            if (!rc) rc = fcpt_batch_time_kernel(b, FCPT_KERNEL_RADIAL_SWEEP, reps, &ms);
-            if (rc) return rc;
-            if (ms < best) {
-                best = ms;
-                best_t = t;
-                best_w = w;
-            }
+    for (int t : tiles) {
+        if (cur_t == 0) break;  // no member's tile is the batch's to choose
+        for (size_t k = 0; k < b->host.size(); ++k)
+            if (b->auto_radial[k]) b->host[k].radial_tile = t;
+        int rc = upload_batch_plan(b);
+        double ms = 0.0;
+        if (!rc) rc = fcpt_batch_time_kernel(b, FCPT_KERNEL_RADIAL_SWEEP, reps, &ms);
+        if (rc) return rc;
+        if (ms < best) {
+            best = ms;
+            best_t = t;
         }
     }
     for (size_t k = 0; k < b->host.size(); ++k)
         if (b->auto_radial[k]) b->host[k].radial_tile = best_t;
-    b->radial_waves = best_w;
     const int rc = upload_batch_plan(b);
     if (rc) return rc;
     if (radial_tile) *radial_tile = best_t;
-    if (radial_waves) *radial_waves = best_w;
+    if (radial_waves) *radial_waves = b->radial_waves;
     return FCPT_OK;
 }
 

@@ -62,6 +62,9 @@ struct DevScalars {
     DevPlanet planet_first[kMaxPlanets];
 };
 
+// values per ring of KParams::sweep_tab
+enum SweepTab { SW_RMED = 0, SW_INV_DIFF_RMED, SW_RINF, SW_INV_SURF, SW_WIDTH, SW_DXTHETA, SW_INV_DXTHETA, kSweepTabs = 8 };
+
 struct KParams {
     int nr, ns;
     double dphi, invdphi;
@@ -96,8 +99,8 @@ struct KParams {
     // storage: 0 = FP64 fields; 1 = FP32 deviations from FP64 per-ring backgrounds
     int split;
     int split_rounding;  // split storage: 0 rounds deviations to nearest, 1 stochastically
-    int radial_tile;     // rings per thread of the radial sweep (0: size-based choice)
-    int radial_waves;    // register budget of the radial sweep: wavefronts per SIMD (2 or 3)
+    int radial_tile;     // rings per walk of the transport's sweeps (0: size-based choice)
+    int radial_waves;    // FCPT_PARAM_RADIAL_WAVES as set (2 or 3); the sweeps have one register budget
     int visc_tile;       // rings per thread of the fused viscous pass (0: size-based choice)
     int kick_tile;       // rings per thread of the kick walk (0: size-based choice, 1: off)
     int kv_tile;         // batches: the kick walk's rings per thread, chosen over the batch
@@ -119,14 +122,10 @@ struct KParams {
     // split storage: per-ring backgrounds of every field (nr + 2 values each;
     // null in FP64 mode); the potential's is rewritten by the potential kernel
     double *bg[FCPT_NUM_FIELDS];
-    // transport work arrays: the momenta between the sweeps (mom_b) have the
-    // fields' element type; the azimuthal sweep's momenta (mom, read by the
-    // end of the step) and the density and energy between the sweeps are
-    // FP64 in both storage modes
-    void *mom[4];        // radial momentum +/-, angular momentum +/- (FP64)
-    void *mom_b[4];      // the radial sweep's momenta
-    void *sig_b, *en_b;  // radial-sweep outputs
-    void *sig_c, *en_c;  // azimuthal-sweep outputs
+    // what the transport's sweeps write and the end of the step reads, FP64 in
+    // both storage modes (rounded once per step, on the final store)
+    void *mom[4];        // radial momentum +/-, angular momentum +/-
+    void *sig_c, *en_c;  // density and energy
     void *valt[2];       // partners of v_r and v_phi for the fused step kernels
     void *ealt;          // partner of E (adiabatic disks)
     double *bgm[4];      // backgrounds of the four momenta (split storage)
@@ -134,6 +133,8 @@ struct KParams {
     // kRingTabs values per ring, nr + 2 rings (k_ring_tables): one base pointer
     // and one run of memory per ring for the walks' scalar loads
     double *ring_tab;
+    // the transport's ring constants, kSweepTabs per ring of one 64-byte line (k_ring_tables)
+    double *sweep_tab;
     double *damp_tab;     // per ring: the damping's squared ramp and time scale: scalar inner, outer, vector inner, outer
     double energy_per_t;  // R / mu / (gamma - 1): energy_at's factor, to rounding
     int const_ok;         // the physical constants lie in the range quot_in assumes

@@ -1699,6 +1699,14 @@ __global__ void __launch_bounds__(256) k_ring_tables(KParams P, double *out)
     tab[TAB_SIGMA_FLOOR10] = 10.0 * P.sigma0 * P.sigma_floor;
     tab[TAB_BETA_INV] = 1 / P.cooling_beta;
     tab[TAB_ARTVISC_SQ] = P.artvisc_factor * P.artvisc_factor;
+    double *sw = P.sweep_tab + (size_t)i * kSweepTabs;
+    sw[SW_RMED] = P.Rmed[i];
+    sw[SW_INV_DIFF_RMED] = P.InvDiffRmed[i];
+    sw[SW_RINF] = P.Rinf[i];
+    sw[SW_INV_SURF] = P.InvSurf[i];
+    sw[SW_WIDTH] = P.Rsup[i] - P.Rinf[i];
+    sw[SW_DXTHETA] = dxtheta;
+    sw[SW_INV_DXTHETA] = 1.0 / dxtheta;
     for (int v = 0; v < 2; ++v) {
         double *t = P.damp_tab + 8 * i + 4 * v;
         const double r = v ? P.Rinf[i] : P.Rmed[i < P.nr ? i : P.nr - 1];
@@ -3060,22 +3068,6 @@ FCPT_PAIR1(final_leapfrog, 256, int, advance_time)
 // ---------------------------------------------------------------------------
 // Transport
 
-// One ring of the radial sweep's window: Sigma, the advected quantities other
-// than the density (four momenta, and E when adiabatic: NQ of them), their
-// specific values Q / Sigma, the van Leer slopes of Sigma and of each
-// specific value, and v_r at the ring's inner interface.  The momenta are
-// formed with the expressions of compute_momenta_from_velocities
-// (TransportEuler.cpp:471-495).  Rings outside the grid hold Sigma = 1 and
-// zero quantities; the reference's interface values never reach them.  The
-// density's own specific value Sigma / Sigma is exactly 1 for the positive
-// Sigma the floor guarantees, so its interface value is 1 on interior
-// interfaces and 0 on the two edge interfaces.
-template <int NQ>
-struct RingW {
-    double s, w[NQ], q[NQ], v;
-    double ds, dw[NQ];
-};
-
 // The ring's stored values, loaded a ring ahead of their use so that the
 // loads are in flight while the previous ring is processed.  Loads go to a
 // clamped ring and the results are selected, so the loop body has no branch.
@@ -3104,8 +3096,75 @@ __device__ __forceinline__ void raw_ring(const KParams &P, int r, int j, int jn,
     X.v1 = vr.raw(rv1, j);
 }
 
-template <bool SPLIT, bool ADI, int NQ>
-__device__ __forceinline__ void decode_ring(const KParams &P, const RingRaw<SPLIT, ADI> &X, RingW<NQ> &R)
+// ---------------------------------------------------------------------------
+// Both sweeps of the transport as one walk: OneWindRad and VanLeerRadial
+// (TransportEuler.cpp:138-168, 545-619), then OneWindTheta (:270-289) with
+// QuantitiesAdvection of the residual velocity v - <v> and of the ring's
+// uniform residual (:292-304, VanLeerTheta :630-664) and AdvectSHIFT (:238-268).
+// A wavefront owns 57 sectors (64 with the halo) and walks `tile` rings
+// outward, a sector per lane.  Its window holds the rings k-1 and k with their
+// slopes and ring k+1: each ring is loaded once, each slope and each interface
+// flux formed once.  Ring k-1, once updated by its two radial fluxes, goes
+// through both azimuthal passes in registers, a sector's neighbours being the
+// adjacent lanes (DPP moves), and is written to its shifted place.
+// Why one kernel: two kernels wrote the radially swept Sigma, E and momenta and
+// read them back (96 of 176 bytes per cell).  Those bytes bound them on large
+// grids (4.7 and 4.3 TB/s), and a launch bounds them on small ones; this walk
+// is bound by FP64 instructions (three wavefronts per SIMD).  Step times with
+// two kernels and now: 128x384 isothermal 36.5 -> 29.6 us, 307x1021 beta 80.0
+// -> 69.8, 1024x3072 adiabatic 345.7 -> 306, 2048x6144 isothermal 877 -> 769,
+// 4096x12288 beta 5034 -> 4550, split 4052 -> 3731.
+// Prefetching the ring constants an iteration ahead costs scalar registers:
+// 2 to 4 % slower.
+__device__ __forceinline__ double sweep_tab(const KParams &P, int t, int i)
+{
+    return cst(P.sweep_tab)[i * kSweepTabs + t];
+}
+
+// n / D.d by the shared reciprocal, for |n| below 2^900 and D.d in
+// [2^-100, 2^100); below 2^-900 the quotient may be off by a unit of its last place
+__device__ __forceinline__ double quot_fast(double n, const SharedDen &D)
+{
+    const double q0 = n * D.r;
+    return fma(fma(-D.d, q0, n), D.r, q0);
+}
+
+// half the van Leer limiter of the differences a and b: a b / (a + b) where
+// they have one sign, else zero.  FINE: both below 2^500 in magnitude, so the
+// quotient by the refined reciprocal is the IEEE one (of products below
+// 2^-900 but for its last place)
+template <bool SPLIT, bool FINE>
+__device__ __forceinline__ double vl_half(double a, double b)
+{
+    if constexpr (SPLIT || !FINE) {
+        return 0.5 * vl_lim<SPLIT>(a, b);
+    } else {
+        const double p = a * b;
+        const double q = quot_fast(p, shared_den(a + b));
+        return p > 0.0 ? q : 0.0;
+    }
+}
+// magnitude below 2^400 (false for NaN)
+__device__ __forceinline__ bool sweep_range(double x) { return fabs(x) < 0x1p400; }
+
+// One ring of the walk's window: Sigma, v_phi, NQ advected quantities, their
+// specific values, v_r at the inner interface and the half slopes.  The
+// momenta are formed with the expressions of compute_momenta_from_velocities
+// (TransportEuler.cpp:471-495).  Rings outside the grid hold Sigma = 1 and
+// zero quantities; the reference's interface values never reach them.  The
+// density's own specific value Sigma / Sigma is exactly 1 for the positive
+// Sigma the floor guarantees, so its interface value is 1 on interior
+// interfaces and 0 on the two edge interfaces.
+template <int NQ>
+struct SweepRing {
+    double s, va, v, ds;
+    double w[NQ], q[NQ], dw[NQ];
+    bool fine;  // of the whole wavefront: Sigma and the specific values are in the fast quotients' range
+};
+
+// quantities Q0 .. Q0 + NQ - 1 of (four momenta, E)
+template <bool SPLIT, bool ADI, int Q0, int NQ>
+__device__ __forceinline__ void sweep_decode(const KParams &P, const RingRaw<SPLIT, ADI> &X, SweepRing<NQ> &R)
 {
     const int r = X.r;
     const bool in = r >= 0 && r < P.nr;
@@ -3115,42 +3174,73 @@ __device__ __forceinline__ void decode_ring(const KParams &P, const RingRaw<SPLI
     FLD(vr, FCPT_VRAD);
     FLD(vaz, FCPT_VAZI);
     const double sig = fld<SPLIT>(P, FCPT_SIGMA).dec(rc, X.sig);
-    const double rr = cst(P.Rmed)[rc];
+    const double rr = sweep_tab(P, SW_RMED, rc);
     const double OmegaF = P.omega_frame;
     const double v0 = vr.dec(rv, X.v0);  // v_r(r), r inside the grid or r == nr
-    double q[NQ];
-    q[0] = sig * vr.dec(rv1, X.v1);      // v_r(r + 1) for r inside the grid
-    q[1] = sig * v0;
-    q[2] = sig * (vaz.dec(rc, X.vaj) + rr * OmegaF) * rr;
-    q[3] = sig * (vaz.dec(rc, X.va) + rr * OmegaF) * rr;
-    if constexpr (ADI) q[4] = fld<SPLIT>(P, FCPT_ENERGY).dec(rc, X.e);
+    R.va = vaz.dec(rc, X.va);
+    double all[5];
+    all[0] = sig * vr.dec(rv1, X.v1);    // v_r(r + 1) for r inside the grid
+    all[1] = sig * v0;
+    all[2] = sig * (vaz.dec(rc, X.vaj) + rr * OmegaF) * rr;
+    all[3] = sig * (R.va + rr * OmegaF) * rr;
+    if constexpr (ADI) all[4] = fld<SPLIT>(P, FCPT_ENERGY).dec(rc, X.e);
     R.v = (r >= 0 && r <= P.nr) ? v0 : 0.0;
     R.s = in ? sig : 1.0;
-    const double inv_sig = SPLIT ? recip<true>(sig) : 0.0;
-    const SharedDen dsig = shared_den(sig);
+    const double *q = all + Q0;
+    double w[NQ];
+    R.fine = true;
+    if constexpr (SPLIT) {
+        const double inv_sig = recip<true>(sig);
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) w[k] = q[k] * inv_sig;
+    } else {
+        const SharedDen D = shared_den(sig);
+        bool ok = quot_range(sig);
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) {
+            w[k] = quot_fast(q[k], D);
+            ok = ok && sweep_range(w[k]);
+        }
+        R.fine = __all(ok);
+        if (!R.fine) {
+            __builtin_amdgcn_s_sleep(0);  // a branch: the divisions are not formed and selected
+#pragma unroll
+            for (int k = 0; k < NQ; ++k) w[k] = q[k] / sig;
+        }
+    }
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
         R.q[k] = in ? q[k] : 0.0;
-        const double w = SPLIT ? q[k] * inv_sig : shared_div(q[k], dsig);
-        R.w[k] = in ? w : 0.0;
+        R.w[k] = in ? w[k] : 0.0;
     }
 }
 
-// van Leer slopes of ring k from rings k-1, k, k+1 (compute_star_radial first
-// loop, TransportEuler.cpp:355-371); zero on the ghost rings
-template <bool SPLIT, int NQ>
-__device__ __forceinline__ void ring_slopes(const KParams &P, int k, const RingW<NQ> &M, RingW<NQ> &C,
-                                            const RingW<NQ> &N)
+// half the van Leer slopes of ring k from rings k-1, k, k+1
+// (compute_star_radial first loop, TransportEuler.cpp:355-371); zero on the ghost rings
+template <bool SPLIT, bool FINE, int NQ>
+__device__ __forceinline__ void sweep_slopes_of(double im, double ip, bool act, const SweepRing<NQ> &M,
+                                                SweepRing<NQ> &C, const SweepRing<NQ> &N)
 {
-    const bool act = k > 0 && k < P.nr - 1;
-    const int kc = act ? k : 1;
-    const double im = cst(P.InvDiffRmed)[kc], ip = cst(P.InvDiffRmed)[kc + 1];
-    const double ds = vl_lim<SPLIT>((N.s - C.s) * ip, (C.s - M.s) * im);
+    const double ds = vl_half<SPLIT, FINE>((N.s - C.s) * ip, (C.s - M.s) * im);
     C.ds = act ? ds : 0.0;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const double dw = vl_lim<SPLIT>((N.w[q] - C.w[q]) * ip, (C.w[q] - M.w[q]) * im);
+        const double dw = vl_half<SPLIT, FINE>((N.w[q] - C.w[q]) * ip, (C.w[q] - M.w[q]) * im);
         C.dw[q] = act ? dw : 0.0;
+    }
+}
+template <bool SPLIT, int NQ>
+__device__ __forceinline__ void sweep_slopes(const KParams &P, int k, const SweepRing<NQ> &M, SweepRing<NQ> &C,
+                                             const SweepRing<NQ> &N)
+{
+    const bool act = k > 0 && k < P.nr - 1;
+    const int kc = act ? k : 1;
+    const double im = sweep_tab(P, SW_INV_DIFF_RMED, kc), ip = sweep_tab(P, SW_INV_DIFF_RMED, kc + 1);
+    if (SPLIT || (M.fine && C.fine && N.fine)) {
+        sweep_slopes_of<SPLIT, true, NQ>(im, ip, act, M, C, N);
+    } else {
+        __builtin_amdgcn_s_sleep(0);
+        sweep_slopes_of<SPLIT, false, NQ>(im, ip, act, M, C, N);
     }
 }
 
@@ -3159,324 +3249,188 @@ __device__ __forceinline__ void ring_slopes(const KParams &P, int k, const RingW
 // edge interfaces k = 0 and k = nr) and the flux dt dphi Rinf[k] Q* Sigma* v_r
 // of each quantity through it (VanLeerRadial, :545-619).  The reference's
 // varq_sup of ring k-1 and varq_inf of ring k are this same product, Rsup[k-1]
-// and Rinf[k] being the same radius.
+// and Rinf[k] being the same radius.  The slopes are halved, so the distances
+// are not.
 template <int NQ>
-__device__ __forceinline__ void interface_flux(const KParams &P, int k, const RingW<NQ> &A,
-                                               const RingW<NQ> &B, double dt, double *f, double &fs)
+__device__ __forceinline__ void sweep_flux(const KParams &P, int k, const SweepRing<NQ> &A, const SweepRing<NQ> &B,
+                                           double dt, double *f, double &fs)
 {
     const bool act = k > 0 && k < P.nr;
     const int kc = act ? k : 1;
     const double v = B.v;
-    const double fpos = (cst(P.Rmed)[kc] - cst(P.Rmed)[kc - 1] - v * dt) * 0.5;
-    const double fneg = (cst(P.Rmed)[kc + 1] - cst(P.Rmed)[kc] + v * dt) * 0.5;
+    const double fpos = sweep_tab(P, SW_RMED, kc) - sweep_tab(P, SW_RMED, kc - 1) - v * dt;
+    const double fneg = sweep_tab(P, SW_RMED, kc + 1) - sweep_tab(P, SW_RMED, kc) + v * dt;
     const bool up = v > 0.0;
     const double ds0 = up ? A.s + fpos * A.ds : B.s - fneg * B.ds;
     const double ds = act ? ds0 : 0.0;
-    const double dens = act ? 1.0 : 0.0;
-    const double c = dt * P.dphi * cst(P.Rinf)[k];
+    const double c = dt * P.dphi * sweep_tab(P, SW_RINF, k);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const double qs0 = up ? A.w[q] + fpos * A.dw[q] : B.w[q] - fneg * B.dw[q];
         const double qs = act ? qs0 : 0.0;
         f[q] = c * qs * ds * v;
     }
-    fs = c * dens * ds * v;
+    fs = c * (act ? 1.0 : 0.0) * ds * v;
 }
 
-// OneWindRad, TransportEuler.cpp:138-168 and VanLeerRadial :545-619.  Every
-// advected quantity of ring i is updated from rings i-2..i+2 of itself and of
-// the density before the sweep (DENSITY_INT), so all of them are done in one
-// pass that reads the state and writes separate outputs.  A thread owns one
-// sector and walks `tile` consecutive rings outward.  Its window holds rings
-// k-1 and k with their slopes and ring k+1: each ring is loaded once, each
-// slope and each interface flux formed once, and the upwind choice is a
-// select, so the loop body is one branch-free block the compiler can schedule
-// as a whole.
-template <bool SPLIT, bool ADI>
-__device__ __forceinline__ void radial_sweep(const KParams &P, int bx, int by, int tile)
+// Both FARGO passes (as az_ring) for this lane's sector of one ring, the
+// neighbour sectors in the adjacent lanes: s0, q0 the radially swept density
+// and quantities, v0 = v_phi - <v_phi>; s2, q2 the results.  The second pass
+// has one velocity vu, so each sector's interface value on its downstream
+// side is formed where its slope is, and only the flux moves between lanes.
+// Returns whether the quotients were in the fast form's range.
+template <bool SPLIT, bool FINE, bool UP, int NQ>
+__device__ __forceinline__ bool sweep_theta(double dt, double v0, double vu, double dxtheta, double invdx,
+                                            double dxrad, double invsurf, double s0, const double *q0, double &s2,
+                                            double *q2)
 {
-    constexpr int NQ = ADI ? 5 : 4;
+    auto slope = [&](double x) {
+        const double b = x - from_left(x);
+        return vl_half<SPLIT, FINE>(from_right(b), b) * invdx;
+    };
+    const double ks0 = v0 * dt, ksu = vu * dt;
+    const double lo_d = dxtheta - ks0, hi_d = dxtheta + ks0;
+    const bool up0 = ks0 > 0.0;
+    auto star0 = [&](double x) {  // the first pass's value at the interface to the left
+        const double d = slope(x);
+        const double lo = from_left(x) + lo_d * from_left(d), hi = x - hi_d * d;
+        return up0 ? lo : hi;
+    };
+    auto star1 = [&](double x) {  // the second pass's value at the downstream interface
+        const double d = slope(x);
+        return UP ? x + (dxtheta - ksu) * d : x - (dxtheta + ksu) * d;
+    };
+    auto div1 = [&](double F) { return UP ? from_left(F) - F : F - from_right(F); };
+    bool ok = true;
+    const double ds0 = star0(s0);
+    const double f0 = dxrad * ds0 * v0;
+    const double s1 = s0 + (f0 - from_right(f0)) * invsurf;
+    const double ds1 = star1(s1);
+    s2 = s1 + div1(dxrad * ds1 * vu) * invsurf;
+    const SharedDen D0 = SPLIT ? SharedDen{s0, recip<true>(s0), true} : shared_den(s0);
+    const SharedDen D1 = SPLIT ? SharedDen{s1, recip<true>(s1), true} : shared_den(s1);
+    if (!SPLIT) ok = quot_range(s0) && quot_range(s1);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const double w0 = SPLIT ? q0[q] * D0.r : FINE ? quot_fast(q0[q], D0) : q0[q] / s0;
+        const double fq = dxrad * star0(w0) * ds0 * v0;
+        const double q1 = q0[q] + (fq - from_right(fq)) * invsurf;
+        const double w1 = SPLIT ? q1 * D1.r : FINE ? quot_fast(q1, D1) : q1 / s1;
+        q2[q] = q1 + div1(dxrad * star1(w1) * ds1 * vu) * invsurf;
+        if (!SPLIT) ok = ok && sweep_range(w0) && sweep_range(w1);
+    }
+    return ok;
+}
+
+constexpr int kSweepSegW = 57;  // sectors written per wavefront
+
+template <bool SPLIT, bool ADI, int Q0, int NQ>
+__device__ __forceinline__ void b_sweeps(const KParams &P, int bx, int by, int tile)
+{
     const int ns = P.ns, nr = P.nr;
-    const int j = bx * 64 + (int)threadIdx.x;
+    const int lane = (int)threadIdx.x;
+    const int j0 = bx * kSweepSegW;
     const int i0 = by * tile;
-    if (j >= ns || i0 >= nr) return;
+    if (j0 >= ns || i0 >= nr) return;
+    const int Ls = ns - j0 < kSweepSegW ? ns - j0 : kSweepSegW;
+    int j = (j0 - 4 + lane) % ns;
+    if (j < 0) j += ns;
     const int jn = j == ns - 1 ? 0 : j + 1;
-    const double dt = P.s->dt;
-    RingW<NQ> A, B, C, D;
+    const double dt = *cst(&P.s->dt);
+    SweepRing<NQ> A, B, C, D;
     {
         RingRaw<SPLIT, ADI> X0, X1, X2, X3;
         raw_ring<SPLIT, ADI>(P, i0 - 2, j, jn, X0);
         raw_ring<SPLIT, ADI>(P, i0 - 1, j, jn, X1);
         raw_ring<SPLIT, ADI>(P, i0, j, jn, X2);
         raw_ring<SPLIT, ADI>(P, i0 + 1, j, jn, X3);
-        decode_ring<SPLIT, ADI, NQ>(P, X0, D);
-        decode_ring<SPLIT, ADI, NQ>(P, X1, A);
-        decode_ring<SPLIT, ADI, NQ>(P, X2, B);
-        decode_ring<SPLIT, ADI, NQ>(P, X3, C);
+        sweep_decode<SPLIT, ADI, Q0, NQ>(P, X0, D);
+        sweep_decode<SPLIT, ADI, Q0, NQ>(P, X1, A);
+        sweep_decode<SPLIT, ADI, Q0, NQ>(P, X2, B);
+        sweep_decode<SPLIT, ADI, Q0, NQ>(P, X3, C);
     }
-    ring_slopes<SPLIT, NQ>(P, i0 - 1, D, A, B);
-    ring_slopes<SPLIT, NQ>(P, i0, A, B, C);
+    sweep_slopes<SPLIT, NQ>(P, i0 - 1, D, A, B);
+    sweep_slopes<SPLIT, NQ>(P, i0, A, B, C);
     double f_prev[NQ], fs_prev;
-    interface_flux<NQ>(P, i0, A, B, dt, f_prev, fs_prev);
+    sweep_flux<NQ>(P, i0, A, B, dt, f_prev, fs_prev);
     const int iend = i0 + tile < nr ? i0 + tile : nr;
     RingRaw<SPLIT, ADI> X;
     raw_ring<SPLIT, ADI>(P, i0 + 2, j, jn, X);
+    const Fld<false> Sc = buf<false>(P, P.sig_c, nullptr), Ec = buf<false>(P, P.en_c, nullptr);
     for (int k = i0 + 1; k <= iend; ++k) {
-        decode_ring<SPLIT, ADI, NQ>(P, X, D);      // ring k+1
+        sweep_decode<SPLIT, ADI, Q0, NQ>(P, X, D);     // ring k+1
         raw_ring<SPLIT, ADI>(P, k + 2, j, jn, X);  // in flight during this iteration
-        ring_slopes<SPLIT, NQ>(P, k, B, C, D);            // ring k
+        sweep_slopes<SPLIT, NQ>(P, k, B, C, D);    // ring k
         A = B;
         B = C;
         C = D;
         double f[NQ], fs;
-        interface_flux<NQ>(P, k, A, B, dt, f, fs);
+        sweep_flux<NQ>(P, k, A, B, dt, f, fs);
         // ring k-1 lies between interfaces k-1 and k
         const int i = k - 1;
-        const double invs = cst(P.InvSurf)[i];
+        const double invs = sweep_tab(P, SW_INV_SURF, i);
+        double q0[NQ], q2[NQ], s2;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            buf<SPLIT>(P, P.mom_b[q], P.bgm[q], kBufMom + q).set(i, j, A.q[q] + (f_prev[q] - f[q]) * invs);
-        if constexpr (ADI) buf<false>(P, P.en_b, nullptr).set(i, j, A.q[4] + (f_prev[4] - f[4]) * invs);
-        buf<false>(P, P.sig_b, nullptr).set(i, j, A.s + (fs_prev - fs) * invs);
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) f_prev[q] = f[q];
-        fs_prev = fs;
-    }
-}
-
-// the radial sweep under two register budgets: 3 wavefronts per SIMD (168
-// VGPRs) or 2 (256 VGPRs)
-template <bool SPLIT, bool ADI>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_radial_sweep2(KParams P, int tile)
-{
-    const BlockXY bb = xcd_block();
-    radial_sweep<SPLIT, ADI>(P, bb.x, bb.y, tile);
-}
-template <bool SPLIT, bool ADI>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_radial_sweep3(KParams P, int tile)
-{
-    const BlockXY bb = xcd_block();
-    radial_sweep<SPLIT, ADI>(P, bb.x, bb.y, tile);
-}
-// batched forms: each disk's tile is its resolved radial_tile
-template <bool SPLIT, bool ADI>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
-    kb_radial_sweep2(const KParams *Ps, const BatchEntry *map)
-{
-    const BatchEntry e = batch_entry(map);
-    const KParams &P = batch_disk(Ps, e.disk);
-    radial_sweep<SPLIT, ADI>(P, (int)(e.yx & 0xffffu), (int)(e.yx >> 16), P.radial_tile);
-}
-template <bool SPLIT, bool ADI>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
-    kb_radial_sweep3(const KParams *Ps, const BatchEntry *map)
-{
-    const BatchEntry e = batch_entry(map);
-    const KParams &P = batch_disk(Ps, e.disk);
-    radial_sweep<SPLIT, ADI>(P, (int)(e.yx & 0xffffu), (int)(e.yx >> 16), P.radial_tile);
-}
-
-// van Leer slope of a sector from its two neighbours (the slope half of
-// ComputeStarTheta, TransportEuler.cpp:416-465)
-template <bool SPLIT>
-__device__ __forceinline__ double slope_theta(double q, double invdxtheta)
-{
-    return 0.5 * vl_lim<SPLIT>(from_right(q) - q, q - from_left(q)) * invdxtheta;
-}
-
-// upwind interface value between sector j-1 and sector j (the second half of
-// ComputeStarTheta): q, dq of sector j in this lane, of sector j-1 in the lane
-// to the left
-__device__ __forceinline__ double star_theta(double q, double dq, double dxtheta, double ksi)
-{
-    const double lo = from_left(q) + (dxtheta - ksi) * from_left(dq);
-    const double hi = q - (dxtheta + ksi) * dq;
-    return (ksi > 0.0) ? lo : hi;
-}
-
-// OneWindTheta, TransportEuler.cpp:270-289, in one pass per ring segment:
-// QuantitiesAdvection (:292-304, VanLeerTheta :630-664) with the residual
-// velocity v - <v>, then with the uniform residual of the ring, then
-// AdvectSHIFT (:238-268).  Each wavefront owns kAzSegW consecutive sectors of
-// one ring, two adjacent sectors per lane, and loads them with kAzHalo
-// sectors on either side; a sector's neighbours are the lane's other sector
-// or the adjacent lane's (one DPP move per neighbour pair), so the kernel
-// needs neither LDS nor barriers.  Each stencil step spoils one more sector
-// at either edge; after the two van Leer passes sectors kAzHalo .. 127 -
-// kAzHalo of the wavefront hold exact results, and the result of sector j is
-// written to sector j + Nshift.  The density's own specific value is exactly
-// 1 (positive Sigma), so its interface values are 1 and drop out of its
-// flux.  Every slope is formed once per sector and each interface selects its
-// upwind side.
-constexpr int kAzHalo = 4;
-constexpr int kAzSegW = 128 - 2 * kAzHalo;  // sectors written per wavefront
-constexpr int kAzWaves = 2;                 // wavefronts per block
-
-// the two sectors of a lane: a = 2 lane, b = 2 lane + 1 (within the segment)
-struct D2 {
-    double a, b;
-};
-__device__ __forceinline__ D2 left2(const D2 &x) { return D2{from_left(x.b), x.a}; }
-__device__ __forceinline__ D2 right2(const D2 &x) { return D2{x.b, from_right(x.a)}; }
-
-template <bool SPLIT>
-__device__ __forceinline__ D2 slope2(const D2 &q, double invdxtheta)
-{
-    const D2 r = right2(q), l = left2(q);
-    return D2{0.5 * vl_lim<SPLIT>(r.a - q.a, q.a - l.a) * invdxtheta,
-              0.5 * vl_lim<SPLIT>(r.b - q.b, q.b - l.b) * invdxtheta};
-}
-
-// upwind interface value between each sector and its left neighbour (the
-// second half of ComputeStarTheta)
-__device__ __forceinline__ D2 star2(const D2 &q, const D2 &dq, double dxtheta, const D2 &ksi)
-{
-    const D2 lq = left2(q), ldq = left2(dq);
-    const double loa = lq.a + (dxtheta - ksi.a) * ldq.a, hia = q.a - (dxtheta + ksi.a) * dq.a;
-    const double lob = lq.b + (dxtheta - ksi.b) * ldq.b, hib = q.b - (dxtheta + ksi.b) * dq.b;
-    return D2{(ksi.a > 0.0) ? loa : hia, (ksi.b > 0.0) ? lob : hib};
-}
-
-// star2 for a velocity of one sign on the whole ring (the uniform residual):
-// UP (ksi > 0) takes the left sector's side for both sectors, else the own
-__device__ __forceinline__ D2 star2_up(const D2 &q, const D2 &dq, double dxtheta, double ksi)
-{
-    const D2 lq = left2(q), ldq = left2(dq);
-    return D2{lq.a + (dxtheta - ksi) * ldq.a, lq.b + (dxtheta - ksi) * ldq.b};
-}
-__device__ __forceinline__ D2 star2_down(const D2 &q, const D2 &dq, double dxtheta, double ksi)
-{
-    return D2{q.a - (dxtheta + ksi) * dq.a, q.b - (dxtheta + ksi) * dq.b};
-}
-template <bool UP>
-__device__ __forceinline__ D2 star2_uniform(const D2 &q, const D2 &dq, double dxtheta, double ksi)
-{
-    return UP ? star2_up(q, dq, dxtheta, ksi) : star2_down(q, dq, dxtheta, ksi);
-}
-
-// flux into the sector through its left interface minus flux out through the
-// right one
-__device__ __forceinline__ D2 flux_div2(const D2 &f)
-{
-    const D2 r = right2(f);
-    double va = f.a, vb = f.b;
-    va -= r.a;
-    vb -= r.b;
-    return D2{va, vb};
-}
-
-// Both FARGO passes for this lane's two sectors of ring i (sources at
-// sectors jsa, jsb = jsa + 1): put(-1, .) receives the transported density
-// and put(q, .) each quantity's transported momentum (q = 0 .. 3) and energy
-// (q = 4), before the cyclic shift, as soon as it is formed (so its
-// registers are free for the next quantity).  The second pass's velocity is
-// the ring's uniform residual, so its upwind side is the same for every
-// sector: UP is its sign (ksi > 0), chosen once per ring by the caller.
-template <bool SPLIT, bool ADI, bool UP, class Put>
-__device__ __forceinline__ void az_ring(const KParams &P, int i, int jsa, int jsb, double dt, Put &&put)
-{
-    constexpr int NQ = ADI ? 5 : 4;
-    const double vm = cst(P.vmean)[i];
-    const double vu = cst(P.vuni)[i];
-    const double ksu = vu * dt;
-    const double dxtheta = P.dphi * cst(P.Rmed)[i];
-    const double invdxtheta = 1.0 / dxtheta;
-    const double dxrad = (cst(P.Rsup)[i] - cst(P.Rinf)[i]) * dt;
-    const double invsurf = cst(P.InvSurf)[i];
-    // every global load first
-    FLD(vaz, FCPT_VAZI);
-    const Fld<false> Sb = buf<false>(P, P.sig_b, nullptr);
-    const D2 s0{Sb(i, jsa), Sb(i, jsb)};
-    const D2 v0{vaz(i, jsa) - vm, vaz(i, jsb) - vm};
-    D2 q0[NQ];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const Fld<SPLIT> m = buf<SPLIT>(P, P.mom_b[q], P.bgm[q], kBufMom + q);
-        q0[q] = D2{m(i, jsa), m(i, jsb)};
-    }
-    if constexpr (ADI) {
-        const Fld<false> Eb = buf<false>(P, P.en_b, nullptr);
-        q0[4] = D2{Eb(i, jsa), Eb(i, jsb)};
-    }
-    const D2 ks0{v0.a * dt, v0.b * dt};
-    // density: first pass (residual velocity), then second pass (uniform residual)
-    const D2 ds0 = star2(s0, slope2<SPLIT>(s0, invdxtheta), dxtheta, ks0);
-    const D2 vd0 = flux_div2(D2{dxrad * ds0.a * v0.a, dxrad * ds0.b * v0.b});
-    const D2 s1{s0.a + vd0.a * invsurf, s0.b + vd0.b * invsurf};
-    const D2 ds1 = star2_uniform<UP>(s1, slope2<SPLIT>(s1, invdxtheta), dxtheta, ksu);
-    const D2 vd1 = flux_div2(D2{dxrad * ds1.a * vu, dxrad * ds1.b * vu});
-    put(-1, D2{s1.a + vd1.a * invsurf, s1.b + vd1.b * invsurf});
-    // the other quantities
-    const D2 inv_s0{SPLIT ? recip<true>(s0.a) : 0.0, SPLIT ? recip<true>(s0.b) : 0.0};
-    const D2 inv_s1{SPLIT ? recip<true>(s1.a) : 0.0, SPLIT ? recip<true>(s1.b) : 0.0};
-    const SharedDen s0a = shared_den(s0.a), s0b = shared_den(s0.b);
-    const SharedDen s1a = shared_den(s1.a), s1b = shared_den(s1.b);
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        const D2 w0{SPLIT ? q0[q].a * inv_s0.a : shared_div(q0[q].a, s0a),
-                    SPLIT ? q0[q].b * inv_s0.b : shared_div(q0[q].b, s0b)};
-        const D2 qs0 = star2(w0, slope2<SPLIT>(w0, invdxtheta), dxtheta, ks0);
-        const D2 vq0 = flux_div2(D2{dxrad * qs0.a * ds0.a * v0.a, dxrad * qs0.b * ds0.b * v0.b});
-        const D2 q1{q0[q].a + vq0.a * invsurf, q0[q].b + vq0.b * invsurf};
-        const D2 w1{SPLIT ? q1.a * inv_s1.a : shared_div(q1.a, s1a), SPLIT ? q1.b * inv_s1.b : shared_div(q1.b, s1b)};
-        const D2 qs1 = star2_uniform<UP>(w1, slope2<SPLIT>(w1, invdxtheta), dxtheta, ksu);
-        const D2 vq1 = flux_div2(D2{dxrad * qs1.a * ds1.a * vu, dxrad * qs1.b * ds1.b * vu});
-        put(q, D2{q1.a + vq1.a * invsurf, q1.b + vq1.b * invsurf});
-    }
-}
-
-template <bool SPLIT, bool ADI>
-__device__ __forceinline__ void b_azimuthal_sweep(const KParams &P, int bx, int by)
-{
-    constexpr int NQ = ADI ? 5 : 4;
-    const int ns = P.ns;
-    const int i = by;
-    const int lane = threadIdx.x & 63;
-    const int j0 = __builtin_amdgcn_readfirstlane(bx * kAzWaves + (int)(threadIdx.x >> 6)) * kAzSegW;
-    if (j0 >= ns) return;  // the whole wavefront
-    const int Ls = ns - j0 < kAzSegW ? ns - j0 : kAzSegW;
-    const double dt = P.s->dt;
-    const int nsh = cst(P.nshift)[i];
-    // this lane's sectors (offset k = 2 lane, 2 lane + 1 from the segment's
-    // first halo sector) and where their results go
-    const int ka = 2 * lane, kb = 2 * lane + 1;
-    int jsa = (j0 - kAzHalo + ka) % ns;
-    if (jsa < 0) jsa += ns;
-    const int jsb = jsa + 1 == ns ? 0 : jsa + 1;
-    int jda = (j0 - kAzHalo + ka + nsh) % ns;
-    if (jda < 0) jda += ns;
-    const int jdb = jda + 1 == ns ? 0 : jda + 1;
-    const bool wa = ka >= kAzHalo && ka < kAzHalo + Ls;
-    const bool wb = kb >= kAzHalo && kb < kAzHalo + Ls;
-    auto put = [&](int q, const D2 &v) {
-        if (q < 0) {
-            const Fld<false> Sc = buf<false>(P, P.sig_c, nullptr);
-            if (wa) Sc.set(i, jda, v.a);
-            if (wb) Sc.set(i, jdb, v.b);
-        } else if (q < 4) {
-            const Fld<false> m = mom_out(P, q);
-            if (wa) m.set(i, jda, v.a);
-            if (wb) m.set(i, jdb, v.b);
-        } else {
-            const Fld<false> Ec = buf<false>(P, P.en_c, nullptr);
-            if (wa) Ec.set(i, jda, v.a);
-            if (wb) Ec.set(i, jdb, v.b);
+        for (int q = 0; q < NQ; ++q) {
+            q0[q] = A.q[q] + (f_prev[q] - f[q]) * invs;
+            if (SPLIT && Q0 + q < 4)
+                q0[q] = buf<SPLIT>(P, nullptr, P.bgm[Q0 + q], kBufMom + Q0 + q).stored(i, j, q0[q]);
+            f_prev[q] = f[q];
         }
-    };
-    if (cst(P.vuni)[i] * dt > 0.0) az_ring<SPLIT, ADI, true>(P, i, jsa, jsb, dt, put);
-    else az_ring<SPLIT, ADI, false>(P, i, jsa, jsb, dt, put);
+        const double s0 = A.s + (fs_prev - fs) * invs;
+        fs_prev = fs;
+        const double v0 = A.va - cst(P.vmean)[i], vu = cst(P.vuni)[i];
+        const double dxtheta = sweep_tab(P, SW_DXTHETA, i), invdx = sweep_tab(P, SW_INV_DXTHETA, i);
+        const double dxrad = sweep_tab(P, SW_WIDTH, i) * dt;
+        const bool up = vu * dt > 0.0;
+        bool ok = up ? sweep_theta<SPLIT, true, true, NQ>(dt, v0, vu, dxtheta, invdx, dxrad, invs, s0, q0, s2, q2)
+                     : sweep_theta<SPLIT, true, false, NQ>(dt, v0, vu, dxtheta, invdx, dxrad, invs, s0, q0, s2, q2);
+        // lanes 0, 1, 62 and 63 hold no exact second pass and no result depends on it
+        if (!SPLIT && !__all(ok || lane < 2 || lane > 61)) {
+            __builtin_amdgcn_s_sleep(0);
+            if (up) sweep_theta<SPLIT, false, true, NQ>(dt, v0, vu, dxtheta, invdx, dxrad, invs, s0, q0, s2, q2);
+            else sweep_theta<SPLIT, false, false, NQ>(dt, v0, vu, dxtheta, invdx, dxrad, invs, s0, q0, s2, q2);
+        }
+        // the upstream side loses four lanes, the downstream one three
+        const int k0 = lane - (up ? 4 : 3);
+        int nsh = cst(P.nshift)[i];
+        if (nsh >= ns || nsh <= -ns) nsh %= ns;
+        int jd = j + nsh;
+        if (jd >= ns) jd -= ns;
+        if (jd < 0) jd += ns;
+        if (k0 >= 0 && k0 < Ls) {
+            if (Q0 == 0) Sc.set(i, jd, s2);
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) (Q0 + q < 4 ? mom_out(P, Q0 + q) : Ec).set(i, jd, q2[q]);
+        }
+    }
 }
 template <bool SPLIT, bool ADI>
-__global__ void __launch_bounds__(64 * kAzWaves) k_azimuthal_sweep(KParams P)
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_sweeps(KParams P, int tile)
 {
     const BlockXY bb = xcd_block();
-    b_azimuthal_sweep<SPLIT, ADI>(P, bb.x, bb.y);
+    b_sweeps<SPLIT, ADI, 0, ADI ? 5 : 4>(P, bb.x, bb.y, tile);
 }
 template <bool SPLIT, bool ADI>
-__global__ void __launch_bounds__(64 * kAzWaves) kb_azimuthal_sweep(const KParams *Ps, const BatchEntry *map)
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) kb_sweeps(const KParams *Ps, const BatchEntry *map)
 {
     const BatchEntry e = batch_entry(map);
-    b_azimuthal_sweep<SPLIT, ADI>(batch_disk(Ps, e.disk), (int)(e.yx & 0xffffu), (int)(e.yx >> 16));
+    const KParams &P = batch_disk(Ps, e.disk);
+    b_sweeps<SPLIT, ADI, 0, ADI ? 5 : 4>(P, (int)(e.yx & 0xffffu), (int)(e.yx >> 16), P.radial_tile);
+}
+// one quantity per block (the grid's z; the first one's blocks also write Sigma)
+template <bool SPLIT, bool ADI>
+__global__ void __launch_bounds__(64) k_sweeps_each(KParams P, int tile)
+{
+    const int bx = (int)blockIdx.x, by = (int)blockIdx.y;
+    switch (blockIdx.z) {
+    case 0: b_sweeps<SPLIT, ADI, 0, 1>(P, bx, by, tile); break;
+    case 1: b_sweeps<SPLIT, ADI, 1, 1>(P, bx, by, tile); break;
+    case 2: b_sweeps<SPLIT, ADI, 2, 1>(P, bx, by, tile); break;
+    case 3: b_sweeps<SPLIT, ADI, 3, 1>(P, bx, by, tile); break;
+    default:
+        if constexpr (ADI) b_sweeps<SPLIT, ADI, 4, 1>(P, bx, by, tile);
+    }
 }
 
 // compute_velocities_from_momenta (TransportEuler.cpp:498-535), then
@@ -3691,7 +3645,10 @@ __global__ void __launch_bounds__(256) k_copy4(KParams P, size_t n8)
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[q] = static_cast<const double *>(P.mom[q])[k];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) static_cast<double *>(P.mom_b[q])[k] = v[q];
+    for (int q = 0; q < 4; ++q) {
+        void *const to = q == 0 ? P.sig_c : q == 1 ? P.en_c : P.valt[q - 2];
+        static_cast<double *>(to)[k] = v[q];
+    }
 }
 
 // split storage: re-express a field's deviations about a new ring background
@@ -3903,55 +3860,68 @@ void launch_boundaries(const KParams &P, hipStream_t st, int final_call, int adv
     LAUNCH(k_ghost_bc, dim3((unsigned)((P.ns + 255) / 256)), dim3(256), st, P, advance_time);
 }
 
-// rings per radial-sweep thread: the longest walk that still gives every SIMD
-// of the 256 CUs three wavefronts (the kernel's register budget allows about
-// three), so that the four-ring window start is amortised where the grid is
-// large and the chip stays full where it is small
-int radial_tile_for(int nr, int ns, int requested)
+// Rings per walk of the transport's sweeps: a walk of t rings costs about
+// t + 1.5 ring times (its window start), and a ring time with n wavefronts on a
+// SIMD is 0.7 n + 1.2 us up to the three its registers allow, as latency is
+// left over, and 1.1 n beyond.  Measured step times at 512x1536 (tiles 1, 3,
+// 8, 16): 116, 107, 109, 120 us; at 1024x3072 (3, 8, 16, 32): 316, 306, 318,
+// 325; at 4096x12288 (8, 16, 32, 48): 4646, 4567, 4550, 4623.
+template <class Waves>
+static int sweep_best_tile(Waves &&waves)
 {
-    if (requested > 0) return requested;
-    const long waves_per_band = (long)((ns + 63) / 64);
-    int tile = 32;
-    while (tile > 2 && waves_per_band * ((nr + tile - 1) / tile) < 3072) tile /= 2;
-    return tile;
+    int best = 1;
+    double best_cost = 1e300;
+    for (int t = 1; t <= 32; ++t) {
+        const double n = std::ceil((double)waves(t) / 1024.0);
+        const double cost = (t + 1.5) * (n <= 3.0 ? 0.7 * n + 1.2 : 1.1 * n);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = t;
+        }
+    }
+    return best;
+}
+static long sweep_waves(const KParams &P, int tile)
+{
+    return (long)((P.ns + kSweepSegW - 1) / kSweepSegW) * ((P.nr + tile - 1) / tile);
+}
+int resolve_sweep_tile(const KParams &P)
+{
+    return P.radial_tile > 0 ? P.radial_tile : sweep_best_tile([&](int t) { return sweep_waves(P, t); });
+}
+int resolve_sweep_tile(const std::vector<KParams> &D)
+{
+    return sweep_best_tile([&](int t) {
+        long w = 0;
+        for (const KParams &P : D) w += sweep_waves(P, P.radial_tile > 0 ? P.radial_tile : t);
+        return w;
+    });
 }
 
-void launch_radial_sweep(const KParams &P, hipStream_t st)
+void launch_sweeps(const KParams &P, hipStream_t st)
 {
-    const int tile = P.radial_tile > 0 ? P.radial_tile : radial_tile_for(P.nr, P.ns, 0);
-    const dim3 g((unsigned)((P.ns + 63) / 64), (unsigned)((P.nr + tile - 1) / tile));
-    // register budget: 3 wavefronts per SIMD (168 VGPRs) or 2 (256 VGPRs)
-    const bool w2 = P.radial_waves == 2;
+    const int tile = resolve_sweep_tile(P);
+    dim3 g((unsigned)((P.ns + kSweepSegW - 1) / kSweepSegW), (unsigned)((P.nr + tile - 1) / tile));
+    // One quantity per block where every SIMD still gets at most one walk:
+    // each walk is then a third as long (32x64 isothermal step 26.2 -> 25.1 us),
+    // while on more walks the shared work repeated in each block costs more
+    // (128x384: 29.8 -> 32.1)
+    const int quantities = P.adiabatic ? 5 : 4;
+    const bool each = sweep_waves(P, tile) * quantities <= 1024;
+    if (each) g.z = (unsigned)quantities;
+#define SW(SP, AD)                                                                                \
+    do {                                                                                          \
+        if (each) hipLaunchKernelGGL((k_sweeps_each<SP, AD>), g, dim3(64), 0, st, P, tile);       \
+        else hipLaunchKernelGGL((k_sweeps<SP, AD>), g, dim3(64), 0, st, P, tile);                 \
+    } while (0)
     if (P.split) {
-        if (P.adiabatic) {
-            if (w2) hipLaunchKernelGGL((k_radial_sweep2<true, true>), g, dim3(64), 0, st, P, tile);
-            else hipLaunchKernelGGL((k_radial_sweep3<true, true>), g, dim3(64), 0, st, P, tile);
-        } else {
-            if (w2) hipLaunchKernelGGL((k_radial_sweep2<true, false>), g, dim3(64), 0, st, P, tile);
-            else hipLaunchKernelGGL((k_radial_sweep3<true, false>), g, dim3(64), 0, st, P, tile);
-        }
+        if (P.adiabatic) SW(true, true);
+        else SW(true, false);
     } else {
-        if (P.adiabatic) {
-            if (w2) hipLaunchKernelGGL((k_radial_sweep2<false, true>), g, dim3(64), 0, st, P, tile);
-            else hipLaunchKernelGGL((k_radial_sweep3<false, true>), g, dim3(64), 0, st, P, tile);
-        } else {
-            if (w2) hipLaunchKernelGGL((k_radial_sweep2<false, false>), g, dim3(64), 0, st, P, tile);
-            else hipLaunchKernelGGL((k_radial_sweep3<false, false>), g, dim3(64), 0, st, P, tile);
-        }
+        if (P.adiabatic) SW(false, true);
+        else SW(false, false);
     }
-}
-void launch_azimuthal_sweep(const KParams &P, hipStream_t st)
-{
-    const int waves = (P.ns + kAzSegW - 1) / kAzSegW;
-    const dim3 g((unsigned)((waves + kAzWaves - 1) / kAzWaves), (unsigned)P.nr);
-    const dim3 b(64 * kAzWaves);
-    if (P.split) {
-        if (P.adiabatic) hipLaunchKernelGGL((k_azimuthal_sweep<true, true>), g, b, 0, st, P);
-        else hipLaunchKernelGGL((k_azimuthal_sweep<true, false>), g, b, 0, st, P);
-    } else {
-        if (P.adiabatic) hipLaunchKernelGGL((k_azimuthal_sweep<false, true>), g, b, 0, st, P);
-        else hipLaunchKernelGGL((k_azimuthal_sweep<false, false>), g, b, 0, st, P);
-    }
+#undef SW
 }
 
 void launch_copy4(const KParams &P, hipStream_t st)
@@ -3968,9 +3938,8 @@ void launch_transport(const KParams &P, hipStream_t st) { launch_transport_to(P,
 // transported density and momenta and writes the velocities of view out
 void launch_transport_to(const KParams &P, const KParams &out, hipStream_t st)
 {
-    launch_radial_sweep(P, st);
     launch_ring_mean(P, st, 1);
-    launch_azimuthal_sweep(P, st);
+    launch_sweeps(P, st);
     LAUNCH(k_velocities, cell_grid(out, out.nr), kBlock, st, out);
 }
 
@@ -3978,8 +3947,7 @@ void launch_transport_ghost(const KParams &P, const KParams &out, hipStream_t st
 {
     const int gb = (P.ns + 255) / 256;
     LAUNCH(k_ghost_ring_mean, dim3((unsigned)(gb + P.nr)), dim3(256), st, P);
-    launch_radial_sweep(P, st);
-    launch_azimuthal_sweep(P, st);
+    launch_sweeps(P, st);
     if (final_advance) LAUNCH(k_velocities_final, cell_grid(out, out.nr - 2), kBlock, st, out, final_advance);
     else LAUNCH(k_velocities, cell_grid(out, out.nr), kBlock, st, out);
 }
@@ -4420,12 +4388,9 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
     auto ghosts = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         add_grid(v, d, (unsigned)((P.ns + 255) / 256), 1);
     };
-    auto radial = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
-        add_grid(v, d, sector_grid(P), (unsigned)((P.nr + P.radial_tile - 1) / P.radial_tile));
-    };
-    auto azim = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
-        const int waves = (P.ns + kAzSegW - 1) / kAzSegW;
-        add_grid(v, d, (unsigned)((waves + kAzWaves - 1) / kAzWaves), (unsigned)P.nr);
+    auto sweeps = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
+        add_grid(v, d, (unsigned)((P.ns + kSweepSegW - 1) / kSweepSegW),
+                 (unsigned)((P.nr + P.radial_tile - 1) / P.radial_tile));
     };
     auto damp = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         const int n_inner = (P.damp_ids[0] > P.damp_ids[1] ? P.damp_ids[0] : P.damp_ids[1]) + 1;
@@ -4489,10 +4454,8 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
     stage(B_GHOST_MEAN, 0, all, [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         add_grid(v, d, (unsigned)((P.ns + 255) / 256 + P.nr), 1);
     });
-    stage(B_RADIAL_ISO, 0, iso, radial);
-    stage(B_RADIAL_ADI, 0, adi, radial);
-    stage(B_AZIM_ISO, 0, iso, azim);
-    stage(B_AZIM_ADI, 0, adi, azim);
+    stage(B_SWEEPS_ISO, 0, iso, sweeps);
+    stage(B_SWEEPS_ADI, 0, adi, sweeps);
     // the velocity kernel with the final boundary call and the derived
     // fields writes the fields of every disk
     stage_v(B_VEL_FINAL, 2, all, rows(2), false, true);
@@ -4509,8 +4472,7 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
         else hipLaunchKernelGGL(kern<false>, dim3(S.n), block, 0, st, Ps, S.map, ##__VA_ARGS__);       \
     } while (0)
 
-void launch_batch_stage(const KParams *Ps, const BatchStageDev &S, int split, int radial_waves,
-                        hipStream_t st)
+void launch_batch_stage(const KParams *Ps, const BatchStageDev &S, int split, hipStream_t st)
 {
     const dim3 b256(256);
     switch (S.kind) {
@@ -4573,35 +4535,16 @@ void launch_batch_stage(const KParams *Ps, const BatchStageDev &S, int split, in
         }
         break;
     }
-    case B_RADIAL_ISO:
-    case B_RADIAL_ADI: {
-        const bool a = S.kind == B_RADIAL_ADI, w2 = radial_waves == 2;
-        const dim3 g(S.n), b(64);
-#define RADB(SP, AD)                                                                           \
-    do {                                                                                       \
-        if (w2) hipLaunchKernelGGL((kb_radial_sweep2<SP, AD>), g, b, 0, st, Ps, S.map);        \
-        else hipLaunchKernelGGL((kb_radial_sweep3<SP, AD>), g, b, 0, st, Ps, S.map);           \
-    } while (0)
+    case B_SWEEPS_ISO:
+    case B_SWEEPS_ADI: {
+        const bool a = S.kind == B_SWEEPS_ADI;
+        const dim3 g(S.n);
         if (split) {
-            if (a) RADB(true, true);
-            else RADB(true, false);
+            if (a) hipLaunchKernelGGL((kb_sweeps<true, true>), g, dim3(64), 0, st, Ps, S.map);
+            else hipLaunchKernelGGL((kb_sweeps<true, false>), g, dim3(64), 0, st, Ps, S.map);
         } else {
-            if (a) RADB(false, true);
-            else RADB(false, false);
-        }
-#undef RADB
-        break;
-    }
-    case B_AZIM_ISO:
-    case B_AZIM_ADI: {
-        const bool a = S.kind == B_AZIM_ADI;
-        const dim3 g(S.n), b(64 * kAzWaves);
-        if (split) {
-            if (a) hipLaunchKernelGGL((kb_azimuthal_sweep<true, true>), g, b, 0, st, Ps, S.map);
-            else hipLaunchKernelGGL((kb_azimuthal_sweep<true, false>), g, b, 0, st, Ps, S.map);
-        } else {
-            if (a) hipLaunchKernelGGL((kb_azimuthal_sweep<false, true>), g, b, 0, st, Ps, S.map);
-            else hipLaunchKernelGGL((kb_azimuthal_sweep<false, false>), g, b, 0, st, Ps, S.map);
+            if (a) hipLaunchKernelGGL((kb_sweeps<false, true>), g, dim3(64), 0, st, Ps, S.map);
+            else hipLaunchKernelGGL((kb_sweeps<false, false>), g, dim3(64), 0, st, Ps, S.map);
         }
         break;
     }

@@ -71,8 +71,7 @@ void launch_kick(const KParams &P, hipStream_t st, int fold_mode);
 // the potential; fold_mode >= 0: in the same launch, the CFL fold of
 // k_cfl_rings' slots (launch_cfl_cells) with that mode
 void launch_potential_fold(const KParams &P, hipStream_t st, int fold_mode);
-void launch_radial_sweep(const KParams &P, hipStream_t st);
-void launch_azimuthal_sweep(const KParams &P, hipStream_t st);
+void launch_sweeps(const KParams &P, hipStream_t st);
 void launch_cfl_cells(const KParams &P, hipStream_t st);
 void launch_copy4(const KParams &P, hipStream_t st);
 void launch_derived(const KParams &P, hipStream_t st);
@@ -101,8 +100,10 @@ void launch_export(const KParams &P, hipStream_t st, const ExportFields &x);
 size_t element_size(const KParams &P);
 // bytes per value of one field: the potential is FP64 in both storage modes
 size_t field_element_size(const KParams &P, int field);
-// rings per thread of the radial sweep (requested > 0 overrides the size-based choice)
-int radial_tile_for(int nr, int ns, int requested);
+// rings per walk of the transport's sweeps (a set tile, else the size-based choice)
+int resolve_sweep_tile(const KParams &P);
+// one tile for the disks of a batch that set none themselves
+int resolve_sweep_tile(const std::vector<KParams> &D);
 // fills the launch-shape fields of a disk's parameters (the CFL grid)
 void init_launch_fields(KParams &P);
 
@@ -125,7 +126,7 @@ struct BatchEntry {
 enum BatchKind {
     B_RING_MEAN, B_CFL_CELLS, B_CFL_FINAL, B_POTENTIAL, B_SRC_VR, B_SRC_VPHI,
     B_SRC_ENERGY, B_TW_Q, B_TW_VEL, B_SN_Q, B_SN_VEL, B_TEMP_FLOOR, B_RECALC_VISC, B_STRESS,
-    B_VISC_UPDATE, B_SUBSTEP3, B_GHOST, B_RADIAL_ISO, B_RADIAL_ADI, B_AZIM_ISO, B_AZIM_ADI,
+    B_VISC_UPDATE, B_SUBSTEP3, B_GHOST, B_SWEEPS_ISO, B_SWEEPS_ADI,
     B_VELOCITIES, B_DAMPING, B_DERIVED, B_SRC_FUSED, B_AV_FUSED, B_VISC_FUSED, B_FINAL_DERIVED,
     B_CFL_RINGS, B_CFL_FINAL_RINGS, B_KV_WALK, B_VISC_WALK, B_GHOST_MEAN, B_VEL_FINAL
 };
@@ -141,7 +142,6 @@ struct BatchStageDev {
 // the stages of one sim::run iteration for a set of disks (parameters as the
 // kernels see them, radial_tile resolved); stages no disk takes part in are left out
 std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &disks);
-void launch_batch_stage(const KParams *Ps, const BatchStageDev &s, int split, int radial_waves,
-                        hipStream_t st);
+void launch_batch_stage(const KParams *Ps, const BatchStageDev &s, int split, hipStream_t st);
 
 }  // namespace fcpt

@@ -261,6 +261,8 @@ int fcpt_run_steps(fcpt_ctx *ctx, int32_t n_steps, int32_t use_graph);
    and the mean duration of one launch of a single kernel of the step, timed
    the same way over `reps` back-to-back launches on the current state
    (FCPT_KERNEL_* below; the listed kernels do not modify their inputs).
+   FCPT_KERNEL_RADIAL_SWEEP and _AZIMUTHAL both time the kernel that runs the
+   transport's two sweeps.
    FCPT_KERNEL_DISK_FORCE times the launches of fcpt_disk_on_planet_accel
    (ring means, cell reduction, block reduction; no copy to the host) for two
    bodies, a star at the origin and a planet at (1, 0), with the self-gravity
@@ -286,10 +288,11 @@ int fcpt_time_copy(fcpt_ctx *ctx, int32_t reps, double *ms_per_launch, double *b
 
 /* Launch-shape tuning (no counterpart in the reference).  Results do not
    depend on the shapes:
-   FCPT_PARAM_RADIAL_TILE   rings walked by one thread of the radial sweep
-                            (1 .. 64; 0 restores the size-based default);
-   FCPT_PARAM_RADIAL_WAVES  the sweep's register budget in wavefronts per
-                            SIMD (2 or 3; default 3);
+   FCPT_PARAM_RADIAL_TILE   rings walked by one thread of the transport's
+                            sweeps (1 .. 64; 0 restores the size-based default);
+   FCPT_PARAM_RADIAL_WAVES  kept as set (2 or 3; default 3), without effect:
+                            the sweeps run as one kernel with one register
+                            budget;
    FCPT_PARAM_KICK_TILE     rings walked by one thread of the kick walk, which
                             runs the source terms, the artificial viscosity,
                             the viscous update and SubStep3 of the fused step
@@ -324,8 +327,7 @@ int fcpt_time_copy(fcpt_ctx *ctx, int32_t reps, double *ms_per_launch, double *b
    deterministic hash of the value, the cell, the field and the step count
    drawing the variate: unbiased, so a slowly changing value does not lose its
    sub-unit increments every step) for the evolved fields Sigma, v_r, v_phi, E
-   and the transported momenta between the two sweeps (after the second sweep
-   they are FP64), to nearest for the fields derived afresh every
+   and the radially swept momenta (after the azimuthal sweep they are FP64), to nearest for the fields derived afresh every
    step (1); stochastically for every field (2); to nearest everywhere (0). */
 /* FCPT_PARAM_REBASE_INTERVAL (split storage only; default 1000) moves the
    backgrounds to the current ring means (fcpt_rebase_backgrounds) after every
@@ -383,14 +385,14 @@ int fcpt_batch_create(fcpt_ctx *const *disks, int32_t n_disks, fcpt_batch **out)
 int fcpt_batch_destroy(fcpt_batch *batch);
 const char *fcpt_batch_last_error(const fcpt_batch *batch);
 int fcpt_batch_synchronize(fcpt_batch *batch);
-/* radial-sweep register budget for the whole batch (2 or 3 wavefronts per SIMD) */
+/* kept as set (2 or 3), without effect (FCPT_PARAM_RADIAL_WAVES) */
 int fcpt_batch_set_radial_waves(fcpt_batch *batch, int32_t waves);
-/* Autotuner (no counterpart in the reference): the radial sweep's tile of the
-   members that left it to the size rule (one tile for all of them, 4 .. 32
-   rings) and the batch's register budget, by the time of the batched radial
-   stage over `reps` launches on the current state (the timed launches write
-   the transport's scratch arrays only).  Keeps and returns the fastest;
-   drops a captured batch graph.  Results do not depend on the choice. */
+/* Autotuner (no counterpart in the reference): the sweeps' tile of the members
+   that left it to the size rule (one tile for all of them, 4 .. 32 rings), by
+   the time of the batched sweeps over `reps` launches on the current state
+   (the timed launches write the transport's scratch arrays only).  Keeps and
+   returns the fastest, and the register budget as set; drops a captured batch
+   graph.  Results do not depend on the choice. */
 int fcpt_batch_autotune(fcpt_batch *batch, int32_t reps, int32_t *radial_tile, int32_t *radial_waves);
 /* n_steps sim::run iterations of every disk; use_graph != 0 replays captured
    HIP graphs as fcpt_run_steps does.  No host synchronisation. */
