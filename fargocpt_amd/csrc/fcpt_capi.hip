@@ -44,10 +44,8 @@ struct fcpt_ctx {
     double *totals_ring = nullptr;
     double *totals_out = nullptr;
     double *totals_host = nullptr;
-    double *force_sig1d = nullptr;  // ring means of Sigma for the disk-force reduction
-    double *force_part = nullptr;   // per-block partial sums
-    double *force_out = nullptr;
-    double *force_host = nullptr;
+    double *force_part = nullptr;  // the disk force's partial sums per ring
+    double *force_host = nullptr;  // its result (pinned, written by the kernel)
     hipGraphExec_t step_graph[2] = {nullptr, nullptr};  // of one iteration and of kGraphSteps
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::string err;
@@ -509,9 +507,7 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
     if (!rc) rc = dev_alloc(c, &c->s_dev, 1);
     if (!rc) rc = dev_alloc(c, &c->totals_ring, 4 * (size_t)nr);
     if (!rc) rc = dev_alloc(c, &c->totals_out, 2);
-    if (!rc) rc = dev_alloc(c, &c->force_sig1d, (size_t)nr + 2);
-    if (!rc) rc = dev_alloc(c, &c->force_part, (size_t)kCflMaxBlocks * 4 * kForceMaxBodies);
-    if (!rc) rc = dev_alloc(c, &c->force_out, (size_t)4 * kForceMaxBodies);
+    if (!rc) rc = dev_alloc(c, &c->force_part, (size_t)nr * 4 * kForceMaxBodies);
     if (rc) {
         fcpt_destroy(c);
         return rc;
@@ -1438,9 +1434,11 @@ static void enqueue_step(const KParams &P, hipStream_t st, int count_monitor, bo
 // one sim::run iteration: CalculateTimeStep with the monitor clip (mode 2),
 // then the step; the fused Euler step folds the CFL minima inside its
 // potential launch (one launch less)
-static void enqueue_iteration(const fcpt_ctx *ctx, bool fused)
+// `report`: the step's clock goes to the pinned mirror as well
+static void enqueue_iteration(const fcpt_ctx *ctx, bool fused, bool report = false)
 {
-    const KParams V = step_view(ctx, fused);
+    KParams V = step_view(ctx, fused);
+    if (report) V.s_out = ctx->s_host;
     if (fused && V.integrator != FCPT_INTEGRATOR_LEAPFROG) {
         launch_cfl_cells(V, ctx->stream);
         enqueue_euler(V, ctx->stream, 1, true, 2);
@@ -1501,11 +1499,10 @@ int fcpt_run_step(fcpt_ctx *ctx, double *dt_out)
     CTX_CHECK(ctx);
     const bool fused = next_fused(ctx);
     if (!fused) sync_derived(ctx);
-    enqueue_iteration(ctx, fused);
+    enqueue_iteration(ctx, fused, true);
     LAUNCH_CHECK(ctx);
     stepped(ctx, fused);
-    int rc = read_scalars(ctx);
-    if (rc) return rc;
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     if (take_nonfinite(ctx))
         return fail(ctx, FCPT_ERR_NONFINITE, "CFL time step is not finite and positive");
     if (dt_out) *dt_out = ctx->s_host->dt;
@@ -1615,8 +1612,7 @@ int fcpt_time_kernel(fcpt_ctx *ctx, int32_t kernel, int32_t reps, double *ms_per
     auto one = [&]() {
         switch (kernel) {
         case FCPT_KERNEL_DISK_FORCE:
-            launch_disk_force(ctx->P, ctx->stream, fb, ctx->force_sig1d, ctx->force_part,
-                              ctx->force_out);
+            launch_disk_force(ctx->P, ctx->stream, fb, ctx->force_part, ctx->force_host);
             break;
         case FCPT_KERNEL_RADIAL_SWEEP:  // one kernel runs both sweeps
         case FCPT_KERNEL_AZIMUTHAL: launch_sweeps(ctx->P, ctx->stream); break;
@@ -1868,10 +1864,8 @@ int fcpt_disk_on_planet_accel(fcpt_ctx *ctx, const fcpt_force_body *bodies, int3
         else
             B.smooth_fixed[k] = -1.0;
     }
-    launch_disk_force(ctx->P, ctx->stream, B, ctx->force_sig1d, ctx->force_part, ctx->force_out);
+    launch_disk_force(ctx->P, ctx->stream, B, ctx->force_part, ctx->force_host);
     LAUNCH_CHECK(ctx);
-    HIP_TRY(ctx, hipMemcpyAsync(ctx->force_host, ctx->force_out, 4 * kForceMaxBodies * sizeof(double),
-                                hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     for (int k = 0; k < n_bodies; ++k) {
         const double *o = ctx->force_host + 4 * k;

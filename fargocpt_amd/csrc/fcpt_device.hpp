@@ -143,6 +143,7 @@ struct KParams {
     int *nshift;         // per-ring integer shift
     double *ring_min;    // CFL minima: per block (kCflMaxBlocks slots) or per ring (nr)
     DevScalars *s;
+    DevScalars *s_out;  // pinned host mirror that the step's clock is written to, or null
 };
 
 }  // namespace fcpt

@@ -2845,13 +2845,23 @@ FCPT_PAIR0(damping, 256)
 // Keplerian v_phi (boundary_conditions.cpp:67-97 and the BC files it dispatches to)
 // end of a sim::run iteration: time += dt and the monitor counter
 // (simulation.cpp:244, 545-551); nothing else in the kernels that call it
-// reads them
+// reads them.  A step whose caller waits for it writes the clock to the pinned
+// mirror from here: a copy after the step costs 6 to 8 us.
 __device__ __forceinline__ void advance_clock(const KParams &P, int advance_time)
 {
     DevScalars *s = P.s;
     const double time_next_monitor = (s->n_monitor + 1) * P.monitor_timestep;
     s->time = s->time + s->dt;
     if (advance_time == 2 && fabs(time_next_monitor - s->time) < 1e-6 * s->last_dt) s->n_monitor++;
+    if (DevScalars *out = P.s_out) {
+        out->dt = s->dt;
+        out->time = s->time;
+        out->last_dt = s->last_dt;
+        out->cfl_dt = s->cfl_dt;
+        out->n_monitor = s->n_monitor;
+        out->error_flags = s->error_flags;
+        out->step_count = s->step_count;
+    }
 }
 
 // the inner / outer ghost rings of sector j (rows 2 and nr-2 are never
@@ -4181,39 +4191,32 @@ void launch_totals(const KParams &P, hipStream_t st, double radius, double *ring
 // ---------------------------------------------------------------------------
 // The disk's gravity on the N bodies (ComputeDiskOnPlanetAccel, Force.cpp:23-122)
 
-// ComputeAverageDensity, Pframeforce.cpp:174-187: ring means of Sigma over the
-// active rings (pairwise tree order), one block per ring
-template <bool SPLIT>
-__global__ void __launch_bounds__(256) k_sigma_ring_mean(KParams P, double *sig1d)
-{
-    __shared__ double sh[256];
-    const int ns = P.ns;
-    const int i = blockIdx.x;
-    FLD(S, FCPT_SIGMA);
-    double acc = 0.0;
-    strided_row<256>(ns, (int)threadIdx.x, [&](int j) { return S(i, j); }, [&](double x) { acc += x; });
-    const double sum = block_sum<256>(acc, sh);
-    if (threadIdx.x == 0) sig1d[i] = sum / ns;
-}
-
 // Per cell and body, the reference's expression (the smoothing of
 // compute_smoothing, Force.cpp:145-159, chosen by the flags; the Klahr-Kley
 // factor 4q^3 - 3q^4 inside r_cubic); inner (Rmed < r_body) and outer sums
 // kept apart as in the reference.  NB bodies per launch (a template argument,
-// so only their accumulators live in registers).  A thread owns one sector
-// and walks the rings with a grid stride, loading the next ring's cell before
-// it works on the current one; 1 / d^3 comes from the reciprocal square root
-// with two Newton steps (a few ulp from the reference's sqrt and division).
-// Each block folds its 4 NB partial sums with wavefront shuffles and LDS into
-// its own slot (component-major, slot = block), and k_disk_force_final sums
-// each component's slots in a fixed order: deterministic, no atomics.
+// so only their accumulators live in registers).  One block per active ring:
+// it first forms the ring's mean Sigma where the flags ask for it
+// (ComputeAverageDensity, Pframeforce.cpp:174-187, pairwise tree order), with
+// the first cells' loads in flight, then a thread adds every 256th cell,
+// loading the next one before it works on the current one; 1 / d^3 comes from
+// the reciprocal square root with two Newton steps (a few ulp from the
+// reference's sqrt and division).  Each block folds its 4 NB partial sums with
+// wavefront shuffles and LDS into its own slot (component-major, slot = ring),
+// and k_disk_force_final sums each component's slots in a fixed order:
+// deterministic, no atomics.
+// What bounds it: latency on the grids that follow every step with it.  With
+// the means in a launch of their own and threads that walk several rings, the
+// force took 10.0 us for four bodies at 48x144 and 24.4 at 512x1536; now 7.7
+// and 11.2.  The result goes straight to pinned memory: the call took 35 us at
+// 48x144 with a copy, 24 without.
 template <bool SPLIT, int NB>
-__global__ void __launch_bounds__(256) k_disk_force(KParams P, ForceBodies B, const double *sig1d,
-                                                    double *part)
+__global__ void __launch_bounds__(256) k_disk_force(KParams P, ForceBodies B, double *part)
 {
     const int ns = P.ns;
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nslots = (int)(gridDim.x * gridDim.y);
+    const int t = (int)threadIdx.x;
+    const int i = 1 + (int)blockIdx.x;  // rings 1 .. nr - 2
+    const int nslots = (int)gridDim.x;
     double acc[NB][4];
 #pragma unroll
     for (int k = 0; k < NB; ++k) acc[k][0] = acc[k][1] = acc[k][2] = acc[k][3] = 0.0;
@@ -4221,59 +4224,56 @@ __global__ void __launch_bounds__(256) k_disk_force(KParams P, ForceBodies B, co
     FLD(Hf, FCPT_SCALE_HEIGHT);
     const double G = P.G;
     const double thick = P.thickness_smoothing;
-    const bool correct = (B.flags & FCPT_FORCE_CORRECT_SELFGRAVITY) != 0;
-    const int last = P.nr - 1;  // rings 1 .. nr - 2
-    const int stride = P.cfl_gy * (int)blockDim.y;
-    int i = wave_ring(1, (int)blockIdx.y);
-    if (j < ns && i < last) {
-        const double cphi = P.cosphi[j];
-        const double sphi = P.sinphi[j];
-        double sig = S(i, j);
-        double H = P.adiabatic ? Hf(i, j) : 0.0;
-        for (;;) {
-            const int in = i + stride;
-            const int ip = in < last ? in : i;
-            const double sig_n = S(ip, j);
-            const double H_n = P.adiabatic ? Hf(ip, j) : 0.0;
-            const double rmed = cst(P.Rmed)[i];
-            const double Hc = P.adiabatic ? H : cst(P.iso_h)[i];
-            const double xc = rmed * cphi;
-            const double yc = rmed * sphi;
-            const double cell_sigma = correct ? sig - cst(sig1d)[i] : sig;
-            const double gm = G * (cst(P.Surf)[i] * cell_sigma);
+    const double rmed = cst(P.Rmed)[i], surf = cst(P.Surf)[i];
+    const double H_ring = P.adiabatic ? 0.0 : cst(P.iso_h)[i];
+    const int j0 = t < ns ? t : 0;
+    double sig = S(i, j0), cphi = P.cosphi[j0], sphi = P.sinphi[j0];
+    double H = P.adiabatic ? Hf(i, j0) : H_ring;
+    double mean = 0.0;
+    if (B.flags & FCPT_FORCE_CORRECT_SELFGRAVITY) {
+        __shared__ double sh[256];
+        double sum = 0.0;
+        strided_row<256>(ns, t, [&](int j) { return S(i, j); }, [&](double x) { sum += x; });
+        mean = block_sum<256>(sum, sh) / ns;
+    }
+    for (int j = t; j < ns; j += 256) {
+        const int jn = j + 256 < ns ? j + 256 : j;
+        const double sig_n = S(i, jn), cphi_n = P.cosphi[jn], sphi_n = P.sinphi[jn];
+        const double H_n = P.adiabatic ? Hf(i, jn) : H_ring;
+        const double xc = rmed * cphi;
+        const double yc = rmed * sphi;
+        const double gm = G * (surf * (sig - mean));
 #pragma unroll
-            for (int k = 0; k < NB; ++k) {
-                const double smooth = B.smooth_fixed[k] >= 0.0 ? B.smooth_fixed[k] : thick * Hc;
-                const double dx = xc - B.x[k];
-                const double dy = yc - B.y[k];
-                const double d2 = (dx * dx + dy * dy) + smooth * smooth;
-                const double inv_d = inv_sqrt<true>(d2);
-                const double inv_d3 = inv_d * inv_d * inv_d;
-                double fx = gm * dx * inv_d3;
-                double fy = gm * dy * inv_d3;
-                const double r_sm = B.r_cubic[k];
-                if (r_sm > 0.0) {  // uniform: the body's cubic smoothing radius
-                    const double q = (d2 * inv_d) / r_sm;
-                    const double klahr = q < 1.0 ? q * q * q * (4.0 - 3.0 * q) : 1.0;
-                    fx *= klahr;
-                    fy *= klahr;
-                }
-                if (rmed < B.r[k]) {  // uniform: one ring against one body
-                    acc[k][0] += fx;
-                    acc[k][1] += fy;
-                } else {
-                    acc[k][2] += fx;
-                    acc[k][3] += fy;
-                }
+        for (int k = 0; k < NB; ++k) {
+            const double smooth = B.smooth_fixed[k] >= 0.0 ? B.smooth_fixed[k] : thick * H;
+            const double dx = xc - B.x[k];
+            const double dy = yc - B.y[k];
+            const double d2 = (dx * dx + dy * dy) + smooth * smooth;
+            const double inv_d = inv_sqrt<true>(d2);
+            const double inv_d3 = inv_d * inv_d * inv_d;
+            double fx = gm * dx * inv_d3;
+            double fy = gm * dy * inv_d3;
+            const double r_sm = B.r_cubic[k];
+            if (r_sm > 0.0) {  // uniform: the body's cubic smoothing radius
+                const double q = (d2 * inv_d) / r_sm;
+                const double klahr = q < 1.0 ? q * q * q * (4.0 - 3.0 * q) : 1.0;
+                fx *= klahr;
+                fy *= klahr;
             }
-            if (in >= last) break;
-            i = in;
-            sig = sig_n;
-            H = H_n;
+            if (rmed < B.r[k]) {  // uniform: one ring against one body
+                acc[k][0] += fx;
+                acc[k][1] += fy;
+            } else {
+                acc[k][2] += fx;
+                acc[k][3] += fy;
+            }
         }
+        sig = sig_n;
+        cphi = cphi_n;
+        sphi = sphi_n;
+        H = H_n;
     }
     __shared__ double wsum[4][NB * 4];
-    const int t = threadIdx.y * blockDim.x + threadIdx.x;
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
 #pragma unroll
@@ -4285,12 +4285,11 @@ __global__ void __launch_bounds__(256) k_disk_force(KParams P, ForceBodies B, co
     }
     __syncthreads();
     if (t < NB * 4)
-        part[(size_t)t * nslots + (blockIdx.y * gridDim.x + blockIdx.x)] =
-            (wsum[0][t] + wsum[1][t]) + (wsum[2][t] + wsum[3][t]);
+        part[(size_t)t * nslots + blockIdx.x] = (wsum[0][t] + wsum[1][t]) + (wsum[2][t] + wsum[3][t]);
 }
 
 // one block per component: the slots summed with a 256-wide stride, then a
-// pairwise tree over the 256 partial sums
+// pairwise tree over the 256 partial sums; out may be pinned host memory
 __global__ void __launch_bounds__(256) k_disk_force_final(const double *part, int nslots, double *out)
 {
     __shared__ double sh[256];
@@ -4301,41 +4300,31 @@ __global__ void __launch_bounds__(256) k_disk_force_final(const double *part, in
     if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
-template <bool SPLIT, int NB>
-static void launch_force_nb(const KParams &P, hipStream_t st, const ForceBodies &B, const double *sig1d,
-                            double *part, dim3 g)
-{
-    hipLaunchKernelGGL((k_disk_force<SPLIT, NB>), g, kBlock, 0, st, P, B, sig1d, part);
-}
-
 template <bool SPLIT>
-static void launch_force_split(const KParams &P, hipStream_t st, const ForceBodies &B,
-                               const double *sig1d, double *part, dim3 g)
+static void launch_force_split(const KParams &P, hipStream_t st, const ForceBodies &B, double *part, dim3 g)
 {
+#define FORCE(N) hipLaunchKernelGGL((k_disk_force<SPLIT, N>), g, dim3(256), 0, st, P, B, part)
     switch (B.n) {
-    case 1: launch_force_nb<SPLIT, 1>(P, st, B, sig1d, part, g); break;
-    case 2: launch_force_nb<SPLIT, 2>(P, st, B, sig1d, part, g); break;
-    case 3: launch_force_nb<SPLIT, 3>(P, st, B, sig1d, part, g); break;
-    case 4: launch_force_nb<SPLIT, 4>(P, st, B, sig1d, part, g); break;
-    case 5: launch_force_nb<SPLIT, 5>(P, st, B, sig1d, part, g); break;
-    case 6: launch_force_nb<SPLIT, 6>(P, st, B, sig1d, part, g); break;
-    case 7: launch_force_nb<SPLIT, 7>(P, st, B, sig1d, part, g); break;
-    default: launch_force_nb<SPLIT, 8>(P, st, B, sig1d, part, g); break;
+    case 1: FORCE(1); break;
+    case 2: FORCE(2); break;
+    case 3: FORCE(3); break;
+    case 4: FORCE(4); break;
+    case 5: FORCE(5); break;
+    case 6: FORCE(6); break;
+    case 7: FORCE(7); break;
+    default: FORCE(8); break;
     }
+#undef FORCE
 }
 
-void launch_disk_force(const KParams &P, hipStream_t st, const ForceBodies &B, double *sig1d,
-                       double *part, double *out4)
+void launch_disk_force(const KParams &P, hipStream_t st, const ForceBodies &B, double *part, double *out4)
 {
     static_assert(kForceMaxBodies == 8, "launch_force_split dispatches 1 .. 8 bodies");
     if (B.n < 1 || B.n > kForceMaxBodies) return;
-    if (B.flags & FCPT_FORCE_CORRECT_SELFGRAVITY)
-        LAUNCH(k_sigma_ring_mean, dim3((unsigned)P.nr), dim3(256), st, P, sig1d);
-    const dim3 g((unsigned)P.cfl_gx, (unsigned)P.cfl_gy);
-    if (P.split) launch_force_split<true>(P, st, B, sig1d, part, g);
-    else launch_force_split<false>(P, st, B, sig1d, part, g);
-    hipLaunchKernelGGL(k_disk_force_final, dim3((unsigned)(4 * B.n)), dim3(256), 0, st, part,
-                       (int)(g.x * g.y), out4);
+    const dim3 g((unsigned)(P.nr - 2));
+    if (P.split) launch_force_split<true>(P, st, B, part, g);
+    else launch_force_split<false>(P, st, B, part, g);
+    hipLaunchKernelGGL(k_disk_force_final, dim3((unsigned)(4 * B.n)), dim3(256), 0, st, part, (int)g.x, out4);
 }
 
 // ---------------------------------------------------------------------------

@@ -114,10 +114,9 @@ struct ForceBodies {
     double x[kForceMaxBodies], y[kForceMaxBodies], r[kForceMaxBodies], r_cubic[kForceMaxBodies];
     double smooth_fixed[kForceMaxBodies];  // >= 0: that smoothing length, < 0: thickness x H(cell)
 };
-// sig1d: nr doubles (ring means of Sigma), part: kCflMaxBlocks x 4 kForceMaxBodies
-// doubles, out4: 4 kForceMaxBodies doubles (inner x, inner y, outer x, outer y per body)
-void launch_disk_force(const KParams &P, hipStream_t st, const ForceBodies &B, double *sig1d,
-                       double *part, double *out4);
+// part: nr x 4 kForceMaxBodies doubles, out4: 4 kForceMaxBodies doubles (inner x, inner y,
+// outer x, outer y per body), device or pinned host memory
+void launch_disk_force(const KParams &P, hipStream_t st, const ForceBodies &B, double *part, double *out4);
 
 // Batched step: one work-table entry per block of one disk's grid
 struct BatchEntry {

@@ -264,7 +264,7 @@ int fcpt_run_steps(fcpt_ctx *ctx, int32_t n_steps, int32_t use_graph);
    FCPT_KERNEL_RADIAL_SWEEP and _AZIMUTHAL both time the kernel that runs the
    transport's two sweeps.
    FCPT_KERNEL_DISK_FORCE times the launches of fcpt_disk_on_planet_accel
-   (ring means, cell reduction, block reduction; no copy to the host) for two
+   (ring means with the cell reduction, then the rings' sum) for two
    bodies, a star at the origin and a planet at (1, 0), with the self-gravity
    correction.  FCPT_KERNEL_CFL is the per-ring CFL kernel (ring means of
    v_phi and the cells' limits; the fold of the ring minima is not timed).
