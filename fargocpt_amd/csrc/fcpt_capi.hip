@@ -348,7 +348,6 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
     P.split_emul = 0;
     P.kick = P.pad_ = 0;
     P.ealt = nullptr;
-    init_launch_fields(P);
     // Interpret.cpp:230-231
     P.dphi = 2.0 * M_PI / (double)ns;
     P.invdphi = (double)ns / (2.0 * M_PI);
@@ -498,12 +497,12 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
     if (!rc) rc = dev_alloc(c, &P.iso_nu, (size_t)nr + 2);
     if (!rc) rc = dev_alloc(c, &P.ring_tab, (size_t)kRingTabs * ((size_t)nr + 2));
     if (!rc) rc = dev_alloc(c, &P.sweep_tab, kSweepTabs * ((size_t)nr + 2));
+    if (!rc) rc = dev_alloc(c, &P.cfl_tab, 8 * ((size_t)nr + 2));
     if (!rc) rc = dev_alloc(c, &P.damp_tab, 8 * ((size_t)nr + 2));
     if (!rc) rc = dev_alloc(c, &P.vmean, (size_t)nr + 1);
     if (!rc) rc = dev_alloc(c, &P.vuni, (size_t)nr + 1);
     if (!rc) rc = dev_alloc(c, &P.nshift, (size_t)nr + 1);
-    // CFL slots: per block of k_cfl_cells (batches) or per ring of k_cfl_rings
-    if (!rc) rc = dev_alloc(c, &P.ring_min, (size_t)(nr > (int)kCflMaxBlocks ? nr : (int)kCflMaxBlocks));
+    if (!rc) rc = dev_alloc(c, &P.ring_min, (size_t)nr);
     if (!rc) rc = dev_alloc(c, &c->s_dev, 1);
     if (!rc) rc = dev_alloc(c, &c->totals_ring, 4 * (size_t)nr);
     if (!rc) rc = dev_alloc(c, &c->totals_out, 2);
@@ -513,6 +512,7 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
         return rc;
     }
     P.s = c->s_dev;
+    P.step_at = &c->s_dev->step_count;
     e = hipHostMalloc((void **)&c->s_host, sizeof(DevScalars), hipHostMallocDefault);
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->totals_host, 2 * sizeof(double), hipHostMallocDefault);
     if (e == hipSuccess)
@@ -531,6 +531,7 @@ int fcpt_create(const fcpt_disk_desc *desc, fcpt_ctx **out)
     for (int k = 0; P.split && k < 4; ++k)
         e = e == hipSuccess ? hipMemset(P.bgm[k], 0, ((size_t)nr + 2) * sizeof(double)) : e;
     std::memset(c->s_host, 0, sizeof(DevScalars));
+    c->s_host->count_next = 1;
     if (e == hipSuccess) e = hipMemcpy(c->s_dev, c->s_host, sizeof(DevScalars), hipMemcpyHostToDevice);
     if (e == hipSuccess) {
         launch_ring_tables(P, c->stream);
@@ -1402,6 +1403,7 @@ static void enqueue_leapfrog(const KParams &P, hipStream_t st, int count_monitor
         launch_kick(K, st, fold_mode);
         launch_transport_ghost(Q, P, st, 0);
         K.kick = 2;
+        K.fold_in_kick = 0;
         launch_kick(K, st, -1);
         launch_final_leapfrog(P, st, count_monitor ? 2 : 1);
         return;
@@ -1439,12 +1441,14 @@ static void enqueue_iteration(const fcpt_ctx *ctx, bool fused, bool report = fal
 {
     KParams V = step_view(ctx, fused);
     if (report) V.s_out = ctx->s_host;
-    if (fused && V.integrator != FCPT_INTEGRATOR_LEAPFROG) {
-        launch_cfl_cells(V, ctx->stream);
-        enqueue_euler(V, ctx->stream, 1, true, 2);
-    } else if (V.lazy_derived) {
-        launch_cfl_cells(V, ctx->stream);
-        enqueue_leapfrog(V, ctx->stream, 1, true, 2);
+    const bool leapfrog = V.integrator == FCPT_INTEGRATOR_LEAPFROG;
+    if (V.lazy_derived || (fused && !leapfrog)) {
+        if (V.cfl_pot) launch_cfl_potential(V, ctx->stream);
+        else launch_cfl_cells(V, ctx->stream);
+        V.fold_in_kick = fold_in_kick(V);
+        const int fold_mode = V.cfl_pot ? kFoldDone : 2;
+        if (leapfrog) enqueue_leapfrog(V, ctx->stream, 1, true, fold_mode);
+        else enqueue_euler(V, ctx->stream, 1, true, fold_mode);
     } else {
         launch_cfl(V, ctx->stream, 2);
         enqueue_step(V, ctx->stream, 1, fused);
@@ -1840,7 +1844,7 @@ int fcpt_autotune(fcpt_ctx *ctx, int32_t reps, int32_t *radial_tile, int32_t *ra
 int fcpt_disk_on_planet_accel(fcpt_ctx *ctx, const fcpt_force_body *bodies, int32_t n_bodies,
                               int32_t flags, double *accel_xy)
 {
-    CTX_CHECK(ctx);  // reads Sigma and H, which every step stores
+    CTX_CHECK(ctx);
     if (n_bodies < 0 || n_bodies > kForceMaxBodies || (n_bodies > 0 && (!bodies || !accel_xy)))
         return fail(ctx, FCPT_ERR_ARG, "1 .. %d bodies", kForceMaxBodies);
     if (flags & ~(FCPT_FORCE_NO_STAR_SMOOTHING | FCPT_FORCE_SMOOTHING_PLANETLOC |
@@ -1864,7 +1868,9 @@ int fcpt_disk_on_planet_accel(fcpt_ctx *ctx, const fcpt_force_body *bodies, int3
         else
             B.smooth_fixed[k] = -1.0;
     }
-    launch_disk_force(ctx->P, ctx->stream, B, ctx->force_part, ctx->force_host);
+    KParams P = ctx->P;
+    P.h_lazy = ctx->derived_stale && step_view(ctx, true).h_lazy;  // no step stored H
+    launch_disk_force(P, ctx->stream, B, ctx->force_part, ctx->force_host);
     LAUNCH_CHECK(ctx);
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     for (int k = 0; k < n_bodies; ++k) {
@@ -2254,6 +2260,7 @@ int fcpt_batch_create(fcpt_ctx *const *disks, int32_t n_disks, fcpt_batch **out)
         // the batch runs the fused step (its rounding points in split storage
         // are the disk's own, whatever tile the batch chooses below)
         set_step_modes(P, true);
+        P.fold_in_kick = fold_in_kick(P);
         b->lazy.push_back(P.lazy_derived != 0);
         host.push_back(P);
     }

@@ -15,7 +15,6 @@
 namespace fcpt {
 
 constexpr int kMaxPlanets = FCPT_MAX_PLANETS;
-constexpr unsigned kCflMaxBlocks = 4096;  // slots of the block-minimum array
 // a ring's values in KParams::ring_tab: the metric the walks read, and the
 // ring-uniform products and quotients of their formulas
 enum {
@@ -60,6 +59,10 @@ struct DevScalars {
     double indirect_mid_x, indirect_mid_y, indirect_first_x, indirect_first_y;
     DevPlanet planet_mid[kMaxPlanets];
     DevPlanet planet_first[kMaxPlanets];
+    // last_dt and the next step_count as the last step left them: what a kick that folds
+    // the CFL minima reads while one of its wavefronts writes last_dt and step_count
+    double last_prev;
+    unsigned count_next, pad3_;
 };
 
 // values per ring of KParams::sweep_tab
@@ -116,7 +119,6 @@ struct KParams {
     // the fused LeapFrog step's kick: 1 and 2 run over dt / 2, 2 from the midstep
     // time and with the midstep bodies; 0 elsewhere (the whole dt)
     int kick, pad_;
-    int cfl_gx, cfl_gy;  // grid of the CFL cell kernel (its block-minimum slots)
     // fields in HBM (indexed by fcpt_field): double, or float when split
     void *f[FCPT_NUM_FIELDS];
     // split storage: per-ring backgrounds of every field (nr + 2 values each;
@@ -135,14 +137,20 @@ struct KParams {
     double *ring_tab;
     // the transport's ring constants, kSweepTabs per ring of one 64-byte line (k_ring_tables)
     double *sweep_tab;
+    double *cfl_tab;     // per ring: radial, azimuthal, smaller and squared smaller cell size, each with its reciprocal
     double *damp_tab;     // per ring: the damping's squared ramp and time scale: scalar inner, outer, vector inner, outer
     double energy_per_t;  // R / mu / (gamma - 1): energy_at's factor, to rounding
     int const_ok;         // the physical constants lie in the range quot_in assumes
     double *vmean;       // per-ring mean azimuthal velocity
     double *vuni;        // per-ring uniform residual velocity (FARGO)
     int *nshift;         // per-ring integer shift
-    double *ring_min;    // CFL minima: per block (kCflMaxBlocks slots) or per ring (nr)
+    double *ring_min;    // the smallest CFL limit of each ring (nr)
     DevScalars *s;
+    int cfl_pot;         // the CFL limits and the potential run as one launch (set_step_modes)
+    int h_lazy;          // and H is formed there, stored in the ghost rings only
+    int fold_in_kick;    // the kick walk folds the ring minima of the CFL limits itself
+    int pad1_;
+    const unsigned *step_at;  // the count the rounding keys of this launch take
     DevScalars *s_out;  // pinned host mirror that the step's clock is written to, or null
 };
 

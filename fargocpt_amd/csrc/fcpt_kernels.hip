@@ -86,6 +86,14 @@ __device__ __forceinline__ double shared_div(double n, const SharedDen &D)
     return q;
 }
 
+// n / D.d by the shared reciprocal, for |n| below 2^900 and D.d in
+// [2^-100, 2^100); below 2^-900 the quotient may be off by a unit of its last place
+__device__ __forceinline__ double quot_fast(double n, const SharedDen &D)
+{
+    const double q0 = n * D.r;
+    return fma(fma(-D.d, q0, n), D.r, q0);
+}
+
 // A denominator with its refined reciprocal, shared by several quotients: in
 // FP64 storage shared_den's, so that in range (ok) the quotient is the IEEE one
 // at three instructions; in split storage recip<true>'s, a product.  ok says
@@ -330,7 +338,14 @@ __device__ __forceinline__ double ring_tab(const KParams &P, int t, int i)
 struct KWalk : KParams {
     const double *rows;
     int row0;
+    double dt;  // of the running kick
 };
+__device__ __forceinline__ double kick_dt(const KWalk &P) { return P.dt; }
+__device__ __forceinline__ double kick_time(const KWalk &P)
+{
+    const double t = *(const __attribute__((address_space(4))) double *)&P.s->time;
+    return P.kick == 2 ? t + P.dt : t;
+}
 __device__ __forceinline__ double ring_tab(const KWalk &P, int t, int i)
 {
     return P.rows[(i - P.row0) * kRingTabs + t];
@@ -351,7 +366,7 @@ __device__ __forceinline__ unsigned store_key(const KParams &P, int id)
 {
     if constexpr (SPLIT) {
         const int mode = P.split_rounding;
-        return (mode == 2 || (mode == 1 && carries_state(id))) ? sr_key(id, cst(&P.s->step_count)[0]) : 0u;
+        return (mode == 2 || (mode == 1 && carries_state(id))) ? sr_key(id, *cst(P.step_at)) : 0u;
     } else {
         return 0u;
     }
@@ -615,16 +630,12 @@ __device__ __forceinline__ void b_ring_mean(const KParams &P, int bx, int by, in
 }
 FCPT_PAIR1(ring_mean, 256, int, mode)
 
-// cfl.cpp:210-376, per cell dt and the per-ring shear limit.  Each thread
-// walks rows with a grid stride; the block minimum (wavefront shuffles, then
-// LDS) goes to its own slot of P.ring_min and k_cfl_finalize folds the slots,
-// so the result is deterministic and free of atomics.
+// The fold of the CFL limits (cfl.cpp:210-376): the rings' smallest
+// (b_cfl_ring's slots) and the shear limits between the rings' means.
 // mode 0: condition_cfl only; 1: sim::CalculateTimeStep (simulation.cpp:100-118);
 // 2: CalculateTimeStep + the monitor clip of sim::run (simulation.cpp:526-542).
-// One block of 256 threads (thread index t) folds the block minima in a fixed
-// pairwise order.
-// With `rings` the slots are the per-ring minima of k_cfl_rings (nr of them)
-// and the fold adds the per-ring shear limits from the ring means.
+// One block of 256 threads (thread index t) folds them in a fixed pairwise
+// order: deterministic and free of atomics.
 __device__ __forceinline__ double cfl_shear(const KParams &P, int k)
 {
     // the limit of the shear between rings k and k + 1 (cfl.cpp:223-233)
@@ -633,14 +644,23 @@ __device__ __forceinline__ double cfl_shear(const KParams &P, int k)
     return P.cfl * P.dphi / denom;
 }
 
-__device__ __forceinline__ void b_cfl_fold(const KParams &P, int mode, int t, bool rings = false)
+// the monitor clip of sim::run (simulation.cpp:526-542)
+__device__ __forceinline__ double monitor_clip(const KParams &P, double rv, int n_monitor, double time)
 {
-    const int nblocks = rings ? P.nr : P.cfl_gx * P.cfl_gy;
+    const double time_next_monitor = (n_monitor + 1) * P.monitor_timestep;
+    const double time_left_till_write = time_next_monitor - time;
+    const bool overshoot = rv > time_left_till_write;
+    const double dt_stretch_factor = 0.05;
+    const bool almost_there = time_left_till_write < rv * (1 + dt_stretch_factor);
+    return (overshoot || almost_there) ? time_left_till_write : rv;
+}
+
+__device__ __forceinline__ void b_cfl_fold(const KParams &P, int mode, int t)
+{
     __shared__ double sh[256];
     double m = __longlong_as_double(0x7FF0000000000000ll);
-    for (int k = t; k < nblocks; k += 256) m = std_min(m, P.ring_min[k]);
-    if (rings)
-        for (int k = t; k < P.nr - 1; k += 256) m = std_min(m, cfl_shear(P, k));
+    for (int k = t; k < P.nr; k += 256) m = std_min(m, P.ring_min[k]);
+    for (int k = t; k < P.nr - 1; k += 256) m = std_min(m, cfl_shear(P, k));
     sh[t] = m;
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
@@ -652,22 +672,58 @@ __device__ __forceinline__ void b_cfl_fold(const KParams &P, int mode, int t, bo
     const double cfl_dt = sh[0];
     s->cfl_dt = cfl_dt;
     s->step_count += 1u;
+    s->count_next = s->step_count + 1u;
     if (!(cfl_dt > 0.0) || !isfinite(cfl_dt)) s->error_flags |= 1;
     if (mode >= 1) {
         const double rv = std_min(P.cfl_max_var * s->last_dt, cfl_dt);
         s->last_dt = rv;
+        s->last_prev = rv;
         s->cfl_dt = rv;
-        if (mode == 2) {
-            const double time_next_monitor = (s->n_monitor + 1) * P.monitor_timestep;
-            const double time_left_till_write = time_next_monitor - s->time;
-            const bool overshoot = rv > time_left_till_write;
-            const double dt_stretch_factor = 0.05;
-            const bool almost_there = time_left_till_write < rv * (1 + dt_stretch_factor);
-            s->dt = (overshoot || almost_there) ? time_left_till_write : rv;
-        }
+        if (mode == 2) s->dt = monitor_clip(P, rv, s->n_monitor, s->time);
     }
 }
-__device__ __forceinline__ void b_cfl_finalize(const KParams &P, int mode) { b_cfl_fold(P, mode, (int)threadIdx.x); }
+
+// The fold (mode 2) by one wavefront of the kick walk: every wavefront forms
+// the same dt from the ring minima and means, and the one with `writes` stores
+// the clock; none reads what that one writes (last_prev and count_next are
+// the last_dt and the next step_count that the last step left).  The shear limits take
+// one division: the smallest quotient is that of the largest shear.
+constexpr int kFoldRings = 512;  // most rings: eight per lane
+__device__ __forceinline__ double cfl_fold_wave(const KParams &P, int lane, bool writes)
+{
+    double m = __longlong_as_double(0x7FF0000000000000ll), shear = 1.0e-100;
+    double lim[kFoldRings / 64], vm[kFoldRings / 64];
+#pragma unroll
+    for (int q = 0; q < kFoldRings / 64; ++q) {
+        const int k = lane + 64 * q;
+        if (64 * q >= P.nr) break;
+        const int c = k < P.nr ? k : P.nr - 1, cn = c + 1 < P.nr ? c + 1 : c;
+        lim[q] = P.ring_min[c];
+        vm[q] = fabs(P.vmean[c] * P.InvRmed[c] - P.vmean[cn] * P.InvRmed[cn]) + 1.0e-100;
+    }
+#pragma unroll
+    for (int q = 0; q < kFoldRings / 64; ++q) {
+        if (64 * q >= P.nr) break;
+        m = std_min(m, lim[q]);
+        shear = std_max(shear, vm[q]);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        m = std_min(m, __shfl_xor(m, off, 64));
+        shear = std_max(shear, __shfl_xor(shear, off, 64));
+    }
+    const double cfl_dt = std_min(m, P.cfl * P.dphi / shear);
+    const double rv = std_min(P.cfl_max_var * *cst(&P.s->last_prev), cfl_dt);
+    const double dt = monitor_clip(P, rv, *cst(&P.s->n_monitor), *cst(&P.s->time));
+    if (writes && lane == 0) {
+        DevScalars *s = P.s;
+        if (!(cfl_dt > 0.0) || !isfinite(cfl_dt)) s->error_flags |= 1;
+        s->step_count = s->count_next;
+        s->last_dt = rv;
+        s->cfl_dt = rv;
+        s->dt = dt;
+    }
+    return dt;
+}
 
 // adiabatic sound speed, scale height and viscosity of one cell
 // (compute_sound_speed, compute_scale_height, compute_viscosity)
@@ -732,180 +788,145 @@ __device__ __forceinline__ AdiDerived adi_derived_stored(const KParams &P, int i
     return a;
 }
 
-// the CFL limit of cell (i, j) (cfl.cpp:235-376), vm_i the ring's mean v_phi
+// The CFL limit of cell (i, j) is CFL / sqrt(sum) (cfl.cpp:235-376), sum the
+// squares of six inverse times added in their order; vm_i is the ring's mean
+// v_phi, and h receives the scale height where the derived fields are formed
+// here.  Division and root round monotonically, so the smallest limit is that
+// of the largest sum: the kernels take the largest sums and form one limit
+// (cfl_limit).  FAST divides by the ring's cell sizes and by E through refined
+// reciprocals, which gives the same bits for finite numerators below 2^400 and
+// sizes and E in [2^-100, 2^100); the caller forms a sum that is not below
+// 2^400 again without it.
+struct CflRing {
+    double inv_cell2;  // split storage
+    SharedDen dr, daz, cell, cell2;
+    bool fast;
+};
+// the ring's cell sizes and their reciprocals: in FP64 storage from
+// KParams::cfl_tab through scalar loads, in split storage (no fall-back, two
+// reciprocals) formed here, where as many scalars would spill
 template <bool SPLIT>
-__device__ __forceinline__ double cfl_cell(const KParams &P, int i, int j, double vm_i)
+__device__ __forceinline__ CflRing cfl_ring(const KParams &P, int i)
 {
-    const int ns = P.ns;
+    CflRing R{};
+    if constexpr (SPLIT) {
+        const double dr = cst(P.Rsup)[i] - cst(P.Rinf)[i], daz = cst(P.Rmed)[i] * P.dphi;
+        R.dr.r = cst(P.InvDiffRsup)[i];
+        R.daz.r = recip<true>(daz);
+        R.cell.r = recip<true>(std_min(dr, daz));
+        R.inv_cell2 = R.cell.r * R.cell.r;
+    } else {
+        const auto t = cst(P.cfl_tab) + 8 * i;
+        R.dr = SharedDen{t[0], t[1], true};
+        R.daz = SharedDen{t[2], t[3], true};
+        R.cell = SharedDen{t[4], t[5], true};
+        R.cell2 = SharedDen{t[6], t[7], true};
+        R.fast = quot_range(R.dr.d) && quot_range(R.daz.d) && quot_range(R.cell2.d);
+    }
+    return R;
+}
+template <bool SPLIT>
+struct CflCell {
+    double vr0, vr1, va0, va1, e, qp, qm, cs, nu, h;
+};
+template <bool SPLIT>
+__device__ __forceinline__ CflCell<SPLIT> cfl_load(const KParams &P, int i, int j)
+{
     FLD(vr, FCPT_VRAD);
     FLD(vaz, FCPT_VAZI);
-    FLD(cs, FCPT_SOUNDSPEED);
-    FLD(nu, FCPT_VISCOSITY);
-    const bool iso = !P.adiabatic;  // c_s and nu are ring profiles
-    const double CFL = P.cfl, dphi = P.dphi;
-    const double fac2 = P.artvisc_factor * P.artvisc_factor;
-    const double dxRadial = cst(P.Rsup)[i] - cst(P.Rinf)[i];
-    const double dxAzimuthal = cst(P.Rmed)[i] * dphi;
-    const double cell_size = std_min(dxRadial, dxAzimuthal);
-    const int jn = j == ns - 1 ? 0 : j + 1;
-    const double vr0 = vr(i, j), vr1 = vr(i + 1, j), va0 = vaz(i, j), va1 = vaz(i, jn);
-    const double v_residual = va0 - vm_i;
-    // split storage: divisions by the ring's cell sizes become products
-    const double inv_dr = SPLIT ? cst(P.InvDiffRsup)[i] : 0.0;
-    const double inv_daz = SPLIT ? recip<true>(dxAzimuthal) : 0.0;
-    const double inv_cell = SPLIT ? recip<true>(cell_size) : 0.0;
-    double csv, nuv;
-    if (iso) {
-        csv = cst(P.iso_cs)[i];
-        nuv = cst(P.iso_nu)[i];
+    const double vr0 = vr(i, j), vr1 = vr(i + 1, j);
+    const double va0 = vaz(i, j), va1 = vaz(i, j == P.ns - 1 ? 0 : j + 1);
+    // one block of loads: a value decoded in a block of its own waits there
+    double e = 0.0, qp = 0.0, qm = 0.0, cs, nu, h = 0.0;
+    if (!P.adiabatic) {  // ring profiles
+        cs = cst(P.iso_cs)[i];
+        nu = cst(P.iso_nu)[i];
     } else if (P.lazy_derived) {
+        e = fld<SPLIT>(P, FCPT_ENERGY)(i, j);
+        const double sig = fld<SPLIT>(P, FCPT_SIGMA)(i, j);
+        qp = fld<SPLIT>(P, FCPT_QPLUS)(i, j);
+        qm = fld<SPLIT>(P, FCPT_QMINUS)(i, j);
         // as recalculate_derived forms them from the same E and Sigma
-        const AdiDerived a = adi_derived_stored<SPLIT>(P, i, j, fld<SPLIT>(P, FCPT_ENERGY)(i, j),
-                                                       fld<SPLIT>(P, FCPT_SIGMA)(i, j));
-        csv = a.cs;
-        nuv = a.nu;
+        const AdiDerived a = adi_derived_stored<SPLIT>(P, i, j, e, sig);
+        cs = a.cs;
+        nu = a.nu;
+        h = a.h;
     } else {
-        csv = cs(i, j);
-        nuv = nu(i, j);
+        e = fld<SPLIT>(P, FCPT_ENERGY)(i, j);
+        qp = fld<SPLIT>(P, FCPT_QPLUS)(i, j);
+        qm = fld<SPLIT>(P, FCPT_QMINUS)(i, j);
+        cs = fld<SPLIT>(P, FCPT_SOUNDSPEED)(i, j);
+        nu = fld<SPLIT>(P, FCPT_VISCOSITY)(i, j);
     }
-    const double invdt1 = SPLIT ? csv * inv_cell : csv / cell_size;
-    const double invdt2 = SPLIT ? vr0 * inv_dr : vr0 / dxRadial;
-    const double invdt3 = SPLIT ? v_residual * inv_daz : v_residual / dxAzimuthal;
+    return CflCell<SPLIT>{vr0, vr1, va0, va1, e, qp, qm, cs, nu, h};
+}
+template <bool SPLIT, bool FAST>
+__device__ __forceinline__ double cfl_sum(const KParams &P, int i, double vm_i, const CflRing &R, const CflCell<SPLIT> &c)
+{
+    auto by = [](double n, const SharedDen &D) { return FAST ? quot_fast(n, D) : n / D.d; };
+    const double fac2 = P.artvisc_factor * P.artvisc_factor;
+    const double v_residual = c.va0 - vm_i;
+    const double csv = c.cs, nuv = c.nu;
+    const double invdt1 = SPLIT ? csv * R.cell.r : by(csv, R.cell);
+    const double invdt2 = SPLIT ? c.vr0 * R.dr.r : by(c.vr0, R.dr);
+    const double invdt3 = SPLIT ? v_residual * R.daz.r : by(v_residual, R.daz);
     // the LeapFrog scheme applies the source terms twice with dt / 2 and
     // relaxes their limits (cfl.cpp:254-261); the Euler factor 1.0 is exact
     const double lf = P.integrator == FCPT_INTEGRATOR_LEAPFROG ? 0.6 : 1.0;
     double invdt4;
     if (P.artvisc == FCPT_ARTVISC_SN) {
-        double dvRadial = vr1 - vr0;
-        double dvAzimuthal = va1 - va0;
+        double dvRadial = c.vr1 - c.vr0;
+        double dvAzimuthal = c.va1 - c.va0;
         if (dvRadial > 0.0) dvRadial = 0.0;
         else dvRadial = -dvRadial;
         if (dvAzimuthal > 0.0) dvAzimuthal = 0.0;
         else dvAzimuthal = -dvAzimuthal;
         if constexpr (SPLIT)
-            invdt4 = 4.0 * fac2 * std_max(dvRadial * inv_dr, dvAzimuthal * inv_daz) * lf;
+            invdt4 = 4.0 * fac2 * std_max(dvRadial * R.dr.r, dvAzimuthal * R.daz.r) * lf;
         else
-            invdt4 = 4.0 * fac2 * std_max(dvRadial / dxRadial, dvAzimuthal / dxAzimuthal) * lf;
+            invdt4 = 4.0 * fac2 * std_max(by(dvRadial, R.dr), by(dvAzimuthal, R.daz)) * lf;
     } else {
-        const double eps_rr = (vr1 - vr0) * cst(P.InvDiffRsup)[i];
-        const double eps_pp = cst(P.InvRmed)[i] * ((va1 - va0) * P.invdphi + 0.5 * (vr1 + vr0));
+        const double eps_rr = (c.vr1 - c.vr0) * cst(P.InvDiffRsup)[i];
+        const double eps_pp = cst(P.InvRmed)[i] * ((c.va1 - c.va0) * P.invdphi + 0.5 * (c.vr1 + c.vr0));
         const double mdiv_V = -std_min(eps_rr + eps_pp, 0.0);
         invdt4 = 4.0 * fac2 * mdiv_V * lf;
     }
-    const double invdt5 = SPLIT ? 4.0 * nuv * (inv_cell * inv_cell) * lf
-                                : 4.0 * nuv / (cell_size * cell_size) * lf;
+    const double invdt5 = SPLIT ? 4.0 * nuv * R.inv_cell2 * lf : by(4.0 * nuv, R.cell2) * lf;
     double invdt6 = 0.0;
     if (P.adiabatic) {
-        FLD(qp, FCPT_QPLUS);
-        FLD(qm, FCPT_QMINUS);
-        FLD(E, FCPT_ENERGY);
         const double inv_limit = 1.0 / P.heating_cooling_cfl_limit;
-        if constexpr (SPLIT) invdt6 = inv_limit * fabs((qp(i, j) - qm(i, j)) * recip<true>(E(i, j))) * lf;
-        else invdt6 = inv_limit * fabs((qp(i, j) - qm(i, j)) / E(i, j)) * lf;
+        double q;
+        if constexpr (SPLIT) q = (c.qp - c.qm) * recip<true>(c.e);
+        else if constexpr (FAST) q = quot_fast(c.qp - c.qm, shared_den(c.e));
+        else q = (c.qp - c.qm) / c.e;
+        invdt6 = inv_limit * fabs(q) * lf;
     }
-    const double sum2 = invdt1 * invdt1 + invdt2 * invdt2 + invdt3 * invdt3 + invdt4 * invdt4 +
-                        invdt5 * invdt5 + invdt6 * invdt6;
-    const double dt_cell = SPLIT ? CFL * inv_sqrt<true>(sum2) : CFL / sqrt(sum2);
-    return dt_cell;
+    return invdt1 * invdt1 + invdt2 * invdt2 + invdt3 * invdt3 + invdt4 * invdt4 + invdt5 * invdt5 + invdt6 * invdt6;
 }
-
-// per-cell CFL limits (cfl.cpp:185-382) and this block's minimum in its slot
-// (k_cfl_finalize folds the slots: a device-wide fold inside this kernel
-// would need a device-scope release per block, which on gfx950 writes back
-// the XCD's L2 and costs more than the separate launch)
 template <bool SPLIT>
-__device__ __forceinline__ void b_cfl_cells(const KParams &P, int bx, int by)
+__device__ __forceinline__ double cfl_cell_sum(const KParams &P, int i, double vm_i, const CflRing &R,
+                                               const CflCell<SPLIT> &c)
 {
-    const int ns = P.ns;
-    const int j = bx * blockDim.x + threadIdx.x;
-    double cand = __longlong_as_double(0x7FF0000000000000ll);
-    const auto vm = cst(P.vmean);
-    for (int i = wave_ring(1, by); i < P.nr - 1 && j < ns; i += P.cfl_gy * (int)blockDim.y) {
-        if (j == 0) {
-            cand = std_min(cand, cfl_shear(P, i));
-            if (i == 1) cand = std_min(cand, cfl_shear(P, 0));
+    double sum = cfl_sum<SPLIT, true>(P, i, vm_i, R, c);
+    if constexpr (!SPLIT) {
+        if (!(R.fast && sum < 0x1p400 && (!P.adiabatic || quot_range(c.e)))) {
+            __builtin_amdgcn_s_sleep(0);  // a branch: not both sums formed and selected
+            sum = cfl_sum<SPLIT, false>(P, i, vm_i, R, c);
         }
-        // NaN never wins a comparison, exactly like the reference's "if (dt_cell < dt_core)"
-        cand = std_min(cand, cfl_cell<SPLIT>(P, i, j, vm[i]));
     }
-    for (int off = 32; off > 0; off >>= 1) cand = std_min(cand, __shfl_xor(cand, off, 64));
-    __shared__ double wmin[4];
-    const int t = threadIdx.y * blockDim.x + threadIdx.x;
-    if ((t & 63) == 0) wmin[t >> 6] = cand;
-    __syncthreads();
-    if (t == 0) {
-        const double m = std_min(std_min(wmin[0], wmin[1]), std_min(wmin[2], wmin[3]));
-        P.ring_min[by * P.cfl_gx + bx] = m;
-    }
-}
-FCPT_PAIR0(cfl_cells, 256)
-
-// The CFL ring mean and cell limits in one launch, one block of 256 threads
-// per ring: the block forms the ring's mean v_phi exactly as k_ring_mean does
-// (same per-thread sums, same tree) and stores it, then the limits of the
-// ring's cells (rings 1 .. nr-2) with that mean, and puts the block minimum in
-// the ring's slot; the fold (rings = true) adds the shear limits between
-// neighbouring rings' means.  The minimum over the same values as
-// k_ring_mean + k_cfl_cells form.
-// 512 threads: the first 256 form the mean (the 256-thread sums and tree of
-// k_ring_mean; the others take part in the barriers only), all 512 the cells.
-template <bool SPLIT>
-__device__ __forceinline__ void b_cfl_rings(const KParams &P, int i)
-{
-    __shared__ double sh[256];
-    __shared__ double wmin[8];
-    const int ns = P.ns;
-    const int t = (int)threadIdx.x;
-    FLD(v, FCPT_VAZI);
-    double acc = 0.0;
-    if (t < 256) strided_row<256>(ns, t, [&](int j) { return v(i, j); }, [&](double x) { acc += x; });
-    if (t < 256) sh[t] = acc;
-    __syncthreads();
-#pragma unroll
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w) sh[t] = sh[t] + sh[t + w];
-        __syncthreads();
-    }
-    const double vm = sh[0] / (double)ns;
-    if (t == 0) P.vmean[i] = vm;
-    double cand = __longlong_as_double(0x7FF0000000000000ll);
-    if (i >= 1 && i < P.nr - 1)
-        for (int j = t; j < ns; j += 512) cand = std_min(cand, cfl_cell<SPLIT>(P, i, j, vm));
-    for (int off = 32; off > 0; off >>= 1) cand = std_min(cand, __shfl_xor(cand, off, 64));
-    if ((t & 63) == 0) wmin[t >> 6] = cand;
-    __syncthreads();
-    if (t == 0) {
-        double m = wmin[0];
-        for (int k = 1; k < 8; ++k) m = std_min(m, wmin[k]);
-        P.ring_min[i] = m;
-    }
+    return sum;
 }
 template <bool SPLIT>
-__global__ void __launch_bounds__(512) k_cfl_rings(KParams P)
+__device__ __forceinline__ double cfl_limit(const KParams &P, double sum)
 {
-    b_cfl_rings<SPLIT>(P, (int)blockIdx.x);
-}
-template <bool SPLIT>
-__global__ void __launch_bounds__(512) kb_cfl_rings(const KParams *Ps, const BatchEntry *map)
-{
-    const BatchEntry e = batch_entry(map);
-    b_cfl_rings<SPLIT>(batch_disk(Ps, e.disk), (int)(e.yx & 0xffffu));
+    return SPLIT ? P.cfl * inv_sqrt<true>(sum) : P.cfl / sqrt(sum);
 }
 
-__global__ void __launch_bounds__(256) k_cfl_finalize(KParams P, int mode) { b_cfl_finalize(P, mode); }
-__global__ void __launch_bounds__(256) k_cfl_finalize_rings(KParams P, int mode)
+__global__ void __launch_bounds__(256) k_cfl_fold(KParams P, int mode) { b_cfl_fold(P, mode, (int)threadIdx.x); }
+__global__ void __launch_bounds__(256) kb_cfl_fold(const KParams *Ps, const BatchEntry *map, int mode)
 {
-    b_cfl_fold(P, mode, (int)threadIdx.x, true);
+    b_cfl_fold(batch_disk(Ps, batch_entry(map).disk), mode, (int)threadIdx.x);
 }
-__global__ void __launch_bounds__(256) kb_cfl_finalize_rings(const KParams *Ps, const BatchEntry *map, int mode)
-{
-    b_cfl_fold(batch_disk(Ps, batch_entry(map).disk), mode, (int)threadIdx.x, true);
-}
-__global__ void __launch_bounds__(256) kb_cfl_finalize(const KParams *Ps, const BatchEntry *map, int mode)
-{
-    b_cfl_finalize(batch_disk(Ps, batch_entry(map).disk), mode);
-}
-
 __global__ void k_set_dt(KParams P, double dt) { P.s->dt = dt; }
 __global__ void k_set_clock(KParams P, double time) { P.s->time = time; }
 
@@ -913,6 +934,7 @@ __global__ void k_set_time(KParams P, double time, double last_dt, int n_monitor
 {
     P.s->time = time;
     P.s->last_dt = last_dt;
+    P.s->last_prev = last_dt;
     P.s->n_monitor = n_monitor;
 }
 
@@ -1091,7 +1113,7 @@ FCPT_PAIR0(potential, 256)
 
 // The potential of a single disk in one launch (b_potential); fold_mode >= 0:
 // one extra block row runs the CFL fold of the step's start
-// (k_cfl_finalize_rings; the potential reads none of the scalars the fold
+// (k_cfl_fold; the potential reads none of the scalars the fold
 // writes, and dt is first read by the kernels after this one).
 template <bool SPLIT>
 __global__ void __launch_bounds__(256) k_potential_fold(KParams P, int fold_mode)
@@ -1100,10 +1122,98 @@ __global__ void __launch_bounds__(256) k_potential_fold(KParams P, int fold_mode
     const int bx = (int)blockIdx.x, by = (int)blockIdx.y - 1;
     if (by < 0) {
         if (bx == 0 && fold_mode >= 0)
-            b_cfl_fold(P, fold_mode, (int)(threadIdx.y * blockDim.x + threadIdx.x), true);
+            b_cfl_fold(P, fold_mode, (int)(threadIdx.y * blockDim.x + threadIdx.x));
         return;
     }
     b_potential<SPLIT>(P, bx, by);
+}
+
+// The CFL ring means and the cells' limits, one block per ring: the block forms
+// the ring's mean v_phi exactly as k_ring_mean does (same per-thread sums, same
+// tree) and stores it, then the limits of the ring's cells (rings 1 .. nr-2)
+// with that mean, and puts the ring's smallest in its slot; the fold adds the
+// shear limits between neighbouring rings' means (cfl.cpp:185-382).  512
+// threads: the first 256 form the mean (the others take part in the barriers
+// only), all 512 the cells.
+// POT: also the potential of the ring's cells, for steps whose derived fields
+// are formed where they are needed; the scale height of its smoothing comes with
+// the sound speed of the limits, so no step stores it.
+// 4096x12288 beta, FP64: 731 us where the two launches took 520 + 314, and the end
+// of the step 795 us instead of 880 without the store of H; 3.8 TB/s, with FP64
+// instructions for about two thirds of its time.
+template <bool SPLIT, bool POT>
+__device__ __forceinline__ void b_cfl_ring(const KParams &P, int i)
+{
+    __shared__ double sh[256];
+    __shared__ double wmax[8];
+    const int ns = P.ns;
+    const int t = (int)threadIdx.x;
+    FLD(v, FCPT_VAZI);
+    FLD(Hf, FCPT_SCALE_HEIGHT);
+    double acc = 0.0;
+    if (t < 256) strided_row<256>(ns, t, [&](int j) { return v(i, j); }, [&](double x) { acc += x; });
+    if (t < 256) sh[t] = acc;
+    __syncthreads();
+#pragma unroll
+    for (int w = 128; w > 0; w >>= 1) {
+        if (t < w) sh[t] = sh[t] + sh[t + w];
+        __syncthreads();
+    }
+    const double vm = sh[0] / (double)ns;
+    if (t == 0) P.vmean[i] = vm;
+    const CflRing R = cfl_ring<SPLIT>(P, i);
+    const double r = cst(P.Rmed)[i];
+    const DevScalars *s = P.s;
+    const int np = POT ? *cst(&s->n_planets) : 0;
+    const double ix = POT ? *cst(&s->indirect_x) : 0.0, iy = POT ? *cst(&s->indirect_y) : 0.0;
+    double most = 0.0;
+    // a loop for the active rings and one for the ghost rings: a test of the
+    // ring in the loop keeps its scalar loads there
+    auto cells = [&](auto act) {
+        for (int j = t; j < ns; j += 512) {
+            double H = P.adiabatic ? 0.0 : cst(P.iso_h)[i];
+            if constexpr (decltype(act)::value) {
+                const CflCell<SPLIT> x = cfl_load<SPLIT>(P, i, j);
+                // NaN never wins a comparison, exactly like the reference's "if (dt_cell < dt_core)"
+                most = std_max(most, cfl_cell_sum<SPLIT>(P, i, vm, R, x));
+                if (POT && P.adiabatic) H = Hf.stored(i, j, x.h);
+            } else {
+                if (P.adiabatic) H = Hf(i, j);  // the ghost rings' is stored
+            }
+            if constexpr (POT) {
+                const double sm = P.thickness_smoothing * H;
+                const double px = r * P.cosphi[j], py = r * P.sinphi[j];
+                double a = 0.0;
+                for (int k = 0; k < np; ++k) {
+                    const auto b = cst(s->planet) + k;
+                    const double smk = b->smooth;
+                    a += potential_body<SPLIT>(P, px, py, smk >= 0.0 ? smk : sm, b->x, b->y, b->mass, b->r_cubic);
+                }
+                phi_fld(P).set(i, j, a + (-ix * px - iy * py));
+            }
+        }
+    };
+    if (i >= 1 && i < P.nr - 1) cells(std::true_type{});
+    else if (POT) cells(std::false_type{});
+    for (int off = 32; off > 0; off >>= 1) most = std_max(most, __shfl_xor(most, off, 64));
+    if ((t & 63) == 0) wmax[t >> 6] = most;
+    __syncthreads();
+    if (t == 0) {
+        double m = wmax[0];
+        for (int k = 1; k < 8; ++k) m = std_max(m, wmax[k]);
+        P.ring_min[i] = m > 0.0 ? cfl_limit<SPLIT>(P, m) : __longlong_as_double(0x7FF0000000000000ll);
+    }
+}
+template <bool SPLIT, bool POT>
+__global__ void __launch_bounds__(512) k_cfl_ring(KParams P)
+{
+    b_cfl_ring<SPLIT, POT>(P, (int)blockIdx.x);
+}
+template <bool SPLIT, bool POT>
+__global__ void __launch_bounds__(512) kb_cfl_ring(const KParams *Ps, const BatchEntry *map)
+{
+    const BatchEntry e = batch_entry(map);
+    b_cfl_ring<SPLIT, POT>(batch_disk(Ps, e.disk), (int)(e.yx & 0xffffu));
 }
 
 // ---------------------------------------------------------------------------
@@ -1303,8 +1413,11 @@ __device__ __forceinline__ void derived_store(const KParams &P, int i, int j, co
 {
     double c_s, h;
     if (P.lazy_derived) {
-        // the only derived field the step reads stored: H (the potential's smoothing)
-        if (P.adiabatic) fld<SPLIT>(P, FCPT_SCALE_HEIGHT).set(i, j, adi_derived<SPLIT>(P, i, d.e, d.sig).h);
+        // the only derived field a step reads stored: H, by the potential where
+        // that is a launch of its own (h_lazy 0) and in the ghost rings, whose
+        // Sigma and E a boundary call of the caller's may change alone
+        if (P.adiabatic && (!P.h_lazy || i == 0 || i == P.nr - 1))
+            fld<SPLIT>(P, FCPT_SCALE_HEIGHT).set(i, j, adi_derived<SPLIT>(P, i, d.e, d.sig).h);
         return;
     }
     if (P.adiabatic) {
@@ -1706,6 +1819,12 @@ __global__ void __launch_bounds__(256) k_ring_tables(KParams P, double *out)
     sw[SW_INV_SURF] = P.InvSurf[i];
     sw[SW_WIDTH] = P.Rsup[i] - P.Rinf[i];
     sw[SW_DXTHETA] = dxtheta;
+    const double dr = P.Rsup[i] - P.Rinf[i], daz = P.Rmed[i] * P.dphi, cell = std_min(dr, daz);
+    const double size[4] = {dr, daz, cell, cell * cell};
+    for (int q = 0; q < 4; ++q) {
+        P.cfl_tab[8 * i + 2 * q] = size[q];
+        P.cfl_tab[8 * i + 2 * q + 1] = shared_den(size[q]).r;
+    }
     sw[SW_INV_DXTHETA] = 1.0 / dxtheta;
     for (int v = 0; v < 2; ++v) {
         double *t = P.damp_tab + 8 * i + 4 * v;
@@ -2484,7 +2603,8 @@ __device__ __forceinline__ void b_kv_walk(const KParams &K, int bx, int by, int 
     const int j = (j0 - kKvHalo + k + ns) % ns;
     const bool own = k >= kKvHalo && k < kKvHalo + Ls;  // lanes that write
     // this wavefront's rows of the ring table: rings i0 - 3 .. i1 + 1
-    const KWalk P{K, lds + (int)threadIdx.y * kv_lds_doubles(tile), i0 >= 3 ? i0 - 3 : 0};
+    KWalk P{K, lds + (int)threadIdx.y * kv_lds_doubles(tile), i0 >= 3 ? i0 - 3 : 0, 0.0};
+    if (K.fold_in_kick) P.step_at = &K.s->count_next;
     {
         const int last = i1 + 1 <= nr ? i1 + 1 : nr, n = (last - P.row0 + 1) * kRingTabs;
         const double *src = K.ring_tab + (size_t)P.row0 * kRingTabs;
@@ -2497,7 +2617,13 @@ __device__ __forceinline__ void b_kv_walk(const KParams &K, int bx, int by, int 
     FLD(E, FCPT_ENERGY);
     const Fld<SPLIT> vr_o = alt_vr<SPLIT>(P);
     const Fld<SPLIT> vaz_o = alt_vaz<SPLIT>(P);
-    const double dt = kick_dt(P);
+    if (K.fold_in_kick) {
+        P.dt = cfl_fold_wave(K, k, bx == 0 && i0 == 0);
+        if (P.kick) P.dt = P.dt / 2;
+    } else {
+        P.dt = kick_dt(K);
+    }
+    const double dt = P.dt;
     const bool diss = ADI && P.artvisc_dissipation;
     const bool emul_derived = EMUL && (P.split_emul & SPLIT_EMUL_DERIVED);
     const bool emul_stages = EMUL && (P.split_emul & SPLIT_EMUL_STAGES);
@@ -2852,6 +2978,8 @@ __device__ __forceinline__ void advance_clock(const KParams &P, int advance_time
     DevScalars *s = P.s;
     const double time_next_monitor = (s->n_monitor + 1) * P.monitor_timestep;
     s->time = s->time + s->dt;
+    s->last_prev = s->last_dt;
+    s->count_next = s->step_count + 1u;
     if (advance_time == 2 && fabs(time_next_monitor - s->time) < 1e-6 * s->last_dt) s->n_monitor++;
     if (DevScalars *out = P.s_out) {
         out->dt = s->dt;
@@ -3129,14 +3257,6 @@ __device__ __forceinline__ void raw_ring(const KParams &P, int r, int j, int jn,
 __device__ __forceinline__ double sweep_tab(const KParams &P, int t, int i)
 {
     return cst(P.sweep_tab)[i * kSweepTabs + t];
-}
-
-// n / D.d by the shared reciprocal, for |n| below 2^900 and D.d in
-// [2^-100, 2^100); below 2^-900 the quotient may be off by a unit of its last place
-__device__ __forceinline__ double quot_fast(double n, const SharedDen &D)
-{
-    const double q0 = n * D.r;
-    return fma(fma(-D.d, q0, n), D.r, q0);
 }
 
 // half the van Leer limiter of the differences a and b: a b / (a + b) where
@@ -3712,34 +3832,27 @@ void launch_ring_mean(const KParams &P, hipStream_t st, int mode)
     LAUNCH(k_ring_mean, dim3(P.nr), dim3(256), st, P, mode);
 }
 
-// CFL grid: at most kCflMaxBlocks blocks, rows walked with a grid stride
-static dim3 cfl_grid(const KParams &P)
+template <bool POT>
+static void launch_cfl_ring(const KParams &P, hipStream_t st)
 {
-    const unsigned gx = (unsigned)((P.ns + 63) / 64);
-    unsigned gy = (unsigned)((P.nr - 2 + 3) / 4);
-    unsigned cap = kCflMaxBlocks / gx;
-    if (cap < 1) cap = 1;
-    if (gy > cap) gy = cap;
-    if (gy < 1) gy = 1;
-    return dim3(gx, gy);
+    const dim3 g((unsigned)P.nr), b(512);
+    if (P.split) hipLaunchKernelGGL((k_cfl_ring<true, POT>), g, b, 0, st, P);
+    else hipLaunchKernelGGL((k_cfl_ring<false, POT>), g, b, 0, st, P);
 }
-
-void init_launch_fields(KParams &P)
-{
-    const dim3 g = cfl_grid(P);
-    P.cfl_gx = (int)g.x;
-    P.cfl_gy = (int)g.y;
-}
-
 void launch_cfl(const KParams &P, hipStream_t st, int mode)
 {
-    LAUNCH(k_cfl_rings, dim3((unsigned)P.nr), dim3(512), st, P);
-    hipLaunchKernelGGL(k_cfl_finalize_rings, dim3(1), dim3(256), 0, st, P, mode);
+    launch_cfl_ring<false>(P, st);
+    hipLaunchKernelGGL(k_cfl_fold, dim3(1), dim3(256), 0, st, P, mode);
+}
+
+void launch_cfl_potential(const KParams &P, hipStream_t st)
+{
+    launch_cfl_ring<true>(P, st);
 }
 
 void launch_cfl_cells(const KParams &P, hipStream_t st)
 {
-    LAUNCH(k_cfl_rings, dim3((unsigned)P.nr), dim3(512), st, P);
+    launch_cfl_ring<false>(P, st);
 }
 
 void launch_set_dt(const KParams &P, hipStream_t st, double dt)
@@ -4052,9 +4165,25 @@ bool kv_walk_applies(const KParams &P)
     return (P.artvisc == FCPT_ARTVISC_TW || P.artvisc == FCPT_ARTVISC_SN) && P.kick_tile != 1 && P.visc_tile != 1;
 }
 
+// whether the kick walk folds the ring minima of launch_cfl_potential itself
+int fold_in_kick(const KParams &P) { return P.cfl_pot && P.nr <= kFoldRings; }
+
 void set_step_modes(KParams &P, bool fused)
 {
     P.lazy_derived = fused && kv_walk_applies(P) ? 1 : 0;
+    // The CFL limits and the potential in one launch where that is the faster:
+    // in FP64 storage on adiabatic disks, which then store and load no scale
+    // height (4096x12288 beta step 4513 -> 4322 us, 1024x3072 307.9 -> 304.9),
+    // and on grids whose kick folds the ring minima, a launch less (128x384
+    // isothermal 29.5 -> 28.0; 2048x6144 isothermal 769 -> 774 is left apart);
+    // in split storage, whose limits and potential are bound by instructions
+    // together, on small grids only (128x384 beta 42.9 -> 40.7; 512x1536
+    // adiabatic 109.2 -> 110.8 is left apart).
+    const bool folds = P.nr <= kFoldRings;
+    P.cfl_pot = P.lazy_derived && (P.split ? folds && (long)P.nr * P.ns <= 131072 : P.adiabatic || folds);
+    // LeapFrog's second kick reads the H of the step's start
+    P.h_lazy = P.cfl_pot && P.adiabatic && P.integrator == FCPT_INTEGRATOR_EULER;
+    P.fold_in_kick = 0;
     P.split_emul = 0;
     if (P.split && P.lazy_derived) {
         const bool walk = walk_rounding(P);
@@ -4124,7 +4253,11 @@ void launch_kick(const KParams &P, hipStream_t st, int fold_mode)
     // with four, 370 with one)
     const dim3 g((unsigned)((P.ns + kKvSegW - 1) / kKvSegW), (unsigned)((P.nr + tile - 1) / tile)), b(64);
     const size_t lds = kv_lds_doubles(tile) * sizeof(double);
-    launch_potential_fold(P, st, fold_mode);
+    if (fold_mode == kFoldDone) {  // launch_cfl_potential before it
+        if (!P.fold_in_kick) hipLaunchKernelGGL(k_cfl_fold, dim3(1), dim3(256), 0, st, P, 2);
+    } else {
+        launch_potential_fold(P, st, fold_mode);
+    }
 #define KV(SP, EM)                                                                                        \
     do {                                                                                                  \
         const bool sn = P.artvisc == FCPT_ARTVISC_SN;                                                     \
@@ -4228,7 +4361,13 @@ __global__ void __launch_bounds__(256) k_disk_force(KParams P, ForceBodies B, do
     const double H_ring = P.adiabatic ? 0.0 : cst(P.iso_h)[i];
     const int j0 = t < ns ? t : 0;
     double sig = S(i, j0), cphi = P.cosphi[j0], sphi = P.sinphi[j0];
-    double H = P.adiabatic ? Hf(i, j0) : H_ring;
+    // a step that forms its derived fields where it needs them stores no H
+    auto height = [&](int j, double sg) {
+        if (!P.adiabatic) return H_ring;
+        if (!P.h_lazy) return Hf(i, j);
+        return Hf.stored(i, j, adi_derived<SPLIT>(P, i, fld<SPLIT>(P, FCPT_ENERGY)(i, j), sg).h);
+    };
+    double H = height(j0, sig);
     double mean = 0.0;
     if (B.flags & FCPT_FORCE_CORRECT_SELFGRAVITY) {
         __shared__ double sh[256];
@@ -4239,7 +4378,7 @@ __global__ void __launch_bounds__(256) k_disk_force(KParams P, ForceBodies B, do
     for (int j = t; j < ns; j += 256) {
         const int jn = j + 256 < ns ? j + 256 : j;
         const double sig_n = S(i, jn), cphi_n = P.cosphi[jn], sphi_n = P.sinphi[jn];
-        const double H_n = P.adiabatic ? Hf(i, jn) : H_ring;
+        const double H_n = height(jn, sig_n);
         const double xc = rmed * cphi;
         const double yc = rmed * sphi;
         const double gm = G * (surf * (sig - mean));
@@ -4371,9 +4510,6 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
     auto rings = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         add_grid(v, d, (unsigned)P.nr, 1);
     };
-    auto cfl = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
-        add_grid(v, d, (unsigned)P.cfl_gx, (unsigned)P.cfl_gy);
-    };
     auto ghosts = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         add_grid(v, d, (unsigned)((P.ns + 255) / 256), 1);
     };
@@ -4389,10 +4525,13 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
     auto one = [](std::vector<BatchEntry> &v, unsigned d, const KParams &) { add_grid(v, d, 1, 1); };
     // sim::CalculateTimeStep and the monitor clip (simulation.cpp:100-118, 526-542):
     // the per-ring CFL blocks and the fold, as launch_cfl
-    stage(B_CFL_RINGS, 0, all, rings);
-    stage(B_CFL_FINAL_RINGS, 2, all, one);
+    auto merged = [](const KParams &P) { return P.cfl_pot != 0; };
+    auto apart = [](const KParams &P) { return P.cfl_pot == 0; };
+    stage(B_CFL_POT, 0, merged, rings);
+    stage(B_CFL_RINGS, 0, apart, rings);
+    stage(B_CFL_FINAL_RINGS, 2, [](const KParams &P) { return !P.fold_in_kick; }, one);
     // step_Euler (simulation.cpp:148-267), in the order of enqueue_euler
-    stage(B_POTENTIAL, 0, all, [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
+    stage(B_POTENTIAL, 0, apart, [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         add_grid(v, d, (unsigned)((P.ns + 64 * kPotCells - 1) / (64 * kPotCells)), rows_grid(P, P.nr));
     });
     // the kick: the walk where the disk's own launch uses it (its tile in
@@ -4450,7 +4589,6 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
     stage_v(B_VEL_FINAL, 2, all, rows(2), false, true);
     std::fill(view.begin(), view.end(), 0u);
     (void)ghosts;
-    (void)cfl;
     (void)damp;
     return st;
 }
@@ -4466,10 +4604,6 @@ void launch_batch_stage(const KParams *Ps, const BatchStageDev &S, int split, hi
     const dim3 b256(256);
     switch (S.kind) {
     case B_RING_MEAN: LAUNCHB(kb_ring_mean, b256, S.arg); break;
-    case B_CFL_CELLS: LAUNCHB(kb_cfl_cells, kBlock); break;
-    case B_CFL_FINAL:
-        hipLaunchKernelGGL(kb_cfl_finalize, dim3(S.n), b256, 0, st, Ps, S.map, S.arg);
-        break;
     case B_POTENTIAL: LAUNCHB(kb_potential, kBlock); break;
     case B_SRC_VR: LAUNCHB(kb_src_vr, kBlock); break;
     case B_SRC_VPHI: LAUNCHB(kb_src_vphi, kBlock); break;
@@ -4491,9 +4625,16 @@ void launch_batch_stage(const KParams *Ps, const BatchStageDev &S, int split, hi
     case B_DAMPING: LAUNCHB(kb_damping, kBlock); break;
     case B_DERIVED: LAUNCHB(kb_derived, kBlock); break;
     case B_FINAL_DERIVED: LAUNCHB(kb_final_derived, kBlock, S.arg); break;
-    case B_CFL_RINGS: LAUNCHB(kb_cfl_rings, dim3(512)); break;
+    case B_CFL_RINGS:
+        if (split) hipLaunchKernelGGL((kb_cfl_ring<true, false>), dim3(S.n), dim3(512), 0, st, Ps, S.map);
+        else hipLaunchKernelGGL((kb_cfl_ring<false, false>), dim3(S.n), dim3(512), 0, st, Ps, S.map);
+        break;
+    case B_CFL_POT:
+        if (split) hipLaunchKernelGGL((kb_cfl_ring<true, true>), dim3(S.n), dim3(512), 0, st, Ps, S.map);
+        else hipLaunchKernelGGL((kb_cfl_ring<false, true>), dim3(S.n), dim3(512), 0, st, Ps, S.map);
+        break;
     case B_CFL_FINAL_RINGS:
-        hipLaunchKernelGGL(kb_cfl_finalize_rings, dim3(S.n), b256, 0, st, Ps, S.map, S.arg);
+        hipLaunchKernelGGL(kb_cfl_fold, dim3(S.n), b256, 0, st, Ps, S.map, S.arg);
         break;
     case B_GHOST_MEAN: LAUNCHB(kb_ghost_ring_mean, b256); break;
     case B_VEL_FINAL: LAUNCHB(kb_velocities_final, kBlock, S.arg); break;

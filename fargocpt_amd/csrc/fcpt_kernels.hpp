@@ -71,6 +71,12 @@ void launch_kick(const KParams &P, hipStream_t st, int fold_mode);
 // the potential; fold_mode >= 0: in the same launch, the CFL fold of
 // k_cfl_rings' slots (launch_cfl_cells) with that mode
 void launch_potential_fold(const KParams &P, hipStream_t st, int fold_mode);
+// the CFL limits' ring minima and the potential in one launch; a launch_kick with
+// fold_mode kFoldDone after it folds the minima (mode 2) and launches no potential
+void launch_cfl_potential(const KParams &P, hipStream_t st);
+constexpr int kFoldDone = 3;
+// whether the kick walk folds them itself (else a launch of its own does)
+int fold_in_kick(const KParams &P);
 void launch_sweeps(const KParams &P, hipStream_t st);
 void launch_cfl_cells(const KParams &P, hipStream_t st);
 void launch_copy4(const KParams &P, hipStream_t st);
@@ -104,8 +110,6 @@ size_t field_element_size(const KParams &P, int field);
 int resolve_sweep_tile(const KParams &P);
 // one tile for the disks of a batch that set none themselves
 int resolve_sweep_tile(const std::vector<KParams> &D);
-// fills the launch-shape fields of a disk's parameters (the CFL grid)
-void init_launch_fields(KParams &P);
 
 // The disk's gravity on up to kForceMaxBodies bodies (ComputeDiskOnPlanetAccel)
 constexpr int kForceMaxBodies = FCPT_MAX_PLANETS;
@@ -123,7 +127,7 @@ struct BatchEntry {
     unsigned disk, yx;  // yx = by << 16 | bx
 };
 enum BatchKind {
-    B_RING_MEAN, B_CFL_CELLS, B_CFL_FINAL, B_POTENTIAL, B_SRC_VR, B_SRC_VPHI,
+    B_RING_MEAN, B_CFL_POT, B_POTENTIAL, B_SRC_VR, B_SRC_VPHI,
     B_SRC_ENERGY, B_TW_Q, B_TW_VEL, B_SN_Q, B_SN_VEL, B_TEMP_FLOOR, B_RECALC_VISC, B_STRESS,
     B_VISC_UPDATE, B_SUBSTEP3, B_GHOST, B_SWEEPS_ISO, B_SWEEPS_ADI,
     B_VELOCITIES, B_DAMPING, B_DERIVED, B_SRC_FUSED, B_AV_FUSED, B_VISC_FUSED, B_FINAL_DERIVED,
