@@ -515,34 +515,34 @@ __device__ __forceinline__ KParams batch_disk(const KParams *Ps, unsigned d)
 // ---------------------------------------------------------------------------
 // ring sums (cfl.cpp:196-205, TransportEuler.cpp:174-190): one block per ring,
 // pairwise tree order
-template <int BS>
-__device__ double block_sum(double v, double *sh)
+// 256 threads' values, the first 256 of the block, summed in pairwise tree order
+// (t + 128, t + 64, ..., t + 1): every wavefront adds the four wavefronts'
+// values and then its lanes' (the two lanes of a pair form the same sum), so
+// the tree takes one barrier and every thread has the result.  With a barrier
+// per level the step took 0.4 to 0.8 us longer (128x384: 28.3 -> 27.6).
+__device__ __forceinline__ double wave_tree(double v)
 {
-    const int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
 #pragma unroll
-    for (int s = BS / 2; s > 0; s >>= 1) {
-        if (t < s) sh[t] = sh[t] + sh[t + s];
-        __syncthreads();
-    }
-    return sh[0];
+    for (int s = 32; s > 0; s >>= 1) v = v + __shfl_xor(v, s, 64);
+    return v;
+}
+__device__ __forceinline__ double block_sum(double v, double *sh)
+{
+    const int t = (int)(threadIdx.y * blockDim.x + threadIdx.x), l = t & 63;
+    if (t < 256) sh[t] = v;
+    __syncthreads();
+    return wave_tree((sh[l] + sh[l + 128]) + (sh[l + 64] + sh[l + 192]));
 }
 
 // The ring sum and the sum of the magnitudes of its terms in one tree: the
-// sum's additions are exactly those of block_sum<BS>.
-template <int BS>
-__device__ double2 block_sum_abs(double v, double a, double2 *sh)
+// sum's additions are exactly those of block_sum.
+__device__ __forceinline__ double2 block_sum_abs(double v, double a, double2 *sh)
 {
-    const int t = threadIdx.x;
+    const int t = (int)threadIdx.x, l = t & 63;
     sh[t] = double2{v, a};
     __syncthreads();
-#pragma unroll
-    for (int s = BS / 2; s > 0; s >>= 1) {
-        if (t < s) sh[t] = double2{sh[t].x + sh[t + s].x, sh[t].y + sh[t + s].y};
-        __syncthreads();
-    }
-    return sh[0];
+    const double2 p = sh[l], q = sh[l + 64], r = sh[l + 128], u = sh[l + 192];
+    return double2{wave_tree((p.x + r.x) + (q.x + u.x)), wave_tree((p.y + r.y) + (q.y + u.y))};
 }
 
 // FARGO shift of ring i from a ring sum (TransportEuler.cpp:215-220)
@@ -621,7 +621,7 @@ __device__ __forceinline__ void b_ring_mean(const KParams &P, int bx, int by, in
         acc += x;
         aacc += fabs(x);
     });
-    const double2 r = block_sum_abs<256>(acc, aacc, sh);
+    const double2 r = block_sum_abs(acc, aacc, sh);
     ring_mean_store(P, i, r.x, r.y, mode, [&]() {
         double seq = 0.0;
         for (int j = 0; j < ns; ++j) seq += v(i, j);
@@ -1132,34 +1132,29 @@ __global__ void __launch_bounds__(256) k_potential_fold(KParams P, int fold_mode
 // the ring's mean v_phi exactly as k_ring_mean does (same per-thread sums, same
 // tree) and stores it, then the limits of the ring's cells (rings 1 .. nr-2)
 // with that mean, and puts the ring's smallest in its slot; the fold adds the
-// shear limits between neighbouring rings' means (cfl.cpp:185-382).  512
-// threads: the first 256 form the mean (the others take part in the barriers
-// only), all 512 the cells.
+// shear limits between neighbouring rings' means (cfl.cpp:185-382).  The first
+// 256 threads form the mean, all of them the cells: 512 where a disk is alone
+// (256: 128x384 27.6 -> 28.6 us per step, 2048x6144 adiabatic 1112 -> 1133; 1024
+// slower everywhere), 256 in a batch, whose rings fill the device anyway and
+// leave fewer of them idle (16 disks of 128 to 512 rings: 437 -> 418 us).
 // POT: also the potential of the ring's cells, for steps whose derived fields
 // are formed where they are needed; the scale height of its smoothing comes with
 // the sound speed of the limits, so no step stores it.
 // 4096x12288 beta, FP64: 731 us where the two launches took 520 + 314, and the end
 // of the step 795 us instead of 880 without the store of H; 3.8 TB/s, with FP64
 // instructions for about two thirds of its time.
-template <bool SPLIT, bool POT>
+template <bool SPLIT, bool POT, int THREADS>
 __device__ __forceinline__ void b_cfl_ring(const KParams &P, int i)
 {
     __shared__ double sh[256];
-    __shared__ double wmax[8];
+    __shared__ double wmax[THREADS / 64];
     const int ns = P.ns;
     const int t = (int)threadIdx.x;
     FLD(v, FCPT_VAZI);
     FLD(Hf, FCPT_SCALE_HEIGHT);
     double acc = 0.0;
     if (t < 256) strided_row<256>(ns, t, [&](int j) { return v(i, j); }, [&](double x) { acc += x; });
-    if (t < 256) sh[t] = acc;
-    __syncthreads();
-#pragma unroll
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w) sh[t] = sh[t] + sh[t + w];
-        __syncthreads();
-    }
-    const double vm = sh[0] / (double)ns;
+    const double vm = block_sum(acc, sh) / (double)ns;
     if (t == 0) P.vmean[i] = vm;
     const CflRing R = cfl_ring<SPLIT>(P, i);
     const double r = cst(P.Rmed)[i];
@@ -1170,7 +1165,7 @@ __device__ __forceinline__ void b_cfl_ring(const KParams &P, int i)
     // a loop for the active rings and one for the ghost rings: a test of the
     // ring in the loop keeps its scalar loads there
     auto cells = [&](auto act) {
-        for (int j = t; j < ns; j += 512) {
+        for (int j = t; j < ns; j += THREADS) {
             double H = P.adiabatic ? 0.0 : cst(P.iso_h)[i];
             if constexpr (decltype(act)::value) {
                 const CflCell<SPLIT> x = cfl_load<SPLIT>(P, i, j);
@@ -1200,20 +1195,20 @@ __device__ __forceinline__ void b_cfl_ring(const KParams &P, int i)
     __syncthreads();
     if (t == 0) {
         double m = wmax[0];
-        for (int k = 1; k < 8; ++k) m = std_max(m, wmax[k]);
+        for (int k = 1; k < THREADS / 64; ++k) m = std_max(m, wmax[k]);
         P.ring_min[i] = m > 0.0 ? cfl_limit<SPLIT>(P, m) : __longlong_as_double(0x7FF0000000000000ll);
     }
 }
 template <bool SPLIT, bool POT>
 __global__ void __launch_bounds__(512) k_cfl_ring(KParams P)
 {
-    b_cfl_ring<SPLIT, POT>(P, (int)blockIdx.x);
+    b_cfl_ring<SPLIT, POT, 512>(P, (int)blockIdx.x);
 }
 template <bool SPLIT, bool POT>
-__global__ void __launch_bounds__(512) kb_cfl_ring(const KParams *Ps, const BatchEntry *map)
+__global__ void __launch_bounds__(256) kb_cfl_ring(const KParams *Ps, const BatchEntry *map)
 {
     const BatchEntry e = batch_entry(map);
-    b_cfl_ring<SPLIT, POT>(batch_disk(Ps, e.disk), (int)(e.yx & 0xffffu));
+    b_cfl_ring<SPLIT, POT, 256>(batch_disk(Ps, e.disk), (int)(e.yx & 0xffffu));
 }
 
 // ---------------------------------------------------------------------------
@@ -2898,7 +2893,7 @@ __global__ void __launch_bounds__(64, ADI ? 3 : 4) k_kv_walk(KParams P, int tile
 }
 // batched form: each disk's tile is its kv_tile
 template <bool SPLIT, bool ADI, bool SN>
-__global__ void __launch_bounds__(256) kb_kv_walk(const KParams *Ps, const BatchEntry *map)
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ADI ? 3 : 4))) kb_kv_walk(const KParams *Ps, const BatchEntry *map)
 {
     const BatchEntry e = batch_entry(map);
     const KParams &P = batch_disk(Ps, e.disk);
@@ -3105,7 +3100,7 @@ __device__ __forceinline__ void b_ghost_ring_mean(const KParams &P, int bx)
             acc += gj;
             aacc += fabs(gj);
         }
-        const double2 r = block_sum_abs<256>(acc, aacc, sh);
+        const double2 r = block_sum_abs(acc, aacc, sh);
         ring_mean_store(P, i, r.x, r.y, 1, [&]() {
             double seq = 0.0;
             for (int j = 0; j < P.ns; ++j) seq += vaz.stored(i, j, g);
@@ -3802,7 +3797,7 @@ __global__ void __launch_bounds__(256) k_split_ring_mean(const float *d, const d
     const float *row = d + (size_t)i * (size_t)ns;
     double acc = 0.0;
     strided_row<256>(ns, (int)threadIdx.x, [&](int j) { return (double)row[j]; }, [&](double x) { acc += x; });
-    const double sum = block_sum<256>(acc, sh);
+    const double sum = block_sum(acc, sh);
     if (threadIdx.x == 0) out[i] = bg[i] + sum / ns;
 }
 
@@ -3986,19 +3981,23 @@ void launch_boundaries(const KParams &P, hipStream_t st, int final_call, int adv
 // Rings per walk of the transport's sweeps: a walk of t rings costs about
 // t + 1.5 ring times (its window start), and a ring time with n wavefronts on a
 // SIMD is 0.7 n + 1.2 us up to the three its registers allow, as latency is
-// left over, and 1.1 n beyond.  Measured step times at 512x1536 (tiles 1, 3,
-// 8, 16): 116, 107, 109, 120 us; at 1024x3072 (3, 8, 16, 32): 316, 306, 318,
-// 325; at 4096x12288 (8, 16, 32, 48): 4646, 4567, 4550, 4623.
+// left over, and 1.1 n beyond; one disk's walks are alike, so n rounds up.
+// Measured step times at 512x1536 (tiles 1, 3, 5, 8, 16): 116, 107, 103, 109,
+// 120 us; at 1024x3072 (3, 8, 16, 19, 32): 316, 306, 318, 303, 325; at
+// 4096x12288 (8, 16, 32, 48): 4646, 4567, 4550, 4623.  A batch's walks end at
+// different times, so one full round leaves SIMDs idle and n gets one more
+// instead: the sweeps of 16 disks of 128 to 512 rings (4, 8, 12, 16, 32): 188,
+// 171, 174, 177, 206.
 template <class Waves>
-static int sweep_best_tile(Waves &&waves)
+static int sweep_best_tile(Waves &&waves, bool batch)
 {
     int best = 1;
     double best_cost = 1e300;
     for (int t = 1; t <= 32; ++t) {
-        const double n = std::ceil((double)waves(t) / 1024.0);
-        const double cost = (t + 1.5) * (n <= 3.0 ? 0.7 * n + 1.2 : 1.1 * n);
-        if (cost < best_cost) {
-            best_cost = cost;
+        const double w = (double)waves(t) / 1024.0, n = std::ceil(w);
+        const double ring = batch ? std::max(1.9, 1.1 * (w + 1.0)) : n <= 3.0 ? 0.7 * n + 1.2 : 1.1 * n;
+        if ((t + 1.5) * ring < best_cost) {
+            best_cost = (t + 1.5) * ring;
             best = t;
         }
     }
@@ -4010,7 +4009,7 @@ static long sweep_waves(const KParams &P, int tile)
 }
 int resolve_sweep_tile(const KParams &P)
 {
-    return P.radial_tile > 0 ? P.radial_tile : sweep_best_tile([&](int t) { return sweep_waves(P, t); });
+    return P.radial_tile > 0 ? P.radial_tile : sweep_best_tile([&](int t) { return sweep_waves(P, t); }, false);
 }
 int resolve_sweep_tile(const std::vector<KParams> &D)
 {
@@ -4018,7 +4017,7 @@ int resolve_sweep_tile(const std::vector<KParams> &D)
         long w = 0;
         for (const KParams &P : D) w += sweep_waves(P, P.radial_tile > 0 ? P.radial_tile : t);
         return w;
-    });
+    }, true);
 }
 
 void launch_sweeps(const KParams &P, hipStream_t st)
@@ -4373,7 +4372,7 @@ __global__ void __launch_bounds__(256) k_disk_force(KParams P, ForceBodies B, do
         __shared__ double sh[256];
         double sum = 0.0;
         strided_row<256>(ns, t, [&](int j) { return S(i, j); }, [&](double x) { sum += x; });
-        mean = block_sum<256>(sum, sh) / ns;
+        mean = block_sum(sum, sh) / ns;
     }
     for (int j = t; j < ns; j += 256) {
         const int jn = j + 256 < ns ? j + 256 : j;
@@ -4435,7 +4434,7 @@ __global__ void __launch_bounds__(256) k_disk_force_final(const double *part, in
     const double *p = part + (size_t)blockIdx.x * nslots;
     double s = 0.0;
     for (int b = threadIdx.x; b < nslots; b += 256) s += p[b];
-    s = block_sum<256>(s, sh);
+    s = block_sum(s, sh);
     if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
@@ -4541,7 +4540,7 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
     auto walk = [](const KParams &P) { return kv_walk_applies(P); };
     auto kick_grid = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         const int tiles = (P.nr + P.kv_tile - 1) / P.kv_tile;
-        add_grid(v, d, (unsigned)((P.ns + kKvSegW - 1) / kKvSegW), (unsigned)((tiles + 3) / 4));
+        add_grid(v, d, (unsigned)((P.ns + kKvSegW - 1) / kKvSegW), (unsigned)tiles);
     };
     auto visc_grid = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         const int tiles = (P.nr + P.visc_tile - 1) / P.visc_tile;
@@ -4626,12 +4625,12 @@ void launch_batch_stage(const KParams *Ps, const BatchStageDev &S, int split, hi
     case B_DERIVED: LAUNCHB(kb_derived, kBlock); break;
     case B_FINAL_DERIVED: LAUNCHB(kb_final_derived, kBlock, S.arg); break;
     case B_CFL_RINGS:
-        if (split) hipLaunchKernelGGL((kb_cfl_ring<true, false>), dim3(S.n), dim3(512), 0, st, Ps, S.map);
-        else hipLaunchKernelGGL((kb_cfl_ring<false, false>), dim3(S.n), dim3(512), 0, st, Ps, S.map);
+        if (split) hipLaunchKernelGGL((kb_cfl_ring<true, false>), dim3(S.n), b256, 0, st, Ps, S.map);
+        else hipLaunchKernelGGL((kb_cfl_ring<false, false>), dim3(S.n), b256, 0, st, Ps, S.map);
         break;
     case B_CFL_POT:
-        if (split) hipLaunchKernelGGL((kb_cfl_ring<true, true>), dim3(S.n), dim3(512), 0, st, Ps, S.map);
-        else hipLaunchKernelGGL((kb_cfl_ring<false, true>), dim3(S.n), dim3(512), 0, st, Ps, S.map);
+        if (split) hipLaunchKernelGGL((kb_cfl_ring<true, true>), dim3(S.n), b256, 0, st, Ps, S.map);
+        else hipLaunchKernelGGL((kb_cfl_ring<false, true>), dim3(S.n), b256, 0, st, Ps, S.map);
         break;
     case B_CFL_FINAL_RINGS:
         hipLaunchKernelGGL(kb_cfl_fold, dim3(S.n), b256, 0, st, Ps, S.map, S.arg);
@@ -4640,9 +4639,9 @@ void launch_batch_stage(const KParams *Ps, const BatchStageDev &S, int split, hi
     case B_VEL_FINAL: LAUNCHB(kb_velocities_final, kBlock, S.arg); break;
     case B_KV_WALK: {
         const dim3 g(S.n);
-#define KWB(SP, AD, SN)                                                                            hipLaunchKernelGGL((kb_kv_walk<SP, AD, SN>), g, kBlock, lds, st, Ps, S.map)
+#define KWB(SP, AD, SN)                                                                            hipLaunchKernelGGL((kb_kv_walk<SP, AD, SN>), g, dim3(64), lds, st, Ps, S.map)
         const int v = (split ? 4 : 0) + (S.arg & 3);
-        const size_t lds = 4 * kv_lds_doubles(S.arg >> 2) * sizeof(double);
+        const size_t lds = kv_lds_doubles(S.arg >> 2) * sizeof(double);
         if (v == 0) KWB(false, false, false);
         else if (v == 1) KWB(false, false, true);
         else if (v == 2) KWB(false, true, false);
