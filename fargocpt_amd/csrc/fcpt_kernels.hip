@@ -545,16 +545,9 @@ __device__ __forceinline__ double2 block_sum_abs(double v, double a, double2 *sh
     return double2{wave_tree((p.x + r.x) + (q.x + u.x)), wave_tree((p.y + r.y) + (q.y + u.y))};
 }
 
-// FARGO shift of ring i from a ring sum (TransportEuler.cpp:215-220)
-__device__ __forceinline__ double fargo_ntilde(const KParams &P, int i, double sum, double dt)
-{
-    const double vm = sum / (double)P.ns;
-    return vm * cst(P.InvRmed)[i] * dt * P.invdphi;
-}
-
 // mode 0: CFL ring mean
-// mode 1: transport ring mean + FARGO shift + uniform residual
-//         (TransportEuler.cpp:207-236)
+// mode 1: transport ring mean + FARGO shift (TransportEuler.cpp:215-220) +
+//         uniform residual (:207-236)
 // The reference sums a ring left to right (TransportEuler.cpp:178-183); the
 // block's tree sums the same terms in another order.  Any two summation
 // orders of n terms differ by at most 2 gamma_(n-1) sum |term| (gamma_k =
@@ -565,27 +558,42 @@ __device__ __forceinline__ double fargo_ntilde(const KParams &P, int i, double s
 // gives it too; otherwise thread 0 forms the left-to-right sum itself
 // (seq_sum: the ring's terms in order) and the ring's mean, shift and
 // residual come from it, as in the reference.
+// What a ring's FARGO shift needs besides its sum, loaded (and 1 / dt formed)
+// while the ring's values are under way
+struct MeanConst {
+    double dt, invdt, inv_rmed, rmed;
+};
+__device__ __forceinline__ MeanConst mean_const(const KParams &P, int i)
+{
+    const double dt = P.s->dt;
+    return MeanConst{dt, 1.0 / dt, cst(P.InvRmed)[i], cst(P.Rmed)[i]};
+}
+// the first wavefront's lanes 0, 1 and 2 form the shift of the sum and of its
+// interval's ends at once
 template <typename SeqSum>
 __device__ __forceinline__ void ring_mean_store(const KParams &P, int i, double sum, double asum, int mode,
-                                                SeqSum seq_sum)
+                                                const MeanConst &c, SeqSum seq_sum)
 {
-    if (threadIdx.x != 0) return;
+    const int t = (int)threadIdx.x;
+    if (t >= 64) return;
+    const double nsd = (double)P.ns;
     if (mode == 1) {
-        const double dt = P.s->dt;
-        const double nsd = (double)P.ns;
         const double bound = asum * (2.02 * nsd * 0x1p-53) + fabs(sum) * 0x1p-50;
-        const double lo = floor(fargo_ntilde(P, i, sum - bound, dt) + 0.5);
-        const double hi = floor(fargo_ntilde(P, i, sum + bound, dt) + 0.5);
-        if (!(lo == hi)) sum = seq_sum();
-        const double vm = sum / nsd;
+        double vm = (t == 1 ? sum - bound : t == 2 ? sum + bound : sum) / nsd;
+        double Ntilde = vm * c.inv_rmed * c.dt * P.invdphi;
+        double Nround = floor(Ntilde + 0.5);
+        const double lo = __shfl(Nround, 1, 64), hi = __shfl(Nround, 2, 64);
+        if (t != 0) return;
+        if (!(lo == hi)) {
+            vm = seq_sum() / nsd;
+            Ntilde = vm * c.inv_rmed * c.dt * P.invdphi;
+            Nround = floor(Ntilde + 0.5);
+        }
         P.vmean[i] = vm;
-        const double invdt = 1.0 / dt;
-        const double Ntilde = vm * cst(P.InvRmed)[i] * dt * P.invdphi;
-        const double Nround = floor(Ntilde + 0.5);
         P.nshift[i] = (int)Nround;
-        P.vuni[i] = (Ntilde - Nround) * cst(P.Rmed)[i] * invdt * P.dphi;
-    } else {
-        P.vmean[i] = sum / (double)P.ns;
+        P.vuni[i] = (Ntilde - Nround) * c.rmed * c.invdt * P.dphi;
+    } else if (t == 0) {
+        P.vmean[i] = sum / nsd;
     }
 }
 
@@ -616,13 +624,14 @@ __device__ __forceinline__ void b_ring_mean(const KParams &P, int bx, int by, in
     const int ns = P.ns;
     const int i = bx;
     FLD(v, FCPT_VAZI);
+    const MeanConst c = mode == 1 ? mean_const(P, i) : MeanConst{};
     double acc = 0.0, aacc = 0.0;
     strided_row<256>(ns, (int)threadIdx.x, [&](int j) { return v(i, j); }, [&](double x) {
         acc += x;
         aacc += fabs(x);
     });
     const double2 r = block_sum_abs(acc, aacc, sh);
-    ring_mean_store(P, i, r.x, r.y, mode, [&]() {
+    ring_mean_store(P, i, r.x, r.y, mode, c, [&]() {
         double seq = 0.0;
         for (int j = 0; j < ns; ++j) seq += v(i, j);
         return seq;
@@ -689,23 +698,32 @@ __device__ __forceinline__ void b_cfl_fold(const KParams &P, int mode, int t)
 // the last_dt and the next step_count that the last step left).  The shear limits take
 // one division: the smallest quotient is that of the largest shear.
 constexpr int kFoldRings = 512;  // most rings: eight per lane
-__device__ __forceinline__ double cfl_fold_wave(const KParams &P, int lane, bool writes)
+struct FoldLoads {
+    double lim[kFoldRings / 64], vm[kFoldRings / 64], rm[kFoldRings / 64];
+};
+__device__ __forceinline__ void cfl_fold_load(const KParams &P, int lane, FoldLoads &x)
 {
-    double m = __longlong_as_double(0x7FF0000000000000ll), shear = 1.0e-100;
-    double lim[kFoldRings / 64], vm[kFoldRings / 64];
 #pragma unroll
     for (int q = 0; q < kFoldRings / 64; ++q) {
-        const int k = lane + 64 * q;
-        if (64 * q >= P.nr) break;
-        const int c = k < P.nr ? k : P.nr - 1, cn = c + 1 < P.nr ? c + 1 : c;
-        lim[q] = P.ring_min[c];
-        vm[q] = fabs(P.vmean[c] * P.InvRmed[c] - P.vmean[cn] * P.InvRmed[cn]) + 1.0e-100;
+        if (64 * q >= P.nr) continue;  // uniform
+        const int c = lane + 64 * q < P.nr ? lane + 64 * q : P.nr - 1;
+        x.lim[q] = P.ring_min[c];
+        x.vm[q] = P.vmean[c];
+        x.rm[q] = P.InvRmed[c];
     }
+}
+__device__ __forceinline__ double cfl_fold_wave(const KParams &P, int lane, bool writes, const FoldLoads &x)
+{
+    double m = __longlong_as_double(0x7FF0000000000000ll), shear = 1.0e-100, next = 0.0;
 #pragma unroll
-    for (int q = 0; q < kFoldRings / 64; ++q) {
-        if (64 * q >= P.nr) break;
-        m = std_min(m, lim[q]);
-        shear = std_max(shear, vm[q]);
+    for (int q = kFoldRings / 64 - 1; q >= 0; --q) {
+        if (64 * q >= P.nr) continue;
+        m = std_min(m, x.lim[q]);
+        // the ring outside is the next lane's; the last lane's the next round's first
+        const double om = x.vm[q] * x.rm[q], right = from_right(om);
+        const double out = lane == 63 ? next : right;
+        if (lane + 64 * q < P.nr - 1) shear = std_max(shear, fabs(om - out) + 1.0e-100);
+        next = __shfl(om, 0, 64);
     }
     for (int off = 32; off > 0; off >>= 1) {
         m = std_min(m, __shfl_xor(m, off, 64));
@@ -1154,13 +1172,19 @@ __device__ __forceinline__ void b_cfl_ring(const KParams &P, int i)
     FLD(Hf, FCPT_SCALE_HEIGHT);
     double acc = 0.0;
     if (t < 256) strided_row<256>(ns, t, [&](int j) { return v(i, j); }, [&](double x) { acc += x; });
-    const double vm = block_sum(acc, sh) / (double)ns;
-    if (t == 0) P.vmean[i] = vm;
+    const bool active = i >= 1 && i < P.nr - 1;
+    // a disk alone waits for its first cells' loads during the sum; a batch has
+    // other rings to run and keeps the registers
+    constexpr bool AHEAD = THREADS == 512;
+    CflCell<SPLIT> c;
+    if constexpr (AHEAD) c = cfl_load<SPLIT>(P, active ? i : 1, t < ns ? t : 0);
     const CflRing R = cfl_ring<SPLIT>(P, i);
     const double r = cst(P.Rmed)[i];
     const DevScalars *s = P.s;
     const int np = POT ? *cst(&s->n_planets) : 0;
     const double ix = POT ? *cst(&s->indirect_x) : 0.0, iy = POT ? *cst(&s->indirect_y) : 0.0;
+    const double vm = block_sum(acc, sh) / (double)ns;
+    if (t == 0) P.vmean[i] = vm;
     double most = 0.0;
     // a loop for the active rings and one for the ghost rings: a test of the
     // ring in the loop keeps its scalar loads there
@@ -1168,10 +1192,10 @@ __device__ __forceinline__ void b_cfl_ring(const KParams &P, int i)
         for (int j = t; j < ns; j += THREADS) {
             double H = P.adiabatic ? 0.0 : cst(P.iso_h)[i];
             if constexpr (decltype(act)::value) {
-                const CflCell<SPLIT> x = cfl_load<SPLIT>(P, i, j);
+                if (!AHEAD || j != t) c = cfl_load<SPLIT>(P, i, j);
                 // NaN never wins a comparison, exactly like the reference's "if (dt_cell < dt_core)"
-                most = std_max(most, cfl_cell_sum<SPLIT>(P, i, vm, R, x));
-                if (POT && P.adiabatic) H = Hf.stored(i, j, x.h);
+                most = std_max(most, cfl_cell_sum<SPLIT>(P, i, vm, R, c));
+                if (POT && P.adiabatic) H = Hf.stored(i, j, c.h);
             } else {
                 if (P.adiabatic) H = Hf(i, j);  // the ghost rings' is stored
             }
@@ -1188,7 +1212,7 @@ __device__ __forceinline__ void b_cfl_ring(const KParams &P, int i)
             }
         }
     };
-    if (i >= 1 && i < P.nr - 1) cells(std::true_type{});
+    if (active) cells(std::true_type{});
     else if (POT) cells(std::false_type{});
     for (int off = 32; off > 0; off >>= 1) most = std_max(most, __shfl_xor(most, off, 64));
     if ((t & 63) == 0) wmax[t >> 6] = most;
@@ -2600,29 +2624,12 @@ __device__ __forceinline__ void b_kv_walk(const KParams &K, int bx, int by, int 
     // this wavefront's rows of the ring table: rings i0 - 3 .. i1 + 1
     KWalk P{K, lds + (int)threadIdx.y * kv_lds_doubles(tile), i0 >= 3 ? i0 - 3 : 0, 0.0};
     if (K.fold_in_kick) P.step_at = &K.s->count_next;
-    {
-        const int last = i1 + 1 <= nr ? i1 + 1 : nr, n = (last - P.row0 + 1) * kRingTabs;
-        const double *src = K.ring_tab + (size_t)P.row0 * kRingTabs;
-        for (int t = k; t < n; t += 64) const_cast<double *>(P.rows)[t] = src[t];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    }
     FLD(vr, FCPT_VRAD);
     FLD(vaz, FCPT_VAZI);
     FLD(S, FCPT_SIGMA);
     FLD(E, FCPT_ENERGY);
     const Fld<SPLIT> vr_o = alt_vr<SPLIT>(P);
     const Fld<SPLIT> vaz_o = alt_vaz<SPLIT>(P);
-    if (K.fold_in_kick) {
-        P.dt = cfl_fold_wave(K, k, bx == 0 && i0 == 0);
-        if (P.kick) P.dt = P.dt / 2;
-    } else {
-        P.dt = kick_dt(K);
-    }
-    const double dt = P.dt;
-    const bool diss = ADI && P.artvisc_dissipation;
-    const bool emul_derived = EMUL && (P.split_emul & SPLIT_EMUL_DERIVED);
-    const bool emul_stages = EMUL && (P.split_emul & SPLIT_EMUL_STAGES);
-    const bool launch_ok = P.const_ok && quot_range(dt);  // the quotients' numerators are in range
     // one ring of the lane's sector as loaded
     struct Raw {
         typename Fld<SPLIT>::T vr, va, s, e;
@@ -2638,6 +2645,40 @@ __device__ __forceinline__ void b_kv_walk(const KParams &K, int bx, int by, int 
         w.phi = phi_fld(P)(c, j);
         return w;
     };
+    // The walk's start issues every load before it waits for one: the window's
+    // rings, the rows of the ring table and the fold's ring minima (with a wait
+    // per round of them a 1024x3072 step took 301.7 us, now 299.4).
+    const int m0 = i0 >= 1 ? i0 - 1 : 0;  // the first ring of the artificial viscosity
+    const Raw x2 = load(m0 >= 2 ? m0 - 2 : 0), x1 = load(m0 >= 1 ? m0 - 1 : 0), x0 = load(m0);
+    Raw X = load(m0 + 1);  // ring m + 1, in flight
+    FoldLoads fold;
+    if (K.fold_in_kick) cfl_fold_load(K, k, fold);
+    {
+        constexpr int U = 6;
+        const int last = i1 + 1 <= nr ? i1 + 1 : nr, n = (last - P.row0 + 1) * kRingTabs;
+        const double *src = K.ring_tab + (size_t)P.row0 * kRingTabs;
+        double *dst = const_cast<double *>(P.rows);
+        for (int t0 = 0; t0 < n; t0 += 64 * U) {
+            double row[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) row[u] = src[min(t0 + 64 * u + k, n - 1)];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (t0 + 64 * u + k < n) dst[t0 + 64 * u + k] = row[u];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    if (K.fold_in_kick) {
+        P.dt = cfl_fold_wave(K, k, bx == 0 && i0 == 0, fold);
+        if (P.kick) P.dt = P.dt / 2;
+    } else {
+        P.dt = kick_dt(K);
+    }
+    const double dt = P.dt;
+    const bool diss = ADI && P.artvisc_dissipation;
+    const bool emul_derived = EMUL && (P.split_emul & SPLIT_EMUL_DERIVED);
+    const bool emul_stages = EMUL && (P.split_emul & SPLIT_EMUL_STAGES);
+    const bool launch_ok = P.const_ok && quot_range(dt);  // the quotients' numerators are in range
     struct Ring {
         double vr, va, s, p, phi, e;  // p: pressure, phi: potential
         double sL, vaR;               // Sigma of sector j - 1, v_phi of sector j + 1
@@ -2713,15 +2754,11 @@ __device__ __forceinline__ void b_kv_walk(const KParams &K, int bx, int by, int 
         Rcp rcp;
         bool fine;  // its E and Sigma are in range
     };
-    const int m0 = i0 >= 1 ? i0 - 1 : 0;  // the first ring of the artificial viscosity
     Ring R0;                              // ring m
     double v1r0, v1a0;                    // its source-term velocities
     Rcp rcp0;
     double qr_m = 0.0, qp_m = 0.0, s_m = 0.0;  // tensor and Sigma of cell (m - 1, j)
-    Raw X;                                // ring m + 1, in flight
     {
-        const Raw x2 = load(m0 >= 2 ? m0 - 2 : 0), x1 = load(m0 >= 1 ? m0 - 1 : 0), x0 = load(m0);
-        X = load(m0 + 1);
         const Ring Rm2 = ring(m0 >= 2 ? m0 - 2 : 0, x2);  // read by rings m0 - 1 >= 2 only
         const Ring Rm = ring(m0 >= 1 ? m0 - 1 : 0, x1);
         R0 = ring(m0, x0);
@@ -3094,6 +3131,7 @@ __device__ __forceinline__ void b_ghost_ring_mean(const KParams &P, int bx)
         // this launch (split storage with stochastic rounding: per sector)
         const Fld<SPLIT> vaz = fld<SPLIT>(P, FCPT_VAZI);
         const double g = ghost_vaz(P, i);
+        const MeanConst c = mean_const(P, i);
         double acc = 0.0, aacc = 0.0;
         for (int j = (int)threadIdx.x; j < P.ns; j += 256) {
             const double gj = vaz.stored(i, j, g);
@@ -3101,7 +3139,7 @@ __device__ __forceinline__ void b_ghost_ring_mean(const KParams &P, int bx)
             aacc += fabs(gj);
         }
         const double2 r = block_sum_abs(acc, aacc, sh);
-        ring_mean_store(P, i, r.x, r.y, 1, [&]() {
+        ring_mean_store(P, i, r.x, r.y, 1, c, [&]() {
             double seq = 0.0;
             for (int j = 0; j < P.ns; ++j) seq += vaz.stored(i, j, g);
             return seq;
