@@ -24,9 +24,9 @@ VECTOR_FIELDS = {"VRAD", "VRAD0", "TAU_R_PHI"}
 
 ARTVISC = {"none": 0, "tw": 1, "sn": 2}
 # kernels of the (fused) step that fcpt_time_kernel can time on their own
-KERNELS = {"radial_sweep": 0, "azimuthal_sweep": 1, "cfl": 3, "visc_fused": 7, "potential": 5}
+KERNELS = {"sweeps": 0, "cfl": 3, "visc_fused": 7, "potential": 5}
 # the same on a batch (the viscous pass is not timed there)
-BATCH_KERNELS = {"radial_sweep": 0, "azimuthal_sweep": 1, "cfl": 3, "potential": 5}
+BATCH_KERNELS = {"sweeps": 0, "cfl": 3, "potential": 5}
 KERNEL_STRESS = 4      # the separate stress-tensor kernel of fcpt_viscous_stress_tensor
 KERNEL_DISK_FORCE = 6  # the disk-on-planet reduction (not part of the hydro step)
 # storage modes (fcpt_disk_desc.precision) and launch parameters of include/fcpt.h

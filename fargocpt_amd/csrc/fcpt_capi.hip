@@ -2399,8 +2399,8 @@ int fcpt_batch_time_kernel(fcpt_batch *b, int32_t kernel, int32_t reps, double *
     switch (kernel) {
     case FCPT_KERNEL_RADIAL_SWEEP:  // one kernel runs both sweeps
     case FCPT_KERNEL_AZIMUTHAL: kinds[0] = B_SWEEPS_ISO; kinds[1] = B_SWEEPS_ADI; break;
-    case FCPT_KERNEL_CFL: kinds[0] = B_CFL_RINGS; break;
-    case FCPT_KERNEL_POTENTIAL: kinds[0] = B_POTENTIAL; break;
+    case FCPT_KERNEL_CFL: kinds[0] = B_CFL_RINGS; kinds[1] = B_CFL_POT; break;  // some members' limits and
+    case FCPT_KERNEL_POTENTIAL: kinds[0] = B_POTENTIAL; kinds[1] = B_CFL_POT; break;  // potential are one launch
     case FCPT_KERNEL_STRESS:
     case FCPT_KERNEL_VISC_FUSED:
         // the batched step runs the fused viscous pass, on views that differ

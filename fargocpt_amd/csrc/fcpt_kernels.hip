@@ -385,11 +385,10 @@ __device__ __forceinline__ Fld<SPLIT> buf(const KParams &P, void *p, const doubl
 
 #define FLD(name, id) const Fld<SPLIT> name = fld<SPLIT>(P, id)
 
-// The transported momenta after the azimuthal sweep, read by the end of the
-// step: FP64 in both storage modes (in split storage their FP32 rounding,
-// once per step, was the largest part of the error near the planets, and
-// the sweep that stores them is bound by its instructions, which the
-// stochastic rounding of four stores per cell adds to)
+// The transported momenta, read by the end of the step: FP64 in both storage
+// modes (in split storage their FP32 rounding, once per step, was the largest
+// part of the error near the planets, and the sweeps are bound by their
+// instructions, which the stochastic rounding of four stores per cell adds to)
 __device__ __forceinline__ Fld<false> mom_out(const KParams &P, int q)
 {
     return Fld<false>{static_cast<double *>(P.mom[q]), nullptr, P.ns, 0u};
@@ -3110,8 +3109,7 @@ FCPT_PAIR1(ghost_bc, 256, int, advance_time)
 // other blocks (one of 256 threads per ring) form the ring means.  The ghost
 // rings' v_phi is one Keplerian value per ring, so their blocks sum that value
 // as stored in place of a load (the same sums, the same tree) and no block
-// reads what another writes.  Only the azimuthal sweep reads the ring means,
-// so they may be formed before the radial sweep.
+// reads what another writes.  Only the sweeps read the ring means.
 template <bool SPLIT>
 __device__ __forceinline__ void b_ghost_ring_mean(const KParams &P, int bx)
 {

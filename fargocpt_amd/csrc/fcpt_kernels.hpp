@@ -69,7 +69,7 @@ long kv_waves(const KParams &P, int tile);
 void resolve_kv_tiles(std::vector<KParams> &disks);
 void launch_kick(const KParams &P, hipStream_t st, int fold_mode);
 // the potential; fold_mode >= 0: in the same launch, the CFL fold of
-// k_cfl_rings' slots (launch_cfl_cells) with that mode
+// the ring minima of launch_cfl_cells with that mode
 void launch_potential_fold(const KParams &P, hipStream_t st, int fold_mode);
 // the CFL limits' ring minima and the potential in one launch; a launch_kick with
 // fold_mode kFoldDone after it folds the minima (mode 2) and launches no potential

@@ -23,12 +23,12 @@ import re
 
 # bench.py times these kernels with fcpt_time_kernel: 3 rounds of 1 warm-up + 20
 # launches (the viscous pass timed is the walk without SubStep3)
-TIMED = (r"k_radial_sweep", r"k_azimuthal_sweep", r"k_cfl_rings", r"k_visc_walk<(true|false), false>",
+TIMED = (r"k_sweeps<", r"k_cfl_ring<(true|false), false>", r"k_visc_walk<(true|false), false>",
          r"k_potential_fold<")
 TIMING_LAUNCHES = 63
 KT_STEPS = 55
-JSON_NAMES = {r"k_radial_sweep": "radial_sweep", r"k_azimuthal_sweep": "azimuthal_sweep",
-              r"k_cfl_rings": "cfl", r"k_visc_walk<(true|false), false>": "visc_fused",
+JSON_NAMES = {r"k_sweeps<": "sweeps",
+              r"k_cfl_ring<(true|false), false>": "cfl", r"k_visc_walk<(true|false), false>": "visc_fused",
               r"k_potential_fold<": "potential", r"k_disk_force<": "disk_force"}
 
 
@@ -69,9 +69,8 @@ def summarise(workload: str, prec: str, base: str, outdir: str) -> dict:
     rows = list(csv.DictReader(open(kt[0])))
     L += ["## Kernel time (kernel_stats.csv)\n",
           f"Calls include the {TIMING_LAUNCHES} launches with which bench.py times each of the "
-          "radial sweep, azimuthal sweep, CFL rings, potential and the viscous walk without "
-          "SubStep3 (an adiabatic step runs the walk with SubStep3, so there this one shows 0 "
-          "launches per step); launches per "
+          "sweeps, CFL rings, potential and the viscous walk without SubStep3 (those that the "
+          "step does not run show 0 launches per step); launches per "
           f"step excludes them and divides by the {KT_STEPS} traced steps.\n",
           "| kernel | calls | launches per step | average µs | % of GPU time |",
           "|---|---|---|---|---|"]
@@ -140,8 +139,8 @@ ISSUE_PASSES = {
             "SQ_INSTS_VALU_TRANS_F64", "SQ_INSTS_VALU_INT32", "SQ_INSTS_VALU_CVT", "SQ_INSTS_VALU_INT64",
             "SQ_INSTS_SMEM"),
 }
-STEP_KERNELS = ("k_azimuthal_sweep", "k_radial_sweep3", "k_visc_walk<(true|false), true>", "k_velocities_final",
-                "k_kick_walk", "k_cfl_rings", "k_potential_fold", "k_ghost_ring_mean")
+STEP_KERNELS = ("k_sweeps<", "k_kv_walk", "k_velocities_final", "k_cfl_ring", "k_potential_fold",
+                "k_ghost_ring_mean")
 SIMDS, CLOCK_HZ = 1024, 2.4e9  # MI355X: 256 CUs x 4 SIMDs, 2.4 GHz peak engine clock
 
 

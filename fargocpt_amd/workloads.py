@@ -153,8 +153,7 @@ def algorithmic_bytes(kernel: str, adiabatic: bool, element: int = 8) -> int:
     per value (8 for FP64 storage, 4 for split storage)."""
     e = 1 if adiabatic else 0
     reads_writes = {
-        "radial_sweep": (3 + e, 5 + e),        # Sigma, v_r, v_phi, (E) -> 4 momenta, Sigma, (E)
-        "azimuthal_sweep": (6 + e, 5 + e),     # Sigma, 4 momenta, (E), v_phi -> 5/6, shifted
+        "sweeps": (3 + e, 5 + e),              # Sigma, v_r, v_phi, (E) -> 4 momenta, Sigma, (E)
         "cfl": (4 + 3 * e, 0),                 # v_r, v_phi, c_s, nu, (Q+, Q-, E)
         "stress": (4, 4),                      # v_r, v_phi, nu, Sigma -> div v, tau_rr, tau_pp, tau_rp
         # v_r, v_phi, Sigma, (nu) -> v_r, v_phi, (div v and the tensor for the heating)
@@ -163,7 +162,8 @@ def algorithmic_bytes(kernel: str, adiabatic: bool, element: int = 8) -> int:
         "disk_force": (2 + e, 0),              # Sigma (ring means, then cells), (H)
     }
     r, w = reads_writes[kernel]
-    return element * (r + w)
+    # what the sweeps hand to the end of the step is FP64 in both storage modes
+    return element * r + (8 if kernel == "sweeps" else element) * w
 
 
 def step_bytes(adiabatic: bool, element: int = 8) -> int:

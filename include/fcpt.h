@@ -268,9 +268,10 @@ int fcpt_run_steps(fcpt_ctx *ctx, int32_t n_steps, int32_t use_graph);
    bodies, a star at the origin and a planet at (1, 0), with the self-gravity
    correction.  FCPT_KERNEL_CFL is the per-ring CFL kernel (ring means of
    v_phi and the cells' limits; the fold of the ring minima is not timed).
-   FCPT_KERNEL_VISC_FUSED is the fused viscous stress + velocity pass of the
-   step (FCPT_PARAM_FUSED_STEP) without SubStep3: the viscous walk, or the
-   cell-parallel pass where the viscous tile is 1; it writes only the
+   FCPT_KERNEL_VISC_FUSED is the fused viscous stress + velocity pass that the
+   step of a disk without artificial viscosity runs (others run it inside the
+   kick walk), without SubStep3: the viscous walk, or the cell-parallel pass
+   where the viscous tile is 1; it writes only the
    velocities' partner buffers (and, in an adiabatic disk with viscous
    heating, the stress tensor). */
 enum { FCPT_KERNEL_RADIAL_SWEEP = 0, FCPT_KERNEL_AZIMUTHAL = 1, FCPT_KERNEL_CFL = 3,
@@ -400,8 +401,9 @@ int fcpt_batch_run_steps(fcpt_batch *batch, int32_t n_steps, int32_t use_graph);
 /* as fcpt_batch_run_steps, timed with HIP events on the batch's stream */
 int fcpt_batch_time_steps(fcpt_batch *batch, int32_t n_steps, int32_t use_graph, double *ms_total);
 /* mean duration of one batched launch of one step kernel over all disks
-   (FCPT_KERNEL_RADIAL_SWEEP, _AZIMUTHAL, _CFL, _POTENTIAL; they do not
-   modify their inputs) */
+   (FCPT_KERNEL_RADIAL_SWEEP and _AZIMUTHAL, which are one kernel, _CFL,
+   _POTENTIAL, both with the launch of the members that run the two as one;
+   they do not modify their inputs) */
 int fcpt_batch_time_kernel(fcpt_batch *batch, int32_t kernel, int32_t reps, double *ms_per_launch);
 
 /* ---- snapshots (output files of the reference) ------------------------ */
