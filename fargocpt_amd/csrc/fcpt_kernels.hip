@@ -3283,8 +3283,11 @@ __device__ __forceinline__ void raw_ring(const KParams &P, int r, int j, int jn,
 // two kernels and now: 128x384 isothermal 36.5 -> 29.6 us, 307x1021 beta 80.0
 // -> 69.8, 1024x3072 adiabatic 345.7 -> 306, 2048x6144 isothermal 877 -> 769,
 // 4096x12288 beta 5034 -> 4550, split 4052 -> 3731.
-// Prefetching the ring constants an iteration ahead costs scalar registers:
-// 2 to 4 % slower.
+// Rings at and beyond the edges take branches of their own: a select per value
+// on every ring was 6 % of the instructions (2048x6144 split 697 -> 684 us per
+// step).  Prefetching the ring constants an iteration ahead costs scalar
+// registers (2 to 4 % slower), the loop unrolled by three so that the window
+// needs no copies vector ones (4096x12288 FP64 4390 -> 4882 us).
 __device__ __forceinline__ double sweep_tab(const KParams &P, int t, int i)
 {
     return cst(P.sweep_tab)[i * kSweepTabs + t];
@@ -3345,8 +3348,8 @@ __device__ __forceinline__ void sweep_decode(const KParams &P, const RingRaw<SPL
     all[2] = sig * (vaz.dec(rc, X.vaj) + rr * OmegaF) * rr;
     all[3] = sig * (R.va + rr * OmegaF) * rr;
     if constexpr (ADI) all[4] = fld<SPLIT>(P, FCPT_ENERGY).dec(rc, X.e);
-    R.v = (r >= 0 && r <= P.nr) ? v0 : 0.0;
-    R.s = in ? sig : 1.0;
+    R.v = v0;
+    R.s = sig;
     const double *q = all + Q0;
     double w[NQ];
     R.fine = true;
@@ -3371,24 +3374,27 @@ __device__ __forceinline__ void sweep_decode(const KParams &P, const RingRaw<SPL
     }
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
-        R.q[k] = in ? q[k] : 0.0;
-        R.w[k] = in ? w[k] : 0.0;
+        R.q[k] = q[k];
+        R.w[k] = w[k];
+    }
+    if (!in) {
+        __builtin_amdgcn_s_sleep(0);  // a branch: selects on every ring are 6 % of the walk's instructions
+        R.s = 1.0;
+        if (r != P.nr) R.v = 0.0;
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) R.q[k] = R.w[k] = 0.0;
     }
 }
 
 // half the van Leer slopes of ring k from rings k-1, k, k+1
 // (compute_star_radial first loop, TransportEuler.cpp:355-371); zero on the ghost rings
 template <bool SPLIT, bool FINE, int NQ>
-__device__ __forceinline__ void sweep_slopes_of(double im, double ip, bool act, const SweepRing<NQ> &M,
+__device__ __forceinline__ void sweep_slopes_of(double im, double ip, const SweepRing<NQ> &M,
                                                 SweepRing<NQ> &C, const SweepRing<NQ> &N)
 {
-    const double ds = vl_half<SPLIT, FINE>((N.s - C.s) * ip, (C.s - M.s) * im);
-    C.ds = act ? ds : 0.0;
+    C.ds = vl_half<SPLIT, FINE>((N.s - C.s) * ip, (C.s - M.s) * im);
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        const double dw = vl_half<SPLIT, FINE>((N.w[q] - C.w[q]) * ip, (C.w[q] - M.w[q]) * im);
-        C.dw[q] = act ? dw : 0.0;
-    }
+    for (int q = 0; q < NQ; ++q) C.dw[q] = vl_half<SPLIT, FINE>((N.w[q] - C.w[q]) * ip, (C.w[q] - M.w[q]) * im);
 }
 template <bool SPLIT, int NQ>
 __device__ __forceinline__ void sweep_slopes(const KParams &P, int k, const SweepRing<NQ> &M, SweepRing<NQ> &C,
@@ -3398,10 +3404,16 @@ __device__ __forceinline__ void sweep_slopes(const KParams &P, int k, const Swee
     const int kc = act ? k : 1;
     const double im = sweep_tab(P, SW_INV_DIFF_RMED, kc), ip = sweep_tab(P, SW_INV_DIFF_RMED, kc + 1);
     if (SPLIT || (M.fine && C.fine && N.fine)) {
-        sweep_slopes_of<SPLIT, true, NQ>(im, ip, act, M, C, N);
+        sweep_slopes_of<SPLIT, true, NQ>(im, ip, M, C, N);
     } else {
         __builtin_amdgcn_s_sleep(0);
-        sweep_slopes_of<SPLIT, false, NQ>(im, ip, act, M, C, N);
+        sweep_slopes_of<SPLIT, false, NQ>(im, ip, M, C, N);
+    }
+    if (!act) {
+        __builtin_amdgcn_s_sleep(0);
+        C.ds = 0.0;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) C.dw[q] = 0.0;
     }
 }
 
@@ -3422,16 +3434,20 @@ __device__ __forceinline__ void sweep_flux(const KParams &P, int k, const SweepR
     const double fpos = sweep_tab(P, SW_RMED, kc) - sweep_tab(P, SW_RMED, kc - 1) - v * dt;
     const double fneg = sweep_tab(P, SW_RMED, kc + 1) - sweep_tab(P, SW_RMED, kc) + v * dt;
     const bool up = v > 0.0;
-    const double ds0 = up ? A.s + fpos * A.ds : B.s - fneg * B.ds;
-    const double ds = act ? ds0 : 0.0;
+    const double ds = up ? A.s + fpos * A.ds : B.s - fneg * B.ds;
     const double c = dt * P.dphi * sweep_tab(P, SW_RINF, k);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const double qs0 = up ? A.w[q] + fpos * A.dw[q] : B.w[q] - fneg * B.dw[q];
-        const double qs = act ? qs0 : 0.0;
+        const double qs = up ? A.w[q] + fpos * A.dw[q] : B.w[q] - fneg * B.dw[q];
         f[q] = c * qs * ds * v;
     }
-    fs = c * (act ? 1.0 : 0.0) * ds * v;
+    fs = c * ds * v;
+    if (!act) {
+        __builtin_amdgcn_s_sleep(0);
+        fs = 0.0;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) f[q] = 0.0;
+    }
 }
 
 // Both FARGO passes (as az_ring) for this lane's sector of one ring, the
