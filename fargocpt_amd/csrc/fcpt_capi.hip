@@ -55,8 +55,9 @@ struct fcpt_ctx {
     // a device ring array for re-expressing a field about a new background
     std::vector<double> hbg[FCPT_NUM_FIELDS];
     double *bg_tmp = nullptr;
-    // the fused step leaves derived fields to be formed (lazy_derived)
-    bool derived_stale = false;
+    // the last step left derived fields to be formed (its lazy_derived), the scale
+    // height among them (its h_lazy)
+    bool derived_stale = false, h_stale = false;
     // the derived fields are those of the current E and Sigma (stored or
     // stale); false once a caller has set a field or stage of its own, which
     // the next step then reads as stored (one iteration of separate kernels)
@@ -121,6 +122,8 @@ int fail(fcpt_ctx *c, int code, const char *fmt, ...)
 // When the fused step runs the kick walk, the derived fields are formed where
 // the step needs them and left stale (KParams::lazy_derived) until
 // sync_derived stores them (the same expressions on the stored E and Sigma).
+// What is stale is the last step's doing, a batch's perhaps, and not a question
+// of the parameters in force when the fields are read.
 static bool lazy_applies(const fcpt_ctx *ctx) { return ctx->fused && kv_walk_applies(ctx->P); }
 // whether the next iteration runs fused, and the parameters it runs with
 // (the fused step of an isothermal disk forms its pressure from Sigma anyway)
@@ -134,18 +137,25 @@ static KParams step_view(const fcpt_ctx *ctx, bool fused)
     set_step_modes(P, fused);
     return P;
 }
-// after a whole iteration that ran with `fused`
-static void stepped(fcpt_ctx *ctx, bool fused)
+// after a whole iteration that ran with the parameters V
+static void stepped(fcpt_ctx *ctx, const KParams &V)
 {
-    ctx->derived_stale = fused && lazy_applies(ctx);
+    ctx->derived_stale = V.lazy_derived != 0;
+    ctx->h_stale = V.h_lazy != 0;
     ctx->derived_own = true;
 }
 static int sync_derived(fcpt_ctx *ctx)
 {
     if (!ctx->derived_stale) return FCPT_OK;
     launch_derived(ctx->P, ctx->stream);
-    ctx->derived_stale = false;
+    LAUNCH_CHECK(ctx);
+    ctx->derived_stale = ctx->h_stale = false;
     return FCPT_OK;
+}
+// before an iteration with the parameters V: the stale fields it reads, stored
+static int sync_for(fcpt_ctx *ctx, const KParams &V)
+{
+    return V.lazy_derived && (V.h_lazy || !ctx->h_stale) ? FCPT_OK : sync_derived(ctx);
 }
 // the fields sync_derived stores (an isothermal disk: the pressure alone)
 static bool derived_field(int f)
@@ -891,7 +901,8 @@ int fcpt_download_field(fcpt_ctx *ctx, int32_t field, double *host)
 {
     CTX_CHECK(ctx);
     if (field < 0 || field >= FCPT_NUM_FIELDS || !host) return fail(ctx, FCPT_ERR_ARG, "bad field");
-    if (derived_field(field)) sync_derived(ctx);
+    if (derived_field(field))
+        if (const int rc = sync_derived(ctx)) return rc;
     return copy_to_host(ctx, {{field, host}});
 }
 
@@ -1437,9 +1448,8 @@ static void enqueue_step(const KParams &P, hipStream_t st, int count_monitor, bo
 // then the step; the fused Euler step folds the CFL minima inside its
 // potential launch (one launch less)
 // `report`: the step's clock goes to the pinned mirror as well
-static void enqueue_iteration(const fcpt_ctx *ctx, bool fused, bool report = false)
+static void enqueue_iteration(const fcpt_ctx *ctx, KParams V, bool fused, bool report = false)
 {
-    KParams V = step_view(ctx, fused);
     if (report) V.s_out = ctx->s_host;
     const bool leapfrog = V.integrator == FCPT_INTEGRATOR_LEAPFROG;
     if (V.lazy_derived || (fused && !leapfrog)) {
@@ -1460,9 +1470,10 @@ int fcpt_step_euler(fcpt_ctx *ctx, double dt)
     CTX_SYNCED(ctx);
     launch_set_dt(ctx->P, ctx->stream, dt);
     const bool fused = next_fused(ctx);
-    enqueue_euler(step_view(ctx, fused), ctx->stream, 0, fused, -1);
+    const KParams V = step_view(ctx, fused);
+    enqueue_euler(V, ctx->stream, 0, fused, -1);
     LAUNCH_CHECK(ctx);
-    stepped(ctx, fused);
+    stepped(ctx, V);
     return FCPT_OK;
 }
 
@@ -1476,7 +1487,7 @@ int fcpt_step_leapfrog(fcpt_ctx *ctx, double dt)
     set_step_modes(V, fused);
     enqueue_leapfrog(V, ctx->stream, 0, fused, -1);
     LAUNCH_CHECK(ctx);
-    stepped(ctx, fused);
+    stepped(ctx, V);
     return FCPT_OK;
 }
 
@@ -1502,10 +1513,11 @@ int fcpt_run_step(fcpt_ctx *ctx, double *dt_out)
 {
     CTX_CHECK(ctx);
     const bool fused = next_fused(ctx);
-    if (!fused) sync_derived(ctx);
-    enqueue_iteration(ctx, fused, true);
+    const KParams V = step_view(ctx, fused);
+    if (const int rc = sync_for(ctx, V)) return rc;
+    enqueue_iteration(ctx, V, fused, true);
     LAUNCH_CHECK(ctx);
-    stepped(ctx, fused);
+    stepped(ctx, V);
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     if (take_nonfinite(ctx))
         return fail(ctx, FCPT_ERR_NONFINITE, "CFL time step is not finite and positive");
@@ -1521,7 +1533,7 @@ static int ensure_step_graph(fcpt_ctx *ctx, bool many)
     if (exec) return FCPT_OK;
     hipGraph_t g = nullptr;
     HIP_TRY(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < (many ? kGraphSteps : 1); ++k) enqueue_iteration(ctx, ctx->fused);
+    for (int k = 0; k < (many ? kGraphSteps : 1); ++k) enqueue_iteration(ctx, step_view(ctx, ctx->fused), ctx->fused);
     hipError_t e = hipStreamEndCapture(ctx->stream, &g);
     if (e != hipSuccess) return fail(ctx, FCPT_ERR_DEVICE, "graph capture: %s", hipGetErrorString(e));
     e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
@@ -1551,19 +1563,18 @@ int fcpt_run_steps(fcpt_ctx *ctx, int32_t n_steps, int32_t use_graph)
         int m = left;
         if (periodic_rebase(ctx)) m = std::min(m, ctx->rebase_interval - ctx->steps_since_rebase);
         const bool fused = next_fused(ctx);
-        if (fused != ctx->fused) {  // fields of the caller's own: one step of separate kernels
-            m = 1;
-            sync_derived(ctx);
-        }
+        const KParams V = step_view(ctx, fused);
+        if (fused != ctx->fused) m = 1;  // fields of the caller's own: one step of separate kernels
+        if (const int rc = sync_for(ctx, V)) return rc;
         int k = 0;
         if (use_graph && fused == ctx->fused) {
             const int per = many ? kGraphSteps : 1;
             for (; k + per <= m; k += per) HIP_TRY(ctx, hipGraphLaunch(ctx->step_graph[many ? 1 : 0], ctx->stream));
         }
-        for (; k < m; ++k) enqueue_iteration(ctx, fused);
+        for (; k < m; ++k) enqueue_iteration(ctx, V, fused);
         LAUNCH_CHECK(ctx);
         left -= m;
-        stepped(ctx, fused);
+        stepped(ctx, V);
         if (periodic_rebase(ctx) && (ctx->steps_since_rebase += m) >= ctx->rebase_interval) {
             const int rc = rebase_backgrounds(ctx);
             if (rc) return rc;
@@ -1685,6 +1696,8 @@ int fcpt_set_launch_param(fcpt_ctx *ctx, int32_t param, int32_t value)
     } else {
         return fail(ctx, FCPT_ERR_ARG, "unknown launch parameter");
     }
+    // stale fields as the steps that left them would have stored them
+    if (const int rc = sync_derived(ctx)) return rc;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     if (param == FCPT_PARAM_RADIAL_TILE) ctx->P.radial_tile = value;
     else if (param == FCPT_PARAM_RADIAL_WAVES) ctx->P.radial_waves = value;
@@ -1752,7 +1765,7 @@ int fcpt_autotune_walks(fcpt_ctx *ctx, int32_t reps, int32_t *kick_tile, int32_t
         hipError_t e = copy_fields(false);
         if (e == hipSuccess) e = hipMemcpyAsync(ctx->s_dev, &s0, sizeof(DevScalars), hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-        ctx->derived_stale = false;
+        ctx->derived_stale = ctx->h_stale = false;
         return e;
     };
     hipError_t e = copy_fields(true);
@@ -1869,7 +1882,7 @@ int fcpt_disk_on_planet_accel(fcpt_ctx *ctx, const fcpt_force_body *bodies, int3
             B.smooth_fixed[k] = -1.0;
     }
     KParams P = ctx->P;
-    P.h_lazy = ctx->derived_stale && step_view(ctx, true).h_lazy;  // no step stored H
+    P.h_lazy = ctx->h_stale;
     launch_disk_force(P, ctx->stream, B, ctx->force_part, ctx->force_host);
     LAUNCH_CHECK(ctx);
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
@@ -2160,7 +2173,6 @@ struct fcpt_batch {
     int split = 0;
     int radial_waves = 3;
     std::vector<fcpt_ctx *> disks;
-    std::vector<bool> lazy;  // the disk's batched step forms c_s, nu and T where needed
     KParams *Ps = nullptr;  // device array: every disk's parameters, then their swapped views
     std::vector<BatchStageDev> stages;
     hipStream_t stream = nullptr;
@@ -2261,7 +2273,6 @@ int fcpt_batch_create(fcpt_ctx *const *disks, int32_t n_disks, fcpt_batch **out)
         // are the disk's own, whatever tile the batch chooses below)
         set_step_modes(P, true);
         P.fold_in_kick = fold_in_kick(P);
-        b->lazy.push_back(P.lazy_derived != 0);
         host.push_back(P);
     }
     // The walks' tiles of the members that leave them to the size rule,
@@ -2364,6 +2375,13 @@ int fcpt_batch_run_steps(fcpt_batch *b, int32_t n_steps, int32_t use_graph)
         }
         --n_steps;
     }
+    // what a member's own steps left stale and its batched step reads
+    for (size_t k = 0; n_steps > 0 && k < b->disks.size(); ++k) {
+        fcpt_ctx *c = b->disks[k];
+        if (!c->derived_stale) continue;
+        if (sync_for(c, b->host[k])) return bfail(b, FCPT_ERR_DEVICE, c->err.c_str());
+        BHIP(b, hipStreamSynchronize(c->stream));
+    }
     for (int left = n_steps; left > 0;) {
         // up to the next background move of a member in split storage
         int m = left;
@@ -2381,8 +2399,7 @@ int fcpt_batch_run_steps(fcpt_batch *b, int32_t n_steps, int32_t use_graph)
         // after the batched steps on the disk's own stream
         BHIP(b, hipEventRecord(b->done, b->stream));
         for (fcpt_ctx *c : b->disks) BHIP(b, hipStreamWaitEvent(c->stream, b->done, 0));
-        for (size_t k = 0; k < b->disks.size(); ++k)
-            if (b->lazy[k]) b->disks[k]->derived_stale = true;
+        for (size_t k = 0; k < b->disks.size(); ++k) stepped(b->disks[k], b->host[k]);
         for (fcpt_ctx *c : b->disks) {
             if (!periodic_rebase(c) || (c->steps_since_rebase += m) < c->rebase_interval) continue;
             if (rebase_backgrounds(c)) return bfail(b, FCPT_ERR_DEVICE, c->err.c_str());
