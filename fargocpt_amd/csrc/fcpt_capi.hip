@@ -1749,6 +1749,7 @@ int fcpt_autotune_walks(fcpt_ctx *ctx, int32_t reps, int32_t *kick_tile, int32_t
         off[k] = total;
         total += (field_rows(k, P.nr) * P.ns * field_element_size(P, k) + 255) / 256 * 256;
     }
+    const bool own = ctx->derived_own;
     char *save = nullptr;
     HIP_TRY(ctx, hipMalloc((void **)&save, total));
     DevScalars s0;
@@ -1766,6 +1767,7 @@ int fcpt_autotune_walks(fcpt_ctx *ctx, int32_t reps, int32_t *kick_tile, int32_t
         if (e == hipSuccess) e = hipMemcpyAsync(ctx->s_dev, &s0, sizeof(DevScalars), hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
         ctx->derived_stale = ctx->h_stale = false;
+        ctx->derived_own = own;
         return e;
     };
     hipError_t e = copy_fields(true);

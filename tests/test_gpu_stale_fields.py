@@ -82,3 +82,19 @@ def test_batch_of_separate_passes(physics):
         _force(a, b)
     _same(a, b, physics)
     batch.close()
+
+
+@pytest.mark.parametrize("field", ["PRESSURE", "ENERGY", "SCALE_HEIGHT"])
+def test_autotune_keeps_uploaded_field(field):
+    """The autotuner's trials leave the next step a field of the caller's own
+    to read."""
+    print(field, flush=True)
+    disks = [_disk(NAMES["adi"], 40, 97, fused=f) for f in (True, True, False)]
+    for d in disks:
+        d.run_steps(3)
+        d.upload_field(field, d.download_field(field) * 1.01)
+    disks[0].autotune_walks(2)
+    for d in disks:
+        d.run_steps(3)
+    _same(disks[1], disks[2], field)
+    _same(disks[0], disks[2], field)
