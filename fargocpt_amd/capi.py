@@ -23,10 +23,28 @@ FIELD_ID = {name: i for i, name in enumerate(FIELDS)}
 VECTOR_FIELDS = {"VRAD", "VRAD0", "TAU_R_PHI"}
 
 ARTVISC = {"none": 0, "tw": 1, "sn": 2}
+
+
+class KernelIds(dict):
+    """Kernel ids by name, an entry per kernel.  The transport's two sweeps run
+    as one kernel; each one's own name stands for it in a lookup."""
+
+    ALIASES = {"radial_sweep": 0, "azimuthal_sweep": 1}
+
+    def __missing__(self, name):
+        return self.ALIASES[name]
+
+    def __contains__(self, name):
+        return super().__contains__(name) or name in self.ALIASES
+
+    def get(self, name, default=None):
+        return self[name] if name in self else default
+
+
 # kernels of the (fused) step that fcpt_time_kernel can time on their own
-KERNELS = {"sweeps": 0, "cfl": 3, "visc_fused": 7, "potential": 5}
+KERNELS = KernelIds({"sweeps": 0, "cfl": 3, "visc_fused": 7, "potential": 5})
 # the same on a batch (the viscous pass is not timed there)
-BATCH_KERNELS = {"sweeps": 0, "cfl": 3, "potential": 5}
+BATCH_KERNELS = KernelIds({"sweeps": 0, "cfl": 3, "potential": 5})
 KERNEL_STRESS = 4      # the separate stress-tensor kernel of fcpt_viscous_stress_tensor
 KERNEL_DISK_FORCE = 6  # the disk-on-planet reduction (not part of the hydro step)
 # storage modes (fcpt_disk_desc.precision) and launch parameters of include/fcpt.h

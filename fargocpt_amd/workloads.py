@@ -161,6 +161,8 @@ def algorithmic_bytes(kernel: str, adiabatic: bool, element: int = 8) -> int:
         "potential": (1, 1),                   # H -> Phi
         "disk_force": (2 + e, 0),              # Sigma (ring means, then cells), (H)
     }
+    if kernel in ("radial_sweep", "azimuthal_sweep"):  # they run as one kernel
+        kernel = "sweeps"
     r, w = reads_writes[kernel]
     # what the sweeps hand to the end of the step is FP64 in both storage modes
     return element * r + (8 if kernel == "sweeps" else element) * w
