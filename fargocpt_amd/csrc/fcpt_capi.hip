@@ -60,7 +60,7 @@ struct fcpt_ctx {
     bool derived_stale = false, h_stale = false;
     // the derived fields are those of the current E and Sigma (stored or
     // stale); false once a caller has set a field or stage of its own, which
-    // the next step then reads as stored (one iteration of separate kernels)
+    // the next step then reads as stored
     bool derived_own = true;
     // split storage: steps between background moves (FCPT_PARAM_REBASE_INTERVAL;
     // 0 = only on request) and steps since the last one
@@ -125,16 +125,20 @@ int fail(fcpt_ctx *c, int code, const char *fmt, ...)
 // What is stale is the last step's doing, a batch's perhaps, and not a question
 // of the parameters in force when the fields are read.
 static bool lazy_applies(const fcpt_ctx *ctx) { return ctx->fused && kv_walk_applies(ctx->P); }
-// whether the next iteration runs fused, and the parameters it runs with
-// (the fused step of an isothermal disk forms its pressure from Sigma anyway)
-static bool next_fused(const fcpt_ctx *ctx)
+// Whether the next step has to read derived fields as the caller left them: it
+// then runs the fused step's cell passes, which read them stored, in place of
+// the walk (the fused step of an isothermal disk forms its pressure from Sigma
+// anyway).  A final boundary call and the step after it, with the separate kernels
+// and so: 512x1536 adiabatic 187 and 157 us, 1024x3072 553 and 481.
+static bool reads_stored(const fcpt_ctx *ctx)
 {
-    return ctx->fused && (ctx->derived_own || !ctx->P.adiabatic || !lazy_applies(ctx));
+    return !ctx->derived_own && ctx->P.adiabatic && lazy_applies(ctx);
 }
-static KParams step_view(const fcpt_ctx *ctx, bool fused)
+// the parameters of a step that forms its derived fields itself, or reads them
+static KParams step_view(const fcpt_ctx *ctx, bool stored = false)
 {
     KParams P = ctx->P;
-    set_step_modes(P, fused);
+    set_step_modes(P, ctx->fused && !stored);
     return P;
 }
 // after a whole iteration that ran with the parameters V
@@ -1448,11 +1452,11 @@ static void enqueue_step(const KParams &P, hipStream_t st, int count_monitor, bo
 // then the step; the fused Euler step folds the CFL minima inside its
 // potential launch (one launch less)
 // `report`: the step's clock goes to the pinned mirror as well
-static void enqueue_iteration(const fcpt_ctx *ctx, KParams V, bool fused, bool report = false)
+static void enqueue_iteration(const fcpt_ctx *ctx, KParams V, bool report = false)
 {
     if (report) V.s_out = ctx->s_host;
     const bool leapfrog = V.integrator == FCPT_INTEGRATOR_LEAPFROG;
-    if (V.lazy_derived || (fused && !leapfrog)) {
+    if (V.lazy_derived || (ctx->fused && !leapfrog)) {
         if (V.cfl_pot) launch_cfl_potential(V, ctx->stream);
         else launch_cfl_cells(V, ctx->stream);
         V.fold_in_kick = fold_in_kick(V);
@@ -1461,7 +1465,7 @@ static void enqueue_iteration(const fcpt_ctx *ctx, KParams V, bool fused, bool r
         else enqueue_euler(V, ctx->stream, 1, true, fold_mode);
     } else {
         launch_cfl(V, ctx->stream, 2);
-        enqueue_step(V, ctx->stream, 1, fused);
+        enqueue_step(V, ctx->stream, 1, ctx->fused);
     }
 }
 
@@ -1469,9 +1473,8 @@ int fcpt_step_euler(fcpt_ctx *ctx, double dt)
 {
     CTX_SYNCED(ctx);
     launch_set_dt(ctx->P, ctx->stream, dt);
-    const bool fused = next_fused(ctx);
-    const KParams V = step_view(ctx, fused);
-    enqueue_euler(V, ctx->stream, 0, fused, -1);
+    const KParams V = step_view(ctx, reads_stored(ctx));
+    enqueue_euler(V, ctx->stream, 0, ctx->fused, -1);
     LAUNCH_CHECK(ctx);
     stepped(ctx, V);
     return FCPT_OK;
@@ -1481,11 +1484,10 @@ int fcpt_step_leapfrog(fcpt_ctx *ctx, double dt)
 {
     CTX_SYNCED(ctx);
     launch_set_dt(ctx->P, ctx->stream, dt);
-    const bool fused = next_fused(ctx);
     KParams V = ctx->P;
     V.integrator = FCPT_INTEGRATOR_LEAPFROG;  // the scheme, whatever the descriptor's own
-    set_step_modes(V, fused);
-    enqueue_leapfrog(V, ctx->stream, 0, fused, -1);
+    set_step_modes(V, ctx->fused && !reads_stored(ctx));
+    enqueue_leapfrog(V, ctx->stream, 0, ctx->fused, -1);
     LAUNCH_CHECK(ctx);
     stepped(ctx, V);
     return FCPT_OK;
@@ -1512,10 +1514,9 @@ int fcpt_set_midstep_params(fcpt_ctx *ctx, const fcpt_step_params *params)
 int fcpt_run_step(fcpt_ctx *ctx, double *dt_out)
 {
     CTX_CHECK(ctx);
-    const bool fused = next_fused(ctx);
-    const KParams V = step_view(ctx, fused);
+    const KParams V = step_view(ctx, reads_stored(ctx));
     if (const int rc = sync_for(ctx, V)) return rc;
-    enqueue_iteration(ctx, V, fused, true);
+    enqueue_iteration(ctx, V, true);
     LAUNCH_CHECK(ctx);
     stepped(ctx, V);
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
@@ -1533,7 +1534,7 @@ static int ensure_step_graph(fcpt_ctx *ctx, bool many)
     if (exec) return FCPT_OK;
     hipGraph_t g = nullptr;
     HIP_TRY(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < (many ? kGraphSteps : 1); ++k) enqueue_iteration(ctx, step_view(ctx, ctx->fused), ctx->fused);
+    for (int k = 0; k < (many ? kGraphSteps : 1); ++k) enqueue_iteration(ctx, step_view(ctx));
     hipError_t e = hipStreamEndCapture(ctx->stream, &g);
     if (e != hipSuccess) return fail(ctx, FCPT_ERR_DEVICE, "graph capture: %s", hipGetErrorString(e));
     e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
@@ -1562,16 +1563,16 @@ int fcpt_run_steps(fcpt_ctx *ctx, int32_t n_steps, int32_t use_graph)
     for (int left = n_steps; left > 0;) {
         int m = left;
         if (periodic_rebase(ctx)) m = std::min(m, ctx->rebase_interval - ctx->steps_since_rebase);
-        const bool fused = next_fused(ctx);
-        const KParams V = step_view(ctx, fused);
-        if (fused != ctx->fused) m = 1;  // fields of the caller's own: one step of separate kernels
+        const bool stored = reads_stored(ctx);
+        if (stored) m = 1;  // one step, then as captured
+        const KParams V = step_view(ctx, stored);
         if (const int rc = sync_for(ctx, V)) return rc;
         int k = 0;
-        if (use_graph && fused == ctx->fused) {
+        if (use_graph && !stored) {
             const int per = many ? kGraphSteps : 1;
             for (; k + per <= m; k += per) HIP_TRY(ctx, hipGraphLaunch(ctx->step_graph[many ? 1 : 0], ctx->stream));
         }
-        for (; k < m; ++k) enqueue_iteration(ctx, V, fused);
+        for (; k < m; ++k) enqueue_iteration(ctx, V);
         LAUNCH_CHECK(ctx);
         left -= m;
         stepped(ctx, V);

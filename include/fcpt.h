@@ -318,8 +318,7 @@ int fcpt_time_copy(fcpt_ctx *ctx, int32_t reps, double *ms_per_launch, double *b
    points above, which always store them.  The derived fields a fused step
    needs are formed from E and Sigma; a step that follows a field or stage of
    the caller's own (fcpt_upload_field of Sigma, E or a derived field, or a
-   stage entry point that changes them) reads the fields as stored, through
-   the separate kernels.  Every parameter change drops a
+   stage entry point that changes them) reads the fields as stored.  Every parameter change drops a
    captured step graph so that the next fcpt_run_steps captures the new
    shape. */
 /* FCPT_PARAM_SPLIT_ROUNDING (split storage only; default 1) chooses how a

@@ -98,3 +98,26 @@ def test_autotune_keeps_uploaded_field(field):
         d.run_steps(3)
     _same(disks[1], disks[2], field)
     _same(disks[0], disks[2], field)
+
+
+@pytest.mark.parametrize("integrator", [0, 1])
+@pytest.mark.parametrize("how", ["pressure", "damping"])
+def test_own_fields_keep_the_fused_passes(integrator, how):
+    """A step that reads the fields as the caller left them is still a fused
+    one: the tensors that only the separate kernels store keep their marks."""
+    print(f"integrator {integrator} {how}", flush=True)
+    a, b = _pair("adi", integrator)
+    for d in (a, b):
+        d.run_step()
+        if how == "pressure":
+            d.upload_field("PRESSURE", d.download_field("PRESSURE") * 1.01)
+        else:
+            d.apply_boundary_condition(1e-3, True)
+    mark = np.full((40, 97), 7.0)
+    for f in ("Q_R", "Q_PHI"):
+        a.upload_field(f, mark)
+    for d in (a, b):
+        d.run_step()
+    for f in ("Q_R", "Q_PHI"):
+        assert np.array_equal(a.download_field(f), mark), f
+    _same(a, b, (integrator, how))
