@@ -51,16 +51,20 @@ def build(verbose: bool = False) -> str:
 
 
 def build_host_check() -> str:
-    """The C++ host-interface check program used by the GPU tests."""
-    src = os.path.join(os.path.dirname(HERE), "tests", "cpp", "host_api_check.cpp")
-    exe = os.path.join(os.path.dirname(HERE), "tests", "cpp", "host_api_check.bin")
-    cmd = [HIPCC, "-O2", "-std=c++17", "-ffp-contract=off", src, "-o", exe,
-           f"-L{HERE}", f"-Wl,-rpath,{HERE}", "-lfcpt_hip"]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        sys.stderr.write(r.stdout + r.stderr)
-        raise RuntimeError("build of host_api_check failed")
-    return exe
+    """The C++ programs used by the GPU tests: the host-interface check, whose
+    path is returned, and the copies with and without pinned memory."""
+    cpp = os.path.join(os.path.dirname(HERE), "tests", "cpp")
+    exes = []
+    for name, extra in (("pinned_check", ["-rdynamic", "-ldl"]), ("host_api_check", [])):
+        src, exe = (os.path.join(cpp, f"{name}.{x}") for x in ("cpp", "bin"))
+        cmd = [HIPCC, "-O2", "-std=c++17", "-ffp-contract=off", src, "-o", exe,
+               f"-L{HERE}", f"-Wl,-rpath,{HERE}", "-lfcpt_hip", *extra]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            sys.stderr.write(r.stdout + r.stderr)
+            raise RuntimeError(f"build of {name} failed")
+        exes.append(exe)
+    return exes[-1]
 
 
 if __name__ == "__main__":

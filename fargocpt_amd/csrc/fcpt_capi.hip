@@ -651,7 +651,8 @@ static int upload_split(fcpt_ctx *ctx, int field, const double *host)
 //
 // The slots belong to the process (a disk's own would cost each disk their
 // pinning, ~10 ms): allocated by the first copy that needs them, leased to one
-// copy at a time, freed with the last context.
+// copy at a time, freed with the last context.  A copy that gets none goes
+// without.
 constexpr size_t kSlotBytes = size_t(4) << 20;
 constexpr int kSlots = 12, kCopyThreads = 8;
 constexpr size_t kSmallBytes = size_t(1) << 20;  // copies up to this size have a buffer of their own
@@ -691,6 +692,7 @@ static hipError_t host_slots_get(bool large, char **out)
                                            hipHostMallocPortable);
         if (e != hipSuccess) {
             p = nullptr;
+            hipGetLastError();  // the caller goes another way: no later call reports it
             return e;
         }
     }
@@ -702,6 +704,15 @@ struct HostCopy {
     int field;
     double *dst;
 };
+struct HostCopies {
+    HostCopy c[4];
+    size_t n = 0;
+    void add(int field, double *dst) { c[n++] = HostCopy{field, dst}; }
+    size_t size() const { return n; }
+    const HostCopy &operator[](size_t k) const { return c[k]; }
+    const HostCopy *begin() const { return c; }
+    const HostCopy *end() const { return c + n; }
+};
 
 // one piece of a copy: n elements of fields[which] from element `first` on
 struct CopyPiece {
@@ -709,12 +720,33 @@ struct CopyPiece {
     size_t first, n;
 };
 
-static int copy_large(fcpt_ctx *ctx, const std::vector<HostCopy> &fields)
+// without pinned memory: each field straight into the caller's pages
+static int copy_pageable(fcpt_ctx *ctx, const HostCopies &fields)
+{
+    const KParams &P = ctx->P;
+    hipError_t e = hipSuccess;
+    for (const HostCopy &f : fields) {
+        const size_t rows = field_rows(f.field, P.nr), ns = (size_t)P.ns;
+        const bool decode = P.split && f.field != FCPT_POTENTIAL;
+        std::vector<double> bg(decode ? rows : 0);
+        std::vector<float> dev(decode ? rows * ns : 0);
+        void *const to = decode ? (void *)dev.data() : (void *)f.dst;
+        if (decode) e = hipMemcpyAsync(bg.data(), P.bg[f.field], rows * sizeof(double), hipMemcpyDeviceToHost, ctx->stream);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(to, P.f[f.field], rows * ns * field_element_size(P, f.field), hipMemcpyDeviceToHost, ctx->stream);
+        const hipError_t se = hipStreamSynchronize(ctx->stream);  // nothing in flight into bg and dev below
+        if (e == hipSuccess) e = se;
+        HIP_TRY(ctx, e);
+        for (size_t i = 0; decode && i < rows; ++i)
+            for (size_t j = 0; j < ns; ++j) f.dst[i * ns + j] = bg[i] + (double)dev[i * ns + j];
+    }
+    return FCPT_OK;
+}
+
+static int copy_large(fcpt_ctx *ctx, const HostCopies &fields, char *slots)
 {
     const KParams &P = ctx->P;
     const size_t ns = (size_t)P.ns;
-    char *slots = nullptr;
-    HIP_TRY(ctx, host_slots_get(true, &slots));
     std::vector<CopyPiece> pieces;
     std::vector<std::vector<double>> bg(fields.size());
     for (size_t k = 0; k < fields.size(); ++k) {
@@ -819,11 +851,9 @@ static int copy_large(fcpt_ctx *ctx, const std::vector<HostCopy> &fields)
 
 // all fields by one kernel into the slots, then to the caller: by this thread
 // below 1 MB, by several above
-static int copy_export(fcpt_ctx *ctx, const std::vector<HostCopy> &fields, size_t total)
+static int copy_export(fcpt_ctx *ctx, const HostCopies &fields, size_t total, char *out)
 {
     const KParams &P = ctx->P;
-    char *out = nullptr;
-    HIP_TRY(ctx, host_slots_get(total > kSmallBytes, &out));
     ExportFields x{};
     size_t at = 0;
     for (const HostCopy &f : fields) {
@@ -875,14 +905,19 @@ static int copy_export(fcpt_ctx *ctx, const std::vector<HostCopy> &fields, size_
 
 // the fields to the caller's arrays in FP64 (split storage: background +
 // deviation)
-static int copy_to_host(fcpt_ctx *ctx, const std::vector<HostCopy> &fields)
+static int copy_to_host(fcpt_ctx *ctx, const HostCopies &fields)
 {
     const KParams &P = ctx->P;
     size_t total = 0;
     for (const HostCopy &f : fields) total += field_rows(f.field, P.nr) * (size_t)P.ns * sizeof(double);
-    std::lock_guard<std::mutex> lease(host_slots().lease);
     try {
-        return total > kSlotBytes * kSlots ? copy_large(ctx, fields) : copy_export(ctx, fields, total);
+        {
+            std::lock_guard<std::mutex> lease(host_slots().lease);
+            char *out = nullptr;
+            if (host_slots_get(total > kSmallBytes, &out) == hipSuccess)
+                return total > kSlotBytes * kSlots ? copy_large(ctx, fields, out) : copy_export(ctx, fields, total, out);
+        }
+        return copy_pageable(ctx, fields);
     } catch (const std::exception &e) {
         return fail(ctx, FCPT_ERR_DEVICE, "copy to the host: %s", e.what());
     }
@@ -907,7 +942,9 @@ int fcpt_download_field(fcpt_ctx *ctx, int32_t field, double *host)
     if (field < 0 || field >= FCPT_NUM_FIELDS || !host) return fail(ctx, FCPT_ERR_ARG, "bad field");
     if (derived_field(field))
         if (const int rc = sync_derived(ctx)) return rc;
-    return copy_to_host(ctx, {{field, host}});
+    HostCopies one;
+    one.add(field, host);
+    return copy_to_host(ctx, one);
 }
 
 // split storage: re-express a field about a new host-given background
@@ -1178,12 +1215,12 @@ int fcpt_upload_state(fcpt_ctx *ctx, const double *sigma, const double *vrad, co
 int fcpt_download_state(fcpt_ctx *ctx, double *sigma, double *vrad, double *vazi, double *energy)
 {
     CTX_CHECK(ctx);
-    std::vector<HostCopy> fields;
+    HostCopies fields;
     double *const dst[4] = {sigma, vrad, vazi, energy};
     const int f[4] = {FCPT_SIGMA, FCPT_VRAD, FCPT_VAZI, FCPT_ENERGY};
     for (int k = 0; k < 4; ++k)
-        if (dst[k]) fields.push_back({f[k], dst[k]});
-    return fields.empty() ? FCPT_OK : copy_to_host(ctx, fields);
+        if (dst[k]) fields.add(f[k], dst[k]);
+    return fields.n == 0 ? FCPT_OK : copy_to_host(ctx, fields);
 }
 
 int fcpt_set_time(fcpt_ctx *ctx, double time, double last_dt, int32_t n_monitor)

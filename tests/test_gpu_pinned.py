@@ -1,0 +1,35 @@
+"""Copies to the host where pinned memory is refused, and what they pin where it
+is granted: tests/cpp/pinned_check counts and refuses the library's requests.
+Fields and states below, at and above the sizes at which the copies change their
+route (one buffer, the slots as a whole, the slots in pieces)."""
+import os
+import subprocess
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+EXE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "pinned_check.bin")
+
+
+def _run(tmp_path, nr, nphi, precision):
+    from fargocpt_amd import workloads as W
+    from fargocpt_amd.capi import desc_from_dict
+    from fargocpt_amd.ic import log_radii
+    assert os.path.exists(EXE), "build tests/cpp/pinned_check with __graft_entry__.build()"
+    cfg = W.disk_config("adi_512x1536", precision)
+    cfg.update({"nr": nr, "nphi": nphi, "radii": log_radii(nr, cfg["rmin"], cfg["rmax"])})
+    desc, radii = desc_from_dict(cfg)
+    (tmp_path / "desc.bin").write_bytes(bytes(desc))
+    radii.tofile(str(tmp_path / "radii.bin"))
+    print(f"{nr} x {nphi} precision {precision}", flush=True)
+    r = subprocess.run([EXE, str(tmp_path)], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr
+    out = [line.split() for line in r.stdout.splitlines()]
+    return {w[0]: (w[1], int(w[2]), int(w[3])) for w in out if len(w) == 4}
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nr,nphi", [(8, 131), (128, 384), (1001, 1573)])
+def test_without_pinned_memory(tmp_path, nr, nphi, precision):
+    got = _run(tmp_path, nr, nphi, precision)
+    assert got["field"][0] == "same" and got["state"][0] == "same", got
