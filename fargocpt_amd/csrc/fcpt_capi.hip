@@ -649,10 +649,13 @@ static int upload_split(fcpt_ctx *ctx, int field, const double *host)
 // 1536: 1.5 - 3.5 -> 0.9 - 1.5 ms, 32 x 64: 80 -> 21 us; slots filled in smaller
 // pieces were slower than in one).
 //
-// The slots belong to the process (a disk's own would cost each disk their
-// pinning, ~10 ms): allocated by the first copy that needs them, leased to one
-// copy at a time, freed with the last context.  A copy that gets none goes
-// without.
+// The slots belong to the process: allocated by the first copy that needs them,
+// as large as it asks, rounded up to a power of two (pinning 2, 4 and 48 MB costs
+// 0.12 - 0.17, 0.3 and 0.5 ms), replaced by larger ones when one asks for more,
+// leased to one copy at a time, freed with the last context.  A copy that gets
+// none goes without, as does the process's first of each kind that fits them: a
+// process's first pinning and first use of it cost more than one copy gains (first
+// copy of a 128x384 state 0.65 ms with them, 0.1 without; 512x1536 2.9 and 1.5).
 constexpr size_t kSlotBytes = size_t(4) << 20;
 constexpr int kSlots = 12, kCopyThreads = 8;
 constexpr size_t kSmallBytes = size_t(1) << 20;  // copies up to this size have a buffer of their own
@@ -661,6 +664,8 @@ struct HostSlots {
     std::mutex life, lease;  // life: users and the allocations' existence
     int users = 0;
     char *small = nullptr, *slots = nullptr;
+    size_t slots_bytes = 0;
+    bool asked[2] = {false, false};  // by a copy for the small buffer, for the slots
 };
 static HostSlots &host_slots()
 {
@@ -681,20 +686,34 @@ static void host_slots_leave()
     if (h.slots) hipHostFree(h.slots);
     h.small = h.slots = nullptr;
 }
-// (the caller holds the lease)
-static hipError_t host_slots_get(bool large, char **out)
+// a buffer of `bytes` (of all the slots where that is more); the caller holds the lease
+static hipError_t host_slots_get(size_t bytes, char **out)
 {
     HostSlots &h = host_slots();
     std::lock_guard<std::mutex> g(h.life);
+    const bool large = bytes > kSmallBytes;
     char *&p = large ? h.slots : h.small;
+    size_t want = kSmallBytes;
+    if (large) {
+        while (want < bytes && want < kSlotBytes * kSlots) want *= 2;
+        want = std::min(want, kSlotBytes * kSlots);
+        if (p && h.slots_bytes < want) {
+            hipHostFree(p);
+            p = nullptr;
+        }
+    }
     if (!p) {
-        const hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&p), large ? kSlotBytes * kSlots : kSmallBytes,
-                                           hipHostMallocPortable);
+        if (!h.asked[large] && bytes <= kSlotBytes * kSlots) {
+            h.asked[large] = true;
+            return hipErrorNotReady;
+        }
+        const hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&p), want, hipHostMallocPortable);
         if (e != hipSuccess) {
             p = nullptr;
             hipGetLastError();  // the caller goes another way: no later call reports it
             return e;
         }
+        if (large) h.slots_bytes = want;
     }
     *out = p;
     return hipSuccess;
@@ -914,7 +933,7 @@ static int copy_to_host(fcpt_ctx *ctx, const HostCopies &fields)
         {
             std::lock_guard<std::mutex> lease(host_slots().lease);
             char *out = nullptr;
-            if (host_slots_get(total > kSmallBytes, &out) == hipSuccess)
+            if (host_slots_get(total, &out) == hipSuccess)
                 return total > kSlotBytes * kSlots ? copy_large(ctx, fields, out) : copy_export(ctx, fields, total, out);
         }
         return copy_pageable(ctx, fields);

@@ -2,11 +2,11 @@
 // for tests/test_gpu_pinned.py: this program's hipHostMalloc stands before the
 // runtime's, counts what the copies ask for and refuses it on request.
 //
-//   pinned_check <dir>
+//   pinned_check <dir> [once]
 // <dir> holds desc.bin (fcpt_disk_desc bytes, radii pointer ignored) and
 // radii.bin.  Prints one line per copy: its name, "same" or "differ" (the copy
-// without pinned memory against the one with it), the pinned allocations made
-// and their bytes.
+// without pinned memory against the one with it; "once", a process's first copy,
+// against what was uploaded), the pinned allocations made and their bytes.
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
 
@@ -82,6 +82,13 @@ int main(int argc, char **argv)
         std::printf("%s %s %zu %zu\n", name, same ? "same" : "differ", pins, pinned_bytes);
         std::fflush(stdout);
     };
+    if (argc > 2) {
+        for (int f = 0; f < 4; ++f) a[f] = x[f];
+        TRY(state(b));
+        report("once", 0, 3);
+        TRY(fcpt_destroy(c));
+        return 0;
+    }
     refuse = true;
     TRY(fcpt_download_field(c, FCPT_VRAD, a[1].data()));
     refuse = false;

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 EXE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "pinned_check.bin")
 
 
-def _run(tmp_path, nr, nphi, precision):
+def _run(tmp_path, nr, nphi, precision, *mode):
     from fargocpt_amd import workloads as W
     from fargocpt_amd.capi import desc_from_dict
     from fargocpt_amd.ic import log_radii
@@ -22,7 +22,7 @@ def _run(tmp_path, nr, nphi, precision):
     (tmp_path / "desc.bin").write_bytes(bytes(desc))
     radii.tofile(str(tmp_path / "radii.bin"))
     print(f"{nr} x {nphi} precision {precision}", flush=True)
-    r = subprocess.run([EXE, str(tmp_path)], capture_output=True, text=True, timeout=100)
+    r = subprocess.run([EXE, str(tmp_path), *mode], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stderr
     out = [line.split() for line in r.stdout.splitlines()]
     return {w[0]: (w[1], int(w[2]), int(w[3])) for w in out if len(w) == 4}
@@ -33,3 +33,19 @@ def _run(tmp_path, nr, nphi, precision):
 def test_without_pinned_memory(tmp_path, nr, nphi, precision):
     got = _run(tmp_path, nr, nphi, precision)
     assert got["field"][0] == "same" and got["state"][0] == "same", got
+
+
+@pytest.mark.parametrize("nr,nphi", [(8, 131), (128, 384), (400, 800), (1001, 1573)])
+def test_pins_what_it_needs(tmp_path, nr, nphi):
+    """Staging grows with the copies: at most twice a copy's bytes beside the
+    small buffer, and never more than the slots."""
+    got = _run(tmp_path, nr, nphi, 0)
+    mb = 1 << 20
+    need = (4 * nr + 1) * nphi * 8
+    assert got["state"][2] <= mb + min(2 * (need + nr * nphi * 8), 48 * mb + 16 * mb), got
+
+
+@pytest.mark.parametrize("nr,nphi", [(8, 131), (128, 384), (400, 800)])
+def test_first_copy_pins_nothing(tmp_path, nr, nphi):
+    """A program that copies one state pays for no staging."""
+    assert _run(tmp_path, nr, nphi, 0, "once")["once"] == ("same", 0, 0)
