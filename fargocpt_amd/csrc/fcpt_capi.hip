@@ -652,20 +652,24 @@ static int upload_split(fcpt_ctx *ctx, int field, const double *host)
 // The slots belong to the process: allocated by the first copy that needs them,
 // as large as it asks, rounded up to a power of two (pinning 2, 4 and 48 MB costs
 // 0.12 - 0.17, 0.3 and 0.5 ms), replaced by larger ones when one asks for more,
-// leased to one copy at a time, freed with the last context.  A copy that gets
+// leased to one copy at a time once the disk's own queue has run, so that no
+// disk's steps hold up another's copy, and freed with the last context.  Copies
+// up to 1 MB take a buffer each, as many as ever ran at once.  A copy that gets
 // none goes without, as does the process's first of each kind that fits them: a
 // process's first pinning and first use of it cost more than one copy gains (first
 // copy of a 128x384 state 0.65 ms with them, 0.1 without; 512x1536 2.9 and 1.5).
 constexpr size_t kSlotBytes = size_t(4) << 20;
 constexpr int kSlots = 12, kCopyThreads = 8;
-constexpr size_t kSmallBytes = size_t(1) << 20;  // copies up to this size have a buffer of their own
+constexpr size_t kSmallBytes = size_t(1) << 20;  // copies up to this size take a buffer of their own
 
 struct HostSlots {
     std::mutex life, lease;  // life: users and the allocations' existence
     int users = 0;
-    char *small = nullptr, *slots = nullptr;
+    std::vector<char *> small;  // small buffers not in use
+    size_t small_made = 0;
+    char *slots = nullptr;
     size_t slots_bytes = 0;
-    bool asked[2] = {false, false};  // by a copy for the small buffer, for the slots
+    bool asked[2] = {false, false};  // by a copy for a small buffer, for the slots
 };
 static HostSlots &host_slots()
 {
@@ -682,41 +686,67 @@ static void host_slots_leave()
     HostSlots &h = host_slots();
     std::lock_guard<std::mutex> g(h.life);
     if (--h.users > 0) return;
-    if (h.small) hipHostFree(h.small);
+    for (char *p : h.small) hipHostFree(p);
+    h.small.clear();
+    h.small_made = 0;
     if (h.slots) hipHostFree(h.slots);
-    h.small = h.slots = nullptr;
+    h.slots = nullptr;
 }
-// a buffer of `bytes` (of all the slots where that is more); the caller holds the lease
-static hipError_t host_slots_get(size_t bytes, char **out)
+// pinned memory, or null: the caller goes another way, and no later call reports it
+static char *host_pin(size_t bytes)
+{
+    void *p = nullptr;
+    if (hipHostMalloc(&p, bytes, hipHostMallocPortable) == hipSuccess) return static_cast<char *>(p);
+    hipGetLastError();
+    return nullptr;
+}
+// a small buffer for as long as this lives
+struct SmallBuffer {
+    char *p = nullptr;
+    SmallBuffer()
+    {
+        HostSlots &h = host_slots();
+        std::lock_guard<std::mutex> g(h.life);
+        if (!h.small.empty()) {
+            p = h.small.back();
+            h.small.pop_back();
+        } else if (!h.asked[0]) {
+            h.asked[0] = true;
+        } else {
+            h.small.reserve(h.small_made + 1);  // room for its return
+            p = host_pin(kSmallBytes);
+            if (p) ++h.small_made;
+        }
+    }
+    ~SmallBuffer()
+    {
+        if (!p) return;
+        std::lock_guard<std::mutex> g(host_slots().life);
+        host_slots().small.push_back(p);
+    }
+    SmallBuffer(const SmallBuffer &) = delete;
+};
+// the slots, `bytes` or all of them, or null; the caller holds the lease
+static char *host_slots_get(size_t bytes)
 {
     HostSlots &h = host_slots();
     std::lock_guard<std::mutex> g(h.life);
-    const bool large = bytes > kSmallBytes;
-    char *&p = large ? h.slots : h.small;
     size_t want = kSmallBytes;
-    if (large) {
-        while (want < bytes && want < kSlotBytes * kSlots) want *= 2;
-        want = std::min(want, kSlotBytes * kSlots);
-        if (p && h.slots_bytes < want) {
-            hipHostFree(p);
-            p = nullptr;
-        }
+    while (want < bytes && want < kSlotBytes * kSlots) want *= 2;
+    want = std::min(want, kSlotBytes * kSlots);
+    if (h.slots && h.slots_bytes < want) {
+        hipHostFree(h.slots);
+        h.slots = nullptr;
     }
-    if (!p) {
-        if (!h.asked[large] && bytes <= kSlotBytes * kSlots) {
-            h.asked[large] = true;
-            return hipErrorNotReady;
+    if (!h.slots) {
+        if (!h.asked[1] && bytes <= kSlotBytes * kSlots) {
+            h.asked[1] = true;
+            return nullptr;
         }
-        const hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&p), want, hipHostMallocPortable);
-        if (e != hipSuccess) {
-            p = nullptr;
-            hipGetLastError();  // the caller goes another way: no later call reports it
-            return e;
-        }
-        if (large) h.slots_bytes = want;
+        h.slots = host_pin(want);
+        h.slots_bytes = want;
     }
-    *out = p;
-    return hipSuccess;
+    return h.slots;
 }
 
 struct HostCopy {
@@ -930,10 +960,13 @@ static int copy_to_host(fcpt_ctx *ctx, const HostCopies &fields)
     size_t total = 0;
     for (const HostCopy &f : fields) total += field_rows(f.field, P.nr) * (size_t)P.ns * sizeof(double);
     try {
-        {
+        if (total <= kSmallBytes) {
+            SmallBuffer b;
+            if (b.p) return copy_export(ctx, fields, total, b.p);
+        } else {
+            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
             std::lock_guard<std::mutex> lease(host_slots().lease);
-            char *out = nullptr;
-            if (host_slots_get(total, &out) == hipSuccess)
+            if (char *out = host_slots_get(total))
                 return total > kSlotBytes * kSlots ? copy_large(ctx, fields, out) : copy_export(ctx, fields, total, out);
         }
         return copy_pageable(ctx, fields);

@@ -49,3 +49,27 @@ def test_pins_what_it_needs(tmp_path, nr, nphi):
 def test_first_copy_pins_nothing(tmp_path, nr, nphi):
     """A program that copies one state pays for no staging."""
     assert _run(tmp_path, nr, nphi, 0, "once")["once"] == ("same", 0, 0)
+
+
+def test_no_wait_for_another_disk():
+    """A copy does not wait for the steps queued on another disk that another
+    thread is copying: through the slots and through a small buffer."""
+    import threading
+    import time
+    from test_gpu_kick_walk import _disk
+    busy, others = _disk("iso_128x384", 1024, 3072), [_disk("iso_128x384", 200, 384), _disk("iso_128x384", 16, 97)]
+    for d in (busy, *others):
+        for _ in range(3):
+            d.download_state()
+    busy.run_steps(8)
+    busy.synchronize()
+    for d in others:
+        print(d.nr, d.nphi, flush=True)
+        busy.run_steps(1200)  # a quarter of a second
+        t = threading.Thread(target=busy.download_state)
+        t.start()
+        time.sleep(0.03)
+        d.download_state()
+        waited = not t.is_alive()
+        t.join()
+        assert not waited
