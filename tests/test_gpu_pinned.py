@@ -73,3 +73,11 @@ def test_no_wait_for_another_disk():
         waited = not t.is_alive()
         t.join()
         assert not waited
+
+
+@pytest.mark.parametrize("nr,nphi,pins", [(15, 128, 1), (16, 128, 0), (128, 384, 0), (340, 385, 1)])
+def test_one_field_goes_straight(tmp_path, nr, nphi, pins):
+    """One FP64 field above 16 KB (17 rows of v_r and 128 sectors) and up to 1 MB
+    takes no staging; a field of split storage does."""
+    for precision in (0, 1):
+        assert _run(tmp_path, nr, nphi, precision)["field"][:2] == ("same", pins if precision == 0 else 1)
