@@ -24,8 +24,11 @@ using namespace fcpt;
 
 // Iterations in one captured graph.  A graph's start and end cost the device
 // 3 to 5 us beyond the kernels between them (32 x 64: 37.1 us per step with one
-// iteration per graph, 33.1 with 4, 32.2 with 16; 251 x 757: 60.3, 57.6, 56.3),
-// and every captured iteration costs its first use about 15 us.
+// iteration per graph, 33.1 with 4, 32.2 with 16; 251 x 757: 60.3, 57.6, 56.3).
+// Capture and first use of the longer graph cost a context's first call of 8 steps
+// 36 to 51 us more than those of a single iteration's (32 x 64: 292 and 256 us; 12
+// steps 392 and 361, 16 and more no more), which its second call has back (195 and
+// 234).
 constexpr int kGraphSteps = 8;
 
 // split storage: steps of fcpt_run_steps between two moves of the ring
