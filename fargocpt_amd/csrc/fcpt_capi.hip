@@ -2469,20 +2469,28 @@ int fcpt_batch_run_steps(fcpt_batch *b, int32_t n_steps, int32_t use_graph)
         const int rc = ensure_batch_graph(b, many);
         if (rc) return rc;
     }
-    if (n_steps > 0 && std::any_of(b->disks.begin(), b->disks.end(), [](fcpt_ctx *c) { return !c->derived_own; })) {
-        // a member with fields of its caller's own: one iteration disk by disk
+    // the batched step after what has been queued on a disk's own stream since
+    auto after = [b](fcpt_ctx *c) {
+        const hipError_t e = hipEventRecord(b->done, c->stream);
+        return e == hipSuccess ? hipStreamWaitEvent(b->stream, b->done, 0) : e;
+    };
+    // fields of its caller's own that a member's batched step would not read
+    bool stored = false;
+    for (size_t k = 0; k < b->disks.size(); ++k)
+        stored = stored || (!b->disks[k]->derived_own && b->host[k].adiabatic && b->host[k].lazy_derived);
+    if (n_steps > 0 && stored) {  // one iteration disk by disk
         for (fcpt_ctx *c : b->disks) {
             if (fcpt_run_steps(c, 1, 0)) return bfail(b, FCPT_ERR_DEVICE, c->err.c_str());
-            BHIP(b, hipStreamSynchronize(c->stream));
+            BHIP(b, after(c));
         }
         --n_steps;
     }
     // what a member's own steps left stale and its batched step reads
     for (size_t k = 0; n_steps > 0 && k < b->disks.size(); ++k) {
         fcpt_ctx *c = b->disks[k];
-        if (!c->derived_stale) continue;
+        const bool stale = c->derived_stale;
         if (sync_for(c, b->host[k])) return bfail(b, FCPT_ERR_DEVICE, c->err.c_str());
-        BHIP(b, hipStreamSynchronize(c->stream));
+        if (stale && !c->derived_stale) BHIP(b, after(c));
     }
     for (int left = n_steps; left > 0;) {
         // up to the next background move of a member in split storage
