@@ -51,13 +51,13 @@ def build(verbose: bool = False) -> str:
 
 
 def build_host_check() -> str:
-    """The C++ programs used by the GPU tests: the host-interface check, whose
-    path is returned, the copies with and without pinned memory and the
-    batches' host waits."""
+    """The C++ programs used by the tests: the host-interface check, whose path is
+    returned, the copies with and without pinned memory, the batches' host
+    waits and the rules that choose a batch's tiles."""
     cpp = os.path.join(os.path.dirname(HERE), "tests", "cpp")
     exes = []
     for name, extra in (("pinned_check", ["-rdynamic", "-ldl"]), ("batch_check", ["-rdynamic", "-ldl"]),
-                        ("host_api_check", [])):
+                        ("tile_rules", []), ("host_api_check", [])):
         src, exe = (os.path.join(cpp, f"{name}.{x}") for x in ("cpp", "bin"))
         cmd = [HIPCC, "-O2", "-std=c++17", "-ffp-contract=off", src, "-o", exe,
                f"-L{HERE}", f"-Wl,-rpath,{HERE}", "-lfcpt_hip", *extra]

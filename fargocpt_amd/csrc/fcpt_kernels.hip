@@ -4246,13 +4246,13 @@ void set_step_modes(KParams &P, bool fused)
 // Rings per thread of the kick walk: a walk of t rings costs about t + 3.5
 // (its window start), and the device holds `slots` of them at once, so the
 // tile with the fewest rounds of walks times their length.
-template <class Waves>
-static int kv_best_tile(Waves &&waves, long slots)
+template <class Rounds>
+static int kv_best_tile(Rounds &&rounds_of)
 {
     int best = 1;
     double best_cost = 1e300;
     for (int t = 1; t <= 24; ++t) {
-        const double rounds = (double)waves(t) / (double)slots;
+        const double rounds = rounds_of(t);
         const double cost = (t + 3.5) * (rounds <= 3.0 ? std::ceil(rounds) : rounds + 0.5);
         if (cost < best_cost) {
             best_cost = cost;
@@ -4263,27 +4263,22 @@ static int kv_best_tile(Waves &&waves, long slots)
 }
 // walks resident at once: 3 wavefronts per SIMD of an adiabatic walk's
 // registers, 4 of an isothermal one's
-static long kv_slots(const KParams &P) { return P.adiabatic ? 3072 : 4096; }
+static double kv_slots(bool adiabatic) { return adiabatic ? 3072.0 : 4096.0; }
 static int kv_tile(const KParams &P)
 {
     if (P.kick_tile > 1) return P.kick_tile;
     if (P.visc_tile > 1) return P.visc_tile;
-    return kv_best_tile([&](int t) { return kv_waves(P, t); }, kv_slots(P));
+    return kv_best_tile([&](int t) { return (double)kv_waves(P, t) / kv_slots(P.adiabatic); });
 }
+// a batch's walks run in rounds too, each member's in slots of its kind
 void resolve_kv_tiles(std::vector<KParams> &D)
 {
-    const KParams *any = nullptr;
-    for (const KParams &P : D)
-        if (kv_walk_applies(P)) any = &P;
-    if (!any) return;
-    const int t = kv_best_tile(
-        [&](int tile) {
-            long w = 0;
-            for (const KParams &P : D)
-                if (kv_walk_applies(P)) w += kv_waves(P, tile);
-            return w;
-        },
-        kv_slots(*any));
+    const int t = kv_best_tile([&](int tile) {
+        long waves[2] = {0, 0};  // of isothermal and of adiabatic members
+        for (const KParams &P : D)
+            if (kv_walk_applies(P)) waves[P.adiabatic ? 1 : 0] += kv_waves(P, tile);
+        return (double)waves[0] / kv_slots(false) + (double)waves[1] / kv_slots(true);
+    });
     for (KParams &P : D)
         if (kv_walk_applies(P)) P.kv_tile = P.kick_tile > 1 ? P.kick_tile : P.visc_tile > 1 ? P.visc_tile : t;
 }
