@@ -154,7 +154,9 @@ static void stepped(fcpt_ctx *ctx, const KParams &V)
 static int sync_derived(fcpt_ctx *ctx)
 {
     if (!ctx->derived_stale) return FCPT_OK;
-    launch_derived(ctx->P, ctx->stream);
+    KParams P = ctx->P;
+    P.step_at = &ctx->s_dev->count_derived;  // rounded as the step would have
+    launch_derived(P, ctx->stream);
     LAUNCH_CHECK(ctx);
     ctx->derived_stale = ctx->h_stale = false;
     return FCPT_OK;
@@ -1803,7 +1805,11 @@ int fcpt_set_launch_param(fcpt_ctx *ctx, int32_t param, int32_t value)
     else if (param == FCPT_PARAM_RADIAL_WAVES) ctx->P.radial_waves = value;
     else if (param == FCPT_PARAM_VISC_TILE) ctx->P.visc_tile = value;
     else if (param == FCPT_PARAM_KICK_TILE) ctx->P.kick_tile = value;
-    else if (param == FCPT_PARAM_SPLIT_ROUNDING) ctx->P.split_rounding = ctx->P.split ? value : 0;
+    else if (param == FCPT_PARAM_SPLIT_ROUNDING) {
+        const int mode = ctx->P.split ? value : 0;
+        if (mode != ctx->P.split_rounding) ctx->derived_own = false;  // stored as the old mode rounds
+        ctx->P.split_rounding = mode;
+    }
     else ctx->fused = value != 0;
     HIP_TRY(ctx, drop_graphs(ctx->step_graph));
     return FCPT_OK;

@@ -62,7 +62,8 @@ struct DevScalars {
     // last_dt and the next step_count as the last step left them: what a kick that folds
     // the CFL minima reads while one of its wavefronts writes last_dt and step_count
     double last_prev;
-    unsigned count_next, pad3_;
+    unsigned count_next;
+    unsigned count_derived;  // the step count at which the derived fields were last formed to be stored
 };
 
 // values per ring of KParams::sweep_tab

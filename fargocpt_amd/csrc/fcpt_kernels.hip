@@ -376,6 +376,15 @@ __device__ __forceinline__ Fld<SPLIT> fld(const KParams &P, int f)
 {
     return Fld<SPLIT>{static_cast<typename Fld<SPLIT>::T *>(P.f[f]), P.bg[f], P.ns, store_key<SPLIT>(P, f)};
 }
+// a derived field as the end of the last step (or the caller) rounded it
+template <bool SPLIT>
+__device__ __forceinline__ Fld<SPLIT> fld_derived(const KParams &P, int f)
+{
+    Fld<SPLIT> x = fld<SPLIT>(P, f);
+    if constexpr (SPLIT)
+        if (P.split_rounding == 2) x.key = sr_key(f, *cst(&P.s->count_derived));
+    return x;
+}
 // a work buffer; id names it for the rounding key (the momenta: kBufMom + q)
 template <bool SPLIT>
 __device__ __forceinline__ Fld<SPLIT> buf(const KParams &P, void *p, const double *bg, int id = -1)
@@ -799,8 +808,8 @@ __device__ __forceinline__ AdiDerived adi_derived_stored(const KParams &P, int i
 {
     AdiDerived a = adi_derived<SPLIT>(P, i, e, sig);
     if (SPLIT && (P.split_emul & SPLIT_EMUL_DERIVED)) {
-        a.cs = fld<SPLIT>(P, FCPT_SOUNDSPEED).stored(i, j, a.cs);
-        a.nu = fld<SPLIT>(P, FCPT_VISCOSITY).stored(i, j, a.nu);
+        a.cs = fld_derived<SPLIT>(P, FCPT_SOUNDSPEED).stored(i, j, a.cs);
+        a.nu = fld_derived<SPLIT>(P, FCPT_VISCOSITY).stored(i, j, a.nu);
     }
     return a;
 }
@@ -1168,7 +1177,7 @@ __device__ __forceinline__ void b_cfl_ring(const KParams &P, int i)
     const int ns = P.ns;
     const int t = (int)threadIdx.x;
     FLD(v, FCPT_VAZI);
-    FLD(Hf, FCPT_SCALE_HEIGHT);
+    const Fld<SPLIT> Hf = fld_derived<SPLIT>(P, FCPT_SCALE_HEIGHT);
     double acc = 0.0;
     if (t < 256) strided_row<256>(ns, t, [&](int j) { return v(i, j); }, [&](double x) { acc += x; });
     const bool active = i >= 1 && i < P.nr - 1;
@@ -1743,6 +1752,7 @@ template <bool SPLIT>
 __device__ __forceinline__ void b_derived(const KParams &P, int bx, int by)
 {
     CELL_LOOP_HEAD(0, P.nr)
+    if (i == 0 && j == 0) P.s->count_derived = *P.step_at;
     derived_store<SPLIT>(P, i, j, derived_load<SPLIT>(P, i, j, true), true, true);
 }
 FCPT_PAIR0(derived, 256)
@@ -2691,7 +2701,9 @@ __device__ __forceinline__ void b_kv_walk(const KParams &K, int bx, int by, int 
         if constexpr (ADI) {
             g.e = E.dec(c, w.e);
             g.p = (P.gamma - 1.0) * g.e;
-            if (emul_derived) g.p = fld<SPLIT>(P, FCPT_PRESSURE).stored(c, j, g.p);
+            // a LeapFrog step's second kick reads the pressure of its own drift
+            if (emul_derived)
+                g.p = (P.kick == 2 ? fld<SPLIT>(P, FCPT_PRESSURE) : fld_derived<SPLIT>(P, FCPT_PRESSURE)).stored(c, j, g.p);
         } else {
             g.e = 0.0;
             g.p = iso_pressure(P, c, g.s);
@@ -3011,6 +3023,7 @@ __device__ __forceinline__ void advance_clock(const KParams &P, int advance_time
     s->time = s->time + s->dt;
     s->last_prev = s->last_dt;
     s->count_next = s->step_count + 1u;
+    s->count_derived = s->step_count;
     if (advance_time == 2 && fabs(time_next_monitor - s->time) < 1e-6 * s->last_dt) s->n_monitor++;
     if (DevScalars *out = P.s_out) {
         out->dt = s->dt;
@@ -4400,7 +4413,7 @@ __global__ void __launch_bounds__(256) k_disk_force(KParams P, ForceBodies B, do
 #pragma unroll
     for (int k = 0; k < NB; ++k) acc[k][0] = acc[k][1] = acc[k][2] = acc[k][3] = 0.0;
     FLD(S, FCPT_SIGMA);
-    FLD(Hf, FCPT_SCALE_HEIGHT);
+    const Fld<SPLIT> Hf = fld_derived<SPLIT>(P, FCPT_SCALE_HEIGHT);
     const double G = P.G;
     const double thick = P.thickness_smoothing;
     const double rmed = cst(P.Rmed)[i], surf = cst(P.Surf)[i];
