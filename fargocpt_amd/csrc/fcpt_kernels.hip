@@ -470,8 +470,9 @@ __device__ __forceinline__ BlockXY xcd_block()
     if (j >= ns || i >= (r1)) return;
 
 // Every kernel body takes the disk's parameters and its block coordinates
-// (bx, by) in that disk's grid, and comes in two launch forms: k_NAME runs
-// one disk on its own grid; kb_NAME runs many disks in one launch, each
+// (bx, by) in that disk's grid, and comes in up to two launch forms: k_NAME runs
+// one disk on its own grid; kb_NAME, of the batched step's stages, many disks in
+// one launch, each
 // block reading (disk, by << 16 | bx) from a per-stage work table and the
 // disk's parameters from a device array (constant address space: scalar
 // loads).
@@ -493,12 +494,15 @@ __device__ __forceinline__ KParams batch_disk(const KParams *Ps, unsigned d)
     return P;
 }
 
-#define FCPT_PAIR0(name, BOUNDS)                                                                  \
+#define FCPT_ONE0(name, BOUNDS)                                                                   \
     template <bool SPLIT>                                                                         \
     __global__ void __launch_bounds__(BOUNDS) k_##name(KParams P)                                 \
     {                                                                                             \
         b_##name<SPLIT>(P, (int)blockIdx.x, (int)blockIdx.y);                                     \
-    }                                                                                             \
+    }
+
+#define FCPT_PAIR0(name, BOUNDS)                                                                  \
+    FCPT_ONE0(name, BOUNDS)                                                                       \
     template <bool SPLIT>                                                                         \
     __global__ void __launch_bounds__(BOUNDS) kb_##name(const KParams *Ps, const BatchEntry *map)  \
     {                                                                                             \
@@ -506,12 +510,15 @@ __device__ __forceinline__ KParams batch_disk(const KParams *Ps, unsigned d)
         b_##name<SPLIT>(batch_disk(Ps, e.disk), (int)(e.yx & 0xffffu), (int)(e.yx >> 16));        \
     }
 
-#define FCPT_PAIR1(name, BOUNDS, T1, a1)                                                          \
+#define FCPT_ONE1(name, BOUNDS, T1, a1)                                                           \
     template <bool SPLIT>                                                                         \
     __global__ void __launch_bounds__(BOUNDS) k_##name(KParams P, T1 a1)                          \
     {                                                                                             \
         b_##name<SPLIT>(P, (int)blockIdx.x, (int)blockIdx.y, a1);                                 \
-    }                                                                                             \
+    }
+
+#define FCPT_PAIR1(name, BOUNDS, T1, a1)                                                          \
+    FCPT_ONE1(name, BOUNDS, T1, a1)                                                               \
     template <bool SPLIT>                                                                         \
     __global__ void __launch_bounds__(BOUNDS)                                                     \
         kb_##name(const KParams *Ps, const BatchEntry *map, T1 a1)                                \
@@ -645,7 +652,7 @@ __device__ __forceinline__ void b_ring_mean(const KParams &P, int bx, int by, in
         return seq;
     });
 }
-FCPT_PAIR1(ring_mean, 256, int, mode)
+FCPT_ONE1(ring_mean, 256, int, mode)
 
 // The fold of the CFL limits (cfl.cpp:210-376): the rings' smallest
 // (b_cfl_ring's slots) and the shear limits between the rings' means.
@@ -1305,7 +1312,7 @@ __device__ __forceinline__ void b_src_vr(const KParams &P, int bx, int by)
     vr.set(i, j, src_vr_new<SPLIT>(P, i, dt, vr(i, j), S(i, j), S(i - 1, j), Pr(i, j), Pr(i - 1, j), Phi(i, j),
                             Phi(i - 1, j), vaz(i, j), vaz(i, jn), vaz(i - 1, j), vaz(i - 1, jn)));
 }
-FCPT_PAIR0(src_vr, 256)
+FCPT_ONE0(src_vr, 256)
 
 // momentum_update_azimuthal, SourceEuler.cpp:375-428
 template <bool SPLIT>
@@ -1321,7 +1328,7 @@ __device__ __forceinline__ void b_src_vphi(const KParams &P, int bx, int by)
     vaz.set(i, j, src_vphi_new<SPLIT>(P, i, dt, vaz(i, j), S(i, j), S(i, jp), Pr(i, j), Pr(i, jp), Phi(i, j),
                                Phi(i, jp)));
 }
-FCPT_PAIR0(src_vphi, 256)
+FCPT_ONE0(src_vphi, 256)
 
 // compression_heating, SourceEuler.cpp:459-493, for one cell (rings 0 .. nr-2)
 // from v_r(i), v_r(i + 1), v_phi(j), v_phi(j + 1)
@@ -1533,7 +1540,7 @@ __device__ __forceinline__ void b_tw_q(const KParams &P, int bx, int by)
     fld<SPLIT>(P, FCPT_Q_PHI).set(i, j, q.qp);
     if (diss) E.set(i, j, tw_dissipation(P, i, q, sig, dt, e_in));
 }
-FCPT_PAIR0(tw_q, 256)
+FCPT_ONE0(tw_q, 256)
 
 // the TW velocity updates of one cell from the tensors around it
 // (artificial_viscosity.cpp:90-139)
@@ -1611,7 +1618,7 @@ __device__ __forceinline__ void b_tw_vel(const KParams &P, int bx, int by, int w
     vaz.set(i, j, tw_vphi_new<SPLIT>(P, i, dt, va, s0, sjp, qp0, qpj));
     if (radial) vr.set(i, j, tw_vr_new<SPLIT>(P, i, dt, v, s0, sm, qr0, qrm, qp0, qpm));
 }
-FCPT_PAIR1(tw_vel, 256, int, with_viscosity)
+FCPT_ONE1(tw_vel, 256, int, with_viscosity)
 
 // The von Neumann-Richtmyer tensor at one cell (artificial_viscosity.cpp:160-185)
 struct SnQ {
@@ -1669,7 +1676,7 @@ __device__ __forceinline__ void b_sn_q(const KParams &P, int bx, int by)
     fld<SPLIT>(P, FCPT_Q_PHI).set(i, j, q.qp);
     if (diss) E.set(i, j, sn_dissipation(P, i, q, sig, dt, e_in));
 }
-FCPT_PAIR0(sn_q, 256)
+FCPT_ONE0(sn_q, 256)
 
 // the SN velocity updates of one cell (artificial_viscosity.cpp:214-248)
 // (inv = 2 dt / (Sigma + its neighbour's))
@@ -1736,7 +1743,7 @@ __device__ __forceinline__ void b_sn_vel(const KParams &P, int bx, int by, int w
     if (radial) vr.set(i, j, sn_vr_new<SPLIT>(P, i, dt, v, s0, sm, qr0, qrm));
     vaz.set(i, j, sn_vphi_new<SPLIT>(P, i, dt, va, s0, sjp, qp0, qpj));
 }
-FCPT_PAIR1(sn_vel, 256, int, with_viscosity)
+FCPT_ONE1(sn_vel, 256, int, with_viscosity)
 
 // recalculate_viscosity, SourceEuler.cpp:205-223
 template <bool SPLIT>
@@ -1755,7 +1762,7 @@ __device__ __forceinline__ void b_derived(const KParams &P, int bx, int by)
     if (i == 0 && j == 0) P.s->count_derived = *P.step_at;
     derived_store<SPLIT>(P, i, j, derived_load<SPLIT>(P, i, j, true), true, true);
 }
-FCPT_PAIR0(derived, 256)
+FCPT_ONE0(derived, 256)
 
 
 // compute_pressure (SourceEuler.cpp): (gamma - 1) E, or Sigma c_s^2 with the
@@ -1956,7 +1963,7 @@ __device__ __forceinline__ void b_stress(const KParams &P, int bx, int by)
     if (i >= 1)
         fld<SPLIT>(P, FCPT_TAU_R_PHI).set(i, j, stress_rp(P, i, va0, vam, vr0, vrp, n, nm, njp, nmp, s, sm, sjp, smp));
 }
-FCPT_PAIR0(stress, 256)
+FCPT_ONE0(stress, 256)
 
 // update_velocities_with_viscosity, viscosity.cpp:355-426, for one cell
 // (inv = dt / Rmed / Sigma_avg)
@@ -2019,7 +2026,7 @@ __device__ __forceinline__ void b_visc_update(const KParams &P, int bx, int by)
     vaz.set(i, j, visc_vphi_new<SPLIT>(P, i, dt, va, s0, sjp, trp0, trp1, tpp0, tppj));
     if (i >= 2) vr.set(i, j, visc_vr_new<SPLIT>(P, i, dt, v, s0, sm, trr0, trrm, trp0, trpn, tpp0, tppm));
 }
-FCPT_PAIR0(visc_update, 256)
+FCPT_ONE0(visc_update, 256)
 
 // ---------------------------------------------------------------------------
 // Fused kernels of the step.  Each reads the velocities of its view (P.f[VRAD],
@@ -3008,7 +3015,7 @@ __device__ __forceinline__ void b_damping(const KParams &P, int bx, int by)
         X.set(i, j, damp_value(X(i, j), X0(i, j), damp_ring(P, vector, i, dt)));
     }
 }
-FCPT_PAIR0(damping, 256)
+FCPT_ONE0(damping, 256)
 
 // ghost rings: zero-gradient Sigma/E, reflecting / zero-gradient / outflow v_r,
 // Keplerian v_phi (boundary_conditions.cpp:67-97 and the BC files it dispatches to)
@@ -3114,7 +3121,7 @@ __device__ __forceinline__ void b_ghost_bc(const KParams &P, int bx, int by, int
     ghost_inner<SPLIT>(P, j);
     ghost_outer<SPLIT>(P, j);
 }
-FCPT_PAIR1(ghost_bc, 256, int, advance_time)
+FCPT_ONE1(ghost_bc, 256, int, advance_time)
 
 // the boundary call before the transport (ghost rings, b_ghost_bc) and the
 // transport's ring mean with the FARGO shift (b_ring_mean, mode 1) in one
@@ -3184,7 +3191,7 @@ __device__ __forceinline__ void b_final_derived(const KParams &P, int bx, int by
     if (i == P.nr - 1) ghost_outer<SPLIT>(P, j);
     derived_store<SPLIT>(P, i, j, derived_load<SPLIT>(P, i, j, true), true, true);
 }
-FCPT_PAIR1(final_derived, 256, int, advance_time)
+FCPT_ONE1(final_derived, 256, int, advance_time)
 
 // The end of the fused LeapFrog step in one launch: the second kick's
 // velocities and E, in the partner buffers of view P, damped into the fields
@@ -3245,7 +3252,7 @@ __device__ __forceinline__ void b_final_leapfrog(const KParams &P, int bx, int b
     }
     if (advance_time && i == 1 && j == 0) advance_clock(P, advance_time);
 }
-FCPT_PAIR1(final_leapfrog, 256, int, advance_time)
+FCPT_ONE1(final_leapfrog, 256, int, advance_time)
 
 // ---------------------------------------------------------------------------
 // Transport
@@ -3463,7 +3470,8 @@ __device__ __forceinline__ void sweep_flux(const KParams &P, int k, const SweepR
     }
 }
 
-// Both FARGO passes (as az_ring) for this lane's sector of one ring, the
+// Both FARGO passes, with the residual and with the uniform velocity
+// (TransportEuler.cpp:292-304, 630-664), for this lane's sector of one ring, the
 // neighbour sectors in the adjacent lanes: s0, q0 the radially swept density
 // and quantities, v0 = v_phi - <v_phi>; s2, q2 the results.  The second pass
 // has one velocity vu, so each sector's interface value on its downstream
@@ -3655,7 +3663,7 @@ __device__ __forceinline__ void b_velocities(const KParams &P, int bx, int by)
     fld<SPLIT>(P, FCPT_SIGMA).set(i, j, sig);
     if (P.adiabatic) fld<SPLIT>(P, FCPT_ENERGY).set(i, j, temperature_floor<SPLIT>(P, e, sig));
 }
-FCPT_PAIR0(velocities, 256)
+FCPT_ONE0(velocities, 256)
 
 // The end of the fused Euler step in one launch: the velocity kernel, the
 // final boundary call (damping, ghost rings, the clock) and
@@ -4569,17 +4577,9 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
     auto rings = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         add_grid(v, d, (unsigned)P.nr, 1);
     };
-    auto ghosts = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
-        add_grid(v, d, (unsigned)((P.ns + 255) / 256), 1);
-    };
     auto sweeps = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
         add_grid(v, d, (unsigned)((P.ns + kSweepSegW - 1) / kSweepSegW),
                  (unsigned)((P.nr + P.radial_tile - 1) / P.radial_tile));
-    };
-    auto damp = [](std::vector<BatchEntry> &v, unsigned d, const KParams &P) {
-        const int n_inner = (P.damp_ids[0] > P.damp_ids[1] ? P.damp_ids[0] : P.damp_ids[1]) + 1;
-        const int o0 = P.damp_ids[2] < P.damp_ids[3] ? P.damp_ids[2] : P.damp_ids[3];
-        add_grid(v, d, sector_grid(P), rows_grid(P, n_inner + P.nr + 1 - o0));
     };
     auto one = [](std::vector<BatchEntry> &v, unsigned d, const KParams &) { add_grid(v, d, 1, 1); };
     // sim::CalculateTimeStep and the monitor clip (simulation.cpp:100-118, 526-542):
@@ -4646,9 +4646,6 @@ std::vector<BatchStageHost> plan_batch_step(const std::vector<KParams> &D)
     // the velocity kernel with the final boundary call and the derived
     // fields writes the fields of every disk
     stage_v(B_VEL_FINAL, 2, all, rows(2), false, true);
-    std::fill(view.begin(), view.end(), 0u);
-    (void)ghosts;
-    (void)damp;
     return st;
 }
 
@@ -4662,28 +4659,14 @@ void launch_batch_stage(const KParams *Ps, const BatchStageDev &S, int split, hi
 {
     const dim3 b256(256);
     switch (S.kind) {
-    case B_RING_MEAN: LAUNCHB(kb_ring_mean, b256, S.arg); break;
     case B_POTENTIAL: LAUNCHB(kb_potential, kBlock); break;
-    case B_SRC_VR: LAUNCHB(kb_src_vr, kBlock); break;
-    case B_SRC_VPHI: LAUNCHB(kb_src_vphi, kBlock); break;
     case B_SRC_FUSED: LAUNCHB(kb_src_fused, kBlock); break;
     case B_AV_FUSED: LAUNCHB(kb_av_fused, kBlock, S.arg); break;
     case B_VISC_FUSED: LAUNCHB(kb_visc_fused, kBlock); break;
     case B_SRC_ENERGY: LAUNCHB(kb_src_energy, kBlock); break;
-    case B_TW_Q: LAUNCHB(kb_tw_q, kBlock); break;
-    case B_TW_VEL: LAUNCHB(kb_tw_vel, kBlock, S.arg); break;
-    case B_SN_Q: LAUNCHB(kb_sn_q, kBlock); break;
-    case B_SN_VEL: LAUNCHB(kb_sn_vel, kBlock, S.arg); break;
     case B_TEMP_FLOOR: LAUNCHB(kb_temperature_floor, kBlock); break;
     case B_RECALC_VISC: LAUNCHB(kb_recalc_viscosity, kBlock); break;
-    case B_STRESS: LAUNCHB(kb_stress, kBlock); break;
-    case B_VISC_UPDATE: LAUNCHB(kb_visc_update, kBlock); break;
     case B_SUBSTEP3: LAUNCHB(kb_substep3, kBlock); break;
-    case B_GHOST: LAUNCHB(kb_ghost_bc, b256, S.arg); break;
-    case B_VELOCITIES: LAUNCHB(kb_velocities, kBlock); break;
-    case B_DAMPING: LAUNCHB(kb_damping, kBlock); break;
-    case B_DERIVED: LAUNCHB(kb_derived, kBlock); break;
-    case B_FINAL_DERIVED: LAUNCHB(kb_final_derived, kBlock, S.arg); break;
     case B_CFL_RINGS:
         if (split) hipLaunchKernelGGL((kb_cfl_ring<true, false>), dim3(S.n), b256, 0, st, Ps, S.map);
         else hipLaunchKernelGGL((kb_cfl_ring<false, false>), dim3(S.n), b256, 0, st, Ps, S.map);

@@ -127,11 +127,9 @@ struct BatchEntry {
     unsigned disk, yx;  // yx = by << 16 | bx
 };
 enum BatchKind {
-    B_RING_MEAN, B_CFL_POT, B_POTENTIAL, B_SRC_VR, B_SRC_VPHI,
-    B_SRC_ENERGY, B_TW_Q, B_TW_VEL, B_SN_Q, B_SN_VEL, B_TEMP_FLOOR, B_RECALC_VISC, B_STRESS,
-    B_VISC_UPDATE, B_SUBSTEP3, B_GHOST, B_SWEEPS_ISO, B_SWEEPS_ADI,
-    B_VELOCITIES, B_DAMPING, B_DERIVED, B_SRC_FUSED, B_AV_FUSED, B_VISC_FUSED, B_FINAL_DERIVED,
-    B_CFL_RINGS, B_CFL_FINAL_RINGS, B_KV_WALK, B_VISC_WALK, B_GHOST_MEAN, B_VEL_FINAL
+    B_CFL_POT, B_CFL_RINGS, B_CFL_FINAL_RINGS, B_POTENTIAL, B_KV_WALK, B_SRC_FUSED, B_SRC_ENERGY, B_AV_FUSED,
+    B_TEMP_FLOOR, B_RECALC_VISC, B_VISC_WALK, B_VISC_FUSED, B_SUBSTEP3, B_GHOST_MEAN, B_SWEEPS_ISO, B_SWEEPS_ADI,
+    B_VEL_FINAL
 };
 struct BatchStageHost {
     int kind, arg;
