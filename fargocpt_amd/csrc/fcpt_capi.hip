@@ -643,11 +643,12 @@ static int upload_split(fcpt_ctx *ctx, int field, const double *host)
 // ---- fields to the host ----------------------------------------------------
 // A copy into the caller's pageable arrays is bound by the host: its pages are
 // touched for the first time (the kernel clears them) and written by one
-// thread, 1.6 GB in 158 ms where the link takes 30.  So the bytes go through
-// pinned slots, in pieces: the link fills a slot while kCopyThreads threads
-// move earlier ones to the caller (and decode split storage's FP32 deviations
-// there, so half the bytes cross the link): 37 ms, and 21 for split storage
-// instead of 292.  What fits the slots as a whole is decoded and written to
+// thread: 1.6 GB took 158 ms into touched pages and 233 into fresh ones, where the
+// link takes 30.  So the bytes go through pinned slots, in pieces: the link fills
+// a slot while kCopyThreads threads move earlier ones to the caller (and decode
+// split storage's FP32 deviations there, so half the bytes cross the link): 37 ms
+// into touched pages and 83 into fresh ones, and 21 for split storage instead of
+// 292.  What fits the slots as a whole is decoded and written to
 // them by one kernel, all fields at once: each transfer and its event cost
 // tens of microseconds, more than the link's time below some MB (512 x
 // 1536: 1.5 - 3.5 -> 0.9 - 1.5 ms, 32 x 64: 80 -> 21 us; slots filled in smaller

@@ -1173,9 +1173,9 @@ __global__ void __launch_bounds__(256) k_potential_fold(KParams P, int fold_mode
 // POT: also the potential of the ring's cells, for steps whose derived fields
 // are formed where they are needed; the scale height of its smoothing comes with
 // the sound speed of the limits, so no step stores it.
-// 4096x12288 beta, FP64: 731 us where the two launches took 520 + 314, and the end
-// of the step 795 us instead of 880 without the store of H; 3.8 TB/s, with FP64
-// instructions for about two thirds of its time.
+// 4096x12288 beta, FP64: 718 us where the two launches take 506 + 306, and the end
+// of the step 796 us instead of 880 without the store of H; 73 B/cell at 5.1 TB/s,
+// with instruction issue for 0.59 of its time.
 template <bool SPLIT, bool POT, int THREADS>
 __device__ __forceinline__ void b_cfl_ring(const KParams &P, int i)
 {
@@ -2610,12 +2610,13 @@ __global__ void __launch_bounds__(256) kb_visc_walk(const KParams *Ps, const Bat
 // artificial viscosity and the viscous update) as if it had been stored;
 // KParams::split_emul adds the roundings of the forms that store more.
 //
-// What bounds it: the latency of its chain of stages, at the 3 wavefronts per
-// SIMD (4 isothermal) that its registers allow; VALU issue is about half of
-// its time.  Hence one pass for the whole kick (a walk for the sources and
+// What bounds it: its instructions, whose issue is 0.61 of its time at 4096 x
+// 12288 adiabatic (0.74 in split storage), and beyond them the latency of its
+// chain of stages, at the 3 wavefronts per SIMD (4 isothermal) that its registers
+// allow.  Hence one pass for the whole kick (a walk for the sources and
 // artificial viscosity and one for the rest moved 188 B/cell at 4096 x 12288
-// adiabatic, 2161 us; this one 88 B/cell, 1390 us; 2048 x 6144 isothermal 256
-// -> 185 us), the loads of ring m + 2 in flight during ring m, no load behind
+// adiabatic, 2161 us; this one 88 B/cell, 1190 us; 2048 x 6144 isothermal 256
+// -> 170 us), the loads of ring m + 2 in flight during ring m, no load behind
 // a store in the loop (rows that are only copied are copied after it: 240 us
 // at 4096 x 12288), the ring's metric in LDS (KWalk), and quotients that share
 // a denominator through one reciprocal.
@@ -4248,9 +4249,11 @@ void set_step_modes(KParams &P, bool fused)
     // height (4096x12288 beta step 4513 -> 4322 us, 1024x3072 307.9 -> 304.9),
     // and on grids whose kick folds the ring minima, a launch less (128x384
     // isothermal 29.5 -> 28.0; 2048x6144 isothermal 769 -> 774 is left apart);
-    // in split storage, whose limits and potential are bound by instructions
-    // together, on small grids only (128x384 beta 42.9 -> 40.7; 512x1536
-    // adiabatic 109.2 -> 110.8 is left apart).
+    // in split storage on small grids only.  There an isothermal disk gains up to
+    // about 1.2e5 cells (128x384 30.9 -> 30.1 us, 181x543 36.2 -> 35.6, 200x600 40.0
+    // either way, 209x627 41.0 -> 41.3, 256x768 45.9 -> 46.5, 512x1536 81.4 -> 82.7),
+    // an adiabatic one 4 % there and 1 % still at 512x1536 (128x384 41.7 -> 40.0,
+    // 209x627 57.9 -> 56.6, 256x768 64.3 -> 62.3, 512x1536 107.0 -> 105.8).
     const bool folds = P.nr <= kFoldRings;
     P.cfl_pot = P.lazy_derived && (P.split ? folds && (long)P.nr * P.ns <= 131072 : P.adiabatic || folds);
     // LeapFrog's second kick reads the H of the step's start
