@@ -657,10 +657,12 @@ static int upload_split(fcpt_ctx *ctx, int field, const double *host)
 // The slots belong to the process: allocated by the first copy that needs them,
 // as large as it asks, rounded up to a power of two (pinning 2, 4 and 48 MB costs
 // 0.12 - 0.17, 0.3 and 0.5 ms), replaced by larger ones when one asks for more,
-// leased to one copy at a time once the disk's own queue has run, so that no
-// disk's steps hold up another's copy, and freed with the last context.  Copies
-// up to 1 MB take a buffer each, as many as ever ran at once.  A copy that gets
-// none goes without, as does the process's first of each kind that fits them: a
+// lent to one copy at a time, and freed with the last context.  A copy that finds
+// them lent to one whose disk's queue still runs goes without them, so that no
+// disk's steps hold up another's copy (waiting for the own queue before taking the
+// slots cost every copy behind queued steps 10 to 18 us); it waits for one that moves
+// its bytes.  Copies up to 1 MB take a buffer each, as many as ever ran at once.  A
+// copy that gets none goes without, as does the process's first of each kind that fits them: a
 // process's first pinning and first use of it cost more than one copy gains (first
 // copy of a 128x384 state 0.65 ms with them, 0.1 without; 512x1536 2.9 and 1.5).
 constexpr size_t kSlotBytes = size_t(4) << 20;
@@ -673,8 +675,10 @@ constexpr size_t kSmallBytes = size_t(1) << 20;  // copies up to this size take 
 constexpr size_t kDirectAbove = size_t(16) << 10;
 
 struct HostSlots {
-    std::mutex life, lease;  // life: users and the allocations' existence
+    std::mutex life;
     int users = 0;
+    std::condition_variable freed;
+    bool lent = false, queued = false;  // the slots; to a copy whose disk's queue still runs
     std::vector<char *> small;  // small buffers not in use
     size_t small_made = 0;
     char *slots = nullptr;
@@ -736,11 +740,32 @@ struct SmallBuffer {
     }
     SmallBuffer(const SmallBuffer &) = delete;
 };
-// the slots, `bytes` or all of them, or null; the caller holds the lease
-static char *host_slots_get(size_t bytes)
+// the slots for as long as this lives, `bytes` or all of them, or null
+struct SlotsLoan {
+    char *p = nullptr;
+    explicit SlotsLoan(size_t bytes);
+    // the borrower's own queue has run
+    void moving()
+    {
+        std::lock_guard<std::mutex> g(host_slots().life);
+        host_slots().queued = false;
+    }
+    ~SlotsLoan()
+    {
+        if (!p) return;
+        HostSlots &h = host_slots();
+        std::lock_guard<std::mutex> g(h.life);
+        h.lent = h.queued = false;
+        h.freed.notify_all();
+    }
+    SlotsLoan(const SlotsLoan &) = delete;
+};
+SlotsLoan::SlotsLoan(size_t bytes)
 {
     HostSlots &h = host_slots();
-    std::lock_guard<std::mutex> g(h.life);
+    std::unique_lock<std::mutex> g(h.life);
+    h.freed.wait(g, [&] { return !h.lent || h.queued; });
+    if (h.lent) return;
     size_t want = kSmallBytes;
     while (want < bytes && want < kSlotBytes * kSlots) want *= 2;
     want = std::min(want, kSlotBytes * kSlots);
@@ -751,12 +776,13 @@ static char *host_slots_get(size_t bytes)
     if (!h.slots) {
         if (!h.asked[1] && bytes <= kSlotBytes * kSlots) {
             h.asked[1] = true;
-            return nullptr;
+            return;
         }
         h.slots = host_pin(want);
         h.slots_bytes = want;
     }
-    return h.slots;
+    p = h.slots;
+    h.lent = h.queued = p != nullptr;
 }
 
 struct HostCopy {
@@ -802,26 +828,30 @@ static int copy_pageable(fcpt_ctx *ctx, const HostCopies &fields)
     return FCPT_OK;
 }
 
-static int copy_large(fcpt_ctx *ctx, const HostCopies &fields, char *slots)
+static int copy_large(fcpt_ctx *ctx, const HostCopies &fields, SlotsLoan &loan)
 {
     const KParams &P = ctx->P;
+    char *const slots = loan.p;
     const size_t ns = (size_t)P.ns;
     std::vector<CopyPiece> pieces;
     std::vector<std::vector<double>> bg(fields.size());
+    hipError_t err = hipSuccess;
     for (size_t k = 0; k < fields.size(); ++k) {
         const int f = fields[k].field;
         const size_t total = field_rows(f, P.nr) * ns, most = kSlotBytes / field_element_size(P, f);
         for (size_t a = 0; a < total; a += most) pieces.push_back({(int)k, a, std::min(most, total - a)});
         if (P.split && f != FCPT_POTENTIAL) {
             bg[k].resize(field_rows(f, P.nr));
-            HIP_TRY(ctx, hipMemcpyAsync(bg[k].data(), P.bg[f], bg[k].size() * sizeof(double), hipMemcpyDeviceToHost,
-                                        ctx->stream));
+            const hipError_t e = hipMemcpyAsync(bg[k].data(), P.bg[f], bg[k].size() * sizeof(double),
+                                                hipMemcpyDeviceToHost, ctx->stream);
+            if (err == hipSuccess) err = e;
         }
     }
     hipEvent_t ev[kSlots] = {};
-    hipError_t err = hipSuccess;
     for (int k = 0; k < kSlots && err == hipSuccess; ++k) err = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
-    if (err == hipSuccess) err = hipStreamSynchronize(ctx->stream);  // the backgrounds
+    const hipError_t queue = hipStreamSynchronize(ctx->stream);  // the disk's own, and the backgrounds
+    if (err == hipSuccess) err = queue;
+    loan.moving();
     std::mutex m;
     std::condition_variable cv;
     size_t issued = 0, next = 0;
@@ -910,7 +940,7 @@ static int copy_large(fcpt_ctx *ctx, const HostCopies &fields, char *slots)
 
 // all fields by one kernel into the slots, then to the caller: by this thread
 // below 1 MB, by several above
-static int copy_export(fcpt_ctx *ctx, const HostCopies &fields, size_t total, char *out)
+static int copy_export(fcpt_ctx *ctx, const HostCopies &fields, size_t total, char *out, SlotsLoan *loan)
 {
     const KParams &P = ctx->P;
     ExportFields x{};
@@ -948,6 +978,7 @@ static int copy_export(fcpt_ctx *ctx, const HostCopies &fields, size_t total, ch
     } catch (...) {  // this thread takes the strips that have no other
     }
     const hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (loan) loan->moving();
     {
         std::lock_guard<std::mutex> l(m);
         go = e == hipSuccess ? 1 : -1;
@@ -974,12 +1005,11 @@ static int copy_to_host(fcpt_ctx *ctx, const HostCopies &fields)
         if (fields.n == 1 && stored && total > kDirectAbove && total <= kSmallBytes) return copy_pageable(ctx, fields);
         if (total <= kSmallBytes) {
             SmallBuffer b;
-            if (b.p) return copy_export(ctx, fields, total, b.p);
+            if (b.p) return copy_export(ctx, fields, total, b.p, nullptr);
         } else {
-            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-            std::lock_guard<std::mutex> lease(host_slots().lease);
-            if (char *out = host_slots_get(total))
-                return total > kSlotBytes * kSlots ? copy_large(ctx, fields, out) : copy_export(ctx, fields, total, out);
+            SlotsLoan loan(total);
+            if (loan.p && total > kSlotBytes * kSlots) return copy_large(ctx, fields, loan);
+            if (loan.p) return copy_export(ctx, fields, total, loan.p, &loan);
         }
         return copy_pageable(ctx, fields);
     } catch (const std::exception &e) {
