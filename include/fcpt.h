@@ -395,7 +395,8 @@ int fcpt_batch_set_radial_waves(fcpt_batch *batch, int32_t waves);
    graph.  Results do not depend on the choice. */
 int fcpt_batch_autotune(fcpt_batch *batch, int32_t reps, int32_t *radial_tile, int32_t *radial_waves);
 /* n_steps sim::run iterations of every disk; use_graph != 0 replays captured
-   HIP graphs as fcpt_run_steps does.  No host synchronisation. */
+   HIP graphs as fcpt_run_steps does.  The call waits for what is queued on the
+   disks' own streams, not for the steps it queues. */
 int fcpt_batch_run_steps(fcpt_batch *batch, int32_t n_steps, int32_t use_graph);
 /* as fcpt_batch_run_steps, timed with HIP events on the batch's stream */
 int fcpt_batch_time_steps(fcpt_batch *batch, int32_t n_steps, int32_t use_graph, double *ms_total);
